@@ -14,6 +14,7 @@
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -117,14 +118,10 @@ struct hpgx_state_s {
   std::vector<hipStream_t> copy_streams;
   std::vector<hipEvent_t> copied, released;  // per task
   std::vector<bool> released_set;
-  // gridding pipeline: 5 = as 4, but FP32 grids with (hi, lo) pair tiles
-  // are added by one wave per tile quadrant with one lane per CF tap and no
-  // LDS atomics (default; 4 where the quadrant regions do not fit LDS), 4 = block-local
-  // bins of one entry per record and plane, haloed LDS tiles updated by LDS
-  // atomics (falls back to 3 when a CF support reaches the tile edge; grids
-  // with more (plane, tile) keys than one workgroup's LDS histogram holds
-  // take global bins), 3 = block-local bins of one entry per touched tile,
-  // 2 = compact entries binned through global counters
+  // gridding pipeline: 5 = by size (use_patch): haloed tiles for one
+  // polarization and small supports, register patches for all other calls
+  // (default); 4 = as 5, but FP32 grids' haloed tiles updated by LDS atomics
+  // instead of one wave per tile quadrant; 2, 3 = register patches always
   int gridder = 5;
   size_t nkeys = 0;
   size_t pass_blocks = 0;  // bin blocks per pass of the block-local pipelines
@@ -132,9 +129,8 @@ struct hpgx_state_s {
   // hi/lo pairs updated by two-sum (default; under compare-and-swap in
   // gridder 4), 0 = FP64 tile sums
   int fp32_tile = 2;
-  // FP32-compensated grids with supports up to 8 x 8 on the block-local
-  // haloed bins: quadrant-keyed bins and k_sub instead of k_quad
-  // (HPGX_SUB_TILES=0 keeps k_quad)
+  // FP32-compensated grids of one polarization with supports up to 8 x 8:
+  // quadrant-keyed bins and k_sub (HPGX_SUB_TILES=0: register patches)
   bool sub_tiles = true;
   // the finishing chain, deferred until an entry point touches the grid
   // (flush_finishing): normalize_by_weights, an in-place grid FFT and, for
@@ -284,46 +280,48 @@ bool halo_ok(hpgx_state_t st) {
 // haloed tiles fed by block-local bins (grids of up to bin_keys_limit keys)
 bool use_halo(hpgx_state_t st) { return halo_ok(st) && use_block_local(st); }
 
+// binned degridding (k_degrid4): one polarization on those grids; other
+// calls degrid in CF-slice order
+bool use_degrid_binned(hpgx_state_t st) { return st->npol == 1 && use_halo(st); }
+
 // haloed tiles fed by global bins (larger grids: counters are then
 // rarely contended)
 bool use_halo_global(hpgx_state_t st) {
   return halo_ok(st) && st->nkeys > size_t(hpgx::bin_keys_limit());
 }
 
-// the quadrant kernel (gridder 5) for FP32 grids with (hi, lo) pair tiles:
-// its regions and tables fit LDS and CF tap indexes fit 32 bits.  FP64 tile
-// sums stay with k_tile4, whose non-returning FP64 LDS atomics need no
-// read-modify-write per tap.
-bool use_quad(hpgx_state_t st) {
-  return st->gridder == 5 && (use_halo(st) || use_halo_global(st))
+// k_sub's calls: FP32-compensated grids of one polarization with supports up
+// to 8 x 8, CF taps within its 32-bit byte offsets
+bool sub_ok(hpgx_state_t st) {
+  return st->sub_tiles && st->gridder == 5 && st->npol == 1 && halo_ok(st)
     && st->mode != HPGX_GRID_FP64 && st->fp32_tile == 2
-    && hpgx::quad_supported(halo_x(st), halo_y(st), int(st->npol))
-    && st->taps_capacity < (size_t(1) << 32);
-}
-
-// the quadrant-key kernel (k_sub): FP32-compensated grids on block-local
-// haloed bins with supports up to 8 x 8, and 4 bin keys per (plane, tile)
-// within one workgroup's LDS histogram
-bool use_sub(hpgx_state_t st) {
-  return st->sub_tiles && use_quad(st) && use_halo(st)
-    && hpgx::sub_supported(halo_x(st), halo_y(st))
-    && st->taps_capacity * sizeof(float2) <= size_t(0xffffffffu)
-    && 4 * st->nkeys <= size_t(hpgx::bin_quad_keys_limit());
-}
-
-// k_sub on global bins (quadrant keys counted and emitted through global
-// counters): grids of more keys than the block-local histogram holds, one
-// polarization
-bool use_sub_global(hpgx_state_t st) {
-  return st->sub_tiles && use_quad(st) && use_halo_global(st) && st->npol == 1
     && hpgx::sub_supported(halo_x(st), halo_y(st))
     && st->taps_capacity * sizeof(float2) <= size_t(0xffffffffu);
 }
 
-// every CF group has the same support
+// register patches (k_patch)
+bool use_patch(hpgx_state_t st) {
+  if (st->gridder < 4 || st->npol > 1 || !halo_ok(st)) return true;
+  return st->gridder == 5 && st->mode != HPGX_GRID_FP64 && st->fp32_tile == 2 && !sub_ok(st);
+}
+
+// k_sub on block-local haloed bins: 4 bin keys per (plane, tile) within one
+// workgroup's LDS histogram
+bool use_sub(hpgx_state_t st) {
+  return sub_ok(st) && use_halo(st)
+    && 4 * st->nkeys <= size_t(hpgx::bin_quad_keys_limit());
+}
+
+// k_sub on global bins (quadrant keys counted and emitted through global
+// counters): grids of more keys than the block-local histogram holds
+bool use_sub_global(hpgx_state_t st) { return sub_ok(st) && use_halo_global(st); }
+
+// every CF group has the same support and number of Mueller elements
 bool uniform_support(hpgx_state_t st) {
   for (const GroupInfo& g : st->groups)
-    if (g.sx != st->groups[0].sx || g.sy != st->groups[0].sy) return false;
+    if (g.sx != st->groups[0].sx || g.sy != st->groups[0].sy
+        || g.nmueller != st->groups[0].nmueller)
+      return false;
   return !st->groups.empty();
 }
 
@@ -336,9 +334,14 @@ size_t bin_keys(hpgx_state_t st) { return use_sub(st) ? 4 * st->nkeys : st->nkey
 size_t halo_bins_limit(hpgx_state_t st) {
   size_t nb = size_t(hpgx::tile_bins_limit());
   while (nb > 1 && hpgx::halo_lds_bytes(halo_x(st), halo_y(st), int(nb)) > 65536) nb /= 2;
-  if (use_quad(st)) nb = std::min(nb, size_t(hpgx::quad_bins_limit()));
   if (use_sub(st)) nb = std::min(nb, size_t(hpgx::sub_bins_limit()));
   return nb;
+}
+
+// tiles of the register patches that one record's support touches at most
+size_t patch_tiles(hpgx_state_t st) {
+  return hpgx::patch_tiles_per_footprint(
+    int(st->gsize[2]), std::max(1, st->cf.max_sx), std::max(1, st->cf.max_sy));
 }
 
 size_t entries_per_record(hpgx_state_t st) {
@@ -383,26 +386,46 @@ int ensure_call_buffers(hpgx_state_t st) {
     HPGX_HIP(st, dev_alloc(cb.scan_temp, cb.scan_temp_bytes));
   }
   if (st->cf.ngroups > 0) {
+    if (use_patch(st)) {
+      // prepared records and tile lists for the whole batch, up to the entry
+      // memory budget and 2^32 list indexes; larger batches are gridded in
+      // chunks (run_grid)
+      const size_t tiles = patch_tiles(st);
+      const size_t rec = hpgx::patch_rec_bytes(int(st->npol));
+      const size_t recs = std::min(
+        {st->vis_capacity, std::max<size_t>(1, entry_budget_bytes() / (rec + tiles * sizeof(unsigned))),
+         size_t(0xffffffffull) / tiles});
+      if (recs > cb.patch_capacity) {
+        dev_free(cb.patch_recs);
+        cb.patch_capacity = 0;
+        HPGX_HIP(st, dev_alloc(cb.patch_recs, recs * rec));
+        cb.patch_capacity = recs;
+      }
+      if (recs * tiles > cb.patch_list_capacity) {
+        dev_free(cb.patch_list);
+        cb.patch_list_capacity = 0;
+        HPGX_HIP(st, dev_alloc(cb.patch_list, recs * tiles * sizeof(unsigned)));
+        cb.patch_list_capacity = recs * tiles;
+      }
+    }
     // bin entries for the whole batch, up to the entry memory budget; larger
     // batches are gridded in chunks (run_grid)
     const size_t epr = entries_per_record(st);
-    const bool halo = use_halo(st) || use_halo_global(st);
-    const size_t per_entry =
-      (halo ? hpgx::halo_entry_bytes(int(st->npol)) : hpgx::entry_bytes(int(st->npol)))
-      + sizeof(unsigned);
+    // (register patches: the bins of the binned degridder only)
+    const bool halo = use_patch(st) ? use_degrid_binned(st) : use_halo(st) || use_halo_global(st);
+    const size_t per_entry = hpgx::halo_entry_bytes(int(st->npol)) + sizeof(unsigned);
     // entries per pass: at least one record's, and below 2^32 (bin counts,
     // offsets and entry indexes are 32-bit)
     const size_t budget = std::min<size_t>(std::max(entry_budget_bytes() / per_entry, epr),
                                            0xffffffffull);
-    size_t need = std::min(st->vis_capacity * epr, budget);
-    if (use_block_local(st)) {
+    size_t need = halo ? std::min(st->vis_capacity * epr, budget) : 0;
+    if (halo && use_halo(st)) {
       // whole bin blocks of bin_block_records records each
       const size_t block_cap = hpgx::bin_block_records() * epr;
       const size_t blocks_needed =
         (st->vis_capacity + hpgx::bin_block_records() - 1) / hpgx::bin_block_records();
-      const size_t bins_max = halo ? halo_bins_limit(st) : size_t(hpgx::tile_bins_limit());
       const size_t blocks =
-        std::max<size_t>(1, std::min({blocks_needed, budget / block_cap, bins_max}));
+        std::max<size_t>(1, std::min({blocks_needed, budget / block_cap, halo_bins_limit(st)}));
       need = blocks * block_cap;
       st->pass_blocks = blocks;
       const size_t tab = blocks * (bin_keys(st) + 1);
@@ -413,7 +436,7 @@ int ensure_call_buffers(hpgx_state_t st) {
         cb.off_table_capacity = tab;
       }
     }
-    if (halo) {
+    if (halo && !use_patch(st)) {
       const size_t hp = st->nkeys * hpgx::halo_pixels_per_key(halo_x(st), halo_y(st));
       if (hp > cb.halo_capacity) {
         dev_free(cb.halo);
@@ -436,13 +459,15 @@ int ensure_call_buffers(hpgx_state_t st) {
       HPGX_HIP(st, dev_alloc(cb.tally_keys, need * 2 * sizeof(unsigned)));
       cb.tally_capacity = need;
     }
-    // the wave-per-record degridder's record order, once a model is set
-    if (st->model && hpgx::degrid_sorts(st->cf) && st->vis_capacity > cb.order_capacity) {
+    // the slice-ordered degridder's record order, once a model is set
+    if (st->model && !use_degrid_binned(st) && st->vis_capacity > cb.order_capacity) {
       dev_free(cb.degrid_order);
+      dev_free(cb.degrid_recs);
       dev_free(cb.order_temp);
       cb.order_capacity = 0;
       cb.order_temp_bytes = hpgx::degrid_order_temp_bytes(st->vis_capacity);
       HPGX_HIP(st, dev_alloc(cb.degrid_order, 4 * st->vis_capacity * sizeof(unsigned)));
+      HPGX_HIP(st, dev_alloc(cb.degrid_recs, st->vis_capacity * hpgx::degrid_rec_bytes()));
       HPGX_HIP(st, dev_alloc(cb.order_temp, cb.order_temp_bytes));
       cb.order_capacity = st->vis_capacity;
     }
@@ -450,9 +475,7 @@ int ensure_call_buffers(hpgx_state_t st) {
       dev_free(cb.stream_entries);
       dev_free(cb.entry_vis);
       cb.entries_capacity = 0;
-      HPGX_HIP(st, dev_alloc(cb.stream_entries,
-                             need * std::max(hpgx::entry_bytes(int(st->npol)),
-                                             hpgx::halo_entry_bytes(int(st->npol)))));
+      HPGX_HIP(st, dev_alloc(cb.stream_entries, need * hpgx::halo_entry_bytes(int(st->npol))));
       HPGX_HIP(st, dev_alloc(cb.entry_vis, need * sizeof(unsigned)));
       cb.entries_capacity = need;
     }
@@ -491,6 +514,8 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.gvis);
   dev_free(cb.tally_entries);
   dev_free(cb.tally_keys);
+  dev_free(cb.patch_recs);
+  dev_free(cb.patch_list);
   dev_free(cb.hist);
   dev_free(cb.offsets);
   dev_free(cb.cursor);
@@ -502,6 +527,7 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.degrid_acc);
   dev_free(cb.scan_temp);
   dev_free(cb.degrid_order);
+  dev_free(cb.degrid_recs);
   dev_free(cb.order_temp);
   dev_free(cb.invalid_count);
   if (st->plan_z2z.valid) hipfftDestroy(st->plan_z2z.h);
@@ -712,6 +738,19 @@ int upload_model(hpgx_state_t st, const void* values, int layout, int memory) {
   return HPGX_SUCCESS;
 }
 
+// per-record sums of the degridders
+int ensure_degrid_acc(hpgx_state_t st) {
+  CallBuffers& cb = st->cb;
+  const size_t need = std::max<size_t>(st->max_batch, 1) * st->npol;
+  if (need > cb.degrid_acc_capacity) {
+    dev_free(cb.degrid_acc);
+    cb.degrid_acc_capacity = 0;
+    HPGX_HIP(st, dev_alloc(cb.degrid_acc, need * sizeof(double2)));
+    cb.degrid_acc_capacity = need;
+  }
+  return HPGX_SUCCESS;
+}
+
 // gridding / degridding pipeline on records already in cb.vis
 // gridding / degridding pipeline on records already in cb.vis; the records
 // are gridded in chunks whose bin entries fit the entry buffer
@@ -725,13 +764,7 @@ int run_degrid_binned(hpgx_state_t st, size_t n, bool do_grid, const void* recor
   const Geometry geo = st->geometry();
   CallBuffers& cb = st->cb;
   const int np = int(st->npol);
-  const size_t acc_need = std::max<size_t>(st->max_batch, 1) * np;
-  if (acc_need > cb.degrid_acc_capacity) {
-    dev_free(cb.degrid_acc);
-    cb.degrid_acc_capacity = 0;
-    HPGX_HIP(st, dev_alloc(cb.degrid_acc, acc_need * sizeof(double2)));
-    cb.degrid_acc_capacity = acc_need;
-  }
+  if (int rc = ensure_degrid_acc(st)) return rc;
   // one grid row whose Mueller rows (both w signs) index some CF element:
   // every record inside the grid has exactly one entry, and the tile kernel
   // finishes its prediction
@@ -790,19 +823,41 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
   const int np = int(st->npol);
   bool gvis_ready = false;
   if (do_degrid) {
-    if (st->model && use_halo(st)) {
+    if (st->model && use_degrid_binned(st)) {
       if (int rc = run_degrid_binned(st, n, do_grid, records, nullptr, out_records)) return rc;
     } else {
+      // records returned into another buffer: copied there whole, then their
+      // values replaced
+      if (records && out_records && out_records != records)
+        HPGX_HIP(st, hipMemcpyAsync(out_records, records, n * visdata_size(st->npol),
+                                    hipMemcpyDeviceToDevice, st->stream));
+      if (st->model)
+        if (int rc = ensure_degrid_acc(st)) return rc;
       HPGX_HIP(st, hpgx::launch_degrid(
-                     st->stream, np, n, geo, st->cf, st->mu, st->model, do_grid, cb));
+                     st->stream, np, n, geo, st->cf, st->mu, st->model, do_grid, cb, nullptr,
+                     rec_base, records ? out_records : rec_base));
     }
     gvis_ready = true;
   }
   if (!do_grid) return HPGX_SUCCESS;
   const int mode = st->mode == HPGX_GRID_FP64 ? 0 : 1;
+  if (use_patch(st)) {
+    const size_t chunk = std::min(cb.patch_capacity, cb.patch_list_capacity / patch_tiles(st));
+    if (chunk == 0) return fail(st, HPGX_ERR_OTHER, "patch lists not allocated");
+    const size_t rec_bytes = visdata_size(st->npol);
+    for (size_t off = 0; off < n; off += chunk) {
+      CallBuffers c = cb;
+      c.vis = static_cast<char*>(rec_base) + off * rec_bytes;
+      c.gvis = cb.gvis ? cb.gvis + off * np : nullptr;
+      HPGX_HIP(st, hpgx::launch_patch(
+                     st->stream, np, std::min(chunk, n - off), geo, st->cf, st->mu,
+                     update_weights, gvis_ready, src, residuals ? residuals + off * np : nullptr,
+                     c, st->weights, mode, st->grid));
+    }
+    return HPGX_SUCCESS;
+  }
   const size_t epr = entries_per_record(st);
   if (use_block_local(st)) {
-    const bool halo = use_halo(st);
     const size_t block_cap = hpgx::bin_block_records() * epr;
     // bin blocks per pass as sized by ensure_call_buffers (entries, offset
     // table and the tile kernel's LDS segment tables)
@@ -817,20 +872,16 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
       const bool sub = use_sub(st);
       HPGX_HIP(st, hpgx::launch_bin(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, gvis_ready, src,
-                     res, c, block_cap, st->weights, halo, false, nullptr, sub));
+                     res, c, block_cap, st->weights, true, false, nullptr, sub));
       if (sub)
         HPGX_HIP(st, hpgx::launch_tile_sub(
                        st->stream, np, m, st->nkeys, geo, st->cf,
                        st->taps_capacity * sizeof(float2), uniform_support(st), st->mu, c,
                        block_cap, halo_x(st), halo_y(st), st->grid));
-      else if (halo)
+      else
         HPGX_HIP(st, hpgx::launch_tile_halo(
                        st->stream, np, mode, st->fp32_tile, m, st->nkeys, geo, st->cf, st->mu, c,
-                       block_cap, halo_x(st), halo_y(st), st->grid, false, use_quad(st)));
-      else
-        HPGX_HIP(st, hpgx::launch_tile_blocal(
-                       st->stream, np, mode, m, st->nkeys, geo, st->cf, st->mu, c,
-                       block_cap, st->grid));
+                       block_cap, halo_x(st), halo_y(st), st->grid));
     }
     return HPGX_SUCCESS;
   }
@@ -847,7 +898,6 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
     c.vis = static_cast<char*>(rec_base) + off * rec_bytes;
     c.gvis = cb.gvis + off * np;
     const double2* res = residuals ? residuals + off * np : nullptr;
-    const bool halo = use_halo_global(st);
     const bool sub = use_sub_global(st);
     const size_t keys = sub ? 4 * st->nkeys : st->nkeys;
     HPGX_HIP(st, hipMemsetAsync(c.hist, 0, (keys + 1) * sizeof(unsigned), st->stream));
@@ -860,23 +910,20 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
     } else {
       HPGX_HIP(st, hpgx::launch_count(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, true, c,
-                     st->weights, halo));
+                     st->weights, true));
       HPGX_HIP(st, hpgx::launch_scan(st->stream, keys, c));
       HPGX_HIP(st, hpgx::launch_emit(
-                     st->stream, np, m, geo, st->cf, st->mu, gvis_ready, src, res, c, halo));
+                     st->stream, np, m, geo, st->cf, st->mu, gvis_ready, src, res, c, true));
     }
     if (sub)
       HPGX_HIP(st, hpgx::launch_tile_sub(
                      st->stream, np, m, st->nkeys, geo, st->cf,
                      st->taps_capacity * sizeof(float2), uniform_support(st), st->mu, c, 0,
                      halo_x(st), halo_y(st), st->grid, true));
-    else if (halo)
+    else
       HPGX_HIP(st, hpgx::launch_tile_halo(
                      st->stream, np, mode, st->fp32_tile, m, st->nkeys, geo, st->cf, st->mu,
-                     c, 0, halo_x(st), halo_y(st), st->grid, true, use_quad(st)));
-    else
-      HPGX_HIP(st, hpgx::launch_tile_stream(
-                     st->stream, np, mode, st->nkeys, geo, st->cf, st->mu, c, st->grid));
+                     c, 0, halo_x(st), halo_y(st), st->grid, true));
   }
   return HPGX_SUCCESS;
 }
@@ -925,6 +972,34 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
                   + std::to_string(noalloc_scratch_bytes));
   char* p = static_cast<char*>(base);
   c = CallBuffers{};
+  // skipped records are counted in the state's own counter (read by
+  // hpgx_fence), as by hpgx_grid_visibilities
+  c.invalid_count = st->cb.invalid_count;
+  if (use_patch(st)) {
+    const size_t keys = hpgx::patch_keys(st->geometry());
+    const size_t tiles = patch_tiles(st);
+    const size_t rec = hpgx::patch_rec_bytes(int(st->npol));
+    c.hist = reinterpret_cast<unsigned*>(p);
+    p += up((keys + 1) * sizeof(unsigned));
+    c.offsets = reinterpret_cast<unsigned*>(p);
+    p += up((keys + 1) * sizeof(unsigned));
+    c.scan_temp = p;
+    c.scan_temp_bytes = st->cb.scan_temp_bytes;
+    p += up(c.scan_temp_bytes);
+    const size_t used = size_t(p - static_cast<char*>(base)) + 256;
+    const size_t recs = noalloc_scratch_bytes > used
+      ? std::min(n, (noalloc_scratch_bytes - used) / (rec + tiles * sizeof(unsigned)))
+      : 0;
+    if (recs == 0)
+      return fail(st, HPGX_ERR_OTHER, "hpgx_grid_visibilities_noalloc: scratch layout overflow");
+    c.patch_recs = p;
+    c.patch_capacity = recs;
+    p += up(recs * rec);
+    c.patch_list = reinterpret_cast<unsigned*>(p);
+    c.patch_list_capacity = recs * tiles;
+    pass_blocks = 0;
+    return HPGX_SUCCESS;
+  }
   c.off_table = reinterpret_cast<unsigned*>(p);
   c.off_table_capacity = blocks * (bin_keys(st) + 1);
   p += up(c.off_table_capacity * sizeof(unsigned));
@@ -943,9 +1018,6 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
   }
   if (size_t(p - static_cast<char*>(base)) > noalloc_scratch_bytes)
     return fail(st, HPGX_ERR_OTHER, "hpgx_grid_visibilities_noalloc: scratch layout overflow");
-  // skipped records are counted in the state's own counter (read by
-  // hpgx_fence), as by hpgx_grid_visibilities
-  c.invalid_count = st->cb.invalid_count;
   pass_blocks = blocks;
   return HPGX_SUCCESS;
 }
@@ -1314,6 +1386,8 @@ int hpgx_set_convolution_function(
   std::vector<GroupInfo> groups(num_groups);
   long long toff = 0, woff = 0;
   int max_sx = 1, max_sy = 1, max_ncube = 1;
+  int min_nm = num_groups ? INT_MAX : 0, max_nm = 0;
+  bool even_nm = true;
   size_t max_stage = 0;
   for (unsigned g = 0; g < num_groups; ++g) {
     const unsigned* e = extents + 4 * g;
@@ -1331,6 +1405,9 @@ int hpgx_set_convolution_function(
     max_sx = std::max(max_sx, gi.sx);
     max_sy = std::max(max_sy, gi.sy);
     max_ncube = std::max(max_ncube, gi.ncube);
+    min_nm = std::min(min_nm, gi.nmueller);
+    max_nm = std::max(max_nm, gi.nmueller);
+    even_nm = even_nm && gi.nmueller % 2 == 0;
     max_stage = std::max(max_stage, size_t(e[0]) * e[1] * e[2] * e[3]);
   }
   if (int rc = ensure_cf_capacity(st, size_t(toff), size_t(woff))) return rc;
@@ -1365,6 +1442,9 @@ int hpgx_set_convolution_function(
   st->cf.max_sx = max_sx;
   st->cf.max_sy = max_sy;
   st->cf.max_ncube = max_ncube;
+  st->cf.min_nm = min_nm;
+  st->cf.max_nm = max_nm;
+  st->cf.even_nm = even_nm;
   return ensure_call_buffers(st);
 }
 
@@ -1428,21 +1508,14 @@ int hpgx_grid_visibilities(
     return HPGX_SUCCESS;
   }
   if (int rc = ensure_call_buffers(st)) return rc;
-  // Device records are read in place unless degridding rewrites them.  The
-  // binned degridder reads them in place too and writes the returned
-  // records straight into visibilities_out (its binning pass copies each
-  // record there whole, then the predicted or residual values replace the
-  // record's values), or nowhere when they are not returned; other
-  // degridders use the staged copy.
+  // Device records are read in place; degridding writes the returned records
+  // straight into visibilities_out, or nowhere when they are not returned.
   const bool dev = memory == HPGX_DEVICE;
-  const bool binned_degrid = do_degrid && st->model && use_halo(st);
   const void* records = nullptr;  // nullptr: the staged copy
   void* out_records = nullptr;
-  if (dev && !do_degrid) {
+  if (dev) {
     records = vis;
-  } else if (dev && binned_degrid) {
-    records = vis;
-    if (return_visibilities) out_records = vis_out;
+    if (do_degrid && return_visibilities) out_records = vis_out;
   } else if (!dev && st->tasks > 1) {
     // uploaded on the next task's copy stream: overlaps the kernels of the
     // calls before
@@ -1549,17 +1622,17 @@ int hpgx_degrid_forward(
   HPGX_HIP(st, hipMemsetAsync(out, 0, bytes, st->stream));
   if (st->cf.ngroups > 0) {
     if (int rc = ensure_call_buffers(st)) return rc;
-    // device records are read in place by the lane-per-record degridder
-    const bool in_place = memory == HPGX_DEVICE
-      && size_t(st->cf.max_sx) * size_t(st->cf.max_sy) <= hpgx::degrid_lane_max_taps();
+    const bool in_place = memory == HPGX_DEVICE;
     if (!in_place)
       if (int rc = stage_records(st, vis, n, memory)) return rc;
-    if (st->model && use_halo(st)) {
+    if (st->model && use_degrid_binned(st)) {
       if (int rc = run_degrid_binned(st, n, false, in_place ? vis : nullptr, out)) return rc;
     } else {
+      if (st->model)
+        if (int rc = ensure_degrid_acc(st)) return rc;
       HPGX_HIP(st, hpgx::launch_degrid(st->stream, int(npol), n, st->geometry(), st->cf,
                                        st->mu, st->model, false, st->cb, out,
-                                       in_place ? vis : nullptr));
+                                       in_place ? vis : st->cb.vis, nullptr));
     }
   }
   if (tmp) {

@@ -20,16 +20,18 @@ constexpr int tile = 32;
 constexpr int tile_waves = 4;
 
 // Per-group geometry of the device CF.  The device layout of group g is
-// "fine-offset sliced": for every (cube, mueller, fx, fy) -- fx, fy in
-// [-F, F] the visibility's fine offset on each axis, F = (os + 1) / 2 -- the
-// sx x sy taps of the support are contiguous, x fastest:
-//   taps[tap_offset + (((cube * nmueller + m) * nf + fx + F) * nf + fy + F)
-//        * sx * sy + Y * sx + X]
+// "fine-offset sliced": for every (cube, fx, fy) -- fx, fy in [-F, F] the
+// visibility's fine offset on each axis, F = (os + 1) / 2 -- the sx x sy
+// taps of the support are contiguous, x fastest, each with its Mueller
+// elements side by side (a record reads all of them, so whole lines of its
+// slice, wherever a tile border cuts the support):
+//   taps[tap_offset + ((((cube * nf + fx + F) * nf + fy + F) * sx * sy
+//        + Y * sx + X) * nmueller + m]
 //   = CFArray(ix, iy, m, cube, g), ix = (X + padding) * os + fx, iy likewise,
 // which is the element the reference reaches through its 6-D layout
 // (src/hpg_impl.hpp:221-281, src/hpg_core.hpp:422-446: major * os + minor).
 // wsum[wsum_offset + ((cube * nmueller + m) * nf + fx + F) * nf + fy + F]
-// is the FP64 sum of that slice's taps, X outer and Y inner.
+// is the FP64 sum of that element's taps of the slice.
 struct GroupInfo {
   long long tap_offset;
   long long wsum_offset;
@@ -84,8 +86,13 @@ struct CallBuffers {
   void* tally_entries;   // launch_tally: entries in record order (Entry4<N>)
   void* tally_keys;      // launch_tally: (key, place within the key) per slot
   size_t tally_capacity; // slots of both
-  unsigned* degrid_order; // launch_degrid (wave form): keys, sorted keys, record
-                          // indexes, sorted indexes, order_capacity each
+  void* patch_recs;       // launch_patch: prepared records (PatchRec<N>)
+  size_t patch_capacity;
+  unsigned* patch_list;   // and the tiles' lists of record indexes
+  size_t patch_list_capacity;
+  unsigned* degrid_order; // launch_degrid: keys, sorted keys, record indexes,
+                          // sorted indexes, order_capacity each
+  void* degrid_recs;      // and its prepared records (DegridRec)
   size_t order_capacity;
   void* order_temp;       // the sort's temporary storage
   size_t order_temp_bytes;
@@ -98,6 +105,8 @@ struct DeviceCF {
   int os, F, nf, ngroups;
   int max_sx, max_sy;
   int max_ncube;  // CF cubes of the group with the most
+  int min_nm, max_nm;  // Mueller elements of the groups with the fewest and the most
+  bool even_nm;   // every group has an even number of them
 };
 
 // ---- launchers (hpgx_kernels.hip) -------------------------------------
@@ -138,9 +147,6 @@ hipError_t launch_tally(
   const double2* residuals, CallBuffers& cb, double* weights);
 hipError_t launch_place(hipStream_t s, int npol, size_t n, const Geometry& geo,
                         CallBuffers& cb);
-hipError_t launch_tile_stream(
-  hipStream_t s, int npol, int mode, size_t nkeys, const Geometry& geo,
-  const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, void* grid);
 // block-local binning (small key counts)
 int bin_blocks_for(size_t n);
 size_t bin_block_records();
@@ -158,18 +164,12 @@ size_t halo_entry_bytes(int npol);
 size_t halo_pixels_per_key(int hx, int hy);
 int halo_tile_limit();
 size_t halo_lds_bytes(int hx, int hy, int nbins);
-// the quadrant kernel (k_quad): its LDS, bin blocks per pass, and whether it
-// takes halo widths hx, hy (its regions fit LDS, the tile + halo its flush)
-size_t quad_lds_bytes(int hx, int hy, int npol);
-int quad_bins_limit();
-bool quad_supported(int hx, int hy, int npol);
 // acc (FP32 grids): 0 FP64 tile sums, 1 FP32 two-sum via returning atomics,
-// 2 FP32 two-sum of (hi, lo) pairs (compare-and-swap in k_tile4, plain
-// read-modify-write in k_quad).  quad: k_quad (acc 0 or 2) instead of k_tile4
+// 2 FP32 two-sum of (hi, lo) pairs under compare-and-swap
 hipError_t launch_tile_halo(
   hipStream_t s, int npol, int mode, int acc, size_t n, size_t nkeys, const Geometry& geo,
   const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
-  int hx, int hy, void* grid, bool global_bins = false, bool quad = false);
+  int hx, int hy, void* grid, bool global_bins = false);
 // the quadrant-key kernel (k_sub): FP32-compensated grids, supports of at
 // most 8 x 8 (hx, hy <= 7), bins of launch_bin with quad_keys; ntile_keys
 // (plane, tile) keys, whose offset-table rows hold 4 ntile_keys + 1 values;
@@ -183,10 +183,17 @@ hipError_t launch_tile_sub(
   hipStream_t s, int npol, size_t n, size_t ntile_keys, const Geometry& geo, const DeviceCF& cf,
   size_t taps_bytes, bool uni, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
   int hx, int hy, void* grid, bool global_bins = false);
-hipError_t launch_tile_blocal(
-  hipStream_t s, int npol, int mode, size_t n, size_t nkeys, const Geometry& geo,
-  const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
-  void* grid);
+// register patches (k_patch): any number of polarizations and grid rows, any
+// support and grid.  cb.hist and cb.offsets hold patch_keys + 1 values,
+// cb.patch_recs patch_capacity records and cb.patch_list
+// patch_tiles_per_footprint indexes for each
+size_t patch_keys(const Geometry& geo);
+size_t patch_rec_bytes(int npol);
+size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy);
+hipError_t launch_patch(
+  hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
+  const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
+  const double2* residuals, CallBuffers& cb, double* weights, int mode, void* grid);
 // binned degridding from the model's LDS tiles (entries of launch_bin with
 // degrid_pass).  one_plane (every record has exactly one entry): the
 // predictions are finished in the same kernel -- FP64 values to pred64, or
@@ -205,20 +212,16 @@ hipError_t launch_degrid_finish(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, const double2* acc, bool do_grid, const void* records,
   void* out_records, CallBuffers& cb, double2* pred64);
-// degridding; with pred64 the FP64 predictions are written there and the
-// records are only read, from `records` when given (else cb.vis; `records`
-// requires supports of at most degrid_lane_max_taps() taps)
-size_t degrid_lane_max_taps();
-// the wave-per-record degridder runs (supports above degrid_lane_max_taps()
-// taps) and can take its records in CF-slice order: with cb.degrid_order
-// for at least n records it sorts them by (CF group, cube, fine offset)
-// first, so that records reading the same CF slices run together
-bool degrid_sorts(const DeviceCF& cf);
+// slice-ordered degridding of the records at `records`: FP64 predictions to
+// pred64, or predicted values (residuals, and gvis in cb, when do_grid)
+// written into out_records when not null, which may be `records`.  With a
+// model, cb.degrid_order, degrid_recs and degrid_acc hold at least n records.
+size_t degrid_rec_bytes();
 size_t degrid_order_temp_bytes(size_t n);
 hipError_t launch_degrid(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
-  const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb,
-  double2* pred64 = nullptr, const void* records = nullptr);
+  const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb, double2* pred64,
+  const void* records, void* out_records);
 
 hipError_t launch_normalize(
   hipStream_t s, int mode, void* grid, const double* weights, double wfactor,

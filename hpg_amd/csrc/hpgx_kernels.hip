@@ -7,23 +7,21 @@
 //
 // Gridding (VisibilityGridder::kernel, src/hpg_core.hpp:1082-1253) is
 // re-organized for the device in two stages: binning, then one workgroup per
-// (grid plane, 32 x 32 tile) key accumulating the tile in LDS and adding it
-// into the grid with one coalesced read-modify-write, so that no global
-// atomic touches the grid.
-//   k_bin + k_quad / k_tile4 + k_halo   records binned by the tile holding
-//        their support corner (block-local bins, no global atomics); the
-//        tile kernels accumulate the tile plus a halo of (support - 1)
-//        pixels, and k_halo folds each tile's halo into its neighbours.
-//        Supports narrower than a tile on grids of up to 8192 keys.
-//   k_bin<N,false> + k_tile3            one entry per touched tile, clipped
-//        footprints (supports reaching the tile edge, small grids).
-//   k_count + scan + k_emit + k_tile2   the same entries binned through
-//        global counters (grids with more keys than one workgroup's LDS
-//        histogram holds).
+// grid tile accumulating it on chip and adding it into the grid with one
+// coalesced read-modify-write, so that no global atomic touches the grid.
+//   k_bin + k_sub / k_tile4 + k_halo   one polarization, supports narrower
+//        than a tile: records binned by the 32 x 32 tile holding their support
+//        corner (block-local bins, no global atomics; grids of more than 8192
+//        keys bin through global counters: k_tally + k_place, k_count +
+//        k_emit); the tile kernels accumulate the tile plus a halo of
+//        (support - 1) pixels in LDS, and k_halo folds each tile's halo into
+//        its neighbours.
+//   k_patch_prep + k_patch_list + k_patch   several polarizations, larger
+//        supports: each tile's sums of all its grid rows in registers.
 // Degridding (degrid_vis, src/hpg_core.hpp:579-682): k_degrid4 reads the
-// model's tile and halo from LDS for binned records; k_degrid_lane (one lane
-// per record) and k_degrid (one wave per record, cross-lane reduction)
-// gather the model directly.
+// model's tile and halo from LDS for binned records (one polarization, small
+// supports); k_degrid takes the records in CF-slice order, several sharing
+// the CF values that a wave loads.
 
 #include "hpgx_internal.hpp"
 
@@ -56,6 +54,7 @@ static_assert(sizeof(VisRec<3>) == 112, "VisData<3>");
 static_assert(sizeof(VisRec<4>) == 120, "VisData<4>");
 
 typedef int v2i_t __attribute__((ext_vector_type(2)));
+typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -147,10 +146,6 @@ __device__ __forceinline__ Coord vis_coord(
 }
 
 __device__ __forceinline__ int tiles_begin(int corner) { return corner / tile; }
-__device__ __forceinline__ int tiles_end(int corner, int support) {
-  return (corner + support - 1) / tile + 1;
-}
-
 __device__ __forceinline__ bool row_has_index(const int* row, int npol) {
   bool any = false;
   for (int v = 0; v < npol; ++v) any |= row[v] >= 0;
@@ -181,6 +176,17 @@ __device__ __forceinline__ void degrid_norms(
   }
 }
 
+// index of the first tap of Mueller element m in the CF slice (cube, fx,
+// fy); the element's tap t follows at t * g.nmueller
+// (UNIT: its CF group has one element)
+template <bool UNIT = false>
+__device__ __forceinline__ long long slice_start(
+  const GroupInfo& g, int nf, int cube, int m, int fxi, int fyi) {
+  const long long slice = ((long long)cube * nf + fxi) * nf + fyi;
+  const long long ntap = (long long)g.sx * g.sy;
+  return UNIT ? g.tap_offset + slice * ntap : g.tap_offset + slice * (ntap * g.nmueller) + m;
+}
+
 // ---- CF ingestion ----------------------------------------------------
 
 __global__ void k_cf_relayout(
@@ -189,6 +195,8 @@ __global__ void k_cf_relayout(
   const long long o = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (o >= total) return;
   long long q = o;
+  const int m = int(q % gi.nmueller);
+  q /= gi.nmueller;
   const int X = int(q % gi.sx);
   q /= gi.sx;
   const int Y = int(q % gi.sy);
@@ -196,9 +204,7 @@ __global__ void k_cf_relayout(
   const int fyi = int(q % nf);
   q /= nf;
   const int fxi = int(q % nf);
-  q /= nf;
-  const int m = int(q % gi.nmueller);
-  const int c = int(q / gi.nmueller);
+  const int c = int(q / nf);
   const long long ix = (long long)(X + cf_padding) * os + (fxi - F);
   const long long iy = (long long)(Y + cf_padding) * os + (fyi - F);
   float2 v = make_float2(0.0f, 0.0f);
@@ -207,29 +213,93 @@ __global__ void k_cf_relayout(
   taps[gi.tap_offset + o] = v;
 }
 
-// the FP64 sum of each CF slice's taps (the weights' normalization), one
-// wave per slice: lane l sums taps l, l + 64, ... (coalesced reads), then a
-// fixed-order wave reduction.  FP64 sums of FP32 taps: exact while the
-// taps' exponents span fewer than about 29 bits, else within a few FP64
-// ulps of any other order
-constexpr int wsum_block = 256;
+// the same through LDS: one workgroup per cube, support row, fine y offset and
+// xc support columns reads the columns' values of every Mueller element (runs
+// of (xc - 1) os + nf values) and writes each fine x offset's taps (runs of
+// xc nmueller values).  k_cf_relayout reads one value of each line at a time:
+// 221 us a group of 64 with 16 elements and supports of 9 to 65 at oversampling
+// 20, on average, against 58 us here.
+constexpr int relayout_block = 256;
+constexpr size_t relayout_lds = 40960;
+__global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
+  const float2* __restrict__ staging, unsigned ex, unsigned ey, GroupInfo gi,
+  int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc) {
+  extern __shared__ float2 win[];
+  unsigned b = blockIdx.x;
+  const int X0 = int(b % unsigned(nxc)) * xc;
+  b /= unsigned(nxc);
+  const int Y = int(b % unsigned(gi.sy));
+  b /= unsigned(gi.sy);
+  const int fyi = int(b % unsigned(nf));
+  const int c = int(b / unsigned(nf));
+  const int nm = gi.nmueller;
+  const int cols = min(xc, gi.sx - X0);
+  const int width = (xc - 1) * os + nf;
+  const long long ix0 = (long long)(X0 + cf_padding) * os - F;
+  const long long iy = (long long)(Y + cf_padding) * os + (fyi - F);
+  for (int m = 0; m < nm; ++m)
+    for (int k = threadIdx.x; k < width; k += relayout_block) {
+      const long long ix = ix0 + k;
+      float2 v = make_float2(0.0f, 0.0f);
+      if (ix >= 0 && iy >= 0 && ix < ex && iy < ey)
+        v = staging[((long long)(c * nm + m) * ey + iy) * ex + ix];
+      win[m * width + k] = v;
+    }
+  __syncthreads();
+  const unsigned run = unsigned(cols) * unsigned(nm);
+  for (unsigned k = threadIdx.x; k < run * unsigned(nf); k += relayout_block) {
+    const int fxi = int(k / run);
+    const unsigned t = k - unsigned(fxi) * run;
+    const int X = int(t / unsigned(nm));
+    const int m = int(t - unsigned(X) * unsigned(nm));
+    taps[gi.tap_offset
+         + ((((long long)c * nf + fxi) * nf + fyi) * gi.sy + Y) * gi.sx * nm
+         + (long long)X0 * nm + t] = win[m * width + X * os + fxi];
+  }
+}
+
+// the FP64 sum of each Mueller element's taps of each CF slice (the weights'
+// normalization), one workgroup per slice (of 64 to 1024 threads by the
+// slice's size: large supports have few slices): thread t sums the values t,
+// t + threads, ... (coalesced reads), which with per = 2^k <= 64 elements all
+// belong to element t mod per, then a fixed-order reduction.  Other numbers of
+// elements (per = 0): one workgroup per slice and element.  FP64 sums of FP32
+// taps: exact while the taps' exponents span fewer than about 29 bits, else
+// within a few FP64 ulps of any other order
+constexpr int wsum_block = 1024;
 __global__ __launch_bounds__(wsum_block) void k_cf_wsum(
   GroupInfo gi, int nf, const float2* __restrict__ taps,
-  double2* __restrict__ wsum, long long nslices) {
-  const long long s = blockIdx.x * (long long)(wsum_block / wave) + threadIdx.x / wave;
-  const int lane = int(threadIdx.x % wave);
-  if (s >= nslices) return;  // the whole wave
-  const int ntap = gi.sx * gi.sy;
-  const float2* t = taps + gi.tap_offset + s * ntap;
+  double2* __restrict__ wsum, int per) {
+  __shared__ double2 part[wsum_block / wave][wave];
+  const int nm = gi.nmueller;
+  const long long ntap = (long long)gi.sx * gi.sy;
+  const long long slice = per ? blockIdx.x : blockIdx.x / nm;  // (cube * nf + fx) * nf + fy
+  const int step = per ? 1 : nm;
+  const float2* t = taps + gi.tap_offset + slice * ntap * nm + (per ? 0 : int(blockIdx.x % nm));
+  const int keep = per ? per : 1;  // elements of this workgroup
   double re = 0.0, im = 0.0;
-  for (int k = lane; k < ntap; k += wave) {
-    const float2 c = t[k];
+  for (long long k = threadIdx.x; k < ntap * keep; k += blockDim.x) {
+    const float2 c = t[k * step];
     re += double(c.x);
     im += double(c.y);
   }
-  re = wave_sum(re);
-  im = wave_sum(im);
-  if (lane == 0) wsum[gi.wsum_offset + s] = make_double2(re, im);
+  for (int d = wave / 2; d >= keep; d >>= 1) {
+    re += __shfl_xor(re, d, wave);
+    im += __shfl_xor(im, d, wave);
+  }
+  const int lane = int(threadIdx.x % wave);
+  if (lane < keep) part[threadIdx.x / wave][lane] = make_double2(re, im);
+  __syncthreads();
+  if (int(threadIdx.x) >= keep) return;
+  re = im = 0.0;
+  for (int w = 0; w < int(blockDim.x) / wave; ++w) {
+    re += part[w][threadIdx.x].x;
+    im += part[w][threadIdx.x].y;
+  }
+  const int m = per ? int(threadIdx.x) : int(blockIdx.x % nm);
+  const long long nslice = (long long)nf * nf;
+  const long long c = slice / nslice;
+  wsum[gi.wsum_offset + (c * nm + m) * nslice + (slice - c * nslice)] = make_double2(re, im);
 }
 
 // ---- gridding ----------------------------------------------------------
@@ -279,19 +349,16 @@ __device__ __forceinline__ void pair_add(
   }
 }
 
-// ---- gridding, binned-stream form ------------------------------------------
+// ---- gridding, global bins ---------------------------------------------------
 //
 // k_count   one thread per visibility: skip rule, weights, bin counts
-// k_emit    one thread per visibility: writes one compact Entry per touched
-//           (plane, tile) bin -- support corner, fine offsets, CF group and
-//           cube, pre-phased values -- so the tile kernel reads its bin as one
-//           contiguous stream instead of gathering per-visibility records
-// k_tile2   one workgroup per bin, one shared LDS tile: waves load 64 entries
-//           at a time (one per lane), broadcast each to the whole wave with
-//           readlane, and accumulate with LDS atomics (FP64 adds), or
-//           (FP32-compensated grids) with compare-and-swap updates of
-//           (hi, lo) pairs by two-sum
+// k_emit    one thread per visibility: writes one compact Entry4 per grid plane
+//           -- support corner, fine offsets, CF group and cube, pre-phased
+//           values -- into the bin of the tile holding the support corner, so
+//           the tile kernel reads its bin as one contiguous stream instead of
+//           gathering per-visibility records
 
+// an entry under construction in k_bin
 struct EntryHead {
   int gx, gy;
   unsigned fpk;  // fxi | fyi << 8 | flags << 16
@@ -316,7 +383,7 @@ struct Entry4 {
 };
 constexpr unsigned e4_pos_w = 1u << 28;
 constexpr unsigned e4_gradient = 1u << 29;
-// k_emit<N, true> writes this layout as 2 + 2N 32-bit words
+// k_emit writes this layout as 2 + 2N 32-bit words
 static_assert(sizeof(Entry4<1>) == 16 && sizeof(Entry4<4>) == 40, "Entry4 layout");
 
 // bin key of tile key k for a support corner (gx, gy): k itself, or with
@@ -328,9 +395,8 @@ __device__ __forceinline__ int bin_key(int k, int gx, int gy, int quad_keys) {
   return 4 * k + (qx | (qy << 1));
 }
 
-// HALO: one entry per plane, in the bin of the tile holding the support
-// corner (the haloed-tile pipeline; with quad_keys in the bin of the
-// corner's quadrant, bin_key); else one per touched tile
+// one entry per plane, in the bin of the tile holding the support corner (with
+// quad_keys of the corner's quadrant, bin_key)
 // Weights: each wave sums its records' weights per (grid cube, row), and
 // for grids of at most count_planes_lds planes adds the sums into the
 // workgroup's LDS, which adds into the grid weights once at its end (the
@@ -339,7 +405,7 @@ __device__ __forceinline__ int bin_key(int k, int gx, int gy, int quad_keys) {
 constexpr int count_planes_lds = 64;
 constexpr unsigned count_blocks_max = 2048;
 
-template <int N, bool HALO>
+template <int N>
 __global__ __launch_bounds__(block) void k_count(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
@@ -398,15 +464,11 @@ __global__ __launch_bounds__(block) void k_count(
         }
         if (c.inside && do_grid) {
           const int ntiles = geo.ntx * geo.nty;
-          const int tx0 = tiles_begin(c.gx), tx1 = HALO ? tx0 + 1 : tiles_end(c.gx, g.sx);
-          const int ty0 = tiles_begin(c.gy), ty1 = HALO ? ty0 + 1 : tiles_end(c.gy, g.sy);
+          const int t = tiles_begin(c.gy) * geo.ntx + tiles_begin(c.gx);
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
             if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
-            const size_t base = size_t(gcube * geo.nr + gpol) * ntiles;
-            for (int ty = ty0; ty < ty1; ++ty)
-              for (int tx = tx0; tx < tx1; ++tx)
-                atomicAdd(hist + bin_key(int(base) + ty * geo.ntx + tx, c.gx, c.gy, quad_keys),
-                          1u);
+            const int base = int(gcube * geo.nr + gpol) * ntiles;
+            atomicAdd(hist + bin_key(base + t, c.gx, c.gy, quad_keys), 1u);
           }
         }
       }
@@ -439,7 +501,7 @@ __global__ __launch_bounds__(block) void k_count(
   }
 }
 
-template <int N, bool HALO>
+template <int N>
 __global__ __launch_bounds__(block) void k_emit(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
@@ -486,32 +548,21 @@ __global__ __launch_bounds__(block) void k_emit(
     }
   }
   const int ntiles = geo.ntx * geo.nty;
-  const int tx0 = tiles_begin(c.gx), tx1 = HALO ? tx0 + 1 : tiles_end(c.gx, g.sx);
-  const int ty0 = tiles_begin(c.gy), ty1 = HALO ? ty0 + 1 : tiles_end(c.gy, g.sy);
+  const int tx = tiles_begin(c.gx), ty = tiles_begin(c.gy);
   for (int gpol = 0; gpol < geo.nr; ++gpol) {
     if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
-    const size_t base = size_t(gcube * geo.nr + gpol) * ntiles;
-    for (int ty = ty0; ty < ty1; ++ty)
-      for (int tx = tx0; tx < tx1; ++tx) {
-        const unsigned pos =
-          atomicAdd(cursor + bin_key(int(base) + ty * geo.ntx + tx, c.gx, c.gy, quad_keys), 1u);
-        if constexpr (HALO) {
-          // the haloed-tile entry (layout of Entry4 below): corner relative
-          // to the tile, fine offsets, flags
-          const unsigned hpos = unsigned(c.gx - tx0 * tile)
-            | (unsigned(c.gy - ty0 * tile) << 6) | ((e.h.fpk & 0xffffu) << 12)
-            | (pos_w ? (1u << 28) : 0u) | (grad ? (1u << 29) : 0u);
-          unsigned* q = static_cast<unsigned*>(entries_out)
-            + size_t(pos) * (2 + 2 * N);
-          q[0] = hpos;
-          q[1] = e.h.gpk;
-          float2* qg = reinterpret_cast<float2*>(q + 2);
-          for (int v = 0; v < N; ++v) qg[v] = e.g[v];
-        } else {
-          static_cast<Entry<N>*>(entries_out)[pos] = e;
-        }
-        if (grad) entry_vis[pos] = unsigned(i);
-      }
+    const int base = int(gcube * geo.nr + gpol) * ntiles;
+    const unsigned pos =
+      atomicAdd(cursor + bin_key(base + ty * geo.ntx + tx, c.gx, c.gy, quad_keys), 1u);
+    // corner relative to the tile, fine offsets, flags
+    const unsigned hpos = unsigned(c.gx - tx * tile) | (unsigned(c.gy - ty * tile) << 6)
+      | ((e.h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u) | (grad ? e4_gradient : 0u);
+    unsigned* q = static_cast<unsigned*>(entries_out) + size_t(pos) * (2 + 2 * N);
+    q[0] = hpos;
+    q[1] = e.h.gpk;
+    float2* qg = reinterpret_cast<float2*>(q + 2);
+    for (int v = 0; v < N; ++v) qg[v] = e.g[v];
+    if (grad) entry_vis[pos] = unsigned(i);
   }
 }
 
@@ -670,242 +721,6 @@ __device__ __forceinline__ float bcast(float v, int k) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
 }
 
-// k_tile2 with UNR: tap iterations whose loads are issued together (two for
-// four polarizations, whose loads would otherwise take the registers of
-// several waves).  The unrolled kernel holds fewer waves, which pays for
-// large supports only (unroll_min_taps and more taps).
-template <int N>
-constexpr int tap_unroll() { return N <= 2 ? 4 : 2; }
-constexpr int unroll_min_taps = 2048;
-
-template <int N, int MODE, bool UNR>
-__global__ __launch_bounds__(block) void k_tile2(
-  Geometry geo, const GroupInfo* __restrict__ groups,
-  const float2* __restrict__ taps, Mueller mu,
-  const unsigned* __restrict__ offsets, const Entry<N>* __restrict__ entries,
-  const unsigned* __restrict__ entry_vis, const VisRec<N>* __restrict__ recs,
-  void* __restrict__ grid) {
-
-  constexpr int TT = tile * tile;
-  // MODE 0: re[TT], im[TT] (double); MODE 1: hi_re, hi_im, lo_re, lo_im (float)
-  __shared__ double acc64[MODE == 0 ? 2 * TT : 1];
-  // MODE 1: (hi, lo) pairs of re[TT], then im[TT]
-  __shared__ unsigned long long pairs[MODE == 1 ? 2 * TT : 1];
-
-  const unsigned key = blockIdx.x;
-  const unsigned beg = offsets[key];
-  const unsigned end = offsets[key + 1];
-  if (beg == end) return;
-
-  const int ntiles = geo.ntx * geo.nty;
-  const unsigned plane = key / ntiles;
-  const int t = int(key % ntiles);
-  const int x0 = (t % geo.ntx) * tile;
-  const int y0 = (t / geo.ntx) * tile;
-  const int gpol = int(plane % geo.nr);
-
-  if constexpr (MODE == 0) {
-    for (int k = threadIdx.x; k < 2 * TT; k += block) acc64[k] = 0.0;
-  } else {
-    for (int k = threadIdx.x; k < 2 * TT; k += block) pairs[k] = 0ull;
-  }
-  __syncthreads();
-
-  const int w = threadIdx.x / wave;
-  const int lane = threadIdx.x % wave;
-
-  for (unsigned base = beg + w * wave; base < end; base += tile_waves * wave) {
-    const int cnt = int(min(unsigned(wave), end - base));
-    Entry<N> mine;
-    if (lane < cnt) mine = entries[base + lane];
-    for (int k = 0; k < cnt; ++k) {
-      const int gx = bcast(mine.h.gx, k);
-      const int gy = bcast(mine.h.gy, k);
-      const unsigned fpk = unsigned(bcast(int(mine.h.fpk), k));
-      const unsigned gpk = unsigned(bcast(int(mine.h.gpk), k));
-      float2 gv[N];
-      for (int v = 0; v < N; ++v)
-        gv[v] = make_float2(bcast(mine.g[v].x, k), bcast(mine.g[v].y, k));
-      const int fxi = int(fpk & 0xffu);
-      const int fyi = int((fpk >> 8) & 0xffu);
-      const unsigned flags = fpk >> 16;
-      const int grp = int(gpk & 0xffffu);
-      const int cfcube = int(gpk >> 16);
-      const GroupInfo g = groups[grp];
-      const bool pos_w = flags & flag_pos_w;
-      const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
-      const float imf = pos_w ? -1.0f : 1.0f;
-
-      const int xa = max(gx, x0) - gx;
-      const int xb = min(gx + g.sx, x0 + tile) - gx;
-      const int ya = max(gy, y0) - gy;
-      const int yb = min(gy + g.sy, y0 + tile) - gy;
-      const int wdt = xb - xa;
-      const int ntap = wdt * (yb - ya);
-      const unsigned mg = magic(unsigned(wdt));
-
-      const float2* slice[N];
-      bool use[N];
-      const long long slice_taps = (long long)g.sx * g.sy;
-      for (int v = 0; v < N; ++v) {
-        const int m = row[v];
-        use[v] = m >= 0 && m < g.nmueller;
-        slice[v] = taps + g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (use[v] ? m : 0)) * geo.nf + fxi)
-               * geo.nf + fyi) * slice_taps;
-      }
-      const bool grad = flags & flag_gradient;
-      double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
-      if (grad) {
-        const unsigned i = entry_vis[base + k];
-        const double gxr = recs[i].grad[0];
-        const double gyr = recs[i].grad[1];
-        phi0x = -gxr * ((g.sx / 2) * geo.os - (fxi - geo.F));
-        phi0y = -gyr * ((g.sy / 2) * geo.os - (fyi - geo.F));
-        dphix = gxr * geo.os;
-        dphiy = gyr * geo.os;
-      }
-
-      if constexpr (!UNR) {
-        for (int q = lane; q < ntap; q += wave) {
-          const int yl = int(div_magic(unsigned(q), unsigned(wdt), mg));
-          const int X = xa + (q - yl * wdt);
-          const int Y = ya + yl;
-          float2 scr = make_float2(1.0f, 0.0f);
-          if (grad) {
-            const double phX = phi0x + X * dphix;
-            const double phY = phi0y + Y * dphiy;
-            scr = narrow(cphase(phX + phY));
-          }
-          const int li = (gy + Y - y0) * tile + (gx + X - x0);
-          double sr = 0.0, si = 0.0;
-          for (int v = 0; v < N; ++v) {
-            if (!use[v]) continue;
-            float2 c = slice[v][Y * g.sx + X];
-            c.y *= imf;
-            if (grad) c = cmul(c, scr);
-            const float2 pr = cmul(c, gv[v]);
-            sr += double(pr.x);
-            si += double(pr.y);
-          }
-          if constexpr (MODE == 0) {
-            __hip_atomic_fetch_add(acc64 + li, sr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(acc64 + TT + li, si, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-          } else {
-            // split the FP64 tap sum into float hi + lo (exact for N == 1)
-            const float hr = float(sr), hi = float(si);
-            const float lr = float(sr - double(hr)), lim = float(si - double(hi));
-            pair_add<(N > 1)>(pairs + li, pairs[li], hr, lr);
-            pair_add<(N > 1)>(pairs + TT + li, pairs[TT + li], hi, lim);
-          }
-        }
-        continue;
-      }
-      // the footprint tile_unroll x 64 taps at a time: the CF loads of all
-      // of them issued before the first is used (one step for footprints of
-      // at most 64 taps, and for records with a phase gradient: their FP64
-      // screen would not fit the registers of the unrolled loop)
-      constexpr int tile_unroll = tap_unroll<N>();
-      const int unroll = grad || ntap <= wave ? 1 : tile_unroll;
-      for (int q0 = lane; q0 < ntap; q0 += unroll * wave) {
-        float2 cv[tile_unroll][N];
-        int tx[tile_unroll], ty[tile_unroll];
-#pragma unroll
-        for (int u = 0; u < tile_unroll; ++u) {
-          const int q = q0 + u * wave;
-          const bool ok = u < unroll && q < ntap;
-          const int qq = ok ? q : 0;
-          const int yl = int(div_magic(unsigned(qq), unsigned(wdt), mg));
-          tx[u] = xa + (qq - yl * wdt);
-          ty[u] = ya + yl;
-#pragma unroll
-          for (int v = 0; v < N; ++v)
-            cv[u][v] = use[v] && ok ? slice[v][ty[u] * g.sx + tx[u]] : make_float2(0.0f, 0.0f);
-        }
-        if (grad) {
-          // one tap (u = 0) with its phase screen
-          const int X = tx[0], Y = ty[0];
-          const double phX = phi0x + X * dphix;
-          const double phY = phi0y + Y * dphiy;
-          const float2 scr = narrow(cphase(phX + phY));
-          const int li = (gy + Y - y0) * tile + (gx + X - x0);
-          double sr = 0.0, si = 0.0;
-          for (int v = 0; v < N; ++v) {
-            if (!use[v]) continue;
-            float2 c = cv[0][v];
-            c.y *= imf;
-            c = cmul(c, scr);
-            const float2 pr = cmul(c, gv[v]);
-            sr += double(pr.x);
-            si += double(pr.y);
-          }
-          if constexpr (MODE == 0) {
-            __hip_atomic_fetch_add(acc64 + li, sr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(acc64 + TT + li, si, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-          } else {
-            const float hr = float(sr), hi = float(si);
-            const float lr = float(sr - double(hr)), lim = float(si - double(hi));
-            pair_add<(N > 1)>(pairs + li, pairs[li], hr, lr);
-            pair_add<(N > 1)>(pairs + TT + li, pairs[TT + li], hi, lim);
-          }
-          continue;
-        }
-#pragma unroll
-        for (int u = 0; u < tile_unroll; ++u) {
-          if (q0 + u * wave >= ntap) break;
-          const int li = (gy + ty[u] - y0) * tile + (gx + tx[u] - x0);
-          double sr = 0.0, si = 0.0;
-          for (int v = 0; v < N; ++v) {
-            if (!use[v]) continue;
-            float2 c = cv[u][v];
-            c.y *= imf;
-            const float2 pr = cmul(c, gv[v]);
-            sr += double(pr.x);
-            si += double(pr.y);
-          }
-          if constexpr (MODE == 0) {
-            __hip_atomic_fetch_add(acc64 + li, sr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(acc64 + TT + li, si, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-          } else {
-            // split the FP64 tap sum into float hi + lo (exact for N == 1)
-            const float hr = float(sr), hi = float(si);
-            const float lr = float(sr - double(hr)), lim = float(si - double(hi));
-            pair_add<(N > 1)>(pairs + li, pairs[li], hr, lr);
-            pair_add<(N > 1)>(pairs + TT + li, pairs[TT + li], hi, lim);
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();
-
-  for (int k = threadIdx.x; k < TT; k += block) {
-    const int xx = x0 + k % tile;
-    const int yy = y0 + k / tile;
-    if (xx >= geo.nx || yy >= geo.ny) continue;
-    const size_t gi = (size_t(plane) * geo.ny + yy) * geo.nx + xx;
-    if constexpr (MODE == 0) {
-      double2* gp = static_cast<double2*>(grid) + gi;
-      double2 gvl = *gp;
-      gvl.x += acc64[k];
-      gvl.y += acc64[TT + k];
-      *gp = gvl;
-    } else {
-      float2* gp = static_cast<float2*>(grid) + gi;
-      const float2 g0 = *gp;
-      float sr, er, si, ei;
-      const unsigned long long pr = pairs[k], pi = pairs[TT + k];
-      two_sum(g0.x, __uint_as_float(unsigned(pr)), sr, er);
-      two_sum(g0.y, __uint_as_float(unsigned(pi)), si, ei);
-      *gp = make_float2(sr + (er + __uint_as_float(unsigned(pr >> 32))),
-                        si + (ei + __uint_as_float(unsigned(pi >> 32))));
-    }
-  }
-}
-
 // ---- gridding, block-local bins ----------------------------------------------
 //
 // For grids with few (plane, tile) keys (<= bin_keys_max) the bins are built
@@ -915,11 +730,6 @@ __global__ __launch_bounds__(block) void k_tile2(
 //           offset table off[block][key] (nkeys + 1 values), then each entry
 //           written at its block-local position -- one pass over the records.
 //           Weights are reduced per grid plane in LDS first.
-// k_tile3   one workgroup per key: gathers the key's segment from every bin
-//           block (offset table + LDS scan), then processes the virtual
-//           entry list 64 entries per wave; entries with at most 64 taps are
-//           handled four at a time with all their CF-tap loads issued
-//           together (latency overlap), the others tap-chunk by tap-chunk.
 
 constexpr int bin_threads = 1024;
 constexpr int bin_recs_per_thread = 4;
@@ -927,7 +737,7 @@ constexpr int bin_records = bin_threads * bin_recs_per_thread;  // per block
 constexpr int bin_keys_max = 8192;        // (plane, tile) keys of the block-local bins
 constexpr int bin_quad_keys_max = 16384;  // quadrant keys (4 per tile key): LDS histogram
 constexpr int bin_planes_max = 1024;
-constexpr int tile_bins_max = 2048;  // bin blocks per pass (LDS of k_tile3)
+constexpr int tile_bins_max = 2048;  // bin blocks per pass (LDS of k_tile4)
 constexpr int bin_stage_bytes = 65536;  // LDS staging of k_bin's haloed entries (one
                                         // chunk for a block of one-polarization entries)
 
@@ -977,10 +787,8 @@ __device__ unsigned block_exclusive_scan(unsigned* a, int n, unsigned* part) {
 }
 
 
-// HALO = false: one entry per (plane, tile) the support touches (Entry<N>,
-// for k_tile3); HALO = true: one entry per plane, keyed by the tile of the
-// support corner (Entry4<N>, for k_tile4)
-template <int N, bool HALO>
+// one entry per record and plane, keyed by the tile of the support corner
+template <int N>
 __global__ __launch_bounds__(bin_threads) void k_bin(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
@@ -994,7 +802,7 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
   __shared__ double wl[bin_planes_max];
   __shared__ unsigned part[bin_threads / wave + 1];
 
-  // quad_keys (HALO only): a key per 16 x 16 quadrant of each (plane, tile),
+  // quad_keys: a key per 16 x 16 quadrant of each (plane, tile),
   // key = 4 * tile key + quadrant of the support corner, so that the
   // entries of one quadrant are contiguous within each bin block
   const int nkeys = geo.ntx * geo.nty * geo.nr * geo.nc * (quad_keys ? 4 : 1);
@@ -1022,7 +830,6 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
   };
   Entry<N> e[bin_recs_per_thread];
   bool keep[bin_recs_per_thread];
-  unsigned short sxy[bin_recs_per_thread][2];
   unsigned gc[bin_recs_per_thread];
   unsigned ninvalid = 0;
 
@@ -1047,7 +854,7 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
   static_assert(sizeof(VisRec<N>) % sizeof(unsigned long long) == 0, "8-byte record words");
   static_assert(bin_recs_per_thread % 2 == 0, "records loaded in pairs");
   VisRec<N> rc[hoist ? 2 : 1];
-  // HALO: the place of each of this thread's entries (one per record and
+  // the place of each of this thread's entries (one per record and
   // grid row with an index; ~0u for none) within its key, from the count's
   // returned value, then (after the scan) its block-local position; the
   // entries are then written through LDS in position order
@@ -1114,8 +921,6 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
     const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
     keep[j] = true;
     gc[j] = gcube;
-    sxy[j][0] = (unsigned short)g.sx;
-    sxy[j][1] = (unsigned short)g.sy;
     e[j].h.gx = c.gx;
     e[j].h.gy = c.gy;
     e[j].h.fpk = unsigned(fxi) | (unsigned(fyi) << 8)
@@ -1170,25 +975,17 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
         wacc[gp] += t;
       }
     }
-    const int tx0 = tiles_begin(c.gx), tx1 = HALO ? tx0 + 1 : tiles_end(c.gx, g.sx);
-    const int ty0 = tiles_begin(c.gy), ty1 = HALO ? ty0 + 1 : tiles_end(c.gy, g.sy);
+    const int t = tiles_begin(c.gy) * geo.ntx + tiles_begin(c.gx);
     const unsigned rows = (pos_w != bool(degrid_pass)) ? rows_m : rows_mc;
     for (int gpol = 0; gpol < geo.nr; ++gpol) {
       if (!((rows >> gpol) & 1u)) continue;
       const int base = (int(gcube) * geo.nr + gpol) * ntiles;
-      for (int ty = ty0; ty < ty1; ++ty)
-        for (int tx = tx0; tx < tx1; ++tx) {
-          const unsigned place = __hip_atomic_fetch_add(
-            cnt + bin_key(base + ty * geo.ntx + tx, c.gx, c.gy, quad_keys), 1u,
-            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          if constexpr (HALO) {
+      const unsigned place = __hip_atomic_fetch_add(
+        cnt + bin_key(base + t, c.gx, c.gy, quad_keys), 1u,
+        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (r == gpol) hpos[j][r] = place;
-          } else {
-            (void)place;
-          }
-        }
+      for (int r = 0; r < 4; ++r)
+        if (r == gpol) hpos[j][r] = place;
     }
   }
   // the threads' weight sums: one sum per (wave, grid cube) present, the
@@ -1233,289 +1030,53 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
     const size_t i = size_t(j) * bin_threads + threadIdx.x;
     const bool pos_w = (e[j].h.fpk >> 16) & flag_pos_w;
     const bool grad = (e[j].h.fpk >> 16) & flag_gradient;
-    const int tx0 = tiles_begin(e[j].h.gx);
-    const int tx1 = HALO ? tx0 + 1 : tiles_end(e[j].h.gx, sxy[j][0]);
-    const int ty0 = tiles_begin(e[j].h.gy);
-    const int ty1 = HALO ? ty0 + 1 : tiles_end(e[j].h.gy, sxy[j][1]);
+    const int t = tiles_begin(e[j].h.gy) * geo.ntx + tiles_begin(e[j].h.gx);
     const unsigned rows = (pos_w != bool(degrid_pass)) ? rows_m : rows_mc;
     for (int gpol = 0; gpol < geo.nr; ++gpol) {
       if (!((rows >> gpol) & 1u)) continue;
       const int base = (int(gc[j]) * geo.nr + gpol) * ntiles;
-      for (int ty = ty0; ty < ty1; ++ty)
-        for (int tx = tx0; tx < tx1; ++tx) {
-          const int key = bin_key(base + ty * geo.ntx + tx, e[j].h.gx, e[j].h.gy, quad_keys);
-          unsigned pos;
-          if constexpr (HALO) {
-            // the key's offset (cnt holds the scan now) + the entry's place
-            unsigned place = 0;
+      // the key's offset (cnt holds the scan now) + the entry's place
+      unsigned place = 0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (r == gpol) place = hpos[j][r];
-            pos = cnt[key] + place;
+      for (int r = 0; r < 4; ++r)
+        if (r == gpol) place = hpos[j][r];
+      const unsigned pos = cnt[bin_key(base + t, e[j].h.gx, e[j].h.gy, quad_keys)] + place;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (r == gpol) hpos[j][r] = pos;
-          } else {
-            pos = __hip_atomic_fetch_add(cnt + key, 1u, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_WORKGROUP);
-            static_cast<Entry<N>*>(entries_out)[b * block_cap + pos] = e[j];
-          }
-          if (grad || degrid_pass) outv[pos] = unsigned(b * bin_records + i);
-        }
+      for (int r = 0; r < 4; ++r)
+        if (r == gpol) hpos[j][r] = pos;
+      if (grad || degrid_pass) outv[pos] = unsigned(b * bin_records + i);
     }
   }
-  if constexpr (HALO) {
-    // chunks of the block's entry range: each thread puts its entries of
-    // the chunk into LDS, then the block copies the chunk out contiguously
-    // (scattered 16 to 40-byte stores would each write a partial line)
-    constexpr unsigned words = unsigned(sizeof(Entry4<N>) / sizeof(unsigned long long));
-    constexpr unsigned chunk = unsigned(bin_stage_bytes / sizeof(Entry4<N>));
-    __shared__ unsigned long long stage[chunk * words];
-    Entry4<N>* staged = reinterpret_cast<Entry4<N>*>(stage);
-    unsigned long long* dst =
-      reinterpret_cast<unsigned long long*>(static_cast<Entry4<N>*>(entries_out) + b * block_cap);
-    for (unsigned c0 = 0; c0 < btotal; c0 += chunk) {
+  // chunks of the block's entry range: each thread puts its entries of
+  // the chunk into LDS, then the block copies the chunk out contiguously
+  // (scattered 16 to 40-byte stores would each write a partial line)
+  constexpr unsigned ewords = unsigned(sizeof(Entry4<N>) / sizeof(unsigned long long));
+  constexpr unsigned chunk = unsigned(bin_stage_bytes / sizeof(Entry4<N>));
+  __shared__ unsigned long long stage[chunk * ewords];
+  Entry4<N>* staged = reinterpret_cast<Entry4<N>*>(stage);
+  unsigned long long* dst =
+    reinterpret_cast<unsigned long long*>(static_cast<Entry4<N>*>(entries_out) + b * block_cap);
+  for (unsigned c0 = 0; c0 < btotal; c0 += chunk) {
 #pragma unroll
-      for (int j = 0; j < bin_recs_per_thread; ++j) {
-        if (!keep[j]) continue;
-        const bool pos_w = (e[j].h.fpk >> 16) & flag_pos_w;
-        const bool grad = (e[j].h.fpk >> 16) & flag_gradient;
-        Entry4<N> q;
-        q.h.pos = unsigned(e[j].h.gx - tiles_begin(e[j].h.gx) * tile)
-          | (unsigned(e[j].h.gy - tiles_begin(e[j].h.gy) * tile) << 6)
-          | ((e[j].h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u)
-          | (grad ? e4_gradient : 0u);
-        q.h.gpk = e[j].h.gpk;
-        for (int v = 0; v < N; ++v) q.g[v] = e[j].g[v];
+    for (int j = 0; j < bin_recs_per_thread; ++j) {
+      if (!keep[j]) continue;
+      const bool pos_w = (e[j].h.fpk >> 16) & flag_pos_w;
+      const bool grad = (e[j].h.fpk >> 16) & flag_gradient;
+      Entry4<N> q;
+      q.h.pos = unsigned(e[j].h.gx - tiles_begin(e[j].h.gx) * tile)
+        | (unsigned(e[j].h.gy - tiles_begin(e[j].h.gy) * tile) << 6)
+        | ((e[j].h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u)
+        | (grad ? e4_gradient : 0u);
+      q.h.gpk = e[j].h.gpk;
+      for (int v = 0; v < N; ++v) q.g[v] = e[j].g[v];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (hpos[j][r] - c0 < chunk) staged[hpos[j][r] - c0] = q;
-      }
-      __syncthreads();
-      const unsigned n = min(chunk, btotal - c0) * words;
-      for (unsigned k = threadIdx.x; k < n; k += bin_threads) dst[size_t(c0) * words + k] = stage[k];
-      __syncthreads();
+      for (int r = 0; r < 4; ++r)
+        if (hpos[j][r] - c0 < chunk) staged[hpos[j][r] - c0] = q;
     }
-  }
-}
-
-// parameters of one entry, uniform across the wave
-struct EntryParams {
-  int gx, gy, fxi, fyi, grp, cfcube, sx;
-  unsigned flags;
-};
-
-template <int N, int MODE, int U>
-__global__ __launch_bounds__(block) void k_tile3(
-  Geometry geo, const GroupInfo* __restrict__ groups,
-  const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
-  int nbins, size_t block_cap, const Entry<N>* __restrict__ entries,
-  const unsigned* __restrict__ entry_vis, const VisRec<N>* __restrict__ recs,
-  void* __restrict__ grid) {
-
-  constexpr int TT = tile * tile;
-  __shared__ double acc64[MODE == 0 ? 2 * TT : 1];
-  // MODE 1: (hi, lo) pairs of re[TT], then im[TT]
-  __shared__ unsigned long long pairs[MODE == 1 ? 2 * TT : 1];
-  __shared__ unsigned seg_pref[tile_bins_max + 1];
-  __shared__ unsigned seg_beg[tile_bins_max];
-  __shared__ unsigned part[block / wave + 1];
-
-  const unsigned key = blockIdx.x;
-  const int nkeys = geo.ntx * geo.nty * geo.nr * geo.nc;
-  // segment of this key in every bin block
-  for (int bb = threadIdx.x; bb < nbins; bb += block) {
-    const unsigned* tab = off_table + size_t(bb) * (nkeys + 1);
-    const unsigned s0 = tab[key], s1 = tab[key + 1];
-    seg_pref[bb] = s1 - s0;
-    seg_beg[bb] = s0;
-  }
-  __syncthreads();
-  const unsigned total = block_exclusive_scan(seg_pref, nbins, part);
-  if (total == 0) return;
-  if (threadIdx.x == 0) seg_pref[nbins] = total;
-
-  const int ntiles = geo.ntx * geo.nty;
-  const unsigned plane = key / ntiles;
-  const int t = int(key % ntiles);
-  const int x0 = (t % geo.ntx) * tile;
-  const int y0 = (t / geo.ntx) * tile;
-  const int gpol = int(plane % geo.nr);
-
-  if constexpr (MODE == 0) {
-    for (int k = threadIdx.x; k < 2 * TT; k += block) acc64[k] = 0.0;
-  } else {
-    for (int k = threadIdx.x; k < 2 * TT; k += block) pairs[k] = 0ull;
-  }
-  __syncthreads();
-
-  const int w = threadIdx.x / wave;
-  const int lane = threadIdx.x % wave;
-
-  auto accumulate = [&](int li, double sr, double si) {
-    if constexpr (MODE == 0) {
-      __hip_atomic_fetch_add(acc64 + li, sr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_add(acc64 + TT + li, si, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    } else {
-      const float hr = float(sr), hi = float(si);
-      const float lr = float(sr - double(hr)), lim = float(si - double(hi));
-      pair_add<(N > 1)>(pairs + li, pairs[li], hr, lr);
-      pair_add<(N > 1)>(pairs + TT + li, pairs[TT + li], hi, lim);
-    }
-  };
-
-  for (unsigned base = w * wave; base < total; base += tile_waves * wave) {
-    const int cnt = int(min(unsigned(wave), total - base));
-    Entry<N> mine;
-    unsigned mine_idx = 0;
-    if (lane < cnt) {
-      // locate entry base + lane in the concatenated segments
-      const unsigned q = base + lane;
-      int lo = 0, hi = nbins;  // seg_pref[lo] <= q < seg_pref[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (seg_pref[mid] <= q) lo = mid; else hi = mid;
-      }
-      mine_idx = unsigned(lo) * unsigned(block_cap) + seg_beg[lo] + (q - seg_pref[lo]);
-      mine = entries[mine_idx];
-    }
-    for (int k0 = 0; k0 < cnt; k0 += U) {
-      EntryParams P[U];
-      float2 gv[U][N];
-      int xa[U], wdt[U], ya[U], ntap[U];
-      const float2* slice[U][N];
-      bool use[U][N];
-      bool fast = true;
-      for (int u = 0; u < U; ++u) {
-        const int k = min(k0 + u, cnt - 1);
-        P[u].gx = bcast(mine.h.gx, k);
-        P[u].gy = bcast(mine.h.gy, k);
-        const unsigned fpk = unsigned(bcast(int(mine.h.fpk), k));
-        const unsigned gpk = unsigned(bcast(int(mine.h.gpk), k));
-        P[u].fxi = int(fpk & 0xffu);
-        P[u].fyi = int((fpk >> 8) & 0xffu);
-        P[u].flags = fpk >> 16;
-        P[u].grp = int(gpk & 0xffffu);
-        P[u].cfcube = int(gpk >> 16);
-        for (int v = 0; v < N; ++v)
-          gv[u][v] = make_float2(bcast(mine.g[v].x, k), bcast(mine.g[v].y, k));
-        const GroupInfo g = groups[P[u].grp];
-        xa[u] = max(P[u].gx, x0) - P[u].gx;
-        const int xb = min(P[u].gx + g.sx, x0 + tile) - P[u].gx;
-        ya[u] = max(P[u].gy, y0) - P[u].gy;
-        const int yb = min(P[u].gy + g.sy, y0 + tile) - P[u].gy;
-        wdt[u] = xb - xa[u];
-        ntap[u] = k0 + u < cnt ? wdt[u] * (yb - ya[u]) : 0;
-        const bool pos_w = P[u].flags & flag_pos_w;
-        const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
-        const long long slice_taps = (long long)g.sx * g.sy;
-        for (int v = 0; v < N; ++v) {
-          const int m = row[v];
-          use[u][v] = m >= 0 && m < g.nmueller;
-          slice[u][v] = taps + g.tap_offset
-            + (((long long)(P[u].cfcube * g.nmueller + (use[u][v] ? m : 0)) * geo.nf + P[u].fxi)
-                 * geo.nf + P[u].fyi) * slice_taps;
-        }
-        fast = fast && ntap[u] <= wave && !(P[u].flags & flag_gradient);
-        P[u].sx = g.sx;
-      }
-      if (fast) {
-        // all loads first, then the products and the LDS accumulation
-        float2 c[U][N];
-        int li[U];
-        for (int u = 0; u < U; ++u) {
-          const unsigned mg = magic(unsigned(max(wdt[u], 1)));
-          const int yl = int(div_magic(unsigned(lane), unsigned(max(wdt[u], 1)), mg));
-          const int X = xa[u] + (lane - yl * wdt[u]);
-          const int Y = ya[u] + yl;
-          li[u] = (P[u].gy + Y - y0) * tile + (P[u].gx + X - x0);
-          for (int v = 0; v < N; ++v)
-            c[u][v] = (lane < ntap[u] && use[u][v]) ? slice[u][v][Y * P[u].sx + X]
-                                                    : make_float2(0.0f, 0.0f);
-        }
-        for (int u = 0; u < U; ++u) {
-          if (lane >= ntap[u]) continue;
-          const float imf = (P[u].flags & flag_pos_w) ? -1.0f : 1.0f;
-          double sr = 0.0, si = 0.0;
-          for (int v = 0; v < N; ++v) {
-            if (!use[u][v]) continue;
-            float2 cc = c[u][v];
-            cc.y *= imf;
-            const float2 pr = cmul(cc, gv[u][v]);
-            sr += double(pr.x);
-            si += double(pr.y);
-          }
-          accumulate(li[u], sr, si);
-        }
-      } else {
-        for (int u = 0; u < U; ++u) {
-          if (ntap[u] == 0) continue;
-          const int k = k0 + u;
-          const bool grad = P[u].flags & flag_gradient;
-          const float imf = (P[u].flags & flag_pos_w) ? -1.0f : 1.0f;
-          const int sx = P[u].sx;
-          double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
-          if (grad) {
-            const unsigned idx = unsigned(bcast(int(mine_idx), k));
-            const unsigned i = entry_vis[idx];
-            const GroupInfo g = groups[P[u].grp];
-            const double gxr = recs[i].grad[0];
-            const double gyr = recs[i].grad[1];
-            phi0x = -gxr * ((g.sx / 2) * geo.os - (P[u].fxi - geo.F));
-            phi0y = -gyr * ((g.sy / 2) * geo.os - (P[u].fyi - geo.F));
-            dphix = gxr * geo.os;
-            dphiy = gyr * geo.os;
-          }
-          const unsigned mg = magic(unsigned(wdt[u]));
-          for (int q = lane; q < ntap[u]; q += wave) {
-            const int yl = int(div_magic(unsigned(q), unsigned(wdt[u]), mg));
-            const int X = xa[u] + (q - yl * wdt[u]);
-            const int Y = ya[u] + yl;
-            float2 scr = make_float2(1.0f, 0.0f);
-            if (grad) {
-              const double phX = phi0x + X * dphix;
-              const double phY = phi0y + Y * dphiy;
-              scr = narrow(cphase(phX + phY));
-            }
-            double sr = 0.0, si = 0.0;
-            for (int v = 0; v < N; ++v) {
-              if (!use[u][v]) continue;
-              float2 cc = slice[u][v][Y * sx + X];
-              cc.y *= imf;
-              if (grad) cc = cmul(cc, scr);
-              const float2 pr = cmul(cc, gv[u][v]);
-              sr += double(pr.x);
-              si += double(pr.y);
-            }
-            accumulate((P[u].gy + Y - y0) * tile + (P[u].gx + X - x0), sr, si);
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();
-
-  for (int k = threadIdx.x; k < TT; k += block) {
-    const int xx = x0 + k % tile;
-    const int yy = y0 + k / tile;
-    if (xx >= geo.nx || yy >= geo.ny) continue;
-    const size_t gi = (size_t(plane) * geo.ny + yy) * geo.nx + xx;
-    if constexpr (MODE == 0) {
-      double2* gp = static_cast<double2*>(grid) + gi;
-      double2 gvl = *gp;
-      gvl.x += acc64[k];
-      gvl.y += acc64[TT + k];
-      *gp = gvl;
-    } else {
-      float2* gp = static_cast<float2*>(grid) + gi;
-      const float2 g0 = *gp;
-      float sr, er, si, ei;
-      const unsigned long long pr = pairs[k], pi = pairs[TT + k];
-      two_sum(g0.x, __uint_as_float(unsigned(pr)), sr, er);
-      two_sum(g0.y, __uint_as_float(unsigned(pi)), si, ei);
-      *gp = make_float2(sr + (er + __uint_as_float(unsigned(pr >> 32))),
-                        si + (ei + __uint_as_float(unsigned(pi >> 32))));
-    }
+    __syncthreads();
+    const unsigned cw = min(chunk, btotal - c0) * ewords;
+    for (unsigned k = threadIdx.x; k < cw; k += bin_threads) dst[size_t(c0) * ewords + k] = stage[k];
+    __syncthreads();
   }
 }
 
@@ -1566,7 +1127,8 @@ __host__ __device__ inline int halo_pixels(int hx, int hy) {
 constexpr int acc_f64 = 0;
 constexpr int acc_f32_cas = 2;
 
-template <int N, int MODE, int ACC>
+// UNIT: every CF group has one Mueller element
+template <int N, int MODE, int ACC, bool UNIT>
 __global__ __launch_bounds__(halo_block) void k_tile4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
@@ -1681,18 +1243,15 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
       const int grp = int(e.h.gpk & 0xffffu);
       const int cfcube = int(e.h.gpk >> 16);
       const GroupInfo g = groups[grp];
-      const int sx = g.sx, sy = g.sy;
+      const int sx = g.sx, sy = g.sy, nm = UNIT ? 1 : g.nmueller;
       const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
       const float imf = pos_w ? -1.0f : 1.0f;
       const float2* slice[N];
       bool use[N];
-      const long long slice_taps = (long long)sx * sy;
       for (int v = 0; v < N; ++v) {
         const int m = row[v];
         use[v] = m >= 0 && m < g.nmueller;
-        slice[v] = taps + g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (use[v] ? m : 0)) * geo.nf + fxi) * geo.nf
-             + fyi) * slice_taps;
+        slice[v] = taps + slice_start<UNIT>(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
       }
       double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
       if (grad) {
@@ -1809,7 +1368,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
 #pragma unroll
             for (int v = 0; v < N; ++v) {
               float2 tv = make_float2(0.0f, 0.0f);
-              if (ok[k]) tv = slice[v][t0 + k];
+              if (ok[k]) tv = slice[v][(t0 + k) * nm];
               c[k][v] = use[v] ? tv : make_float2(0.0f, 0.0f);
             }
           }
@@ -1944,130 +1503,10 @@ __global__ void k_halo(
   *gp = g;
 }
 
-// ---- gridding: haloed tiles, one wave per tile quadrant, one lane per tap --
-//
-// k_quad accumulates the keys and entries of k_tile4 into an FP32 grid,
-// (hi, lo) pairs per pixel updated by two-sum as in k_tile4's
-// compare-and-swap scheme, without LDS atomics.
-// The workgroup of a (plane, tile) key has four waves; wave w owns quadrant
-// (w & 1, w >> 1) of the 32 x 32 tile -- the entries whose support corner
-// lies in that 16 x 16 quadrant -- and a private LDS region of
-// (16 + hx) x (16 + hy) pixels, which holds those supports whole.  The wave
-// adds one entry at a time, one lane per CF tap: an entry's taps are
-// distinct pixels, a wave's LDS operations execute in order and no other wave
-// writes the region, so each tap is a plain 16-byte read-modify-write.  Per
-// round each thread prepares one entry (CF slice, values, region pixel) and
-// the round's entries are sorted by quadrant into LDS.  The flush sums the
-// four regions over the tile and its halo and writes both as k_tile4 does,
-// so k_halo folds the halos unchanged.
-constexpr int quad_block = 4 * wave;
-constexpr int quad_edge = tile / 2;
-constexpr int quad_bins_max = 256;  // bin blocks per pass (LDS segment tables)
-constexpr int quad_flush = 8;       // tile + halo pixels per thread in the flush
-// entries whose first CF taps are loaded ahead of their turn (2 measured
-// faster than 1, 3 or 4 for one polarization: the pipeline refills at
-// every round)
-template <int N>
-constexpr int quad_depth() { return 2; }
-
-// an entry prepared for its quadrant's wave; gc = (pos_w ? -1 : 1) * g with
-// re and im swapped, so that cmul(conj_w(c), g) = (c.x g.x - c.y gc.x,
-// c.x g.y + c.y gc.y) with the reference's roundings.  Entries with a phase
-// gradient do not use gc: gc[0].x holds the bits of their entry index.
-template <int N>
-struct QuadRec {
-  unsigned w0;        // region pixel | sx << 12 | sy << 18 | use << 24 | flags
-  unsigned slice[N];  // first tap of each polarization's CF slice
-  float2 g[N];
-  float2 gc[N];
-};
-constexpr unsigned quad_gradient = 1u << 28;
+constexpr int quad_edge = tile / 2;  // pixels of a tile quadrant
 constexpr unsigned quad_pos_w = 1u << 29;
-constexpr unsigned quad_skip = 1u << 30;  // not added by the pipelined loop
-                                          // (phase gradient, or no used
-                                          // polarization)
-template <int N>
-constexpr int quad_round() { return N == 1 ? quad_block : quad_block / 2; }
 
-__device__ __forceinline__ unsigned uniform_u(unsigned v) {
-  return unsigned(__builtin_amdgcn_readfirstlane(int(v)));
-}
-
-// adds the tap value h + l (FP32 high and low parts) to the (hi, lo) pairs
-// of a region pixel: hi' = fl(hi + h), lo' = fl(lo + (err + l)), err the
-// exact rounding error of the first sum (two-sum)
-template <int N>
-__device__ __forceinline__ void quad_add(
-  float4* region, int px, float h_r, float h_i, float l_r, float l_i) {
-  float4 a = region[px];
-  float sum, err;
-  two_sum(a.x, h_r, sum, err);
-  a.x = sum;
-  a.z = N > 1 ? a.z + (err + l_r) : a.z + err;
-  two_sum(a.y, h_i, sum, err);
-  a.y = sum;
-  a.w = N > 1 ? a.w + (err + l_i) : a.w + err;
-  region[px] = a;
-}
-
-// an entry with a phase gradient: its CF taps times the phase screen
-// exp(i phi(X, Y)) (FP64 phase, the reference's cphase) added by one wave,
-// one lane per tap.  Not inlined: the FP64 sine and cosine would otherwise
-// raise the register count of k_quad's pipelined loop.
-template <int N>
-__device__ __noinline__ void quad_gradient_entry(
-  const QuadRec<N>& p, unsigned ei, const Geometry& geo, const float2* __restrict__ taps,
-  const Entry4<N>* __restrict__ entries, const unsigned* __restrict__ entry_vis,
-  const VisRec<N>* __restrict__ recs, int QX, float4* region) {
-  const int lane = int(threadIdx.x % wave);
-  const unsigned w0 = uniform_u(p.w0);
-  const int base = int(w0 & 4095u);
-  const int sx = int((w0 >> 12) & 63u);
-  const int sy = int((w0 >> 18) & 63u);
-  const unsigned use = (w0 >> 24) & 15u;
-  const float imf = (w0 & quad_pos_w) ? -1.0f : 1.0f;
-  ei = uniform_u(ei);
-  const unsigned pos = entries[ei].h.pos;
-  const int fxi = int((pos >> 12) & 255u);
-  const int fyi = int((pos >> 20) & 255u);
-  const unsigned ri = entry_vis[ei];
-  const double gxr = recs[ri].grad[0];
-  const double gyr = recs[ri].grad[1];
-  const double phi0x = -gxr * ((sx / 2) * geo.os - (fxi - geo.F));
-  const double phi0y = -gyr * ((sy / 2) * geo.os - (fyi - geo.F));
-  const double dphix = gxr * geo.os;
-  const double dphiy = gyr * geo.os;
-  for (int t0 = 0; t0 < sx * sy; t0 += wave) {
-    const int tp = t0 + lane;
-    if (tp >= sx * sy) continue;
-    const int Y = tp / sx;
-    const int X = tp - Y * sx;
-    const float2 scr = narrow(cphase((phi0x + X * dphix) + (phi0y + Y * dphiy)));
-    double sr = 0.0, si = 0.0;
-    float h_r = 0.0f, h_i = 0.0f, l_r = 0.0f, l_i = 0.0f;
-    for (int v = 0; v < N; ++v) {
-      if (!((use >> v) & 1u)) continue;
-      float2 cc = taps[uniform_u(p.slice[v]) + size_t(tp)];
-      cc.y *= imf;
-      const float2 pr = cmul(cmul(cc, scr), p.g[v]);
-      if constexpr (N == 1) {
-        h_r = pr.x;
-        h_i = pr.y;
-      }
-      sr += double(pr.x);
-      si += double(pr.y);
-    }
-    if constexpr (N > 1) {
-      h_r = float(sr);
-      h_i = float(si);
-      l_r = float(sr - double(h_r));
-      l_i = float(si - double(h_i));
-    }
-    quad_add<N>(region, base + Y * QX + X, h_r, h_i, l_r, l_i);
-  }
-}
-
-// The flush of the quadrant kernels: the sum of the four quadrant regions
+// The flush of the quadrant kernel: the sum of the four quadrant regions
 // of (hi, lo) pairs (LDS, float4 per pixel, quadrant qd at qd * QX * QY)
 // over the tile and its halo.  Tile pixels are added to the FP32 grid with
 // one rounding (a two-sum of the grid value and hi, then hi + (err + lo));
@@ -2145,420 +1584,6 @@ __device__ __forceinline__ void quad_flush_tile(
   }
 }
 
-// ONE: every support fits one step (sx, sy <= 8); the pipelined loop is
-// then free of branches around vector memory loads, so each entry waits for
-// its own CF taps only and not for the loads issued after them
-template <int N, bool ONE>
-__global__ __launch_bounds__(quad_block) void k_quad(
-  Geometry geo, const GroupInfo* __restrict__ groups,
-  const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
-  int nbins, size_t block_cap, const Entry4<N>* __restrict__ entries,
-  const unsigned* __restrict__ entry_vis, const VisRec<N>* __restrict__ recs,
-  int hx, int hy, void* __restrict__ grid, double2* __restrict__ halo,
-  unsigned* __restrict__ halo_set) {
-  constexpr int RB = quad_round<N>();
-  // quadrant regions, 16 bytes per pixel: FP32 (hi_re, hi_im, lo_re, lo_im)
-  extern __shared__ float4 regions[];
-  __shared__ QuadRec<N> list[RB];
-  __shared__ unsigned seg_pref[quad_bins_max + 1];
-  __shared__ unsigned seg_beg[quad_bins_max];
-  __shared__ unsigned part[quad_block / wave + 1];
-  // per round: entries per quadrant, then a gradient flag; two sets, used
-  // by alternate rounds, so that a round needs no barrier before its counts
-  __shared__ unsigned qcnt2[2][5];
-
-  const int QX = quad_edge + hx;
-  const int QY = quad_edge + hy;
-  const int Q = QX * QY;
-  const unsigned key = xcd_key(blockIdx.x, gridDim.x);  // one block per key
-  const int nkeys = geo.ntx * geo.nty * geo.nr * geo.nc;
-  for (int bb = threadIdx.x; bb < nbins; bb += quad_block) {
-    const unsigned* tab = off_table + size_t(bb) * (nkeys + 1);
-    const unsigned s0 = tab[key], s1 = tab[key + 1];
-    seg_pref[bb] = s1 - s0;
-    seg_beg[bb] = s0;
-  }
-  __syncthreads();
-  const unsigned total = block_exclusive_scan(seg_pref, nbins, part);
-  if (total == 0) {
-    if (threadIdx.x == 0) halo_set[key] = 0u;
-    return;
-  }
-  if (threadIdx.x == 0) seg_pref[nbins] = total;
-
-  const int ntiles = geo.ntx * geo.nty;
-  const unsigned plane = key / ntiles;
-  const int t = int(key % ntiles);
-  const int x0 = (t % geo.ntx) * tile;
-  const int y0 = (t / geo.ntx) * tile;
-  const int gpol = int(plane % geo.nr);
-
-  for (int k = threadIdx.x; k < 4 * Q; k += quad_block)
-    regions[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (threadIdx.x < 10) qcnt2[threadIdx.x / 5][threadIdx.x % 5] = 0u;
-  // a single CF group is read once (the common case), not once per entry
-  const bool one_group = geo.ngroups == 1;
-  const GroupInfo group0 = groups[0];
-  __syncthreads();
-
-  const unsigned tid = threadIdx.x;
-  const int w = int(tid) / wave;
-  const int lane = int(tid) % wave;
-  float4* reg32 = regions + size_t(w) * Q;
-
-  auto locate = [&](unsigned q) {
-    int lo = 0, hi = nbins;  // seg_pref[lo] <= q < seg_pref[hi]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (seg_pref[mid] <= q) lo = mid; else hi = mid;
-    }
-    return unsigned(lo) * unsigned(block_cap) + seg_beg[lo] + (q - seg_pref[lo]);
-  };
-  // this thread's raw entry of the next round
-  Entry4<N> ne{};
-  unsigned nidx = 0;
-  auto load_round = [&](unsigned r0) {
-    if (tid < unsigned(RB) && r0 + tid < total) {
-      nidx = locate(r0 + tid);
-      ne = entries[nidx];
-    }
-  };
-  load_round(0);
-
-  // Lane layout of an entry's taps, step st of its steps: supports up to 8
-  // wide put tap (X, Y) = (lane & 7, lane >> 3 + 8 st) on this lane, so that
-  // the rows of one 16-lane LDS phase use distinct banks when the region row
-  // is 8 modulo 16 pixels; wider supports take the taps t = 64 st + lane
-  // contiguously, Y = t / sx from a float reciprocal (exact here: t < 4096
-  // and (t + 1/2) / sx stays 1/(2 sx) > 0.0079 away from an integer, far
-  // beyond the 4e-4 error of the product).
-  const int lane_x8 = lane & 7;
-  const int lane_y8 = lane >> 3;
-  auto tap_xy = [&](int sx, float rsx, int st, int& X, int& Y) {
-    if (ONE || sx <= 8) {
-      X = lane_x8;
-      Y = lane_y8 + st * (wave / 8);
-    } else {
-      const int tp = st * wave + lane;
-      Y = int((float(tp) + 0.5f) * rsx);
-      X = tp - Y * sx;
-    }
-  };
-  auto num_steps = [](int sx, int sy) {
-    return sx <= 8 ? (sy + wave / 8 - 1) / (wave / 8) : (sx * sy + wave - 1) / wave;
-  };
-
-  // an entry in flight: its prepared values and its first step's CF taps
-  struct Slot {
-    unsigned i, w0;
-    const float2* slice[N];
-    float2 c[N];
-    unsigned long long lanes;  // ONE: lanes holding a tap of the support
-  };
-  // Byte offset of this lane's first-step tap in a slice, for the support
-  // last seen (lanes outside the support read tap 0).  The first step's
-  // taps load unconditionally: a load under a condition would need its
-  // register cleared first, which waits for all loads in flight.
-  int tap_key = -1;
-  unsigned tap_off = 0;
-  unsigned long long tap_lanes = 0ull;
-  auto fetch = [&](unsigned i, Slot& s) {
-    const QuadRec<N>& p = list[i];
-    const unsigned w0v = p.w0;
-    unsigned slv[N];
-#pragma unroll
-    for (int v = 0; v < N; ++v) slv[v] = p.slice[v];
-    s.i = i;
-    s.w0 = uniform_u(w0v);
-    const int key_s = int((s.w0 >> 12) & 4095u);  // sx | sy << 6
-    if (key_s != __builtin_amdgcn_readfirstlane(tap_key)) {
-      tap_key = key_s;
-      const int sx = key_s & 63, sy = key_s >> 6;
-      int X, Y;
-      tap_xy(sx, __builtin_amdgcn_rcpf(float(sx)), 0, X, Y);
-      const bool ok = unsigned(X) < unsigned(sx) && unsigned(Y) < unsigned(sy);
-      tap_off = unsigned(ok ? Y * sx + X : 0) * unsigned(sizeof(float2));
-    }
-#pragma unroll
-    for (int v = 0; v < N; ++v) {
-      s.slice[v] = taps + uniform_u(slv[v]);
-      s.c[v] = *reinterpret_cast<const float2*>(
-        reinterpret_cast<const char*>(s.slice[v]) + tap_off);
-    }
-  };
-  auto add_tap = [&](int px, float h_r, float h_i, float l_r, float l_i) {
-    quad_add<N>(reg32, px, h_r, h_i, l_r, l_i);
-  };
-  const int lane_px = lane_y8 * QX + lane_x8;
-  // ONE: the raw record of an entry, read from LDS one pipeline stage before
-  // its fetch, so that the fetch's scalar reads find it there
-  struct RawRec {
-    unsigned w0;
-    unsigned sl[N];
-    float2 g[N], gc[N];
-  };
-  auto read_rec = [&](unsigned i, RawRec& r) {
-    const QuadRec<N>& p = list[i];
-    r.w0 = p.w0;
-#pragma unroll
-    for (int v = 0; v < N; ++v) {
-      r.sl[v] = p.slice[v];
-      r.g[v] = p.g[v];
-      r.gc[v] = p.gc[v];
-    }
-  };
-  auto fetch_raw = [&](const RawRec& r, Slot& s) {
-    s.w0 = uniform_u(r.w0);
-    const int key_s = int((s.w0 >> 12) & 4095u);  // sx | sy << 6
-    if (key_s != __builtin_amdgcn_readfirstlane(tap_key)) {
-      tap_key = key_s;
-      const int sx = key_s & 63, sy = key_s >> 6;
-      const bool ok = lane_x8 < sx && lane_y8 < sy;
-      tap_off = unsigned(ok ? lane_y8 * sx + lane_x8 : 0) * unsigned(sizeof(float2));
-      tap_lanes = __ballot(ok);
-    }
-    s.lanes = (s.w0 & quad_skip) ? 0ull : tap_lanes;
-#pragma unroll
-    for (int v = 0; v < N; ++v) {
-      s.slice[v] = taps + uniform_u(r.sl[v]);
-      s.c[v] = *reinterpret_cast<const float2*>(
-        reinterpret_cast<const char*>(s.slice[v]) + tap_off);
-    }
-  };
-  // an entry of supports up to 8 x 8 (ONE): a single step, no branch when
-  // the entry is live; `live` false (past the wave's entries) adds nothing
-  auto process_one = [&](Slot& s, const RawRec& r, bool live) {
-    const unsigned use = (s.w0 >> 24) & 15u;
-    if (__builtin_amdgcn_inverse_ballot_w64(live ? s.lanes : 0ull)) {
-      const int px = int(s.w0 & 4095u) + lane_px;
-      if constexpr (N == 1) {
-        const float2 c = s.c[0];
-        const float2 g = r.g[0], gc = r.gc[0];
-        const float pr = c.x * g.x - c.y * gc.x;
-        const float pi = c.x * g.y + c.y * gc.y;
-        add_tap(px, pr, pi, 0.0f, 0.0f);
-      } else {
-        double sr = 0.0, si = 0.0;
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          if (!((use >> v) & 1u)) continue;
-          const float2 c = s.c[v];
-          const float2 g = r.g[v], gc = r.gc[v];
-          sr += double(c.x * g.x - c.y * gc.x);
-          si += double(c.x * g.y + c.y * gc.y);
-        }
-        const float h_r = float(sr), h_i = float(si);
-        add_tap(px, h_r, h_i, float(sr - double(h_r)), float(si - double(h_i)));
-      }
-    }
-  };
-  auto process = [&](Slot& s) {
-    if ((s.w0 & quad_gradient) || !((s.w0 >> 24) & 15u)) return;
-    const int base = int(s.w0 & 4095u);
-    const int sx = int((s.w0 >> 12) & 63u);
-    const int sy = int((s.w0 >> 18) & 63u);
-    const unsigned use = (s.w0 >> 24) & 15u;
-    const float rsx = __builtin_amdgcn_rcpf(float(sx));
-    const int steps = num_steps(sx, sy);
-    for (int st = 0; st < steps; ++st) {
-      int X, Y;
-      tap_xy(sx, rsx, st, X, Y);
-      if (st > 0) {
-        const bool okn = unsigned(X) < unsigned(sx) && unsigned(Y) < unsigned(sy);
-        const int tp = okn ? Y * sx + X : 0;
-#pragma unroll
-        for (int v = 0; v < N; ++v) s.c[v] = s.slice[v][tp];
-      }
-      if (!(unsigned(X) < unsigned(sx) && unsigned(Y) < unsigned(sy))) continue;
-      // FP32 products c * g (conjugated c for w > 0), their FP64 sum over
-      // the polarizations
-      const QuadRec<N>& p = list[s.i];
-      if constexpr (N == 1) {
-        const float2 c = s.c[0];
-        const float2 g = p.g[0], gc = p.gc[0];
-        const float pr = c.x * g.x - c.y * gc.x;
-        const float pi = c.x * g.y + c.y * gc.y;
-        add_tap(base + Y * QX + X, pr, pi, 0.0f, 0.0f);
-      } else {
-        double sr = 0.0, si = 0.0;
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          if (!((use >> v) & 1u)) continue;
-          const float2 c = s.c[v];
-          const float2 g = p.g[v], gc = p.gc[v];
-          sr += double(c.x * g.x - c.y * gc.x);
-          si += double(c.x * g.y + c.y * gc.y);
-        }
-        const float h_r = float(sr), h_i = float(si);
-        add_tap(base + Y * QX + X, h_r, h_i, float(sr - double(h_r)), float(si - double(h_i)));
-      }
-    }
-  };
-  unsigned round = 0;
-  for (unsigned r0 = 0; r0 < total; r0 += RB, ++round) {
-    __builtin_amdgcn_s_setprio(0);
-    const unsigned rn = min(unsigned(RB), total - r0);
-    const bool mine = tid < rn;
-    const Entry4<N> e = ne;
-    const unsigned idx = nidx;
-    unsigned* qcnt = qcnt2[round & 1u];
-    unsigned* qgrad = qcnt + 4;
-    QuadRec<N> rec{};
-    int qd = -1;
-    if (mine) {
-      const unsigned pos = e.h.pos;
-      const int lx = int(pos & 63u);
-      const int ly = int((pos >> 6) & 63u);
-      const int fxi = int((pos >> 12) & 255u);
-      const int fyi = int((pos >> 20) & 255u);
-      const bool pos_w = pos & e4_pos_w;
-      const bool grad = pos & e4_gradient;
-      const int grp = int(e.h.gpk & 0xffffu);
-      const int cfcube = int(e.h.gpk >> 16);
-      const GroupInfo g = one_group ? group0 : groups[grp];
-      const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
-      const long long slice_taps = (long long)g.sx * g.sy;
-      const float imf = pos_w ? -1.0f : 1.0f;
-      unsigned use = 0;
-#pragma unroll
-      for (int v = 0; v < N; ++v) {
-        const int m = row[v];
-        const bool u = m >= 0 && m < g.nmueller;
-        use |= u ? 1u << v : 0u;
-        rec.slice[v] = unsigned(
-          g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (u ? m : 0)) * geo.nf + fxi) * geo.nf + fyi)
-            * slice_taps);
-        rec.g[v] = e.g[v];
-        rec.gc[v] = make_float2(imf * e.g[v].y, imf * e.g[v].x);
-      }
-      const int qx = lx >= quad_edge ? 1 : 0;
-      const int qy = ly >= quad_edge ? 1 : 0;
-      qd = qx | (qy << 1);
-      const unsigned base = unsigned((ly - qy * quad_edge) * QX + (lx - qx * quad_edge));
-      rec.w0 = base | (unsigned(g.sx) << 12) | (unsigned(g.sy) << 18) | (use << 24)
-        | (grad ? quad_gradient : 0u) | (pos_w ? quad_pos_w : 0u)
-        | ((grad || use == 0u) ? quad_skip : 0u);
-      if (grad) rec.gc[0].x = __uint_as_float(idx);
-    }
-    // counting sort by quadrant: one LDS atomic per wave and quadrant
-    if (__ballot(mine && (rec.w0 & quad_gradient)) != 0ull && lane == 0)
-      __hip_atomic_fetch_or(qgrad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    unsigned slot = 0;
-    const unsigned long long below = (1ull << lane) - 1ull;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const unsigned long long m = __ballot(qd == k);
-      unsigned wbase = 0;
-      if (lane == 0 && m != 0ull)
-        wbase = __hip_atomic_fetch_add(qcnt + k, unsigned(__popcll(m)), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-      wbase = __shfl(wbase, 0, wave);
-      if (qd == k) slot = wbase + unsigned(__popcll(m & below));
-    }
-    // (the list is free: every wave added the previous round's entries
-    // before its counts above)
-    __syncthreads();
-    const unsigned c0 = qcnt[0], c1 = qcnt[1], c2 = qcnt[2], c3 = qcnt[3];
-    const bool any_gradient = *qgrad != 0u;
-    // the other set was last read in the previous round, before its list
-    // barrier; cleared before this round's list barrier, it is ready for
-    // the next round's counts
-    if (tid < 5) qcnt2[(round + 1u) & 1u][tid] = 0u;
-    if (mine) {
-      const unsigned off = (qd > 0 ? c0 : 0u) + (qd > 1 ? c1 : 0u) + (qd > 2 ? c2 : 0u) + slot;
-      list[off] = rec;
-    }
-    __syncthreads();
-    // this wave's entries of the round, D in flight
-    // (wave-uniform: kept in scalar registers, so that the loops below index
-    // the list with scalar arithmetic)
-    const unsigned beg = uniform_u((w > 0 ? c0 : 0u) + (w > 1 ? c1 : 0u) + (w > 2 ? c2 : 0u));
-    const unsigned end = uniform_u(beg + (w == 0 ? c0 : w == 1 ? c1 : w == 2 ? c2 : c3));
-    // issue priority by the share of the round: the wave with the most
-    // entries sets the round's length, so it goes first on its SIMD (whose
-    // other waves belong to other workgroups)
-    {
-      const unsigned cnt[4] = {c0, c1, c2, c3};
-      const unsigned own = end - beg;
-      int rank = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) rank += (cnt[k] < own || (cnt[k] == own && k < w)) ? 1 : 0;
-      if (rank == 3)
-        __builtin_amdgcn_s_setprio(3);
-      else if (rank == 2)
-        __builtin_amdgcn_s_setprio(2);
-      else if (rank == 1)
-        __builtin_amdgcn_s_setprio(1);
-    }
-    constexpr int D = quad_depth<N>();
-    Slot sl[D];
-    if constexpr (ONE) {
-      // records read 2D entries ahead into 2D banks (entry beg + j in bank
-      // j mod 2D, where it stays until it is added), CF taps loaded D
-      // entries ahead; clamped reads past the end repeat the last entry and
-      // are not added
-      if (beg < end) {
-        RawRec rr[2 * D];
-#pragma unroll
-        for (int b = 0; b < 2 * D; ++b) read_rec(min(beg + b, end - 1), rr[b]);
-#pragma unroll
-        for (int k = 0; k < D; ++k) fetch_raw(rr[k], sl[k]);
-        // the next round's entries load while the first taps are in flight
-        load_round(r0 + RB);
-        unsigned i = beg;
-        // every entry added and every read in range: no checks
-        for (; i + 4 * D <= end; i += 2 * D) {
-#pragma unroll
-          for (int k = 0; k < 2 * D; ++k) {
-            process_one(sl[k % D], rr[k], true);
-            fetch_raw(rr[(k + D) % (2 * D)], sl[k % D]);
-            read_rec(i + k + 2 * D, rr[k]);
-          }
-        }
-        for (; i < end; i += 2 * D) {
-#pragma unroll
-          for (int k = 0; k < 2 * D; ++k) {
-            process_one(sl[k % D], rr[k], i + k < end);
-            fetch_raw(rr[(k + D) % (2 * D)], sl[k % D]);
-            read_rec(min(i + k + 2 * D, end - 1), rr[k]);
-          }
-        }
-      } else {
-        load_round(r0 + RB);
-      }
-    } else {
-      // the next round's entries load while this round's are added
-      load_round(r0 + RB);
-#pragma unroll
-      for (int k = 0; k < D; ++k)
-        if (beg + k < end) fetch(beg + k, sl[k]);
-      for (unsigned i = beg; i < end; i += D) {
-#pragma unroll
-        for (int k = 0; k < D; ++k) {
-          if (i + k < end) {
-            process(sl[k]);
-            if (i + k + D < end) fetch(i + k + D, sl[k]);
-          }
-        }
-      }
-    }
-    if (any_gradient)
-#pragma nounroll
-      for (unsigned i = beg; i < end; ++i)
-        if (uniform_u(list[i].w0) & quad_gradient)
-          quad_gradient_entry<N>(list[i], __float_as_uint(list[i].gc[0].x), geo, taps, entries,
-                                 entry_vis, recs, QX, reg32);
-  }
-  __builtin_amdgcn_s_setprio(0);
-  __syncthreads();
-
-  quad_flush_tile<quad_block, quad_flush>(regions, QX, QY, hx, hy, geo, plane, x0, y0,
-                                         static_cast<float2*>(grid),
-                                         halo + size_t(key) * halo_pixels(hx, hy));
-  if (threadIdx.x == 0) halo_set[key] = 1u;
-}
-
 // ---- gridding: quadrant keys, two waves per quadrant, FP32 block sums ----
 //
 // k_sub grids FP32-compensated tiles for supports of at most 8 x 8 pixels
@@ -2582,8 +1607,7 @@ __global__ __launch_bounds__(quad_block) void k_quad(
 // summed in FP32 over at most sub_fold entries of a region, those sums are
 // accumulated with compensation, and a wave keeps the pairs of half a
 // region in registers.  The flush sums the four quadrants' pairs over the
-// tile and halo (quad_flush_tile), as k_quad does, so k_halo folds the
-// halos unchanged.
+// tile and halo (quad_flush_tile), as k_tile4 does, and k_halo folds the halos.
 constexpr int sub_waves = 8;
 constexpr int sub_block = sub_waves * wave;
 constexpr int sub_bins_max = 256;  // bin blocks per pass (LDS segment tables)
@@ -2626,7 +1650,7 @@ __device__ __forceinline__ float2 screen_f32(double phi) {
 // one wave, one lane per tap, to the wave's FP32 region
 template <int N>
 __device__ __forceinline__ void sub_gradient_entry(
-  unsigned w0, const unsigned* slice, const float2* g, unsigned ri, unsigned pos,
+  unsigned w0, int nm, const unsigned* slice, const float2* g, unsigned ri, unsigned pos,
   const Geometry& geo, const float2* __restrict__ taps, const VisRec<N>* __restrict__ recs,
   int QX, float2* region) {
   const int lane = int(threadIdx.x % wave);
@@ -2651,7 +1675,7 @@ __device__ __forceinline__ void sub_gradient_entry(
   float h_r = 0.0f, h_i = 0.0f;
   for (int v = 0; v < N; ++v) {
     if (!((use >> v) & 1u)) continue;
-    float2 cc = taps[size_t(slice[v]) + size_t(tp)];
+    float2 cc = taps[size_t(slice[v]) + size_t(tp) * nm];
     cc.y *= imf;
     const float2 pr = cmul(cmul(cc, scr), g[v]);
     if constexpr (N == 1) {
@@ -2865,14 +1889,15 @@ void k_sub(
   // reads past taps_bytes return 0
   const __amdgpu_buffer_rsrc_t tap_rsrc = __builtin_amdgcn_make_buffer_rsrc(
     const_cast<float2*>(taps), 0, int(taps_bytes), 0x00020000);
-  // lanes holding a tap of a support (sx, sy), and their tap byte offset
-  auto support_lanes = [&](int sx, int sy, unsigned& off) {
+  // lanes holding a tap of a support (sx, sy) of a CF group with nm Mueller
+  // elements, and their tap byte offset
+  auto support_lanes = [&](int sx, int sy, int nm, unsigned& off) {
     const bool ok = lane_x < sx && lane_y < sy;
-    off = unsigned(ok ? lane_y * sx + lane_x : 0) * unsigned(sizeof(float2));
+    off = unsigned(ok ? (lane_y * sx + lane_x) * nm : 0) * unsigned(sizeof(float2));
     return ok;
   };
   unsigned tap_off = 0;
-  const bool uni_ok = UNI ? support_lanes(group0.sx, group0.sy, tap_off) : true;
+  const bool uni_ok = UNI ? support_lanes(group0.sx, group0.sy, group0.nmueller, tap_off) : true;
   int tap_key = -1;
   unsigned long long tap_lanes = 0ull;
 
@@ -2927,24 +1952,20 @@ void k_sub(
       const int grp = int(e.h.gpk & 0xffffu);
       const int cfcube = int(e.h.gpk >> 16);
       const GroupInfo g = one_group ? group0 : groups[grp];
-      const long long slice_taps = (long long)g.sx * g.sy;
       unsigned use = 0;
 #pragma unroll
       for (int v = 0; v < N; ++v) {
         const int m = pos_w ? row_m[v] : row_mc[v];
         const bool u = m >= 0 && m < g.nmueller;
         use |= u ? 1u << v : 0u;
-        p_sl[v] = unsigned(
-          g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (u ? m : 0)) * geo.nf + fxi) * geo.nf + fyi)
-            * slice_taps);
+        p_sl[v] = unsigned(slice_start(g, geo.nf, cfcube, u ? m : 0, fxi, fyi));
         if (u && !grad) {
           p_gx[v] = e.g[v].x;
           p_gy[v] = e.g[v].y;
         }
       }
       const unsigned base = unsigned((ly - qy * quad_edge) * QX + (lx - qx * quad_edge));
-      p_key = unsigned(g.sx) | (unsigned(g.sy) << 6);
+      p_key = unsigned(g.sx) | (unsigned(g.sy) << 6) | (unsigned(g.nmueller) << 12);
       normal = !grad && use != 0u;
       if constexpr (PK) {
         p_addr = (p_sl[0] << sub_pk_shift) | (normal ? base | (pos_w ? sub_pk_flip : 0u) : 0u);
@@ -2971,7 +1992,7 @@ void k_sub(
         const int key_s = __builtin_amdgcn_readlane(int(p_key), j);
         if (key_s != tap_key) {
           tap_key = key_s;
-          tap_lanes = __ballot(support_lanes(key_s & 63, key_s >> 6, tap_off));
+          tap_lanes = __ballot(support_lanes(key_s & 63, (key_s >> 6) & 63, key_s >> 12, tap_off));
         }
         ring_lanes[r] = tap_lanes;
       }
@@ -3085,7 +2106,8 @@ void k_sub(
         const unsigned w0 = (gbase * unsigned(QX) + ((gpos & 63u) - unsigned(qx * quad_edge)))
           | (unsigned(gg.sx) << 12) | (unsigned(gg.sy) << 18) | (guse << 24)
           | (gpos_w ? quad_pos_w : 0u);
-        sub_gradient_entry<N>(w0, sl, gv, entry_vis[ej], ge.h.pos, geo, taps, recs, QX, region);
+        sub_gradient_entry<N>(w0, gg.nmueller, sl, gv, entry_vis[ej], ge.h.pos, geo, taps, recs,
+                              QX, region);
       }
       if (last_half && ((rd + 1u) % unsigned(sub_fold_rounds) == 0u || rd + 1u == nrounds)) {
         __syncthreads();
@@ -3109,19 +2131,499 @@ void k_sub(
   if (tid == 0) halo_set[tkey] = 1u;
 }
 
+// ---- gridding: pixel patches in registers -----------------------------------
+//
+// The gridder of several polarizations, and of supports beyond the other
+// tile kernels'.  One workgroup owns a tile of all grid rows of one cube and
+// keeps its pixels' FP64 sums in registers, so a tap costs no LDS or global
+// atomic: a lane is a (pixel, grid row), a wave holds 2 x 2 patches of 64 / P
+// pixels (P = lanes per pixel: 1, 2 or 4 rows), the workgroup 2 x 2 waves.
+//
+//   k_patch_prep  one thread per visibility: skip rule, weights, the record's
+//                 prepared form (support corner, CF slice, pre-phased values)
+//                 and the counts of the tiles it touches
+//   (scan)        the tiles' list offsets
+//   k_patch_list  one thread per visibility: its index into the lists of the
+//                 tiles it touches
+//   k_patch       one workgroup per tile: 256 list entries at a time staged in
+//                 LDS; each wave tests them 64 at a time against its own
+//                 pixels, and adds those that overlap one by one
+//
+// A slice holds its Mueller elements side by side, so the 64 lanes of a patch
+// read whole runs of it (4 x 128 bytes for 16 elements), each CF byte once
+// per record whatever the tile borders cut; lanes outside the support read
+// past the buffer resource's end, which fetches nothing.  Small patches keep
+// the lanes busy: a support S wide fills (S / (S + 3))^2 of the 4 x 4 patches
+// it touches, 72% at S = 17.
+//
+// Bound: the CF reads from HBM for large CFs (64 groups of supports 9-65, 16
+// elements, 500,000 records: 104 GB in 19.9 ms, 5.2 TB/s, against 27.7 ms for
+// clipped tiles in LDS, one workgroup per plane and element-major slices;
+// supports 17-129, 150,000 records: 119 GB in 20.3 ms, before 38.4 ms), the
+// vector ALU for CFs that stay in the last-level cache (supports 9-25, 200,000
+// records: 1.17 ms, before 4.31 ms by LDS compare-and-swap).
+
+// lanes per pixel for nr grid rows
+constexpr int patch_lanes(int nr) { return nr <= 1 ? 1 : nr == 2 ? 2 : 4; }
+// pixels of a patch, of a wave's 2 x 2 patches and of a tile along x and y
+__host__ __device__ constexpr int patch_w(int P) { return P == 4 ? 4 : 8; }
+__host__ __device__ constexpr int patch_h(int P) { return P == 1 ? 8 : 4; }
+__host__ __device__ constexpr int patch_tile_x(int P) { return 4 * patch_w(P); }
+__host__ __device__ constexpr int patch_tile_y(int P) { return 4 * patch_h(P); }
+constexpr int patch_block = 4 * wave;
+
+// a record prepared for its tiles; sxy = 0: not gridded
+template <int N>
+struct __align__(16) PatchRec {
+  int gx, gy;               // support corner
+  unsigned long long base;  // first value of its CF slice (element 0, tap 0)
+  unsigned sxy;             // sx | sy << 16
+  unsigned fl;              // flags | fxi << 8 | fyi << 16
+  unsigned nm;              // Mueller elements of its CF group
+  unsigned cube;            // grid cube
+  float2 g[N];
+};
+static_assert(sizeof(PatchRec<1>) == 48 && sizeof(PatchRec<4>) == 64, "PatchRec layout");
+
+// Weights: each wave sums its records' weights per (grid cube, row), and
+// for grids of at most count_planes_lds planes adds the sums into the
+// workgroup's LDS, which adds into the grid weights once at its end (the
+// workgroups stride over the records, so a few thousand global atomics per
+// plane instead of one per wave).
+template <int N>
+__global__ __launch_bounds__(block) void k_patch_prep(
+  const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
+  const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
+  Mueller mu, int update_weights, int gvis_ready, int adjoint,
+  const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
+  int ptx, int pty, int tw, int th, PatchRec<N>* __restrict__ out,
+  unsigned* __restrict__ hist, double* __restrict__ weights,
+  unsigned long long* __restrict__ invalid) {
+
+  __shared__ double wblk[count_planes_lds];
+  const int nplanes = geo.nr * geo.nc;
+  const bool lds_w = update_weights && nplanes <= count_planes_lds;
+  if (lds_w)
+    for (int k = threadIdx.x; k < nplanes; k += blockDim.x) wblk[k] = 0.0;
+  __syncthreads();
+
+  const size_t stride = size_t(gridDim.x) * blockDim.x;
+  const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  // every thread runs the same number of iterations (the wave reductions
+  // below need all lanes)
+  const size_t iters = (n + stride - 1) / stride;
+  for (size_t it = 0; it < iters; ++it) {
+    const size_t i = i0 + it * stride;
+    bool counted = false;
+    unsigned gcube = 0;
+    double tw4[4] = {0.0, 0.0, 0.0, 0.0};
+    if (i < n) {
+      const VisRec<N>& r = recs[i];
+      const unsigned grp = r.cf_index[1];
+      const unsigned cfcube = r.cf_index[0];
+      gcube = r.grid_cube;
+      bool valid = grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc);
+      if (valid) valid = cfcube < unsigned(groups[grp].ncube);
+      PatchRec<N> e;
+      e.sxy = 0u;
+      if (!valid) {
+        atomicAdd(invalid, 1ull);
+      } else {
+        const GroupInfo g = groups[grp];
+        const Coord c = vis_coord(r, geo, g);
+        const bool pos_w = r.uvw[2] > 0;
+        if (c.inside) {
+          const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
+          bool any = false;
+          counted = update_weights != 0;
+#pragma unroll
+          for (int gp = 0; gp < 4; ++gp) {
+            if (gp >= geo.nr) continue;
+            double t = 0.0;
+#pragma unroll
+            for (int v = 0; v < N; ++v) {
+              const int m = pos_w ? mu.M[gp][v] : mu.Mc[gp][v];
+              any |= m >= 0;
+              if (update_weights && m >= 0 && m < g.nmueller) {
+                const double2 sw = wsum[g.wsum_offset
+                                        + ((long long)(cfcube * g.nmueller + m) * geo.nf + fxi)
+                                          * geo.nf + fyi];
+                t += hypot(sw.x, sw.y) * double(r.w[v]);
+              }
+            }
+            tw4[gp] = t;
+          }
+          if (any) {
+            const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
+            e.gx = c.gx;
+            e.gy = c.gy;
+            e.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi);
+            e.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
+            e.fl = unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
+              | (unsigned(fxi) << 8) | (unsigned(fyi) << 16);
+            e.nm = unsigned(g.nmueller);
+            e.cube = gcube;
+            if (gvis_ready) {
+              for (int v = 0; v < N; ++v) e.g[v] = gvis_in[i * N + v];
+            } else {
+              const double2 phasor = cphase(r.phase);
+              if (!adjoint) {
+                for (int v = 0; v < N; ++v) e.g[v] = prephase(r.vis[v], phasor, r.w[v]);
+              } else {
+                double2 W[N];
+                degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
+                for (int v = 0; v < N; ++v) {
+                  double2 d = W[v];
+                  if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
+                  d.y = -d.y;
+                  e.g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
+                }
+              }
+            }
+            const int tx0 = c.gx / tw, tx1 = (c.gx + g.sx - 1) / tw;
+            const int ty0 = c.gy / th, ty1 = (c.gy + g.sy - 1) / th;
+            for (int ty = ty0; ty <= ty1; ++ty)
+              for (int tx = tx0; tx <= tx1; ++tx)
+                atomicAdd(hist + (size_t(gcube) * pty + ty) * ptx + tx, 1u);
+          }
+        }
+      }
+      if (e.sxy) out[i] = e; else out[i].sxy = 0u;
+    }
+    if (update_weights) {
+      unsigned long long active = __ballot(counted);
+      const int lane = threadIdx.x % wave;
+      while (active) {
+        const int leader = __ffsll((long long)active) - 1;
+        const unsigned cube = __shfl(gcube, leader, wave);
+        const bool mine = counted && gcube == cube;
+        active &= ~__ballot(mine);
+#pragma unroll
+        for (int gp = 0; gp < 4; ++gp) {
+          if (gp >= geo.nr) continue;
+          const double sw = wave_sum(mine ? tw4[gp] : 0.0);
+          if (lane == leader) {
+            const size_t k = size_t(cube) * geo.nr + gp;
+            if (lds_w)
+              __hip_atomic_fetch_add(wblk + k, sw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            else
+              atomicAdd(weights + k, sw);
+          }
+        }
+      }
+    }
+  }
+  if (lds_w) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < nplanes; k += blockDim.x)
+      if (wblk[k] != 0.0) atomicAdd(weights + k, wblk[k]);
+  }
+}
+
+// hist counts down: an entry's place in its tile's list is what is left
+template <int N>
+__global__ __launch_bounds__(block) void k_patch_list(
+  size_t n, int ptx, int pty, int tw, int th, const PatchRec<N>* __restrict__ prs,
+  unsigned* __restrict__ hist, const unsigned* __restrict__ offsets,
+  unsigned* __restrict__ list) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const unsigned sxy = prs[i].sxy;
+  if (!sxy) return;
+  const int gx = prs[i].gx, gy = prs[i].gy;
+  const unsigned gcube = prs[i].cube;
+  const int tx0 = gx / tw, tx1 = (gx + int(sxy & 0xffffu) - 1) / tw;
+  const int ty0 = gy / th, ty1 = (gy + int(sxy >> 16) - 1) / th;
+  for (int ty = ty0; ty <= ty1; ++ty)
+    for (int tx = tx0; tx <= tx1; ++tx) {
+      const size_t key = (size_t(gcube) * pty + ty) * ptx + tx;
+      list[offsets[key] + atomicSub(hist + key, 1u) - 1u] = unsigned(i);
+    }
+}
+
+__global__ __launch_bounds__(block) void k_zero(unsigned* __restrict__ p, size_t n) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// exp(i ph): ph less the nearest multiple k of pi / 2 (pi / 2 as a 53-bit
+// head, whose difference is exact, and its tail), then the Taylor series of
+// sine and cosine up to r^15 and r^16, |r| <= pi / 4 (remainders below
+// 1e-16).  As cphase, whose library call would cost the tap loops 40 registers
+// and with them a quarter of their waves.
+__device__ __forceinline__ double2 cphase_taylor(double ph) {
+  const double k = rint(ph * 0.63661977236758134);  // 2 / pi
+  double r = __builtin_fma(-k, 1.5707963267948966, ph);
+  r = __builtin_fma(-k, 6.123233995736766e-17, r);
+  const double z = r * r;
+  double s = -1.0 / 1307674368000.0;
+  s = __builtin_fma(s, z, 1.0 / 6227020800.0);
+  s = __builtin_fma(s, z, -1.0 / 39916800.0);
+  s = __builtin_fma(s, z, 1.0 / 362880.0);
+  s = __builtin_fma(s, z, -1.0 / 5040.0);
+  s = __builtin_fma(s, z, 1.0 / 120.0);
+  s = __builtin_fma(s, z, -1.0 / 6.0);
+  s = __builtin_fma(s * z, r, r);
+  double c = 1.0 / 20922789888000.0;
+  c = __builtin_fma(c, z, -1.0 / 87178291200.0);
+  c = __builtin_fma(c, z, 1.0 / 479001600.0);
+  c = __builtin_fma(c, z, -1.0 / 3628800.0);
+  c = __builtin_fma(c, z, 1.0 / 40320.0);
+  c = __builtin_fma(c, z, -1.0 / 720.0);
+  c = __builtin_fma(c, z, 1.0 / 24.0);
+  c = __builtin_fma(c, z, -0.5);
+  c = __builtin_fma(c, z, 1.0);
+  const int q = int(k - 4.0 * rint(0.25 * k)) & 3;  // quadrant (0 .. 3)
+  const double re = q & 1 ? s : c, im = q & 1 ? c : s;
+  return make_double2(q == 1 || q == 2 ? -re : re, q >= 2 ? -im : im);
+}
+
+// what a row takes of a slice (patch_kind)
+constexpr int patch_any = 0;   // any of the N elements, one load each
+constexpr int patch_full = 1;  // N neighbouring elements, N even, at 16-byte
+                               // alignment: two elements a load
+constexpr int patch_one = 2;   // at most one element
+
+template <int N, int P, int KIND>
+__global__ __launch_bounds__(patch_block) __attribute__((amdgpu_waves_per_eu(5)))
+void k_patch(
+  Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int ptx, int pty,
+  const unsigned* __restrict__ offsets, const unsigned* __restrict__ list,
+  const PatchRec<N>* __restrict__ prs, const VisRec<N>* __restrict__ recs,
+  void* __restrict__ grid) {
+
+  constexpr int PW = patch_w(P), PH = patch_h(P);
+  constexpr int L = KIND == patch_one ? 1 : N;  // elements a lane loads per tap
+  __shared__ PatchRec<N> st[patch_block];
+  __shared__ unsigned st_i[patch_block];
+
+  const unsigned key = blockIdx.x;
+  const unsigned beg = offsets[key];
+  const unsigned cnt = offsets[key + 1] - beg;
+  if (cnt == 0) return;
+  const int tx = int(key % unsigned(ptx));
+  const int tq = int(key / unsigned(ptx));
+  const int ty = tq % pty;
+  const int cube = tq / pty;
+
+  const int w = uniform(int(threadIdx.x) / wave);
+  const int lane = threadIdx.x % wave;
+  const int row = lane % P;
+  const int px = (lane / P) % PW;
+  const int py = (lane / P) / PW;
+  const int bx = tx * patch_tile_x(P) + (w & 1) * 2 * PW;  // the wave's pixels
+  const int by = ty * patch_tile_y(P) + (w >> 1) * 2 * PH;
+
+  // this lane's Mueller row for w <= 0: byte offsets of its elements within a
+  // tap (~0u: none) and, for patch_one, the polarization they multiply; in
+  // eo_x, vs_x what changes of them (xor) for w > 0
+  unsigned eo[L], eo_x[L];
+  unsigned vs = 0u, vs_x = 0u;
+#pragma unroll
+  for (int k = 0; k < L; ++k) {
+    eo[k] = ~0u;
+    eo_x[k] = ~0u;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (r >= geo.nr || r != row) continue;
+#pragma unroll
+    for (int v = 0; v < N; ++v) {
+      const int m0 = mu.Mc[r][v], m1 = mu.M[r][v];
+      constexpr unsigned es = unsigned(sizeof(float2));
+      const int k = KIND == patch_one ? 0 : v;
+      if (m0 >= 0) {
+        eo[k] = unsigned(m0) * es;
+        if (KIND == patch_one) vs = unsigned(v);
+      }
+      if (m1 >= 0) {
+        eo_x[k] = unsigned(m1) * es;
+        if (KIND == patch_one) vs_x = unsigned(v);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < L; ++k) eo_x[k] ^= eo[k];
+  vs_x ^= vs;
+
+  double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
+
+  for (unsigned b0 = 0; b0 < cnt; b0 += patch_block) {
+    const unsigned m = min(unsigned(patch_block), cnt - b0);
+    __syncthreads();
+    if (threadIdx.x < m) {
+      const unsigned i = list[beg + b0 + threadIdx.x];
+      st_i[threadIdx.x] = i;
+      st[threadIdx.x] = prs[i];
+    }
+    __syncthreads();
+    for (unsigned k0 = 0; k0 < m; k0 += wave) {
+      // lane j: does entry k0 + j touch the wave's pixels
+      const unsigned je = min(k0 + unsigned(lane), m - 1u);
+      const int hgx = st[je].gx, hgy = st[je].gy;
+      const unsigned long long hbase = st[je].base;
+      const unsigned hsxy = st[je].sxy, hfl = st[je].fl, hnm = st[je].nm;
+      const bool hit = k0 + unsigned(lane) < m && hgx < bx + 2 * PW
+        && hgx + int(hsxy & 0xffffu) > bx && hgy < by + 2 * PH && hgy + int(hsxy >> 16) > by;
+      unsigned long long todo = __ballot(hit);
+      while (todo) {
+        const int j = __builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        const int gx = __builtin_amdgcn_readlane(hgx, j);
+        const int gy = __builtin_amdgcn_readlane(hgy, j);
+        const unsigned blo = unsigned(__builtin_amdgcn_readlane(int(unsigned(hbase)), j));
+        const unsigned bhi = unsigned(__builtin_amdgcn_readlane(int(hbase >> 32), j));
+        const unsigned sxy = unsigned(__builtin_amdgcn_readlane(int(hsxy), j));
+        const unsigned fl = unsigned(__builtin_amdgcn_readlane(int(hfl), j));
+        const unsigned nm = unsigned(__builtin_amdgcn_readlane(int(hnm), j));
+        const PatchRec<N>& e = st[k0 + unsigned(j)];
+        const int sx = int(sxy & 0xffffu), sy = int(sxy >> 16);
+        const bool pos_w = fl & flag_pos_w;
+        const unsigned pm = pos_w ? ~0u : 0u;
+        // the slice from the first support row within the wave's pixels on,
+        // at most 2 PH rows: offsets of 32 bits for any support
+        const int y0 = max(by - gy, 0);
+        const int rows = min(sy - y0, 2 * PH);
+        const unsigned tap_bytes = nm * unsigned(sizeof(float2));
+        const unsigned row_bytes = unsigned(sx) * tap_bytes;
+        const float2* first = taps + ((unsigned long long)blo | ((unsigned long long)bhi << 32))
+          + (unsigned long long)unsigned(y0) * (unsigned(sx) * nm);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float2*>(first), 0, int(unsigned(rows) * row_bytes), 0x00020000);
+        const int X = bx + px - gx;
+        const int Y = by + py - gy;
+        const unsigned off0 = unsigned(Y - y0) * row_bytes + unsigned(X) * tap_bytes;
+        float2 c[4][L];
+        bool in[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int dx = (k & 1) * PW, dy = (k >> 1) * PH;
+          in[k] = unsigned(X + dx) < unsigned(sx) && unsigned(Y + dy) < unsigned(sy);
+          const unsigned off = off0 + unsigned(dy) * row_bytes + unsigned(dx) * tap_bytes;
+          if constexpr (KIND == patch_full) {
+            const unsigned o = in[k] ? off + (eo[0] ^ (eo_x[0] & pm)) : ~0u;
+#pragma unroll
+            for (int v = 0; v < N; v += 2) {
+              const v4i_t q = __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc, int(o), v * int(sizeof(float2)), 0);
+              c[k][v] = make_float2(__int_as_float(q.x), __int_as_float(q.y));
+              c[k][v + 1] = make_float2(__int_as_float(q.z), __int_as_float(q.w));
+            }
+          } else {
+#pragma unroll
+            for (int v = 0; v < L; ++v) {
+              const unsigned ev = eo[v] ^ (eo_x[v] & pm);
+              const v2i_t q = __builtin_amdgcn_raw_buffer_load_b64(
+                rsrc, int(in[k] && ev < tap_bytes ? off + ev : ~0u), 0, 0);
+              c[k][v] = make_float2(__int_as_float(q.x), __int_as_float(q.y));
+            }
+          }
+        }
+        // conj(c) g for w > 0: c.y g.y and c.y g.x enter with the sign
+        // flipped, which rounds as conjugating c does
+        float imf = pos_w ? -1.0f : 1.0f;
+        if (fl & flag_gradient) {
+          // the taps times the phase screen instead
+          const unsigned i = st_i[k0 + unsigned(j)];
+          const double gxr = recs[i].grad[0], gyr = recs[i].grad[1];
+          const int fxi = int((fl >> 8) & 255u), fyi = int((fl >> 16) & 255u);
+          const double phi0x = -gxr * ((sx / 2) * geo.os - (fxi - geo.F));
+          const double phi0y = -gyr * ((sy / 2) * geo.os - (fyi - geo.F));
+          const double dphix = gxr * geo.os;
+          const double dphiy = gyr * geo.os;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int Xk = X + (k & 1) * PW, Yk = Y + (k >> 1) * PH;
+            const float2 scr =
+              narrow(cphase_taylor((phi0x + Xk * dphix) + (phi0y + Yk * dphiy)));
+#pragma unroll
+            for (int v = 0; v < L; ++v)
+              c[k][v] = cmul(make_float2(c[k][v].x, imf * c[k][v].y), scr);
+            // one patch at a time: the four together would hold the registers
+            // of a wave
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          imf = 1.0f;
+        }
+        float2 g[L], gs[L];
+#pragma unroll
+        for (int v = 0; v < L; ++v) {
+          g[v] = KIND == patch_one ? e.g[vs ^ (vs_x & pm)] : e.g[v];
+          gs[v] = make_float2(imf * g[v].x, imf * g[v].y);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (!in[k]) continue;
+          double sr = 0.0, si = 0.0;
+#pragma unroll
+          for (int v = 0; v < L; ++v) {
+            const float2 cc = c[k][v];
+            const float pr = cc.x * g[v].x - cc.y * gs[v].y;
+            const float pi = cc.x * g[v].y + cc.y * gs[v].x;
+            if constexpr (KIND == patch_full) {
+              sr += double(pr);
+              si += double(pi);
+            } else {
+              const bool use = (eo[v] ^ (eo_x[v] & pm)) < tap_bytes;
+              sr += use ? double(pr) : 0.0;
+              si += use ? double(pi) : 0.0;
+            }
+          }
+          ar[k] += sr;
+          ai[k] += si;
+        }
+      }
+    }
+  }
+
+  // the tile's only writer: a plain read-modify-write of each pixel
+  if (row >= geo.nr) return;
+  const size_t plane = (size_t(cube) * geo.nr + row) * size_t(geo.ny) * geo.nx;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int x = bx + px + (k & 1) * PW, y = by + py + (k >> 1) * PH;
+    if (x >= geo.nx || y >= geo.ny) continue;
+    const size_t gi = plane + size_t(y) * geo.nx + x;
+    if (mode == 0) {
+      double2* gp = static_cast<double2*>(grid) + gi;
+      double2 v = *gp;
+      v.x += ar[k];
+      v.y += ai[k];
+      *gp = v;
+    } else {
+      // one rounding of grid value + FP64 tile sum
+      float2* gp = static_cast<float2*>(grid) + gi;
+      const float2 v = *gp;
+      *gp = make_float2(float(double(v.x) + ar[k]), float(double(v.y) + ai[k]));
+    }
+  }
+}
+
+
 // ---- degridding --------------------------------------------------------
 
-// The wave-per-record degridder's record order: key = the record's CF slice
-// (group, CF cube, fine offsets: grp * stride + (cube * nf + fxi) * nf +
-// fyi), kmax for records it skips (no CF, outside the grid).  Sorted by key,
-// the records that read the same 16 Mueller slices run together and find
-// them in L2 (a record's taps of all Mueller elements are read once per
-// slice set and batch rather than once per record).
+// The slice-ordered degridder, for several polarizations, large supports and
+// large grids: k_degrid_keys prepares the records, a radix sort orders them
+// by CF slice, k_degrid sums c' x model over their supports and
+// k_degrid_finish makes predictions of the sums.
+
+// a record prepared for k_degrid; sxy = 0: not degridded
+struct __align__(16) DegridRec {
+  unsigned long long base;  // first value of its CF slice (element 0, tap 0)
+  long long corner;         // model index of its support corner, grid row 0
+  unsigned sxy;             // sx | sy << 16
+  unsigned fl;              // flags | fxi << 8 | fyi << 16
+  unsigned nm;              // Mueller elements of its CF group
+  unsigned pad;
+};
+
+// key = the record's (grid cube, group, CF cube, fine offsets), kmax for
+// records that are skipped (no CF, outside the grid)
 template <int N>
 __global__ void k_degrid_keys(
   size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const VisRec<N>* __restrict__ recs, unsigned stride, unsigned kmax,
-  unsigned* __restrict__ keys, unsigned* __restrict__ idx) {
+  const VisRec<N>* __restrict__ recs, unsigned stride, unsigned cube_stride, unsigned kmax,
+  unsigned* __restrict__ keys, unsigned* __restrict__ idx, DegridRec* __restrict__ out) {
   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
   const VisRec<N>& r = recs[i];
@@ -3129,251 +2631,300 @@ __global__ void k_degrid_keys(
   const unsigned cfcube = r.cf_index[0];
   const unsigned gcube = r.grid_cube;
   unsigned key = kmax;
+  DegridRec d{};
   if (grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc)) {
     const GroupInfo g = groups[grp];
     if (cfcube < unsigned(g.ncube)) {
       const Coord c = vis_coord(r, geo, g);
-      if (c.inside)
-        key = grp * stride
-          + (cfcube * unsigned(geo.nf) + unsigned(c.fx + geo.F)) * unsigned(geo.nf)
-          + unsigned(c.fy + geo.F);
+      if (c.inside) {
+        const unsigned fxi = unsigned(c.fx + geo.F), fyi = unsigned(c.fy + geo.F);
+        const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
+        key = gcube * cube_stride + grp * stride
+          + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
+        d.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi));
+        d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
+        d.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
+        d.fl = unsigned((r.uvw[2] > 0 ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
+          | (fxi << 8) | (fyi << 16);
+        d.nm = unsigned(g.nmueller);
+      }
     }
   }
-  keys[i] = key;
-  idx[i] = unsigned(i);
+  if (keys) {
+    keys[i] = key;
+    idx[i] = unsigned(i);
+  }
+  out[i] = d;
 }
 
-// order: the records' processing order (k_degrid_keys, sorted), or null
-template <int N>
-__global__ __launch_bounds__(block) void k_degrid(
-  size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const float2* __restrict__ taps, const double2* __restrict__ wsum, Mueller mu,
-  const double2* __restrict__ model, int do_grid, VisRec<N>* __restrict__ recs,
-  float2* __restrict__ gvis, double2* __restrict__ pred64,
-  const unsigned* __restrict__ order) {
+// sums val[0, V) of the lanes that differ in bits P .. 32 of their number.
+// Each step halves the values a lane holds (it keeps one half, and adds its
+// partner's values of that half) while their number is even: V - 1 adds
+// instead of V log2(64 / P).  Value `at` + i is in val[i] afterwards, i below
+// the returned number.
+template <int V, int MASK, int P>
+__device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
+  if constexpr (MASK < P) {
+    return V;
+  } else if constexpr (V % 2 == 0) {
+    constexpr int H = V / 2;
+    const bool up = lane & MASK;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const double keep = up ? val[i + H] : val[i];
+      const double send = up ? val[i] : val[i + H];
+      val[i] = keep + __shfl_xor(send, MASK, wave);
+    }
+    at += up ? H : 0;
+    return reduce_lanes<H, MASK / 2, P>(val, lane, at);
+  } else {
+#pragma unroll
+    for (int i = 0; i < V; ++i) val[i] += __shfl_xor(val[i], MASK, wave);
+    return reduce_lanes<V, MASK / 2, P>(val, lane, at);
+  }
+}
 
-  const size_t wi = blockIdx.x * (size_t)(block / wave) + threadIdx.x / wave;
+// records a wave takes: their sums (N complex values a lane, one where a row
+// uses one element) within 64 registers
+template <int N, int KIND>
+constexpr int degrid_recs() { return KIND == patch_one || N <= 2 ? 8 : 4; }
+
+// One wave takes R records in a row of the order; those of one slice share
+// every CF value it loads (per tap of 4 x 4 elements a record reads 64 bytes
+// of model and 128 of CF: the CF reads are the larger part until four share
+// them).  A lane is a (tap, grid row), 64 / P taps a step; the Mueller
+// elements of a slice lie side by side, so a step's CF loads cover whole
+// lines.  The sums over the support go to acc (record x polarization).
+// order null: the records as they come.  same_rows: M and Mc are equal, so
+// that records of both signs of w share CF values (the model's imaginary part
+// takes the sign: sum conj(c) m = conj(sum c conj(m))).  patch_one: no two
+// rows use one polarization; acc of one that no row uses is not written.
+// Bound: the model gathers (64 bytes per tap from anywhere in the model: 4.4
+// TB/s with their line ends).  500,000 records of supports 9-65 and 16 elements
+// 14.1 ms (26.8 ms one record a wave), 150,000 of 17-129 14.7 ms (27.1), 1e6 of
+// 9-33 and one element a row 6.2 ms (7.3).  Three waves per SIMD: at four the
+// sums spill (15.9 ms the first).
+template <int N, int P, int KIND>
+__global__ __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(3)))
+void k_degrid(
+  size_t n, Geometry geo, const float2* __restrict__ taps, Mueller mu, int same_rows,
+  const double2* __restrict__ model, const DegridRec* __restrict__ drs,
+  const VisRec<N>* __restrict__ recs, const unsigned* __restrict__ order,
+  double* __restrict__ acc) {
+
+  constexpr int R = degrid_recs<N, KIND>();
+  constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
+  constexpr int TPS = wave / P;                 // taps a step
+
+  const int w = uniform(int(threadIdx.x) / wave);
   const int lane = threadIdx.x % wave;
-  if (wi >= n) return;
-  const size_t i = order ? size_t(order[wi]) : wi;
-  VisRec<N>& r = recs[i];
-  const unsigned grp = r.cf_index[1];
-  const unsigned cfcube = r.cf_index[0];
-  const unsigned gcube = r.grid_cube;
-  if (!(grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc))) return;
-  if (!(cfcube < unsigned(groups[grp].ncube))) return;
-  const GroupInfo g = groups[grp];
-  const Coord c = vis_coord(r, geo, g);
-  if (!c.inside) return;  // values left unchanged (src/hpg_core.hpp:1136-1169)
-  const bool pos_w = r.uvw[2] > 0;
-  const double2 phasor = cphase(r.phase);
-  const int fxi = c.fx + geo.F;
-  const int fyi = c.fy + geo.F;
+  const size_t p0 = (blockIdx.x * (size_t)(block / wave) + w) * R;
+  if (p0 >= n) return;
+  const int row = lane % P;
+  const int q = lane / P;
 
-  float2 pred[N];
-  double2 pred_d[N];
-  for (int v = 0; v < N; ++v) {
-    pred[v] = make_float2(0.0f, 0.0f);
-    pred_d[v] = make_double2(0.0, 0.0);
+  // lane r < R: record r of the wave
+  DegridRec d{};
+  unsigned rec_i = 0;
+  if (lane < R && p0 + lane < n) {
+    rec_i = order ? order[p0 + lane] : unsigned(p0 + lane);
+    d = drs[rec_i];
   }
-  if (model) {
-    const float imf = pos_w ? 1.0f : -1.0f;
-    const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-    const double phi0x = -r.grad[0] * ((g.sx / 2) * geo.os - c.fx);
-    const double phi0y = -r.grad[1] * ((g.sy / 2) * geo.os - c.fy);
-    const double dphix = r.grad[0] * geo.os;
-    const double dphiy = r.grad[1] * geo.os;
-    const int ntap = g.sx * g.sy;
-    const unsigned mg = magic(unsigned(g.sx));
-    const long long slice_taps = ntap;
-    double2 a[N];
-    for (int v = 0; v < N; ++v) a[v] = make_double2(0.0, 0.0);
-    for (int gpol = 0; gpol < geo.nr; ++gpol) {
-      const int* row = pos_w ? mu.Mc[gpol] : mu.M[gpol];
-      const float2* slice[N];
-      bool use[N];
-      for (int v = 0; v < N; ++v) {
-        const int m = row[v];
-        use[v] = m >= 0 && m < g.nmueller;
-        slice[v] = taps + g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (use[v] ? m : 0)) * geo.nf + fxi)
-               * geo.nf + fyi) * slice_taps;
+  const unsigned long long live = __ballot(d.sxy != 0u);
+
+  // this lane's Mueller row for w <= 0 (element indexes, -1: none; for
+  // patch_one in [0] only, with its polarization) and what changes of it
+  // (xor) for w > 0
+  int el[L], el_x[L];
+  int vs = 0, vs_x = 0;
+#pragma unroll
+  for (int k = 0; k < L; ++k) el[k] = el_x[k] = -1;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (r >= geo.nr || r != row) continue;
+#pragma unroll
+    for (int v = 0; v < N; ++v) {
+      // degridding uses the other Mueller matrix than gridding
+      // (src/hpg_core.hpp:598-600)
+      const int m0 = mu.M[r][v], m1 = mu.Mc[r][v];
+      const int k = KIND == patch_one ? 0 : v;
+      if (m0 >= 0) {
+        el[k] = m0;
+        vs = v;
       }
-      const double2* mplane =
-        model + (size_t(gcube) * geo.nr + gpol) * size_t(geo.ny) * geo.nx;
-      for (int q = lane; q < ntap; q += wave) {
-        const int Y = int(div_magic(unsigned(q), unsigned(g.sx), mg));
-        const int X = q - Y * g.sx;
-        double2 mv = mplane[size_t(c.gy + Y) * geo.nx + (c.gx + X)];
-        if (grad) {
-          const double phX = phi0x + X * dphix;
-          const double phY = phi0y + Y * dphiy;
-          mv = cmul(mv, cphase(-phX - phY));
-        }
-        for (int v = 0; v < N; ++v) {
-          if (!use[v]) continue;
-          float2 cf = slice[v][q];
-          cf.y *= imf;
-          const double2 p = cmul(cf, mv);
-          a[v].x += p.x;
-          a[v].y += p.y;
-        }
+      if (m1 >= 0) {
+        el_x[k] = m1;
+        vs_x = v;
       }
     }
-    double2 W[N];
-    degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-    const double2 conj_phasor = make_double2(phasor.x, -phasor.y);
-    for (int v = 0; v < N; ++v) {
-      const double2 s = make_double2(wave_sum(a[v].x), wave_sum(a[v].y));
-      const double2 d = (W[v].x != 0.0 || W[v].y != 0.0) ? W[v] : make_double2(1.0, 0.0);
-      pred_d[v] = cmul(kdiv(s, d), conj_phasor);
-      pred[v] = narrow(pred_d[v]);
+  }
+#pragma unroll
+  for (int k = 0; k < L; ++k) el_x[k] ^= el[k];
+  vs_x ^= vs;
+  const long long row_off = (long long)(row < geo.nr ? row : 0) * geo.ny * geo.nx;
+
+  auto lane_u64 = [&](unsigned long long v, int j) {
+    return (unsigned long long)unsigned(__builtin_amdgcn_readlane(int(unsigned(v)), j))
+      | ((unsigned long long)unsigned(__builtin_amdgcn_readlane(int(v >> 32), j)) << 32);
+  };
+  auto lane_u32 = [&](unsigned v, int j) {
+    return unsigned(__builtin_amdgcn_readlane(int(v), j));
+  };
+
+  // the sums of RR records from record r on, which share one slice and
+  // Mueller row; GRAD: one record with a phase gradient
+  auto run = [&](auto rr_c, auto grad_c, int r) {
+    constexpr int RR = decltype(rr_c)::value;
+    constexpr bool GRAD = decltype(grad_c)::value;
+    const unsigned sxy = lane_u32(d.sxy, r);
+    const int sx = int(sxy & 0xffffu);
+    const unsigned ntap = unsigned(sx) * (sxy >> 16);
+    const unsigned nm = lane_u32(d.nm, r);
+    const int pm = (lane_u32(d.fl, r) & flag_pos_w) ? -1 : 0;
+    const float2* cf = taps + lane_u64(d.base, r) + size_t(q) * nm;  // this lane's tap
+    unsigned eo[L];                                                  // its elements
+    bool use[L];
+#pragma unroll
+    for (int v = 0; v < L; ++v) {
+      const int m = el[v] ^ (el_x[v] & pm);
+      use[v] = m >= 0 && m < int(nm);
+      eo[v] = unsigned(use[v] ? m : 0);
     }
-  }
-  if (pred64) {
-    // forward operator of the differentiable form: FP64 predictions
-    if (lane == 0)
-      for (int v = 0; v < N; ++v) pred64[i * N + v] = pred_d[v];
-    return;
-  }
-  if (lane == 0) {
-    for (int v = 0; v < N; ++v) {
-      if (do_grid) {
-        float2 val = r.vis[v];
-        val.x -= pred[v].x;
-        val.y -= pred[v].y;
-        r.vis[v] = val;
-        gvis[i * N + v] = prephase(val, phasor, r.w[v]);
+    const double2* mp[RR];
+    unsigned flip[RR];  // w <= 0: the imaginary parts' sign
+#pragma unroll
+    for (int k = 0; k < RR; ++k) {
+      mp[k] = model + (lane_u64((unsigned long long)d.corner, r + k) + row_off);
+      flip[k] = (lane_u32(d.fl, r + k) & flag_pos_w) ? 0u : 0x80000000u;
+    }
+    double val[RR * L * 2];
+#pragma unroll
+    for (int k = 0; k < RR * L * 2; ++k) val[k] = 0.0;
+    // the tap's (X, Y), from a float reciprocal and one correction either way
+    // (exact: q < 64), and the model offset
+    int Y = int(float(q) * __builtin_amdgcn_rcpf(float(sx)));
+    int X = q - Y * sx;
+    if (X < 0) {
+      X += sx;
+      --Y;
+    }
+    if (X >= sx) {
+      X -= sx;
+      ++Y;
+    }
+    long long off = (long long)Y * geo.nx + X;
+    const int dY = sx > TPS ? 0 : TPS / sx;
+    const int dX = TPS - dY * sx;
+    const long long doff = (long long)dY * geo.nx + dX;
+    const long long wrap = (long long)geo.nx - sx;
+    double gp0 = 0.0, gdx = 0.0, gdy = 0.0, gp1 = 0.0;
+    if constexpr (GRAD) {
+      const unsigned fl = lane_u32(d.fl, r);
+      const VisRec<N>& rc = recs[lane_u32(rec_i, r)];
+      const double gxr = rc.grad[0], gyr = rc.grad[1];
+      gp0 = -gxr * ((sx / 2) * geo.os - (int((fl >> 8) & 255u) - geo.F));
+      gp1 = -gyr * ((int(sxy >> 16) / 2) * geo.os - (int((fl >> 16) & 255u) - geo.F));
+      gdx = gxr * geo.os;
+      gdy = gyr * geo.os;
+    }
+    auto step = [&]() {
+      float2 c[L];
+      double2 m[RR];
+      if constexpr (KIND == patch_full) {
+#pragma unroll
+        for (int v = 0; v < N; v += 2) {
+          const float4 t = *reinterpret_cast<const float4*>(cf + eo[0] + v);
+          c[v] = make_float2(t.x, t.y);
+          c[v + 1] = make_float2(t.z, t.w);
+        }
       } else {
-        r.vis[v] = pred[v];
+#pragma unroll
+        for (int v = 0; v < L; ++v) c[v] = cf[eo[v]];
       }
-    }
-  }
-}
-
-// One lane per visibility (supports up to degrid_lane_taps taps): the lane
-// walks the footprint in chunks of halo_chunk taps, issuing the chunk's
-// model-pixel and CF-tap loads together, and accumulates in FP64 registers;
-// no cross-lane reduction.  Same per-tap arithmetic as k_degrid.
-constexpr int degrid_lane_taps = 1024;
-
-template <int N>
-__global__ __launch_bounds__(block) void k_degrid_lane(
-  size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const float2* __restrict__ taps, const double2* __restrict__ wsum, Mueller mu,
-  const double2* __restrict__ model, int do_grid, const VisRec<N>* recs_in,
-  VisRec<N>* recs, float2* __restrict__ gvis, double2* __restrict__ pred64) {
-  // recs_in and recs may be the same records: each lane reads its record's
-  // fields before writing them back
-
-  const size_t i = blockIdx.x * (size_t)block + threadIdx.x;
-  if (i >= n) return;
-  const VisRec<N>& r = recs_in[i];
-  const unsigned grp = r.cf_index[1];
-  const unsigned cfcube = r.cf_index[0];
-  const unsigned gcube = r.grid_cube;
-  if (!(grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc))) return;
-  const GroupInfo g = groups[grp];
-  if (!(cfcube < unsigned(g.ncube))) return;
-  const Coord c = vis_coord(r, geo, g);
-  if (!c.inside) return;  // values left unchanged (src/hpg_core.hpp:1136-1169)
-  const bool pos_w = r.uvw[2] > 0;
-  const double2 phasor = cphase(r.phase);
-  const int fxi = c.fx + geo.F;
-  const int fyi = c.fy + geo.F;
-
-  float2 pred[N];
-  double2 pred_d[N];
-  for (int v = 0; v < N; ++v) {
-    pred[v] = make_float2(0.0f, 0.0f);
-    pred_d[v] = make_double2(0.0, 0.0);
-  }
-  if (model) {
-    const float imf = pos_w ? 1.0f : -1.0f;
-    const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-    const double phi0x = -r.grad[0] * ((g.sx / 2) * geo.os - c.fx);
-    const double phi0y = -r.grad[1] * ((g.sy / 2) * geo.os - c.fy);
-    const double dphix = r.grad[0] * geo.os;
-    const double dphiy = r.grad[1] * geo.os;
-    const int sx = g.sx, sy = g.sy;
-    const long long slice_taps = (long long)sx * sy;
-    double2 a[N];
-    for (int v = 0; v < N; ++v) a[v] = make_double2(0.0, 0.0);
-    for (int gpol = 0; gpol < geo.nr; ++gpol) {
-      const int* row = pos_w ? mu.Mc[gpol] : mu.M[gpol];
-      const float2* slice[N];
-      bool use[N];
-      bool any = false;
-      for (int v = 0; v < N; ++v) {
-        const int m = row[v];
-        use[v] = m >= 0 && m < g.nmueller;
-        any |= use[v];
-        slice[v] = taps + g.tap_offset
-          + (((long long)(cfcube * g.nmueller + (use[v] ? m : 0)) * geo.nf + fxi) * geo.nf
-             + fyi) * slice_taps;
+      cf += size_t(TPS) * nm;
+#pragma unroll
+      for (int k = 0; k < RR; ++k) m[k] = mp[k][off];
+      if constexpr (GRAD) m[0] = cmul(m[0], cphase_taylor(-(gp0 + X * gdx) - (gp1 + Y * gdy)));
+      X += dX;
+      Y += dY;
+      off += doff;
+      if (X >= sx) {
+        X -= sx;
+        ++Y;
+        off += wrap;
       }
-      if (!any) continue;
-      const double2* mplane =
-        model + (size_t(gcube) * geo.nr + gpol) * size_t(geo.ny) * geo.nx;
-      for (int Y = 0; Y < sy; ++Y) {
-        const double2* mrow = mplane + size_t(c.gy + Y) * geo.nx + c.gx;
-        for (int X0 = 0; X0 < sx; X0 += halo_chunk) {
-          double2 mv[halo_chunk];
-          float2 cf[N][halo_chunk];
 #pragma unroll
-          for (int k = 0; k < halo_chunk; ++k) {
-            const bool in = X0 + k < sx;
-            mv[k] = in ? mrow[X0 + k] : make_double2(0.0, 0.0);
+      for (int k = 0; k < RR; ++k) {
+        const double mx = m[k].x;
+        const double my = __hiloint2double(
+          int(unsigned(__double2hiint(m[k].y)) ^ flip[k]), __double2loint(m[k].y));
 #pragma unroll
-            for (int v = 0; v < N; ++v)
-              cf[v][k] = (in && use[v]) ? slice[v][Y * sx + X0 + k] : make_float2(0.0f, 0.0f);
-          }
-#pragma unroll
-          for (int k = 0; k < halo_chunk; ++k) {
-            if (X0 + k >= sx) break;
-            const int X = X0 + k;
-            double2 m = mv[k];
-            if (grad) {
-              const double phX = phi0x + X * dphix;
-              const double phY = phi0y + Y * dphiy;
-              m = cmul(m, cphase(-phX - phY));
-            }
-#pragma unroll
-            for (int v = 0; v < N; ++v) {
-              if (!use[v]) continue;
-              float2 cc = cf[v][k];
-              cc.y *= imf;
-              const double2 p = cmul(cc, m);
-              a[v].x += p.x;
-              a[v].y += p.y;
-            }
-          }
+        for (int v = 0; v < L; ++v) {
+          if (KIND == patch_any && !use[v]) continue;
+          const double cx = double(c[v].x), cy = double(c[v].y);
+          double& a = val[(k * L + v) * 2];
+          double& b = val[(k * L + v) * 2 + 1];
+          a = __builtin_fma(cx, mx, a);
+          a = __builtin_fma(-cy, my, a);
+          b = __builtin_fma(cx, my, b);
+          b = __builtin_fma(cy, mx, b);
         }
       }
+    };
+    const unsigned full = ntap / TPS;
+#pragma unroll 1
+    for (unsigned s = 0; s < full; ++s) step();
+    if (full * TPS + unsigned(q) < ntap) step();
+    // the other sign's imaginary parts, then the sums over the taps (and,
+    // but for patch_one, the rows)
+#pragma unroll
+    for (int k = 0; k < RR; ++k)
+#pragma unroll
+      for (int v = 0; v < L; ++v) {
+        double& b = val[(k * L + v) * 2 + 1];
+        b = flip[k] ? -b : b;
+        if (KIND != patch_one && !use[v]) val[(k * L + v) * 2] = b = 0.0;
+      }
+    int at = 0;
+    const int left =
+      reduce_lanes<RR * L * 2, wave / 2, KIND == patch_one ? P : 1>(val, lane, at);
+#pragma unroll
+    for (int i = 0; i < RR * L * 2; ++i) {
+      if (i >= left) continue;
+      const int a = at + i;
+      const int k = a / (L * 2);
+      const size_t ri = unsigned(__shfl(int(rec_i), r + k, wave));
+      const int v = KIND == patch_one ? vs ^ (vs_x & pm) : (a / 2) % L;
+      if (KIND != patch_one || use[0]) acc[(ri * N + v) * 2 + (a & 1)] = val[i];
     }
-    double2 W[N];
-    degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-    const double2 conj_phasor = make_double2(phasor.x, -phasor.y);
-    for (int v = 0; v < N; ++v) {
-      const double2 d = (W[v].x != 0.0 || W[v].y != 0.0) ? W[v] : make_double2(1.0, 0.0);
-      pred_d[v] = cmul(kdiv(a[v], d), conj_phasor);
-      pred[v] = narrow(pred_d[v]);
+  };
+
+  for (int r = 0; r < R;) {
+    if (!((live >> r) & 1ull)) {
+      ++r;
+      continue;
     }
-  }
-  if (pred64) {
-    for (int v = 0; v < N; ++v) pred64[i * N + v] = pred_d[v];
-    return;
-  }
-  VisRec<N>& o = recs[i];
-  for (int v = 0; v < N; ++v) {
-    if (do_grid) {
-      float2 val = r.vis[v];
-      val.x -= pred[v].x;
-      val.y -= pred[v].y;
-      o.vis[v] = val;
-      gvis[i * N + v] = prephase(val, phasor, r.w[v]);
+    const unsigned long long base = lane_u64(d.base, r);
+    const unsigned fl = lane_u32(d.fl, r);
+    const unsigned long long same = __ballot(
+      d.sxy != 0u && !(d.fl & flag_gradient) && d.base == base
+      && (same_rows || !((d.fl ^ fl) & flag_pos_w))) >> r;
+    const int len = __builtin_ctzll(~same);  // records in a row, 0 for a gradient
+    if (len >= R) {
+      run(std::integral_constant<int, R>{}, std::false_type{}, r);
+      r += R;
+    } else if (R > 4 && len >= 4) {
+      run(std::integral_constant<int, R / 2>{}, std::false_type{}, r);
+      r += R / 2;
+    } else if (len >= 2) {
+      run(std::integral_constant<int, 2>{}, std::false_type{}, r);
+      r += 2;
+    } else if (len == 1) {
+      run(std::integral_constant<int, 1>{}, std::false_type{}, r);
+      r += 1;
     } else {
-      o.vis[v] = pred[v];
+      run(std::integral_constant<int, 1>{}, std::true_type{}, r);
+      r += 1;
     }
   }
 }
@@ -3396,7 +2947,8 @@ __device__ __noinline__ double2 degrid_screen(double2 m, double ph) {
 // cphase out of line, for the same reason
 __device__ __noinline__ double2 cphase_call(double ph) { return cphase(ph); }
 
-template <int N>
+// UNIT: every CF group has one Mueller element
+template <int N, bool UNIT>
 __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 1))) void k_degrid4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
@@ -3487,20 +3039,17 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
     const int grp = int(eh.gpk & 0xffffu);
     const int cfcube = int(eh.gpk >> 16);
     const GroupInfo g = groups[grp];
-    const int sx = g.sx, sy = g.sy;
+    const int sx = g.sx, sy = g.sy, nm = UNIT ? 1 : g.nmueller;
     // degridding uses the other Mueller matrix and the opposite conjugation
     // of gridding (src/hpg_core.hpp:598-600)
     const int* row = pos_w ? mu.Mc[gpol] : mu.M[gpol];
     const float imf = pos_w ? 1.0f : -1.0f;
     const float2* slice[N];
     bool use[N];
-    const long long slice_taps = (long long)sx * sy;
     for (int v = 0; v < N; ++v) {
       const int m = row[v];
       use[v] = m >= 0 && m < g.nmueller;
-      slice[v] = taps + g.tap_offset
-        + (((long long)(cfcube * g.nmueller + (use[v] ? m : 0)) * geo.nf + fxi) * geo.nf
-           + fyi) * slice_taps;
+      slice[v] = taps + slice_start<UNIT>(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
     }
     double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
     if (grad) {
@@ -3556,7 +3105,7 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
 #pragma unroll
           for (int v = 0; v < N; ++v) {
             float2 tv = make_float2(0.0f, 0.0f);
-            if (ok[k]) tv = slice[v][t0 + k];
+            if (ok[k]) tv = slice[v][(t0 + k) * nm];
             c[k][v] = tv;
           }
         }
@@ -3606,8 +3155,9 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
   }
 }
 
-// predictions from the per-record sums of k_degrid4 (the end of degrid_vis
-// and of the degridding branch of VisibilityGridder::kernel,
+// predictions from the per-record sums of k_degrid and k_degrid4 (acc null: no
+// model, which predicts zero) (the end of degrid_vis and of the degridding
+// branch of VisibilityGridder::kernel,
 // src/hpg_core.hpp:643-682, 1136-1169), one thread per record
 template <int N>
 __global__ __launch_bounds__(block) void k_degrid_finish(
@@ -3636,8 +3186,15 @@ __global__ __launch_bounds__(block) void k_degrid_finish(
   float2 pred[N];
   double2 pred_d[N];
   for (int v = 0; v < N; ++v) {
+    // a polarization that no row uses has no sum
+    bool any = false;
+    for (int gpol = 0; gpol < geo.nr; ++gpol) {
+      const int m = pos_w ? mu.Mc[gpol][v] : mu.M[gpol][v];
+      any |= m >= 0 && m < g.nmueller;
+    }
     const double2 d = (W[v].x != 0.0 || W[v].y != 0.0) ? W[v] : make_double2(1.0, 0.0);
-    pred_d[v] = cmul(kdiv(acc[i * N + v], d), conj_phasor);
+    const double2 a = any && acc ? acc[i * N + v] : make_double2(0.0, 0.0);
+    pred_d[v] = acc ? cmul(kdiv(a, d), conj_phasor) : a;
     pred[v] = narrow(pred_d[v]);
   }
   if (pred64) {
@@ -3767,20 +3324,36 @@ hipError_t launch_cf_relayout(
   const long long total =
     (long long)gi.ncube * gi.nmueller * nf * nf * gi.sx * gi.sy;
   if (total == 0) return hipSuccess;
-  hipLaunchKernelGGL(
-    k_cf_relayout, dim3(blocks_for(size_t(total))), dim3(block), 0, s, staging,
-    ext[0], ext[1], gi, os, F, nf, taps, total);
+  // support columns whose window fits LDS
+  auto lds = [&](int xc) {
+    return (size_t(xc - 1) * os + nf) * gi.nmueller * sizeof(float2);
+  };
+  int xc = std::min(gi.sx, 8);
+  while (xc > 1 && lds(xc) > relayout_lds) --xc;
+  const int nxc = (gi.sx + xc - 1) / xc;
+  const unsigned long long blocks = (unsigned long long)nxc * gi.sy * nf * gi.ncube;
+  if (lds(xc) <= relayout_lds && blocks <= 0x7fffffffull)
+    hipLaunchKernelGGL(
+      k_cf_relayout_lds, dim3(unsigned(blocks)), dim3(relayout_block), lds(xc), s, staging,
+      ext[0], ext[1], gi, os, F, nf, taps, xc, nxc);
+  else
+    hipLaunchKernelGGL(
+      k_cf_relayout, dim3(blocks_for(size_t(total))), dim3(block), 0, s, staging,
+      ext[0], ext[1], gi, os, F, nf, taps, total);
   return hipGetLastError();
 }
 
 hipError_t launch_cf_wsum(
   hipStream_t s, const GroupInfo& gi, int nf, const float2* taps,
   double2* wsum) {
-  const long long ns = (long long)gi.ncube * gi.nmueller * nf * nf;
+  const int nm = gi.nmueller;
+  const int per = nm > 0 && nm <= wave && (nm & (nm - 1)) == 0 ? nm : 0;
+  const long long ns = (long long)gi.ncube * (per ? 1 : nm) * nf * nf;
   if (ns == 0) return hipSuccess;
+  const long long values = (long long)gi.sx * gi.sy * (per ? per : 1);
+  const int threads = values <= 1024 ? wave : values <= 8192 ? 256 : wsum_block;
   hipLaunchKernelGGL(
-    k_cf_wsum, dim3(blocks_for(size_t(ns), wsum_block / wave)), dim3(wsum_block), 0, s, gi,
-    nf, taps, wsum, ns);
+    k_cf_wsum, dim3(unsigned(ns)), dim3(threads), 0, s, gi, nf, taps, wsum, per);
   return hipGetLastError();
 }
 
@@ -3812,31 +3385,13 @@ hipError_t launch_count(
   const Mueller& mu, bool update_weights, bool do_grid, CallBuffers& cb,
   double* weights, bool halo_entries, bool quad_keys) {
   if (n == 0) return hipSuccess;
-#define HPGX_COUNT(NP, H)                                                      \
-  hipLaunchKernelGGL(                                                          \
-    (k_count<NP, H>), dim3(std::min(unsigned(blocks_for(n)), count_blocks_max)), \
-    dim3(block), 0, s,                                                         \
-    static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
-    int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count,     \
-    int(halo_entries && quad_keys))
-  if (halo_entries) {
-    switch (npol) {
-    case 1: HPGX_COUNT(1, true); break;
-    case 2: HPGX_COUNT(2, true); break;
-    case 3: HPGX_COUNT(3, true); break;
-    case 4: HPGX_COUNT(4, true); break;
-    default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (npol) {
-    case 1: HPGX_COUNT(1, false); break;
-    case 2: HPGX_COUNT(2, false); break;
-    case 3: HPGX_COUNT(3, false); break;
-    case 4: HPGX_COUNT(4, false); break;
-    default: return hipErrorInvalidValue;
-    }
-  }
-#undef HPGX_COUNT
+  if (npol != 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(
+    k_count<1>, dim3(std::min(unsigned(blocks_for(n)), count_blocks_max)),
+    dim3(block), 0, s,
+    static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
+    int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count,
+    int(halo_entries && quad_keys));
   return hipGetLastError();
 }
 
@@ -3875,63 +3430,12 @@ hipError_t launch_emit(
   CallBuffers& cb, bool halo_entries, bool quad_keys) {
   if (n == 0) return hipSuccess;
   const int adj = src == GvisSource::Adjoint;
-#define HPGX_EMIT(NP, H)                                                       \
-  hipLaunchKernelGGL(                                                          \
-    (k_emit<NP, H>), dim3(blocks_for(n)), dim3(block), 0, s,                   \
-    static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
-    int(gvis_ready), adj, cb.gvis, residuals, cb.cursor, cb.stream_entries,    \
-    cb.entry_vis, int(halo_entries && quad_keys))
-  if (halo_entries) {
-    switch (npol) {
-    case 1: HPGX_EMIT(1, true); break;
-    case 2: HPGX_EMIT(2, true); break;
-    case 3: HPGX_EMIT(3, true); break;
-    case 4: HPGX_EMIT(4, true); break;
-    default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (npol) {
-    case 1: HPGX_EMIT(1, false); break;
-    case 2: HPGX_EMIT(2, false); break;
-    case 3: HPGX_EMIT(3, false); break;
-    case 4: HPGX_EMIT(4, false); break;
-    default: return hipErrorInvalidValue;
-    }
-  }
-#undef HPGX_EMIT
-  return hipGetLastError();
-}
-
-hipError_t launch_tile_stream(
-  hipStream_t s, int npol, int mode, size_t nkeys, const Geometry& geo,
-  const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, void* grid) {
-  if (nkeys == 0) return hipSuccess;
-  const bool unr = size_t(cf.max_sx) * size_t(cf.max_sy) >= size_t(unroll_min_taps);
-#define HPGX_TILE2(NP, MD)                                                     \
-  hipLaunchKernelGGL(                                                          \
-    unr ? (k_tile2<NP, MD, true>) : (k_tile2<NP, MD, false>),                  \
-    dim3(unsigned(nkeys)), dim3(block), 0, s, geo,                             \
-    cf.groups, cf.taps, mu, cb.offsets,                                        \
-    static_cast<const Entry<NP>*>(cb.stream_entries), cb.entry_vis,            \
-    static_cast<const VisRec<NP>*>(cb.vis), grid)
-  if (mode == 0) {
-    switch (npol) {
-    case 1: HPGX_TILE2(1, 0); break;
-    case 2: HPGX_TILE2(2, 0); break;
-    case 3: HPGX_TILE2(3, 0); break;
-    case 4: HPGX_TILE2(4, 0); break;
-    default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (npol) {
-    case 1: HPGX_TILE2(1, 1); break;
-    case 2: HPGX_TILE2(2, 1); break;
-    case 3: HPGX_TILE2(3, 1); break;
-    case 4: HPGX_TILE2(4, 1); break;
-    default: return hipErrorInvalidValue;
-    }
-  }
-#undef HPGX_TILE2
+  if (npol != 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(
+    k_emit<1>, dim3(blocks_for(n)), dim3(block), 0, s,
+    static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
+    int(gvis_ready), adj, cb.gvis, residuals, cb.cursor, cb.stream_entries,
+    cb.entry_vis, int(halo_entries && quad_keys));
   return hipGetLastError();
 }
 
@@ -3952,31 +3456,13 @@ hipError_t launch_bin(
   const int adj = src == GvisSource::Adjoint;
   const int dg = degrid_pass;
   const unsigned nb = unsigned(bin_blocks_for(n));
-#define HPGX_BIN(NP, H)                                                        \
-  hipLaunchKernelGGL(                                                          \
-    (k_bin<NP, H>), dim3(nb), dim3(bin_threads), 0, s,                         \
-    static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
-    int(update_weights), int(gvis_ready), adj, dg, cb.gvis, residuals,         \
-    cb.off_table, cb.stream_entries, cb.entry_vis, block_cap, weights,         \
-    cb.invalid_count, static_cast<VisRec<NP>*>(copy_records), int(quad_keys))
-  if (halo_entries) {
-    switch (npol) {
-    case 1: HPGX_BIN(1, true); break;
-    case 2: HPGX_BIN(2, true); break;
-    case 3: HPGX_BIN(3, true); break;
-    case 4: HPGX_BIN(4, true); break;
-    default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (npol) {
-    case 1: HPGX_BIN(1, false); break;
-    case 2: HPGX_BIN(2, false); break;
-    case 3: HPGX_BIN(3, false); break;
-    case 4: HPGX_BIN(4, false); break;
-    default: return hipErrorInvalidValue;
-    }
-  }
-#undef HPGX_BIN
+  if (npol != 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(
+    k_bin<1>, dim3(nb), dim3(bin_threads), 0, s,
+    static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
+    int(update_weights), int(gvis_ready), adj, dg, cb.gvis, residuals,
+    cb.off_table, cb.stream_entries, cb.entry_vis, block_cap, weights,
+    cb.invalid_count, static_cast<VisRec<1>*>(copy_records), int(quad_keys));
   return hipGetLastError();
 }
 
@@ -4008,24 +3494,6 @@ hipError_t launch_halo(
       k_halo<float2>, dim3(blocks_for(count)), dim3(block), 0, s, geo, hx, hy,
       cb.halo, cb.halo_set, nkeys, static_cast<float2*>(grid));
   return hipGetLastError();
-}
-
-size_t quad_lds_bytes(int hx, int hy, int npol) {
-  const size_t regions = 4 * size_t(quad_edge + hx) * (quad_edge + hy) * sizeof(float4);
-  size_t rec = 0, rb = 0;
-  switch (npol) {
-  case 1: rec = sizeof(QuadRec<1>); rb = quad_round<1>(); break;
-  case 2: rec = sizeof(QuadRec<2>); rb = quad_round<2>(); break;
-  case 3: rec = sizeof(QuadRec<3>); rb = quad_round<3>(); break;
-  default: rec = sizeof(QuadRec<4>); rb = quad_round<4>(); break;
-  }
-  return regions + rb * rec
-    + sizeof(unsigned) * (2 * size_t(quad_bins_max) + 1 + quad_block / wave + 1 + 5);
-}
-int quad_bins_limit() { return quad_bins_max; }
-bool quad_supported(int hx, int hy, int npol) {
-  return hx >= 0 && hy >= 0 && hx < tile && hy < tile && quad_lds_bytes(hx, hy, npol) <= 65536
-    && (tile + hx) * (tile + hy) <= quad_flush * quad_block;
 }
 
 size_t sub_lds_bytes(int hx, int hy) {
@@ -4061,7 +3529,6 @@ hipError_t launch_tile_sub(
     static_cast<const Entry4<NP>*>(cb.stream_entries), cb.entry_vis,           \
     static_cast<const VisRec<NP>*>(cb.vis), hx, hy, static_cast<float2*>(grid),\
     cb.halo, cb.halo_set)
-#define HPGX_SUB_N(NP, PX, PK) HPGX_SUB_G(NP, PX, PK, false)
 #define HPGX_SUB_1(NP, PX, PK)                                                 \
   do {                                                                         \
     if (global_bins) HPGX_SUB_G(1, PX, PK, true);                              \
@@ -4078,18 +3545,10 @@ hipError_t launch_tile_sub(
   // by tap index below sub_pk_taps
   static_assert(9 * wave < int(sub_pk_flip), "region pixel in the packed word");
   const bool pk = npol == 1 && taps_bytes / sizeof(float2) < sub_pk_taps;
-  switch (npol) {
-  case 1:
-    if (pk) HPGX_SUB_PX(HPGX_SUB_1, 1, true) else HPGX_SUB_PX(HPGX_SUB_1, 1, false)
-    break;
-  case 2: HPGX_SUB_PX(HPGX_SUB_N, 2, false); break;
-  case 3: HPGX_SUB_PX(HPGX_SUB_N, 3, false); break;
-  case 4: HPGX_SUB_PX(HPGX_SUB_N, 4, false); break;
-  default: return hipErrorInvalidValue;
-  }
+  if (npol != 1) return hipErrorInvalidValue;
+  if (pk) HPGX_SUB_PX(HPGX_SUB_1, 1, true) else HPGX_SUB_PX(HPGX_SUB_1, 1, false)
 #undef HPGX_SUB_PX
 #undef HPGX_SUB_1
-#undef HPGX_SUB_N
 #undef HPGX_SUB_G
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -4099,102 +3558,151 @@ hipError_t launch_tile_sub(
 hipError_t launch_tile_halo(
   hipStream_t s, int npol, int mode, int acc, size_t n, size_t nkeys, const Geometry& geo,
   const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
-  int hx, int hy, void* grid, bool global_bins, bool quad) {
+  int hx, int hy, void* grid, bool global_bins) {
   if (nkeys == 0 || n == 0) return hipSuccess;
   if (hx < 0 || hy < 0 || hx >= tile || hy >= tile) return hipErrorInvalidValue;
   // global bins: one contiguous range per key, read as a single bin block
   // whose offset-table row is the scanned offsets
   const int nb = global_bins ? 1 : bin_blocks_for(n);
   const unsigned* table = global_bins ? cb.offsets : cb.off_table;
-  if (quad) {
-    if (nb > quad_bins_max || !quad_supported(hx, hy, npol) || mode != 1 || acc != acc_f32_cas)
-      return hipErrorInvalidValue;
-    const size_t dyn = 4 * size_t(quad_edge + hx) * (quad_edge + hy) * sizeof(float4);
-    // every support within one lane step (hx, hy = largest support - 1)
-    const bool one = hx < 8 && hy < 8;
-#define HPGX_QUAD(NP)                                                          \
-  hipLaunchKernelGGL(                                                          \
-    one ? (k_quad<NP, true>) : (k_quad<NP, false>),                            \
-    dim3(unsigned(nkeys)), dim3(quad_block), dyn, s,                           \
-    geo, cf.groups, cf.taps, mu, table, nb, block_cap,                         \
-    static_cast<const Entry4<NP>*>(cb.stream_entries), cb.entry_vis,           \
-    static_cast<const VisRec<NP>*>(cb.vis), hx, hy, grid, cb.halo, cb.halo_set)
-    switch (npol) {
-    case 1: HPGX_QUAD(1); break;
-    case 2: HPGX_QUAD(2); break;
-    case 3: HPGX_QUAD(3); break;
-    case 4: HPGX_QUAD(4); break;
-    default: return hipErrorInvalidValue;
-    }
-#undef HPGX_QUAD
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_halo(s, mode, nkeys, geo, cb, hx, hy, grid);
-  }
   const size_t lds = halo_lds_bytes(hx, hy, nb);
   if (lds > 65536) return hipErrorInvalidValue;
-#define HPGX_TILE4(NP, MD, AC)                                                 \
+#define HPGX_TILE4(MD, AC)                                                     \
   hipLaunchKernelGGL(                                                          \
-    (k_tile4<NP, MD, AC>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s,    \
+    cf.max_nm == 1 ? (k_tile4<1, MD, AC, true>) : (k_tile4<1, MD, AC, false>), \
+    dim3(unsigned(nkeys)), dim3(halo_block), lds, s,                           \
     geo, cf.groups, cf.taps, mu, table, nb, block_cap,                         \
-    static_cast<const Entry4<NP>*>(cb.stream_entries), cb.entry_vis,           \
-    static_cast<const VisRec<NP>*>(cb.vis), hx, hy, grid, cb.halo, cb.halo_set)
-#define HPGX_TILE4_NP(MD, AC)                                                  \
-  switch (npol) {                                                              \
-  case 1: HPGX_TILE4(1, MD, AC); break;                                        \
-  case 2: HPGX_TILE4(2, MD, AC); break;                                        \
-  case 3: HPGX_TILE4(3, MD, AC); break;                                        \
-  case 4: HPGX_TILE4(4, MD, AC); break;                                        \
-  default: return hipErrorInvalidValue;                                        \
-  }
-  if (mode == 0) {
-    HPGX_TILE4_NP(0, acc_f64)
-  } else if (acc == 0) {
-    HPGX_TILE4_NP(1, acc_f64)
-  } else {
-    HPGX_TILE4_NP(1, acc_f32_cas)
-  }
-#undef HPGX_TILE4_NP
+    static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,            \
+    static_cast<const VisRec<1>*>(cb.vis), hx, hy, grid, cb.halo, cb.halo_set)
+  if (npol != 1) return hipErrorInvalidValue;
+  if (mode == 0)
+    HPGX_TILE4(0, acc_f64);
+  else if (acc == 0)
+    HPGX_TILE4(1, acc_f64);
+  else
+    HPGX_TILE4(1, acc_f32_cas);
 #undef HPGX_TILE4
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_halo(s, mode, nkeys, geo, cb, hx, hy, grid);
 }
 
-hipError_t launch_tile_blocal(
-  hipStream_t s, int npol, int mode, size_t n, size_t nkeys, const Geometry& geo,
-  const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
-  void* grid) {
-  if (nkeys == 0 || n == 0) return hipSuccess;
-  const int nb = bin_blocks_for(n);
-#define HPGX_TILE3(NP, MD, UU)                                                 \
-  hipLaunchKernelGGL(                                                          \
-    (k_tile3<NP, MD, UU>), dim3(unsigned(nkeys)), dim3(block), 0, s, geo,      \
-    cf.groups, cf.taps, mu, cb.off_table, nb, block_cap,                       \
-    static_cast<const Entry<NP>*>(cb.stream_entries), cb.entry_vis,            \
-    static_cast<const VisRec<NP>*>(cb.vis), grid)
-  if (mode == 0) {
-    switch (npol) {
-    case 1: HPGX_TILE3(1, 0, 4); break;
-    case 2: HPGX_TILE3(2, 0, 4); break;
-    case 3: HPGX_TILE3(3, 0, 2); break;
-    case 4: HPGX_TILE3(4, 0, 2); break;
-    default: return hipErrorInvalidValue;
-    }
-  } else {
-    switch (npol) {
-    case 1: HPGX_TILE3(1, 1, 4); break;
-    case 2: HPGX_TILE3(2, 1, 4); break;
-    case 3: HPGX_TILE3(3, 1, 2); break;
-    case 4: HPGX_TILE3(4, 1, 2); break;
-    default: return hipErrorInvalidValue;
-    }
+int patch_tiles_x(const Geometry& geo) {
+  return (geo.nx + patch_tile_x(patch_lanes(geo.nr)) - 1) / patch_tile_x(patch_lanes(geo.nr));
+}
+int patch_tiles_y(const Geometry& geo) {
+  return (geo.ny + patch_tile_y(patch_lanes(geo.nr)) - 1) / patch_tile_y(patch_lanes(geo.nr));
+}
+size_t patch_keys(const Geometry& geo) {
+  return size_t(patch_tiles_x(geo)) * patch_tiles_y(geo) * geo.nc;
+}
+size_t patch_rec_bytes(int npol) {
+  switch (npol) {
+  case 1: return sizeof(PatchRec<1>);
+  case 2: return sizeof(PatchRec<2>);
+  case 3: return sizeof(PatchRec<3>);
+  default: return sizeof(PatchRec<4>);
   }
-#undef HPGX_TILE3
-  return hipGetLastError();
+}
+size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy) {
+  const int tw = patch_tile_x(patch_lanes(nr)), th = patch_tile_y(patch_lanes(nr));
+  return size_t((max_sx - 1 + tw - 1) / tw + 1) * size_t((max_sy - 1 + th - 1) / th + 1);
 }
 
-size_t degrid_lane_max_taps() { return size_t(degrid_lane_taps); }
+// how the rows of both signs of w take their elements of a slice
+int patch_kind(int npol, const Geometry& geo, const DeviceCF& cf, const Mueller& mu) {
+  bool one = true, full = npol % 2 == 0 && cf.even_nm;
+  for (int s = 0; s < 2; ++s)
+    for (int r = 0; r < geo.nr; ++r) {
+      const int* row = s ? mu.M[r] : mu.Mc[r];
+      int used = 0;
+      for (int v = 0; v < npol; ++v) {
+        used += row[v] >= 0;
+        full = full && row[0] >= 0 && row[0] % 2 == 0 && row[v] == row[0] + v
+          && row[v] < cf.min_nm;
+      }
+      one = one && used <= 1;
+    }
+  return one ? patch_one : full ? patch_full : patch_any;
+}
+
+hipError_t launch_patch(
+  hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
+  const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
+  const double2* residuals, CallBuffers& cb, double* weights, int mode, void* grid) {
+  if (n == 0) return hipSuccess;
+  if (n > cb.patch_capacity) return hipErrorInvalidValue;
+  const int P = patch_lanes(geo.nr);
+  const int ptx = patch_tiles_x(geo), pty = patch_tiles_y(geo);
+  const size_t keys = patch_keys(geo);
+  const int kind = patch_kind(npol, geo, cf, mu);
+  // a kernel, not a memset: a captured graph may replay it
+  hipLaunchKernelGGL(k_zero, dim3(blocks_for(keys + 1)), dim3(block), 0, s, cb.hist, keys + 1);
+#define HPGX_PREP(NP)                                                          \
+  hipLaunchKernelGGL(                                                          \
+    k_patch_prep<NP>, dim3(std::min(blocks_for(n), count_blocks_max)), dim3(block), 0, s, \
+    static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
+    int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint), cb.gvis, residuals, \
+    ptx, pty, patch_tile_x(P), patch_tile_y(P), static_cast<PatchRec<NP>*>(cb.patch_recs), \
+    cb.hist, weights, cb.invalid_count)
+#define HPGX_LIST(NP)                                                          \
+  hipLaunchKernelGGL(                                                          \
+    k_patch_list<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, ptx, pty,     \
+    patch_tile_x(P), patch_tile_y(P), static_cast<const PatchRec<NP>*>(cb.patch_recs), \
+    cb.hist, cb.offsets, cb.patch_list)
+#define HPGX_PATCH_P(NP, PP, KD)                                               \
+  hipLaunchKernelGGL(                                                          \
+    (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_block), 0, s, geo, cf.taps, mu, \
+    mode, ptx, pty, cb.offsets, cb.patch_list,                                 \
+    static_cast<const PatchRec<NP>*>(cb.patch_recs),                           \
+    static_cast<const VisRec<NP>*>(cb.vis), grid)
+#define HPGX_PATCH_K(NP, KD)                                                   \
+  do {                                                                         \
+    if (P == 1) HPGX_PATCH_P(NP, 1, KD);                                       \
+    else if (P == 2) HPGX_PATCH_P(NP, 2, KD);                                  \
+    else HPGX_PATCH_P(NP, 4, KD);                                              \
+  } while (0)
+  switch (npol) {
+  case 1: HPGX_PREP(1); break;
+  case 2: HPGX_PREP(2); break;
+  case 3: HPGX_PREP(3); break;
+  case 4: HPGX_PREP(4); break;
+  default: return hipErrorInvalidValue;
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  size_t bytes = cb.scan_temp_bytes;
+  e = hipcub::DeviceScan::ExclusiveSum(cb.scan_temp, bytes, cb.hist, cb.offsets, int(keys + 1), s);
+  if (e != hipSuccess) return e;
+  switch (npol) {
+  case 1:
+    HPGX_LIST(1);
+    HPGX_PATCH_K(1, patch_one);
+    break;
+  case 2:
+    HPGX_LIST(2);
+    if (kind == patch_one) HPGX_PATCH_K(2, patch_one);
+    else if (kind == patch_full) HPGX_PATCH_K(2, patch_full);
+    else HPGX_PATCH_K(2, patch_any);
+    break;
+  case 3:
+    HPGX_LIST(3);
+    if (kind == patch_one) HPGX_PATCH_K(3, patch_one);
+    else HPGX_PATCH_K(3, patch_any);
+    break;
+  default:
+    HPGX_LIST(4);
+    if (kind == patch_one) HPGX_PATCH_K(4, patch_one);
+    else if (kind == patch_full) HPGX_PATCH_K(4, patch_full);
+    else HPGX_PATCH_K(4, patch_any);
+    break;
+  }
+#undef HPGX_PATCH_K
+#undef HPGX_PATCH_P
+#undef HPGX_LIST
+#undef HPGX_PREP
+  return hipGetLastError();
+}
 
 hipError_t launch_degrid_tiles(
   hipStream_t s, int npol, size_t n, size_t nkeys, const Geometry& geo,
@@ -4206,20 +3714,18 @@ hipError_t launch_degrid_tiles(
   const int nb = bin_blocks_for(n);
   const size_t lds = halo_lds_bytes(hx, hy, nb);
   if (lds > 65536) return hipErrorInvalidValue;
-#define HPGX_DEGRID4(NP)                                                       \
+#define HPGX_DEGRID4(UNIT)                                                     \
   hipLaunchKernelGGL(                                                          \
-    k_degrid4<NP>, dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo,       \
+    (k_degrid4<1, UNIT>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo, \
     cf.groups, cf.taps, mu, cb.off_table, nb, block_cap,                       \
-    static_cast<const Entry4<NP>*>(cb.stream_entries), cb.entry_vis,           \
-    static_cast<const VisRec<NP>*>(cb.vis), hx, hy, model, acc, int(one_plane),  \
-    cf.wsum, int(do_grid), static_cast<VisRec<NP>*>(out_recs), cb.gvis, pred64)
-  switch (npol) {
-  case 1: HPGX_DEGRID4(1); break;
-  case 2: HPGX_DEGRID4(2); break;
-  case 3: HPGX_DEGRID4(3); break;
-  case 4: HPGX_DEGRID4(4); break;
-  default: return hipErrorInvalidValue;
-  }
+    static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,            \
+    static_cast<const VisRec<1>*>(cb.vis), hx, hy, model, acc, int(one_plane), \
+    cf.wsum, int(do_grid), static_cast<VisRec<1>*>(out_recs), cb.gvis, pred64)
+  if (npol != 1) return hipErrorInvalidValue;
+  if (cf.max_nm == 1)
+    HPGX_DEGRID4(true);
+  else
+    HPGX_DEGRID4(false);
 #undef HPGX_DEGRID4
   return hipGetLastError();
 }
@@ -4247,9 +3753,7 @@ hipError_t launch_degrid_finish(
   return hipGetLastError();
 }
 
-bool degrid_sorts(const DeviceCF& cf) {
-  return size_t(cf.max_sx) * size_t(cf.max_sy) > size_t(degrid_lane_taps);
-}
+size_t degrid_rec_bytes() { return sizeof(DegridRec); }
 
 size_t degrid_order_temp_bytes(size_t n) {
   size_t bytes = 0;
@@ -4262,55 +3766,43 @@ size_t degrid_order_temp_bytes(size_t n) {
 
 hipError_t launch_degrid(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
-  const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb,
-  double2* pred64, const void* records) {
+  const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb, double2* pred64,
+  const void* records, void* out_records) {
   if (n == 0) return hipSuccess;
-  const void* in = records ? records : cb.vis;
-  if (size_t(cf.max_sx) * size_t(cf.max_sy) <= size_t(degrid_lane_taps)) {
-#define HPGX_DEGRID_LANE(NP)                                                   \
-  hipLaunchKernelGGL(                                                          \
-    k_degrid_lane<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, geo,         \
-    cf.groups, cf.taps, cf.wsum, mu, model, int(do_grid),                      \
-    static_cast<const VisRec<NP>*>(in), static_cast<VisRec<NP>*>(cb.vis),      \
-    cb.gvis, pred64)
-    switch (npol) {
-    case 1: HPGX_DEGRID_LANE(1); break;
-    case 2: HPGX_DEGRID_LANE(2); break;
-    case 3: HPGX_DEGRID_LANE(3); break;
-    case 4: HPGX_DEGRID_LANE(4); break;
-    default: return hipErrorInvalidValue;
-    }
-#undef HPGX_DEGRID_LANE
-    return hipGetLastError();
-  }
-  if (records) return hipErrorInvalidValue;  // the wave form reads cb.vis
-  // (callers stage records for supports above degrid_lane_max_taps())
-  // the records in CF-slice order where the order buffers hold the batch
-  // and the keys fit 32 bits
+  if (!model)
+    return launch_degrid_finish(s, npol, n, geo, cf, mu, nullptr, do_grid, records, out_records,
+                                cb, pred64);
+  if (cb.order_capacity < n || n > 0xffffffffull) return hipErrorInvalidValue;
+  // the records in CF-slice order where the keys fit 32 bits (with the grid
+  // cube first if they still do: its model planes then stay in the last-level
+  // cache), else as they come
   const unsigned* order = nullptr;
   const unsigned long long stride = (unsigned long long)std::max(cf.max_ncube, 1) * cf.nf * cf.nf;
-  const unsigned long long kmax = stride * (unsigned long long)cf.ngroups;
-  if (model && cb.degrid_order && cb.order_capacity >= n && n <= 0x7fffffffull
-      && kmax > 0 && kmax < 0xffffffffull) {
-    unsigned* keys = cb.degrid_order;
-    unsigned* keys_sorted = keys + cb.order_capacity;
-    unsigned* idx = keys + 2 * cb.order_capacity;
-    unsigned* idx_sorted = keys + 3 * cb.order_capacity;
+  const unsigned long long slices = stride * (unsigned long long)cf.ngroups;
+  const bool by_cube = slices * (unsigned long long)geo.nc < 0xffffffffull;
+  const unsigned long long kmax = by_cube ? slices * (unsigned long long)geo.nc : slices;
+  const bool sorted = n <= 0x7fffffffull && kmax > 0 && kmax < 0xffffffffull;
+  DegridRec* drs = static_cast<DegridRec*>(cb.degrid_recs);
+  unsigned* keys = sorted ? cb.degrid_order : nullptr;
+  unsigned* keys_sorted = cb.degrid_order + cb.order_capacity;
+  unsigned* idx = cb.degrid_order + 2 * cb.order_capacity;
+  unsigned* idx_sorted = cb.degrid_order + 3 * cb.order_capacity;
 #define HPGX_DKEYS(NP)                                                         \
   hipLaunchKernelGGL(                                                          \
     k_degrid_keys<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, geo,         \
-    cf.groups, static_cast<const VisRec<NP>*>(cb.vis), unsigned(stride),       \
-    unsigned(kmax), keys, idx)
-    switch (npol) {
-    case 1: HPGX_DKEYS(1); break;
-    case 2: HPGX_DKEYS(2); break;
-    case 3: HPGX_DKEYS(3); break;
-    case 4: HPGX_DKEYS(4); break;
-    default: return hipErrorInvalidValue;
-    }
+    cf.groups, static_cast<const VisRec<NP>*>(records), unsigned(stride),      \
+    unsigned(by_cube ? slices : 0ull), unsigned(kmax), keys, idx, drs)
+  switch (npol) {
+  case 1: HPGX_DKEYS(1); break;
+  case 2: HPGX_DKEYS(2); break;
+  case 3: HPGX_DKEYS(3); break;
+  case 4: HPGX_DKEYS(4); break;
+  default: return hipErrorInvalidValue;
+  }
 #undef HPGX_DKEYS
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (sorted) {
     const int bits = 32 - __builtin_clz(unsigned(kmax));
     size_t bytes = cb.order_temp_bytes;
     e = hipcub::DeviceRadixSort::SortPairs(cb.order_temp, bytes, keys, keys_sorted, idx,
@@ -4318,21 +3810,60 @@ hipError_t launch_degrid(
     if (e != hipSuccess) return e;
     order = idx_sorted;
   }
-  const unsigned nb = unsigned((n + (block / wave) - 1) / (block / wave));
-#define HPGX_DEGRID(NP)                                                        \
-  hipLaunchKernelGGL(                                                          \
-    k_degrid<NP>, dim3(nb), dim3(block), 0, s, n, geo, cf.groups, cf.taps,     \
-    cf.wsum, mu, model, int(do_grid), static_cast<VisRec<NP>*>(cb.vis),        \
-    cb.gvis, pred64, order)
+  const int P = patch_lanes(geo.nr);
+  int kind = patch_kind(npol, geo, cf, mu);
+  bool same_rows = true;
+  for (int v = 0; v < npol; ++v) {
+    int used = 0, used_c = 0;
+    for (int r = 0; r < geo.nr; ++r) {
+      same_rows = same_rows && mu.M[r][v] == mu.Mc[r][v];
+      used += mu.M[r][v] >= 0;
+      used_c += mu.Mc[r][v] >= 0;
+    }
+    if (kind == patch_one && (used > 1 || used_c > 1)) kind = patch_any;
+  }
+#define HPGX_DEGRID_P(NP, PP, KD)                                              \
+  do {                                                                         \
+    constexpr size_t per = size_t(block / wave) * degrid_recs<NP, KD>();       \
+    hipLaunchKernelGGL(                                                        \
+      (k_degrid<NP, PP, KD>), dim3(unsigned((n + per - 1) / per)), dim3(block), 0, s, n, geo, \
+      cf.taps, mu, int(same_rows), model, drs,                                 \
+      static_cast<const VisRec<NP>*>(records), order,                          \
+      reinterpret_cast<double*>(cb.degrid_acc));                               \
+  } while (0)
+#define HPGX_DEGRID_K(NP, KD)                                                  \
+  do {                                                                         \
+    if (P == 1) HPGX_DEGRID_P(NP, 1, KD);                                      \
+    else if (P == 2) HPGX_DEGRID_P(NP, 2, KD);                                 \
+    else HPGX_DEGRID_P(NP, 4, KD);                                             \
+  } while (0)
   switch (npol) {
-  case 1: HPGX_DEGRID(1); break;
-  case 2: HPGX_DEGRID(2); break;
-  case 3: HPGX_DEGRID(3); break;
-  case 4: HPGX_DEGRID(4); break;
+  case 1:
+    if (kind == patch_one) HPGX_DEGRID_K(1, patch_one);
+    else HPGX_DEGRID_K(1, patch_any);
+    break;
+  case 2:
+    if (kind == patch_one) HPGX_DEGRID_K(2, patch_one);
+    else if (kind == patch_full) HPGX_DEGRID_K(2, patch_full);
+    else HPGX_DEGRID_K(2, patch_any);
+    break;
+  case 3:
+    if (kind == patch_one) HPGX_DEGRID_K(3, patch_one);
+    else HPGX_DEGRID_K(3, patch_any);
+    break;
+  case 4:
+    if (kind == patch_one) HPGX_DEGRID_K(4, patch_one);
+    else if (kind == patch_full) HPGX_DEGRID_K(4, patch_full);
+    else HPGX_DEGRID_K(4, patch_any);
+    break;
   default: return hipErrorInvalidValue;
   }
-#undef HPGX_DEGRID
-  return hipGetLastError();
+#undef HPGX_DEGRID_K
+#undef HPGX_DEGRID_P
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_degrid_finish(s, npol, n, geo, cf, mu, cb.degrid_acc, do_grid, records,
+                              out_records, cb, pred64);
 }
 
 bool finish_pre_fits(const Geometry& geo) {
