@@ -27,6 +27,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <cmath>
 #include <type_traits>
 
 namespace hpgx {
@@ -2617,12 +2618,14 @@ struct __align__(16) DegridRec {
   unsigned pad;
 };
 
-// key = the record's (grid cube, group, CF cube, fine offsets), kmax for
-// records that are skipped (no CF, outside the grid)
+// key = the record's (grid cube, region, group, CF cube, fine offsets), kmax
+// for records that are skipped (no CF, outside the grid); region (region_sh
+// below 31) the square of 2^region_sh pixels that holds the support corner
 template <int N>
 __global__ void k_degrid_keys(
   size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const VisRec<N>* __restrict__ recs, unsigned stride, unsigned cube_stride, unsigned kmax,
+  const VisRec<N>* __restrict__ recs, unsigned stride, unsigned slices, int region_sh,
+  unsigned regions_x, unsigned regions, unsigned kmax,
   unsigned* __restrict__ keys, unsigned* __restrict__ idx, DegridRec* __restrict__ out) {
   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -2639,7 +2642,9 @@ __global__ void k_degrid_keys(
       if (c.inside) {
         const unsigned fxi = unsigned(c.fx + geo.F), fyi = unsigned(c.fy + geo.F);
         const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-        key = gcube * cube_stride + grp * stride
+        const unsigned region = (unsigned(c.gy) >> region_sh) * regions_x
+          + (unsigned(c.gx) >> region_sh);
+        key = (gcube * regions + region) * slices + grp * stride
           + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
         d.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi));
         d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
@@ -2657,14 +2662,14 @@ __global__ void k_degrid_keys(
   out[i] = d;
 }
 
-// sums val[0, V) of the lanes that differ in bits P .. 32 of their number.
+// sums val[0, V) of the lanes that differ in bits 1 .. MASK of their number.
 // Each step halves the values a lane holds (it keeps one half, and adds its
 // partner's values of that half) while their number is even: V - 1 adds
-// instead of V log2(64 / P).  Value `at` + i is in val[i] afterwards, i below
+// instead of V log2(lanes).  Value `at` + i is in val[i] afterwards, i below
 // the returned number.
-template <int V, int MASK, int P>
+template <int V, int MASK>
 __device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
-  if constexpr (MASK < P) {
+  if constexpr (MASK == 0) {
     return V;
   } else if constexpr (V % 2 == 0) {
     constexpr int H = V / 2;
@@ -2676,52 +2681,58 @@ __device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
       val[i] = keep + __shfl_xor(send, MASK, wave);
     }
     at += up ? H : 0;
-    return reduce_lanes<H, MASK / 2, P>(val, lane, at);
+    return reduce_lanes<H, MASK / 2>(val, lane, at);
   } else {
 #pragma unroll
     for (int i = 0; i < V; ++i) val[i] += __shfl_xor(val[i], MASK, wave);
-    return reduce_lanes<V, MASK / 2, P>(val, lane, at);
+    return reduce_lanes<V, MASK / 2>(val, lane, at);
   }
 }
 
-// records a wave takes: their sums (N complex values a lane, one where a row
-// uses one element) within 64 registers
-template <int N, int KIND>
-constexpr int degrid_recs() { return KIND == patch_one || N <= 2 ? 8 : 4; }
+// records a wave takes (eight of one element a row, or of two polarizations,
+// measured slower: their registers cost a wave per SIMD)
+constexpr int degrid_recs = 4;
 
 // One wave takes R records in a row of the order; those of one slice share
 // every CF value it loads (per tap of 4 x 4 elements a record reads 64 bytes
 // of model and 128 of CF: the CF reads are the larger part until four share
-// them).  A lane is a (tap, grid row), 64 / P taps a step; the Mueller
-// elements of a slice lie side by side, so a step's CF loads cover whole
-// lines.  The sums over the support go to acc (record x polarization).
+// them).  A lane is a (tap, grid row), 64 / P taps a step, the taps of a row in
+// neighbouring lanes: their model values are neighbours too (the cache takes a
+// load by lines, 16 for 64 lanes of 16 bytes so, 64 with the rows in
+// neighbouring lanes: 1.2 ms against 0.97 for 300,000 records of supports 9-33
+// and one element a row).  The sums over the support go to acc (record x polarization).
 // order null: the records as they come.  same_rows: M and Mc are equal, so
 // that records of both signs of w share CF values (the model's imaginary part
 // takes the sign: sum conj(c) m = conj(sum c conj(m))).  patch_one: no two
 // rows use one polarization; acc of one that no row uses is not written.
-// Bound: the model gathers (64 bytes per tap from anywhere in the model: 4.4
-// TB/s with their line ends).  500,000 records of supports 9-65 and 16 elements
-// 14.1 ms (26.8 ms one record a wave), 150,000 of 17-129 14.7 ms (27.1), 1e6 of
-// 9-33 and one element a row 6.2 ms (7.3).  Three waves per SIMD: at four the
-// sums spill (15.9 ms the first).
+// Bound: the model gathers, from HBM for batches that are sparse on the grid
+// (64 bytes per tap from anywhere in the model, 4.4 TB/s with their line ends:
+// 500,000 records of supports 9-65 and 16 elements 13.8 ms, 26.8 ms one record a
+// wave; 150,000 of 17-129 14.0 ms, before 27.1), from L2 in dense regions
+// (launch_degrid): 1e6 records of supports 9-33 and one element a row 2.9 ms,
+// before 7.3; 300,000 of 7-17, two polarizations, 222 us, before 1250 us one
+// record a lane.  Two steps' loads at once where a row uses one element (3.3 ms
+// one by one).  Three waves per SIMD for several: at four the sums spill
+// (15.9 ms the first).
 template <int N, int P, int KIND>
-__global__ __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(KIND == patch_one ? 4 : 3)))
 void k_degrid(
   size_t n, Geometry geo, const float2* __restrict__ taps, Mueller mu, int same_rows,
-  const double2* __restrict__ model, const DegridRec* __restrict__ drs,
+  const double2* __restrict__ model, int by_xcd, const DegridRec* __restrict__ drs,
   const VisRec<N>* __restrict__ recs, const unsigned* __restrict__ order,
   double* __restrict__ acc) {
 
-  constexpr int R = degrid_recs<N, KIND>();
+  constexpr int R = degrid_recs;
   constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
   constexpr int TPS = wave / P;                 // taps a step
 
   const int w = uniform(int(threadIdx.x) / wave);
   const int lane = threadIdx.x % wave;
-  const size_t p0 = (blockIdx.x * (size_t)(block / wave) + w) * R;
+  const unsigned bi = by_xcd ? xcd_key(blockIdx.x, gridDim.x) : blockIdx.x;
+  const size_t p0 = (bi * (size_t)(block / wave) + w) * R;
   if (p0 >= n) return;
-  const int row = lane % P;
-  const int q = lane / P;
+  const int row = lane / TPS;
+  const int q = lane % TPS;
 
   // lane r < R: record r of the wave
   DegridRec d{};
@@ -2827,54 +2838,69 @@ void k_degrid(
       gdx = gxr * geo.os;
       gdy = gyr * geo.os;
     }
-    auto step = [&]() {
-      float2 c[L];
-      double2 m[RR];
-      if constexpr (KIND == patch_full) {
+    // U steps, their loads issued together
+    auto steps = [&](auto u_c) {
+      constexpr int U = decltype(u_c)::value;
+      float2 c[U][L];
+      double2 m[U][RR];
 #pragma unroll
-        for (int v = 0; v < N; v += 2) {
-          const float4 t = *reinterpret_cast<const float4*>(cf + eo[0] + v);
-          c[v] = make_float2(t.x, t.y);
-          c[v + 1] = make_float2(t.z, t.w);
+      for (int u = 0; u < U; ++u) {
+        if constexpr (KIND == patch_full) {
+#pragma unroll
+          for (int v = 0; v < N; v += 2) {
+            const float4 t = *reinterpret_cast<const float4*>(cf + eo[0] + v);
+            c[u][v] = make_float2(t.x, t.y);
+            c[u][v + 1] = make_float2(t.z, t.w);
+          }
+        } else {
+#pragma unroll
+          for (int v = 0; v < L; ++v) c[u][v] = cf[eo[v]];
         }
-      } else {
+        cf += size_t(TPS) * nm;
 #pragma unroll
-        for (int v = 0; v < L; ++v) c[v] = cf[eo[v]];
-      }
-      cf += size_t(TPS) * nm;
-#pragma unroll
-      for (int k = 0; k < RR; ++k) m[k] = mp[k][off];
-      if constexpr (GRAD) m[0] = cmul(m[0], cphase_taylor(-(gp0 + X * gdx) - (gp1 + Y * gdy)));
-      X += dX;
-      Y += dY;
-      off += doff;
-      if (X >= sx) {
-        X -= sx;
-        ++Y;
-        off += wrap;
+        for (int k = 0; k < RR; ++k) m[u][k] = mp[k][off];
+        if constexpr (GRAD)
+          m[u][0] = cmul(m[u][0], cphase_taylor(-(gp0 + X * gdx) - (gp1 + Y * gdy)));
+        X += dX;
+        Y += dY;
+        off += doff;
+        if (X >= sx) {
+          X -= sx;
+          ++Y;
+          off += wrap;
+        }
       }
 #pragma unroll
-      for (int k = 0; k < RR; ++k) {
-        const double mx = m[k].x;
-        const double my = __hiloint2double(
-          int(unsigned(__double2hiint(m[k].y)) ^ flip[k]), __double2loint(m[k].y));
+      for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int v = 0; v < L; ++v) {
-          if (KIND == patch_any && !use[v]) continue;
-          const double cx = double(c[v].x), cy = double(c[v].y);
-          double& a = val[(k * L + v) * 2];
-          double& b = val[(k * L + v) * 2 + 1];
-          a = __builtin_fma(cx, mx, a);
-          a = __builtin_fma(-cy, my, a);
-          b = __builtin_fma(cx, my, b);
-          b = __builtin_fma(cy, mx, b);
+        for (int k = 0; k < RR; ++k) {
+          const double mx = m[u][k].x;
+          const double my = __hiloint2double(
+            int(unsigned(__double2hiint(m[u][k].y)) ^ flip[k]), __double2loint(m[u][k].y));
+#pragma unroll
+          for (int v = 0; v < L; ++v) {
+            if (KIND == patch_any && !use[v]) continue;
+            const double cx = double(c[u][v].x), cy = double(c[u][v].y);
+            double& a = val[(k * L + v) * 2];
+            double& b = val[(k * L + v) * 2 + 1];
+            a = __builtin_fma(cx, mx, a);
+            a = __builtin_fma(-cy, my, a);
+            b = __builtin_fma(cx, my, b);
+            b = __builtin_fma(cy, mx, b);
+          }
         }
       }
     };
+    constexpr int U = GRAD || RR * (L + 1) > 12 ? 1 : 2;
     const unsigned full = ntap / TPS;
+    unsigned s = 0;
 #pragma unroll 1
-    for (unsigned s = 0; s < full; ++s) step();
-    if (full * TPS + unsigned(q) < ntap) step();
+    for (; s + U <= full; s += U) steps(std::integral_constant<int, U>{});
+    if constexpr (U > 1) {
+#pragma unroll 1
+      for (; s < full; ++s) steps(std::integral_constant<int, 1>{});
+    }
+    if (full * TPS + unsigned(q) < ntap) steps(std::integral_constant<int, 1>{});
     // the other sign's imaginary parts, then the sums over the taps (and,
     // but for patch_one, the rows)
 #pragma unroll
@@ -2887,7 +2913,7 @@ void k_degrid(
       }
     int at = 0;
     const int left =
-      reduce_lanes<RR * L * 2, wave / 2, KIND == patch_one ? P : 1>(val, lane, at);
+      reduce_lanes<RR * L * 2, (KIND == patch_one ? TPS : wave) / 2>(val, lane, at);
 #pragma unroll
     for (int i = 0; i < RR * L * 2; ++i) {
       if (i >= left) continue;
@@ -2913,9 +2939,6 @@ void k_degrid(
     if (len >= R) {
       run(std::integral_constant<int, R>{}, std::false_type{}, r);
       r += R;
-    } else if (R > 4 && len >= 4) {
-      run(std::integral_constant<int, R / 2>{}, std::false_type{}, r);
-      r += R / 2;
     } else if (len >= 2) {
       run(std::integral_constant<int, 2>{}, std::false_type{}, r);
       r += 2;
@@ -3773,15 +3796,58 @@ hipError_t launch_degrid(
     return launch_degrid_finish(s, npol, n, geo, cf, mu, nullptr, do_grid, records, out_records,
                                 cb, pred64);
   if (cb.order_capacity < n || n > 0xffffffffull) return hipErrorInvalidValue;
-  // the records in CF-slice order where the keys fit 32 bits (with the grid
-  // cube first if they still do: its model planes then stay in the last-level
-  // cache), else as they come
+  const int P = patch_lanes(geo.nr);
+  int kind = patch_kind(npol, geo, cf, mu);
+  bool same_rows = true;
+  for (int v = 0; v < npol; ++v) {
+    int used = 0, used_c = 0;
+    for (int r = 0; r < geo.nr; ++r) {
+      same_rows = same_rows && mu.M[r][v] == mu.Mc[r][v];
+      used += mu.M[r][v] >= 0;
+      used_c += mu.Mc[r][v] >= 0;
+    }
+    if (kind == patch_one && (used > 1 || used_c > 1)) kind = patch_any;
+  }
   const unsigned* order = nullptr;
+  // The records in CF-slice order; where the batch is dense, region by region,
+  // whose model then stays in L2: the largest square of 2^k pixels whose model
+  // (all rows, with the supports' halo) fits half of an XCD's 4 MB, each XCD
+  // taking a contiguous share of the records.  Dense: a region's records read
+  // its model four times over at least, and what their shorter runs of one
+  // slice read more of the CF is no more than the model reads that leave HBM.
+  // Degridding kernel without and with regions: 1e6 records of supports 9-33,
+  // one element a row, 2048^2: 5.7 -> 2.9 ms; 300,000 on 1024^2: 1.45 -> 0.92;
+  // 300,000 of 7-17, two polarizations, 2 x 1500^2: 287 -> 222 us.  (Contiguous
+  // shares without regions would give the XCDs different CF groups, the large
+  // supports to one: 14 -> 22 ms on 64 groups.)
+  // Grid cubes one after the other while the keys fit 32 bits; no order if the
+  // slices alone do not.
   const unsigned long long stride = (unsigned long long)std::max(cf.max_ncube, 1) * cf.nf * cf.nf;
   const unsigned long long slices = stride * (unsigned long long)cf.ngroups;
-  const bool by_cube = slices * (unsigned long long)geo.nc < 0xffffffffull;
-  const unsigned long long kmax = by_cube ? slices * (unsigned long long)geo.nc : slices;
-  const bool sorted = n <= 0x7fffffffull && kmax > 0 && kmax < 0xffffffffull;
+  constexpr unsigned long long key_limit = 0xffffffffull;
+  constexpr double l2_bytes = 2.0 * (1 << 20);
+  const double density = double(n) / (double(geo.nx) * geo.ny * geo.nc);
+  const double support = std::max(cf.max_sx, cf.max_sy);
+  int region_sh = 5;
+  while (std::pow(std::ldexp(1.0, region_sh + 1) + support, 2) * geo.nr * sizeof(double2) <= l2_bytes)
+    ++region_sh;
+  {
+    const double in_region = std::ldexp(density, 2 * region_sh);
+    const double cf_bytes = double(kind == patch_one ? 1 : npol) * sizeof(float2);
+    const double run = std::max(1.0, in_region / double(slices));
+    const double run_all = std::max(1.0, double(n) / (double(slices) * geo.nc));
+    const double edge = std::ldexp(1.0, region_sh) + support;
+    if (cf_bytes / run > sizeof(double2) + cf_bytes / run_all
+        || in_region * support * support < 4.0 * edge * edge
+        || edge * edge * geo.nr * sizeof(double2) > l2_bytes)
+      region_sh = 31;
+  }
+  auto count = [&](int size) { return (unsigned long long)((unsigned(size) - 1u) >> region_sh) + 1; };
+  if (slices * geo.nc * count(geo.nx) * count(geo.ny) >= key_limit) region_sh = 31;
+  const unsigned long long regions = count(geo.nx) * count(geo.ny);
+  const bool by_cube = slices * regions * geo.nc < key_limit;
+  const unsigned long long kmax = by_cube ? slices * regions * geo.nc : slices;
+  const bool sorted = n <= 0x7fffffffull && kmax > 0 && kmax < key_limit;
   DegridRec* drs = static_cast<DegridRec*>(cb.degrid_recs);
   unsigned* keys = sorted ? cb.degrid_order : nullptr;
   unsigned* keys_sorted = cb.degrid_order + cb.order_capacity;
@@ -3791,7 +3857,8 @@ hipError_t launch_degrid(
   hipLaunchKernelGGL(                                                          \
     k_degrid_keys<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, geo,         \
     cf.groups, static_cast<const VisRec<NP>*>(records), unsigned(stride),      \
-    unsigned(by_cube ? slices : 0ull), unsigned(kmax), keys, idx, drs)
+    unsigned(slices), region_sh, unsigned(count(geo.nx)), unsigned(by_cube ? regions : 0ull), \
+    unsigned(kmax), keys, idx, drs)
   switch (npol) {
   case 1: HPGX_DKEYS(1); break;
   case 2: HPGX_DKEYS(2); break;
@@ -3810,24 +3877,12 @@ hipError_t launch_degrid(
     if (e != hipSuccess) return e;
     order = idx_sorted;
   }
-  const int P = patch_lanes(geo.nr);
-  int kind = patch_kind(npol, geo, cf, mu);
-  bool same_rows = true;
-  for (int v = 0; v < npol; ++v) {
-    int used = 0, used_c = 0;
-    for (int r = 0; r < geo.nr; ++r) {
-      same_rows = same_rows && mu.M[r][v] == mu.Mc[r][v];
-      used += mu.M[r][v] >= 0;
-      used_c += mu.Mc[r][v] >= 0;
-    }
-    if (kind == patch_one && (used > 1 || used_c > 1)) kind = patch_any;
-  }
 #define HPGX_DEGRID_P(NP, PP, KD)                                              \
   do {                                                                         \
-    constexpr size_t per = size_t(block / wave) * degrid_recs<NP, KD>();       \
+    constexpr size_t per = size_t(block / wave) * degrid_recs;       \
     hipLaunchKernelGGL(                                                        \
       (k_degrid<NP, PP, KD>), dim3(unsigned((n + per - 1) / per)), dim3(block), 0, s, n, geo, \
-      cf.taps, mu, int(same_rows), model, drs,                                 \
+      cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,            \
       static_cast<const VisRec<NP>*>(records), order,                          \
       reinterpret_cast<double*>(cb.degrid_acc));                               \
   } while (0)

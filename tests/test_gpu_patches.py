@@ -141,6 +141,27 @@ def test_slice_runs_vs_oracle(hpg, oracle_mod, monkeypatch, kind, radii, device,
     _planes_close(gs.grid_values(), o.grid_values(), 1e-5)
 
 
+@pytest.mark.parametrize("M,nm,radius", [(DIAG, 4, 4), (FULL, 16, 3), (DIAG, 4, 0)])
+def test_degrid_regions_vs_oracle(hpg, oracle_mod, M, nm, radius):
+    """A batch dense enough to be degridded region by region (2^k pixels
+    squares, several on this grid, edges between and at its ends)."""
+    from hpg_amd import workloads
+    gsz = (520, 300, 4, 2)
+    n = 30_011
+    cf = workloads.random_cf(3, [radius], nmueller=nm, seed=21)
+    rec = workloads.random_visibilities(n, 4, gsz, (0.9, 1.1), cf, seed=22, phase=True,
+                                        margin=-3)
+    gs, o = _pair(hpg, oracle_mod, gsz, M, M, cf, 0, n)
+    rng = np.random.default_rng(9)
+    model = rng.standard_normal(gsz[::-1]) + 1j * rng.standard_normal(gsz[::-1])
+    gs.set_model(hpg.Device.Serial, model)
+    o.set_model(model)
+    pred = gs.degrid_get_predicted_visibilities(hpg.Device.Serial, rec)
+    pexp = o.grid_visibilities(_view(rec, oracle_mod), False, do_degrid=True, do_grid=False)
+    np.testing.assert_allclose(pred["visibilities"], pexp["vis"], rtol=1e-6,
+                               atol=1e-6 * np.abs(pexp["vis"]).max())
+
+
 def test_patches_in_passes(hpg, monkeypatch):
     """Batches whose lists exceed the entry budget take several passes."""
     from hpg_amd import workloads
