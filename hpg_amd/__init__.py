@@ -559,6 +559,24 @@ class GridderState:
             self._h, out.ctypes.data_as(ctypes.c_void_p), int(layout)), self._h)
         return out
 
+    def _device_values(self, call, device):
+        import torch
+        out = torch.empty(self.grid_shape, dtype=torch.complex128, device=device)
+        # the block may have been freed by work still queued on torch's stream
+        _order_after_torch(out.device)
+        _check(call(self._h, ctypes.c_void_p(out.data_ptr())), self._h)
+        return out
+
+    def grid_values_device(self, device="cuda"):
+        """The grid as a torch complex128 GPU tensor (cube, mrow, y, x),
+        copied on the device."""
+        return self._device_values(_lib.lib().hpgx_grid_values_device, device)
+
+    def model_values_device(self, device="cuda"):
+        """The model as a torch complex128 GPU tensor (cube, mrow, y, x),
+        copied on the device."""
+        return self._device_values(_lib.lib().hpgx_model_values_device, device)
+
     def grid_window(self, x0, y0, nx, ny, mrow=0, cube=0):
         """Window [x0, x0+nx) x [y0, y0+ny) of one plane, shape (ny, nx)."""
         out = np.empty((ny, nx), dtype=np.complex128)

@@ -48,6 +48,8 @@ SIGNATURES = [
     ("hpgx_grid_values", i, [vp, vp, i]),
     ("hpgx_grid_weights", i, [vp, vp, i]),
     ("hpgx_model_values", i, [vp, vp, i]),
+    ("hpgx_grid_values_device", i, [vp, vp]),
+    ("hpgx_model_values_device", i, [vp, vp]),
     ("hpgx_grid_window", i, [vp, u, u, u, u, u, u, vp]),
     ("hpgx_grid_device_ptr", i, [vp, vp, vp]),
     ("hpgx_event_record", i, [vp, i]),

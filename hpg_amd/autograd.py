@@ -27,6 +27,15 @@ import torch
 from . import Device, FFTSign, GridderState, ShiftDirection  # noqa: F401
 
 
+def _values(on_device, on_host, device):
+    """the state's grid or model on a tensor's device (through host memory the
+    three copies of a fitting step took 27 of its 32 ms: 1024^2 x 4 pixels,
+    300,000 records)"""
+    if device.type == "cuda":
+        return on_device(device)
+    return torch.from_numpy(np.ascontiguousarray(on_host())).to(device)
+
+
 class Degrid(torch.autograd.Function):
     @staticmethod
     def forward(ctx, model, state, records):
@@ -41,8 +50,7 @@ class Degrid(torch.autograd.Function):
         state = ctx.state
         state.reset_grid()
         state.degrid_adjoint(ctx.records, grad_out.contiguous())
-        g = torch.from_numpy(np.ascontiguousarray(state.grid_values())).to(grad_out.device)
-        return g, None, None
+        return _values(state.grid_values_device, state.grid_values, grad_out.device), None, None
 
 
 def degrid(model, state, records):
@@ -70,7 +78,7 @@ def _model_pass(state, values, sign, direction, fft_first):
     else:
         state.shift_model(direction)
         state.apply_model_fft(1.0, sign, True)
-    return torch.from_numpy(np.ascontiguousarray(state.model_values())).to(values.device)
+    return _values(state.model_values_device, state.model_values, values.device)
 
 
 class ImageToModel(torch.autograd.Function):

@@ -1789,6 +1789,42 @@ int hpgx_model_values(hpgx_state_t st, void* dst, int layout) {
   return copy_grid_to_host(st, st->model, false, dst, layout);
 }
 
+// a grid-shaped device array (null: zeros) as complex<double> into device
+// memory dst, which may lie on another GPU
+static int values_to_device(hpgx_state_t st, const void* src, bool is_float, void* dst) {
+  if (int rc = set_device(st)) return rc;
+  const size_t n = st->grid_elems();
+  hipPointerAttribute_t at{};
+  const bool here = hipPointerGetAttributes(&at, dst) == hipSuccess && at.device == st->device;
+  double2* out = static_cast<double2*>(dst);
+  if (!here) HPGX_HIP(st, dev_alloc(out, n * sizeof(double2)));
+  hipError_t e;
+  if (!src)
+    e = hipMemsetAsync(out, 0, n * sizeof(double2), st->stream);
+  else if (is_float)
+    e = hpgx::launch_widen(st->stream, static_cast<const float2*>(src), out, n);
+  else
+    e = hipMemcpyAsync(out, src, n * sizeof(double2), hipMemcpyDeviceToDevice, st->stream);
+  if (!here && e == hipSuccess)
+    e = hipMemcpyAsync(dst, out, n * sizeof(double2), hipMemcpyDefault, st->stream);
+  const hipError_t w = hipStreamSynchronize(st->stream);
+  if (!here) dev_free(out);
+  if (e == hipSuccess) e = w;
+  return e == hipSuccess ? HPGX_SUCCESS : hip_fail(st, e, "readback to device memory");
+}
+
+int hpgx_grid_values_device(hpgx_state_t st, void* dst) {
+  if (!st || !dst) return HPGX_ERR_OTHER;
+  if (int rc = set_device(st)) return rc;
+  if (int rc = flush_finishing(st)) return rc;
+  return values_to_device(st, st->grid, st->mode != HPGX_GRID_FP64, dst);
+}
+
+int hpgx_model_values_device(hpgx_state_t st, void* dst) {
+  if (!st || !dst) return HPGX_ERR_OTHER;
+  return values_to_device(st, st->model, false, dst);
+}
+
 int hpgx_grid_window(
   hpgx_state_t st, unsigned x0, unsigned y0, unsigned nx, unsigned ny,
   unsigned mrow, unsigned cube, void* dst) {

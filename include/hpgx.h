@@ -291,6 +291,11 @@ HPGX_API int hpgx_reset_grid(hpgx_state_t state);
 HPGX_API int hpgx_grid_values(hpgx_state_t state, void* dst, int layout);
 HPGX_API int hpgx_grid_weights(hpgx_state_t state, double* dst, int layout);
 HPGX_API int hpgx_model_values(hpgx_state_t state, void* dst, int layout);
+/* The grid or the model as complex<double> in HPGX_LAYOUT_LEFT into device
+ * memory dst (grid-sized, on any GPU), complete when the call returns; dst must
+ * not be in use by other queued work.  An unset model reads as zero. */
+HPGX_API int hpgx_grid_values_device(hpgx_state_t state, void* dst);
+HPGX_API int hpgx_model_values_device(hpgx_state_t state, void* dst);
 /* Fence, then copy the window [x0, x0+nx) x [y0, y0+ny) of plane
  * (mrow, cube) of the grid into host memory dst, complex<double>, x fastest.
  * No reference counterpart: a narrow form of grid_values() for large grids. */

@@ -194,3 +194,27 @@ def test_cf_layout_weights(hpg, oracle_mod, nm, os_, radius):
     o.grid_visibilities(_view(rec, oracle_mod), True)
     _planes_close(gs.grid_values(), o.grid_values(), 1e-12)
     np.testing.assert_allclose(gs.grid_weights(), o.grid_weights(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_values_on_device(hpg, mode):
+    """The grid and the model read back into device tensors equal the host
+    copies bit for bit; an unset model reads as zero."""
+    import torch
+    from hpg_amd import workloads
+    gsz = (37, 21, 2, 3)
+    cf = workloads.random_cf(4, [2], nmueller=2, seed=1)
+    rec = workloads.random_visibilities(500, 2, gsz, (1.0, 1.0), cf, seed=2)
+    gs = hpg.GridderState.create(hpg.Device.Hip, 0, 500, cf, gsz, (1.0, 1.0),
+                                 [[0, -1], [-1, 1]], grid_mode=mode)
+    gs.set_convolution_function(hpg.Device.Serial, cf)
+    assert not gs.model_values_device().any()
+    gs.grid_visibilities(hpg.Device.Serial, rec)
+    gs.normalize_by_weights(2.0)
+    gs.apply_grid_fft(1.0, hpg.FFTSign.POSITIVE, True)
+    on_device = gs.grid_values_device()
+    assert on_device.dtype == torch.complex128 and tuple(on_device.shape) == gs.grid_shape
+    assert np.array_equal(on_device.cpu().numpy(), gs.grid_values())
+    model = torch.randn(gs.grid_shape, dtype=torch.complex128, device="cuda")
+    gs.set_model(hpg.Device.Serial, model)
+    assert torch.equal(gs.model_values_device(), model)
