@@ -983,6 +983,8 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
     p += up((keys + 1) * sizeof(unsigned));
     c.offsets = reinterpret_cast<unsigned*>(p);
     p += up((keys + 1) * sizeof(unsigned));
+    c.cursor = reinterpret_cast<unsigned*>(p);
+    p += up(keys * sizeof(unsigned));
     c.scan_temp = p;
     c.scan_temp_bytes = st->cb.scan_temp_bytes;
     p += up(c.scan_temp_bytes);

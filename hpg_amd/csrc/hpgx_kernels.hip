@@ -2138,12 +2138,14 @@ void k_sub(
 // tile kernels'.  One workgroup owns a tile of all grid rows of one cube and
 // keeps its pixels' FP64 sums in registers, so a tap costs no LDS or global
 // atomic: a lane is a (pixel, grid row), a wave holds 2 x 2 patches of 64 / P
-// pixels (P = lanes per pixel: 1, 2 or 4 rows), the workgroup 2 x 2 waves.
+// pixels (P = lanes per pixel: 1, 2 or 4 rows), the workgroup 2 x 2 waves, or
+// twice that, two waves sharing the entries of the same pixels (patch_split).
 //
 //   k_patch_prep  one thread per visibility: skip rule, weights, the record's
 //                 prepared form (support corner, CF slice, pre-phased values)
 //                 and the counts of the tiles it touches
-//   (scan)        the tiles' list offsets
+//   k_patch_scan  the tiles' list offsets and their order (many tiles: hipCUB's
+//                 scan, in grid order)
 //   k_patch_list  one thread per visibility: its index into the lists of the
 //                 tiles it touches
 //   k_patch       one workgroup per tile: 256 list entries at a time staged in
@@ -2158,11 +2160,13 @@ void k_sub(
 // it touches, 72% at S = 17.
 //
 // Bound: the CF reads from HBM for large CFs (64 groups of supports 9-65, 16
-// elements, 500,000 records: 104 GB in 19.9 ms, 5.2 TB/s, against 27.7 ms for
+// elements, 500,000 records: 104 GB in 19.5 ms, 5.3 TB/s, against 27.7 ms for
 // clipped tiles in LDS, one workgroup per plane and element-major slices;
-// supports 17-129, 150,000 records: 119 GB in 20.3 ms, before 38.4 ms), the
-// vector ALU for CFs that stay in the last-level cache (supports 9-25, 200,000
-// records: 1.17 ms, before 4.31 ms by LDS compare-and-swap).
+// supports 17-129, 150,000 records: 119 GB in 19.2 ms, before 38.4 ms), vector
+// issue for CFs that stay in the last-level cache (supports 9-25, 200,000
+// records: 1.00 ms, before 4.31 ms by LDS compare-and-swap). Loading the next
+// one to three entries' CF values ahead of their turn gained nothing there and
+// cost the small supports 10%: the waves cover the loads.
 
 // lanes per pixel for nr grid rows
 constexpr int patch_lanes(int nr) { return nr <= 1 ? 1 : nr == 2 ? 2 : 4; }
@@ -2172,6 +2176,12 @@ __host__ __device__ constexpr int patch_h(int P) { return P == 1 ? 8 : 4; }
 __host__ __device__ constexpr int patch_tile_x(int P) { return 4 * patch_w(P); }
 __host__ __device__ constexpr int patch_tile_y(int P) { return 4 * patch_h(P); }
 constexpr int patch_block = 4 * wave;
+// waves that share the entries of the same pixels: a tile's entries run one
+// after the other, so the fullest tile of a dense uv core sets the kernel's
+// length. Two where a tile is 16 pixels wide (four rows: 300,000 records on
+// 1024^2 1.58 -> 0.97 ms, the large CFs 2 to 5% less), four gained no more; one
+// for the wider tiles, whose entries are cheap (two rows: 244 us against 312).
+__host__ __device__ constexpr int patch_split(int P) { return P == 4 ? 2 : 1; }
 
 // a record prepared for its tiles; sxy = 0: not gridded
 template <int N>
@@ -2342,6 +2352,68 @@ __global__ __launch_bounds__(block) void k_patch_list(
     }
 }
 
+// For tiles of at most patch_scan_keys: the exclusive scan of their counts, and
+// their order by falling count class, so that the tiles of a dense uv core
+// start first: in grid order they came in the middle, and the chip waited for
+// them (200,000 records, supports 9-25: 1172 -> 1071 us, two polarizations,
+// 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
+// in place of hipCUB's scan (10 us).
+constexpr int patch_scan_threads = 1024;
+constexpr int patch_scan_keys = 16384;
+constexpr int patch_classes = 6;
+__global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
+  int keys, const unsigned* __restrict__ hist, unsigned* __restrict__ offsets,
+  unsigned* __restrict__ order) {
+  __shared__ unsigned a[patch_scan_keys + 1];
+  __shared__ unsigned part[patch_scan_threads / wave + 1];
+  __shared__ unsigned cls[patch_classes];
+  for (int k = threadIdx.x; k < keys; k += patch_scan_threads) a[k] = hist[k];
+  if (threadIdx.x < patch_classes) cls[threadIdx.x] = 0u;
+  __syncthreads();
+  const unsigned total = block_exclusive_scan(a, keys, part);
+  if (threadIdx.x == 0) a[keys] = total;
+  __syncthreads();
+  const int lane = threadIdx.x % wave;
+  const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
+  // class 0: over four times the mean, ..., the last: empty
+  auto class_of = [&](int k) {
+    const unsigned long long c = (unsigned long long)(a[k + 1] - a[k]) * unsigned(keys);
+    return c > 4ull * total ? 0 : c > 2ull * total ? 1 : c > total ? 2 : 4ull * c > total ? 3
+      : c ? 4 : 5;
+  };
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int r = 0; r < rounds; ++r) {
+      const int k = r * patch_scan_threads + int(threadIdx.x);
+      const int q = k < keys ? class_of(k) : -1;
+      if (pass == 0 && k < keys) offsets[k] = a[k];
+#pragma unroll
+      for (int c = 0; c < patch_classes; ++c) {
+        const unsigned long long m = __ballot(q == c);
+        if (!m) continue;
+        const int lead = __builtin_ctzll(m);
+        unsigned at = 0;
+        if (lane == lead)
+          at = __hip_atomic_fetch_add(cls + c, unsigned(__builtin_popcountll(m)),
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        at = unsigned(__builtin_amdgcn_readlane(int(at), lead));
+        if (pass == 1 && q == c)
+          order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] = unsigned(k);
+      }
+    }
+    __syncthreads();
+    if (pass == 0 && threadIdx.x == 0) {
+      unsigned run = 0;
+      for (int c = 0; c < patch_classes; ++c) {
+        const unsigned t = cls[c];
+        cls[c] = run;
+        run += t;
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) offsets[keys] = total;
+}
+
 __global__ __launch_bounds__(block) void k_zero(unsigned* __restrict__ p, size_t n) {
   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0u;
@@ -2386,19 +2458,22 @@ constexpr int patch_full = 1;  // N neighbouring elements, N even, at 16-byte
 constexpr int patch_one = 2;   // at most one element
 
 template <int N, int P, int KIND>
-__global__ __launch_bounds__(patch_block) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(patch_split(P) * patch_block)
+__attribute__((amdgpu_waves_per_eu(5)))
 void k_patch(
   Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int ptx, int pty,
-  const unsigned* __restrict__ offsets, const unsigned* __restrict__ list,
-  const PatchRec<N>* __restrict__ prs, const VisRec<N>* __restrict__ recs,
-  void* __restrict__ grid) {
+  const unsigned* __restrict__ offsets, const unsigned* __restrict__ order,
+  const unsigned* __restrict__ list, const PatchRec<N>* __restrict__ prs,
+  const VisRec<N>* __restrict__ recs, void* __restrict__ grid) {
 
   constexpr int PW = patch_w(P), PH = patch_h(P);
   constexpr int L = KIND == patch_one ? 1 : N;  // elements a lane loads per tap
-  __shared__ PatchRec<N> st[patch_block];
-  __shared__ unsigned st_i[patch_block];
+  constexpr int SPLIT = patch_split(P);
+  constexpr unsigned stage = SPLIT * patch_block;
+  __shared__ PatchRec<N> st[stage];
+  __shared__ unsigned st_i[stage];
 
-  const unsigned key = blockIdx.x;
+  const unsigned key = order ? order[blockIdx.x] : blockIdx.x;
   const unsigned beg = offsets[key];
   const unsigned cnt = offsets[key + 1] - beg;
   if (cnt == 0) return;
@@ -2408,12 +2483,13 @@ void k_patch(
   const int cube = tq / pty;
 
   const int w = uniform(int(threadIdx.x) / wave);
+  const int part = w >> 2;  // this wave's share of its pixels' entries
   const int lane = threadIdx.x % wave;
   const int row = lane % P;
   const int px = (lane / P) % PW;
   const int py = (lane / P) / PW;
   const int bx = tx * patch_tile_x(P) + (w & 1) * 2 * PW;  // the wave's pixels
-  const int by = ty * patch_tile_y(P) + (w >> 1) * 2 * PH;
+  const int by = ty * patch_tile_y(P) + ((w >> 1) & 1) * 2 * PH;
 
   // this lane's Mueller row for w <= 0: byte offsets of its elements within a
   // tap (~0u: none) and, for patch_one, the polarization they multiply; in
@@ -2449,8 +2525,8 @@ void k_patch(
 
   double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
 
-  for (unsigned b0 = 0; b0 < cnt; b0 += patch_block) {
-    const unsigned m = min(unsigned(patch_block), cnt - b0);
+  for (unsigned b0 = 0; b0 < cnt; b0 += stage) {
+    const unsigned m = min(stage, cnt - b0);
     __syncthreads();
     if (threadIdx.x < m) {
       const unsigned i = list[beg + b0 + threadIdx.x];
@@ -2459,12 +2535,12 @@ void k_patch(
     }
     __syncthreads();
     for (unsigned k0 = 0; k0 < m; k0 += wave) {
-      // lane j: does entry k0 + j touch the wave's pixels
+      // lane j: does entry k0 + j, of the wave's share, touch its pixels
       const unsigned je = min(k0 + unsigned(lane), m - 1u);
       const int hgx = st[je].gx, hgy = st[je].gy;
       const unsigned long long hbase = st[je].base;
       const unsigned hsxy = st[je].sxy, hfl = st[je].fl, hnm = st[je].nm;
-      const bool hit = k0 + unsigned(lane) < m && hgx < bx + 2 * PW
+      const bool hit = lane % SPLIT == part && k0 + unsigned(lane) < m && hgx < bx + 2 * PW
         && hgx + int(hsxy & 0xffffu) > bx && hgy < by + 2 * PH && hgy + int(hsxy >> 16) > by;
       unsigned long long todo = __ballot(hit);
       while (todo) {
@@ -2500,6 +2576,9 @@ void k_patch(
         for (int k = 0; k < 4; ++k) {
           const int dx = (k & 1) * PW, dy = (k >> 1) * PH;
           in[k] = unsigned(X + dx) < unsigned(sx) && unsigned(Y + dy) < unsigned(sy);
+          // a row without its element takes nothing
+          if constexpr (KIND == patch_one)
+            in[k] = in[k] && (eo[0] ^ (eo_x[0] & pm)) < tap_bytes;
           const unsigned off = off0 + unsigned(dy) * row_bytes + unsigned(dx) * tap_bytes;
           if constexpr (KIND == patch_full) {
             const unsigned o = in[k] ? off + (eo[0] ^ (eo_x[0] & pm)) : ~0u;
@@ -2515,7 +2594,7 @@ void k_patch(
             for (int v = 0; v < L; ++v) {
               const unsigned ev = eo[v] ^ (eo_x[v] & pm);
               const v2i_t q = __builtin_amdgcn_raw_buffer_load_b64(
-                rsrc, int(in[k] && ev < tap_bytes ? off + ev : ~0u), 0, 0);
+                rsrc, int(in[k] && (KIND == patch_one || ev < tap_bytes) ? off + ev : ~0u), 0, 0);
               c[k][v] = make_float2(__int_as_float(q.x), __int_as_float(q.y));
             }
           }
@@ -2561,7 +2640,7 @@ void k_patch(
             const float2 cc = c[k][v];
             const float pr = cc.x * g[v].x - cc.y * gs[v].y;
             const float pi = cc.x * g[v].y + cc.y * gs[v].x;
-            if constexpr (KIND == patch_full) {
+            if constexpr (KIND != patch_any) {
               sr += double(pr);
               si += double(pi);
             } else {
@@ -2573,6 +2652,31 @@ void k_patch(
           ar[k] += sr;
           ai[k] += si;
         }
+      }
+    }
+  }
+
+  if constexpr (SPLIT > 1) {
+    // the parts' sums, added by part 0 in their order
+    static_assert(sizeof(st) >= size_t(SPLIT - 1) * 4 * wave * 8 * sizeof(double), "sums in st");
+    double* sums = reinterpret_cast<double*>(st);
+    __syncthreads();
+    if (part > 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        double* q = sums + ((size_t(w - 4) * 8 + 2 * k) * wave + lane);
+        q[0] = ar[k];
+        q[wave] = ai[k];
+      }
+    }
+    __syncthreads();
+    if (part > 0) return;
+    for (int o = 1; o < SPLIT; ++o) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const double* q = sums + ((size_t(w + 4 * (o - 1)) * 8 + 2 * k) * wave + lane);
+        ar[k] += q[0];
+        ai[k] += q[wave];
       }
     }
   }
@@ -3675,8 +3779,9 @@ hipError_t launch_patch(
     cb.hist, cb.offsets, cb.patch_list)
 #define HPGX_PATCH_P(NP, PP, KD)                                               \
   hipLaunchKernelGGL(                                                          \
-    (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_block), 0, s, geo, cf.taps, mu, \
-    mode, ptx, pty, cb.offsets, cb.patch_list,                                 \
+    (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_split(PP) * patch_block), 0, s, \
+    geo, cf.taps, mu,                                                          \
+    mode, ptx, pty, cb.offsets, order, cb.patch_list,                          \
     static_cast<const PatchRec<NP>*>(cb.patch_recs),                           \
     static_cast<const VisRec<NP>*>(cb.vis), grid)
 #define HPGX_PATCH_K(NP, KD)                                                   \
@@ -3694,8 +3799,17 @@ hipError_t launch_patch(
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  size_t bytes = cb.scan_temp_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(cb.scan_temp, bytes, cb.hist, cb.offsets, int(keys + 1), s);
+  const unsigned* order = nullptr;
+  if (keys <= size_t(patch_scan_keys)) {
+    order = cb.cursor;
+    hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, int(keys), cb.hist,
+                       cb.offsets, cb.cursor);
+    e = hipGetLastError();
+  } else {
+    size_t bytes = cb.scan_temp_bytes;
+    e = hipcub::DeviceScan::ExclusiveSum(cb.scan_temp, bytes, cb.hist, cb.offsets, int(keys + 1),
+                                         s);
+  }
   if (e != hipSuccess) return e;
   switch (npol) {
   case 1:
