@@ -407,6 +407,13 @@ int ensure_call_buffers(hpgx_state_t st) {
         HPGX_HIP(st, dev_alloc(cb.patch_list, recs * tiles * sizeof(unsigned)));
         cb.patch_list_capacity = recs * tiles;
       }
+      const size_t table = hpgx::patch_table_entries(st->geometry(), recs);
+      if (table > cb.patch_table_capacity) {
+        dev_free(cb.patch_table);
+        cb.patch_table_capacity = 0;
+        HPGX_HIP(st, dev_alloc(cb.patch_table, table * sizeof(unsigned)));
+        cb.patch_table_capacity = table;
+      }
     }
     // bin entries for the whole batch, up to the entry memory budget; larger
     // batches are gridded in chunks (run_grid)
@@ -516,6 +523,7 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.tally_keys);
   dev_free(cb.patch_recs);
   dev_free(cb.patch_list);
+  dev_free(cb.patch_table);
   dev_free(cb.hist);
   dev_free(cb.offsets);
   dev_free(cb.cursor);
@@ -988,10 +996,14 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
     c.scan_temp = p;
     c.scan_temp_bytes = st->cb.scan_temp_bytes;
     p += up(c.scan_temp_bytes);
-    const size_t used = size_t(p - static_cast<char*>(base)) + 256;
-    const size_t recs = noalloc_scratch_bytes > used
-      ? std::min(n, (noalloc_scratch_bytes - used) / (rec + tiles * sizeof(unsigned)))
-      : 0;
+    const size_t used = size_t(p - static_cast<char*>(base)) + 2 * 256;
+    auto fits = [&](size_t r) {
+      return used + r * (rec + tiles * sizeof(unsigned))
+          + hpgx::patch_table_entries(st->geometry(), r) * sizeof(unsigned)
+        <= noalloc_scratch_bytes;
+    };
+    size_t recs = n;
+    while (recs > 0 && !fits(recs)) recs -= (recs + 7) / 8;
     if (recs == 0)
       return fail(st, HPGX_ERR_OTHER, "hpgx_grid_visibilities_noalloc: scratch layout overflow");
     c.patch_recs = p;
@@ -999,6 +1011,9 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
     p += up(recs * rec);
     c.patch_list = reinterpret_cast<unsigned*>(p);
     c.patch_list_capacity = recs * tiles;
+    p += up(recs * tiles * sizeof(unsigned));
+    c.patch_table = reinterpret_cast<unsigned*>(p);
+    c.patch_table_capacity = hpgx::patch_table_entries(st->geometry(), recs);
     pass_blocks = 0;
     return HPGX_SUCCESS;
   }

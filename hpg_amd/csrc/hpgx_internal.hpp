@@ -90,6 +90,8 @@ struct CallBuffers {
   size_t patch_capacity;
   unsigned* patch_list;   // and the tiles' lists of record indexes
   size_t patch_list_capacity;
+  unsigned* patch_table;  // and the workgroups' places in them (few tiles)
+  size_t patch_table_capacity;
   unsigned* degrid_order; // launch_degrid: keys, sorted keys, record indexes,
                           // sorted indexes, order_capacity each
   void* degrid_recs;      // and its prepared records (DegridRec)
@@ -189,6 +191,8 @@ hipError_t launch_tile_sub(
 // patch_tiles_per_footprint indexes for each
 size_t patch_keys(const Geometry& geo);
 size_t patch_rec_bytes(int npol);
+// values of cb.patch_table for n records a call (0 for many tiles)
+size_t patch_table_entries(const Geometry& geo, size_t n);
 size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy);
 hipError_t launch_patch(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,

@@ -2201,28 +2201,40 @@ static_assert(sizeof(PatchRec<1>) == 48 && sizeof(PatchRec<4>) == 64, "PatchRec 
 // workgroup's LDS, which adds into the grid weights once at its end (the
 // workgroups stride over the records, so a few thousand global atomics per
 // plane instead of one per wave).
-template <int N>
-__global__ __launch_bounds__(block) void k_patch_prep(
+// LOCAL (at most patch_local_keys tiles): the workgroup, of `batch` records in a
+// row, counts its tiles in LDS, adds its counts to hist once per tile, and
+// keeps each tile's place for it in its row of `table`, so that k_patch_list
+// places the entries without global atomics (10 G/s over the chip: they were
+// all of the two kernels' time: 284 + 265 us for 300,000 records of supports 9-33
+// on 4096 tiles, now 48 + 19).
+constexpr int patch_local_threads = 1024;
+constexpr int patch_local_keys = 16384;
+template <int N, bool LOCAL>
+__global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_prep(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int gvis_ready, int adjoint,
   const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
   int ptx, int pty, int tw, int th, PatchRec<N>* __restrict__ out,
   unsigned* __restrict__ hist, double* __restrict__ weights,
-  unsigned long long* __restrict__ invalid) {
+  unsigned long long* __restrict__ invalid, unsigned batch, unsigned* __restrict__ table) {
 
   __shared__ double wblk[count_planes_lds];
+  __shared__ unsigned cnt[LOCAL ? patch_local_keys : 1];
+  const int keys = ptx * pty * geo.nc;
+  if constexpr (LOCAL)
+    for (int k = threadIdx.x; k < keys; k += blockDim.x) cnt[k] = 0u;
   const int nplanes = geo.nr * geo.nc;
   const bool lds_w = update_weights && nplanes <= count_planes_lds;
   if (lds_w)
     for (int k = threadIdx.x; k < nplanes; k += blockDim.x) wblk[k] = 0.0;
   __syncthreads();
 
-  const size_t stride = size_t(gridDim.x) * blockDim.x;
-  const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  const size_t stride = LOCAL ? blockDim.x : size_t(gridDim.x) * blockDim.x;
+  const size_t i0 = blockIdx.x * (size_t)(LOCAL ? batch : blockDim.x) + threadIdx.x;
   // every thread runs the same number of iterations (the wave reductions
   // below need all lanes)
-  const size_t iters = (n + stride - 1) / stride;
+  const size_t iters = LOCAL ? (batch + stride - 1) / stride : (n + stride - 1) / stride;
   for (size_t it = 0; it < iters; ++it) {
     const size_t i = i0 + it * stride;
     bool counted = false;
@@ -2295,7 +2307,11 @@ __global__ __launch_bounds__(block) void k_patch_prep(
             const int ty0 = c.gy / th, ty1 = (c.gy + g.sy - 1) / th;
             for (int ty = ty0; ty <= ty1; ++ty)
               for (int tx = tx0; tx <= tx1; ++tx)
-                atomicAdd(hist + (size_t(gcube) * pty + ty) * ptx + tx, 1u);
+                if constexpr (LOCAL)
+                  __hip_atomic_fetch_add(cnt + (int(gcube) * pty + ty) * ptx + tx, 1u,
+                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                else
+                  atomicAdd(hist + (size_t(gcube) * pty + ty) * ptx + tx, 1u);
           }
         }
       }
@@ -2324,32 +2340,52 @@ __global__ __launch_bounds__(block) void k_patch_prep(
       }
     }
   }
-  if (lds_w) {
-    __syncthreads();
+  if (lds_w || LOCAL) __syncthreads();
+  if (lds_w)
     for (int k = threadIdx.x; k < nplanes; k += blockDim.x)
       if (wblk[k] != 0.0) atomicAdd(weights + k, wblk[k]);
+  if constexpr (LOCAL) {
+    unsigned* row = table + size_t(blockIdx.x) * keys;
+    for (int k = threadIdx.x; k < keys; k += blockDim.x)
+      row[k] = cnt[k] ? atomicAdd(hist + k, cnt[k]) : 0u;
   }
 }
 
-// hist counts down: an entry's place in its tile's list is what is left
-template <int N>
-__global__ __launch_bounds__(block) void k_patch_list(
-  size_t n, int ptx, int pty, int tw, int th, const PatchRec<N>* __restrict__ prs,
+// an entry's place in its tile's list: hist counts down what is left, or
+// (LOCAL) the workgroup counts up from its place
+template <int N, bool LOCAL>
+__global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_list(
+  size_t n, int nc, int ptx, int pty, int tw, int th, const PatchRec<N>* __restrict__ prs,
   unsigned* __restrict__ hist, const unsigned* __restrict__ offsets,
-  unsigned* __restrict__ list) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const unsigned sxy = prs[i].sxy;
-  if (!sxy) return;
-  const int gx = prs[i].gx, gy = prs[i].gy;
-  const unsigned gcube = prs[i].cube;
-  const int tx0 = gx / tw, tx1 = (gx + int(sxy & 0xffffu) - 1) / tw;
-  const int ty0 = gy / th, ty1 = (gy + int(sxy >> 16) - 1) / th;
-  for (int ty = ty0; ty <= ty1; ++ty)
-    for (int tx = tx0; tx <= tx1; ++tx) {
-      const size_t key = (size_t(gcube) * pty + ty) * ptx + tx;
-      list[offsets[key] + atomicSub(hist + key, 1u) - 1u] = unsigned(i);
-    }
+  unsigned* __restrict__ list, unsigned batch, const unsigned* __restrict__ table) {
+  __shared__ unsigned at[LOCAL ? patch_local_keys : 1];
+  const size_t first = blockIdx.x * (size_t)(LOCAL ? batch : blockDim.x);
+  if constexpr (LOCAL) {
+    const int keys = ptx * pty * nc;
+    const unsigned* row = table + size_t(blockIdx.x) * keys;
+    for (int k = threadIdx.x; k < keys; k += blockDim.x) at[k] = offsets[k] + row[k];
+    __syncthreads();
+  }
+  const size_t last = min(n, first + (LOCAL ? size_t(batch) : size_t(blockDim.x)));
+  for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
+    const unsigned sxy = prs[i].sxy;
+    if (!sxy) continue;
+    const int gx = prs[i].gx, gy = prs[i].gy;
+    const unsigned gcube = prs[i].cube;
+    const int tx0 = gx / tw, tx1 = (gx + int(sxy & 0xffffu) - 1) / tw;
+    const int ty0 = gy / th, ty1 = (gy + int(sxy >> 16) - 1) / th;
+    for (int ty = ty0; ty <= ty1; ++ty)
+      for (int tx = tx0; tx <= tx1; ++tx) {
+        const size_t key = (size_t(gcube) * pty + ty) * ptx + tx;
+        unsigned pos;
+        if constexpr (LOCAL)
+          pos = __hip_atomic_fetch_add(at + key, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+        else
+          pos = offsets[key] + atomicSub(hist + key, 1u) - 1u;
+        list[pos] = unsigned(i);
+      }
+  }
 }
 
 // For tiles of at most patch_scan_keys: the exclusive scan of their counts, and
@@ -2359,7 +2395,7 @@ __global__ __launch_bounds__(block) void k_patch_list(
 // 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
 // in place of hipCUB's scan (10 us).
 constexpr int patch_scan_threads = 1024;
-constexpr int patch_scan_keys = 16384;
+constexpr int patch_scan_keys = patch_local_keys;
 constexpr int patch_classes = 6;
 __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
   int keys, const unsigned* __restrict__ hist, unsigned* __restrict__ offsets,
@@ -3723,6 +3759,15 @@ int patch_tiles_y(const Geometry& geo) {
 size_t patch_keys(const Geometry& geo) {
   return size_t(patch_tiles_x(geo)) * patch_tiles_y(geo) * geo.nc;
 }
+// records of a workgroup that counts in LDS: 2048, or more so that there are
+// at most 512 rows of places
+size_t patch_batch(size_t n) {
+  return std::max<size_t>(2048, ((n + 511) / 512 + 1023) / 1024 * 1024);
+}
+size_t patch_table_entries(const Geometry& geo, size_t n) {
+  const size_t keys = patch_keys(geo);
+  return keys <= size_t(patch_local_keys) ? std::min<size_t>((n + 2047) / 2048, 512) * keys : 0;
+}
 size_t patch_rec_bytes(int npol) {
   switch (npol) {
   case 1: return sizeof(PatchRec<1>);
@@ -3765,18 +3810,26 @@ hipError_t launch_patch(
   const int kind = patch_kind(npol, geo, cf, mu);
   // a kernel, not a memset: a captured graph may replay it
   hipLaunchKernelGGL(k_zero, dim3(blocks_for(keys + 1)), dim3(block), 0, s, cb.hist, keys + 1);
+  const bool local = keys <= size_t(patch_local_keys);
+  const size_t batch = patch_batch(n);
+  const unsigned nb = local ? unsigned((n + batch - 1) / batch) : 0u;
+  if (local && nb * keys > cb.patch_table_capacity) return hipErrorInvalidValue;
 #define HPGX_PREP(NP)                                                          \
   hipLaunchKernelGGL(                                                          \
-    k_patch_prep<NP>, dim3(std::min(blocks_for(n), count_blocks_max)), dim3(block), 0, s, \
+    local ? (k_patch_prep<NP, true>) : (k_patch_prep<NP, false>),              \
+    dim3(local ? nb : std::min(blocks_for(n), count_blocks_max)),              \
+    dim3(local ? patch_local_threads : block), 0, s,                           \
     static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
     int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint), cb.gvis, residuals, \
     ptx, pty, patch_tile_x(P), patch_tile_y(P), static_cast<PatchRec<NP>*>(cb.patch_recs), \
-    cb.hist, weights, cb.invalid_count)
+    cb.hist, weights, cb.invalid_count, unsigned(batch), cb.patch_table)
 #define HPGX_LIST(NP)                                                          \
   hipLaunchKernelGGL(                                                          \
-    k_patch_list<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, ptx, pty,     \
+    local ? (k_patch_list<NP, true>) : (k_patch_list<NP, false>),              \
+    dim3(local ? nb : blocks_for(n)), dim3(local ? patch_local_threads : block), 0, s, n, \
+    geo.nc, ptx, pty,                                                          \
     patch_tile_x(P), patch_tile_y(P), static_cast<const PatchRec<NP>*>(cb.patch_recs), \
-    cb.hist, cb.offsets, cb.patch_list)
+    cb.hist, cb.offsets, cb.patch_list, unsigned(batch), cb.patch_table)
 #define HPGX_PATCH_P(NP, PP, KD)                                               \
   hipLaunchKernelGGL(                                                          \
     (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_split(PP) * patch_block), 0, s, \
@@ -3800,7 +3853,7 @@ hipError_t launch_patch(
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const unsigned* order = nullptr;
-  if (keys <= size_t(patch_scan_keys)) {
+  if (local) {
     order = cb.cursor;
     hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, int(keys), cb.hist,
                        cb.offsets, cb.cursor);
