@@ -470,12 +470,12 @@ int ensure_call_buffers(hpgx_state_t st) {
     if (st->model && !use_degrid_binned(st) && st->vis_capacity > cb.order_capacity) {
       dev_free(cb.degrid_order);
       dev_free(cb.degrid_recs);
-      dev_free(cb.order_temp);
+      dev_free(cb.degrid_bins);
       cb.order_capacity = 0;
-      cb.order_temp_bytes = hpgx::degrid_order_temp_bytes(st->vis_capacity);
       HPGX_HIP(st, dev_alloc(cb.degrid_order, 4 * st->vis_capacity * sizeof(unsigned)));
       HPGX_HIP(st, dev_alloc(cb.degrid_recs, st->vis_capacity * hpgx::degrid_rec_bytes()));
-      HPGX_HIP(st, dev_alloc(cb.order_temp, cb.order_temp_bytes));
+      HPGX_HIP(st, dev_alloc(cb.degrid_bins, hpgx::degrid_bins_entries(st->vis_capacity)
+                                               * sizeof(unsigned)));
       cb.order_capacity = st->vis_capacity;
     }
     if (need > cb.entries_capacity) {
@@ -536,7 +536,7 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.scan_temp);
   dev_free(cb.degrid_order);
   dev_free(cb.degrid_recs);
-  dev_free(cb.order_temp);
+  dev_free(cb.degrid_bins);
   dev_free(cb.invalid_count);
   if (st->plan_z2z.valid) hipfftDestroy(st->plan_z2z.h);
   if (st->plan_c2c.valid) hipfftDestroy(st->plan_c2c.h);

@@ -92,12 +92,12 @@ struct CallBuffers {
   size_t patch_list_capacity;
   unsigned* patch_table;  // and the workgroups' places in them (few tiles)
   size_t patch_table_capacity;
-  unsigned* degrid_order; // launch_degrid: keys, sorted keys, record indexes,
-                          // sorted indexes, order_capacity each
+  unsigned* degrid_order; // launch_degrid: keys, the record order, (key, record)
+                          // pairs, 4 order_capacity values,
+  unsigned* degrid_bins;  // the sort's counts, offsets and places
+                          // (degrid_bins_entries),
   void* degrid_recs;      // and its prepared records (DegridRec)
   size_t order_capacity;
-  void* order_temp;       // the sort's temporary storage
-  size_t order_temp_bytes;
 };
 
 struct DeviceCF {
@@ -219,9 +219,10 @@ hipError_t launch_degrid_finish(
 // slice-ordered degridding of the records at `records`: FP64 predictions to
 // pred64, or predicted values (residuals, and gvis in cb, when do_grid)
 // written into out_records when not null, which may be `records`.  With a
-// model, cb.degrid_order, degrid_recs and degrid_acc hold at least n records.
+// model, cb.degrid_order, degrid_bins, degrid_recs and degrid_acc hold at least n
+// records.
 size_t degrid_rec_bytes();
-size_t degrid_order_temp_bytes(size_t n);
+size_t degrid_bins_entries(size_t n);
 hipError_t launch_degrid(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb, double2* pred64,

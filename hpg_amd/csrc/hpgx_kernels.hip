@@ -2393,7 +2393,7 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_l
 // start first: in grid order they came in the middle, and the chip waited for
 // them (200,000 records, supports 9-25: 1172 -> 1071 us, two polarizations,
 // 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
-// in place of hipCUB's scan (10 us).
+// in place of hipCUB's scan (10 us).  order null: the scan alone.
 constexpr int patch_scan_threads = 1024;
 constexpr int patch_scan_keys = patch_local_keys;
 constexpr int patch_classes = 6;
@@ -2409,6 +2409,10 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
   const unsigned total = block_exclusive_scan(a, keys, part);
   if (threadIdx.x == 0) a[keys] = total;
   __syncthreads();
+  if (!order) {
+    for (int k = threadIdx.x; k <= keys; k += patch_scan_threads) offsets[k] = a[k];
+    return;
+  }
   const int lane = threadIdx.x % wave;
   const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
   // class 0: over four times the mean, ..., the last: empty
@@ -2744,9 +2748,14 @@ void k_patch(
 // ---- degridding --------------------------------------------------------
 
 // The slice-ordered degridder, for several polarizations, large supports and
-// large grids: k_degrid_keys prepares the records, a radix sort orders them
-// by CF slice, k_degrid sums c' x model over their supports and
-// k_degrid_finish makes predictions of the sums.
+// large grids: k_degrid_keys prepares the records, k_degrid_place and
+// k_degrid_sort order them by CF slice, k_degrid sums c' x model over their
+// supports and k_degrid_finish makes predictions of the sums.  The order is a
+// counting sort in two levels, the upper bits of the keys in at most
+// patch_local_keys bins as the tile lists of k_patch (LDS counts, one global
+// atomic per workgroup and bin), the lower 2^low_bits within a bin in LDS: 4
+// short launches, 35 us for 1e6 records of 3e5 keys and 25 for 300,000, against
+// 130 and 104 us of hipCUB's radix sort (two-polarization residuals 752 -> 649 us).
 
 // a record prepared for k_degrid; sxy = 0: not degridded
 struct __align__(16) DegridRec {
@@ -2758,48 +2767,132 @@ struct __align__(16) DegridRec {
   unsigned pad;
 };
 
-// key = the record's (grid cube, region, group, CF cube, fine offsets), kmax
-// for records that are skipped (no CF, outside the grid); region (region_sh
-// below 31) the square of 2^region_sh pixels that holds the support corner
+struct DegridKeys {
+  unsigned slices, stride;  // of the batch, of a group
+  int region_sh;
+  unsigned regions_x, regions;
+  int drop_bits, low_bits, bins;  // the key's bits, from the lowest
+};
+
+// key = the record's (grid cube, region, group, CF cube, fine offsets), ~0 for
+// records that are skipped (no CF, outside the grid); region (region_sh below
+// 31) the square of 2^region_sh pixels that holds the support corner.  keys
+// null: prepared only
 template <int N>
-__global__ void k_degrid_keys(
+__global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
   size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const VisRec<N>* __restrict__ recs, unsigned stride, unsigned slices, int region_sh,
-  unsigned regions_x, unsigned regions, unsigned kmax,
-  unsigned* __restrict__ keys, unsigned* __restrict__ idx, DegridRec* __restrict__ out) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const VisRec<N>& r = recs[i];
-  const unsigned grp = r.cf_index[1];
-  const unsigned cfcube = r.cf_index[0];
-  const unsigned gcube = r.grid_cube;
-  unsigned key = kmax;
-  DegridRec d{};
-  if (grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc)) {
-    const GroupInfo g = groups[grp];
-    if (cfcube < unsigned(g.ncube)) {
-      const Coord c = vis_coord(r, geo, g);
-      if (c.inside) {
-        const unsigned fxi = unsigned(c.fx + geo.F), fyi = unsigned(c.fy + geo.F);
-        const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-        const unsigned region = (unsigned(c.gy) >> region_sh) * regions_x
-          + (unsigned(c.gx) >> region_sh);
-        key = (gcube * regions + region) * slices + grp * stride
-          + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
-        d.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi));
-        d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
-        d.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
-        d.fl = unsigned((r.uvw[2] > 0 ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
-          | (fxi << 8) | (fyi << 16);
-        d.nm = unsigned(g.nmueller);
+  const VisRec<N>* __restrict__ recs, DegridKeys dk, unsigned batch, unsigned* __restrict__ keys,
+  DegridRec* __restrict__ out, unsigned* __restrict__ hist, unsigned* __restrict__ table) {
+  __shared__ unsigned cnt[patch_local_keys];
+  const int shift = dk.low_bits + dk.drop_bits;
+  if (keys)
+    for (int k = threadIdx.x; k < dk.bins; k += blockDim.x) cnt[k] = 0u;
+  __syncthreads();
+  const size_t first = blockIdx.x * (size_t)batch;
+  const size_t last = min(n, first + batch);
+  for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
+    const VisRec<N>& r = recs[i];
+    const unsigned grp = r.cf_index[1];
+    const unsigned cfcube = r.cf_index[0];
+    const unsigned gcube = r.grid_cube;
+    unsigned key = ~0u;
+    DegridRec d{};
+    if (grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc)) {
+      const GroupInfo g = groups[grp];
+      if (cfcube < unsigned(g.ncube)) {
+        const Coord c = vis_coord(r, geo, g);
+        if (c.inside) {
+          const unsigned fxi = unsigned(c.fx + geo.F), fyi = unsigned(c.fy + geo.F);
+          const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
+          const unsigned region = (unsigned(c.gy) >> dk.region_sh) * dk.regions_x
+            + (unsigned(c.gx) >> dk.region_sh);
+          key = (gcube * dk.regions + region) * dk.slices + grp * dk.stride
+            + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
+          d.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi));
+          d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
+          d.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
+          d.fl = unsigned((r.uvw[2] > 0 ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
+            | (fxi << 8) | (fyi << 16);
+          d.nm = unsigned(g.nmueller);
+          if (keys)
+            __hip_atomic_fetch_add(cnt + (key >> shift), 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
       }
     }
+    if (keys) keys[i] = key;
+    out[i] = d;
   }
-  if (keys) {
-    keys[i] = key;
-    idx[i] = unsigned(i);
+  if (!keys) return;
+  __syncthreads();
+  unsigned* row = table + size_t(blockIdx.x) * dk.bins;
+  for (int k = threadIdx.x; k < dk.bins; k += blockDim.x)
+    row[k] = cnt[k] ? atomicAdd(hist + k, cnt[k]) : 0u;
+}
+
+// the records into their bins: (lower key bits, record) pairs
+__global__ __launch_bounds__(patch_local_threads) void k_degrid_place(
+  size_t n, DegridKeys dk, unsigned batch, const unsigned* __restrict__ keys,
+  const unsigned* __restrict__ offsets, const unsigned* __restrict__ table,
+  unsigned* __restrict__ order, uint2* __restrict__ pairs) {
+  __shared__ unsigned at[patch_local_keys];
+  const int shift = dk.low_bits + dk.drop_bits;
+  const unsigned* row = table + size_t(blockIdx.x) * dk.bins;
+  for (int k = threadIdx.x; k < dk.bins; k += blockDim.x) at[k] = offsets[k] + row[k];
+  __syncthreads();
+  const size_t first = blockIdx.x * (size_t)batch;
+  const size_t last = min(n, first + batch);
+  for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
+    const unsigned key = keys[i];
+    if (key == ~0u) continue;
+    const unsigned pos = __hip_atomic_fetch_add(at + (key >> shift), 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (dk.low_bits)
+      pairs[pos] = make_uint2((key >> dk.drop_bits) & ((1u << dk.low_bits) - 1u), unsigned(i));
+    else
+      order[pos] = unsigned(i);  // the bins are the slices
   }
-  out[i] = d;
+}
+
+// one workgroup per bin: its records in order of their lower key bits
+constexpr int degrid_sort_threads = 256;
+constexpr int degrid_sort_loads = 8;
+constexpr int degrid_low_keys = 8192;
+__global__ __launch_bounds__(degrid_sort_threads) void k_degrid_sort(
+  int low_keys, const unsigned* __restrict__ offsets, const uint2* __restrict__ pairs,
+  unsigned* __restrict__ order) {
+  __shared__ unsigned low[degrid_low_keys];
+  __shared__ unsigned part[degrid_sort_threads / wave + 1];
+  constexpr unsigned stride = degrid_sort_threads * degrid_sort_loads;
+  const unsigned beg = offsets[blockIdx.x], end = offsets[blockIdx.x + 1];
+  if (end - beg <= 1u) {
+    if (threadIdx.x == 0 && end != beg) order[beg] = pairs[beg].y;
+    return;
+  }
+  for (int k = threadIdx.x; k < low_keys; k += degrid_sort_threads) low[k] = 0u;
+  __syncthreads();
+  for (int pass = 0; pass < 2; ++pass) {
+    for (size_t first = beg; first < end; first += stride) {
+      uint2 p[degrid_sort_loads];
+#pragma unroll
+      for (int j = 0; j < degrid_sort_loads; ++j) {
+        const size_t k = first + j * degrid_sort_threads + threadIdx.x;
+        p[j] = k < end ? pairs[k] : make_uint2(~0u, 0u);
+      }
+#pragma unroll
+      for (int j = 0; j < degrid_sort_loads; ++j) {
+        if (p[j].x == ~0u) continue;
+        const unsigned at = __hip_atomic_fetch_add(low + p[j].x, 1u, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (pass) order[beg + at] = p[j].y;
+      }
+    }
+    __syncthreads();
+    if (!pass) {
+      block_exclusive_scan(low, low_keys, part);
+      __syncthreads();
+    }
+  }
 }
 
 // sums val[0, V) of the lanes that differ in bits 1 .. MASK of their number.
@@ -2841,7 +2934,7 @@ constexpr int degrid_recs = 4;
 // load by lines, 16 for 64 lanes of 16 bytes so, 64 with the rows in
 // neighbouring lanes: 1.2 ms against 0.97 for 300,000 records of supports 9-33
 // and one element a row).  The sums over the support go to acc (record x polarization).
-// order null: the records as they come.  same_rows: M and Mc are equal, so
+// order null: the records as they come, else *ordered of them.  same_rows: M and Mc are equal, so
 // that records of both signs of w share CF values (the model's imaginary part
 // takes the sign: sum conj(c) m = conj(sum c conj(m))).  patch_one: no two
 // rows use one polarization; acc of one that no row uses is not written.
@@ -2860,7 +2953,7 @@ void k_degrid(
   size_t n, Geometry geo, const float2* __restrict__ taps, Mueller mu, int same_rows,
   const double2* __restrict__ model, int by_xcd, const DegridRec* __restrict__ drs,
   const VisRec<N>* __restrict__ recs, const unsigned* __restrict__ order,
-  double* __restrict__ acc) {
+  const unsigned* __restrict__ ordered, double* __restrict__ acc) {
 
   constexpr int R = degrid_recs;
   constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
@@ -2870,6 +2963,7 @@ void k_degrid(
   const int lane = threadIdx.x % wave;
   const unsigned bi = by_xcd ? xcd_key(blockIdx.x, gridDim.x) : blockIdx.x;
   const size_t p0 = (bi * (size_t)(block / wave) + w) * R;
+  if (order) n = *ordered;  // the records that are not skipped
   if (p0 >= n) return;
   const int row = lane / TPS;
   const int q = lane % TPS;
@@ -3944,14 +4038,8 @@ hipError_t launch_degrid_finish(
 }
 
 size_t degrid_rec_bytes() { return sizeof(DegridRec); }
-
-size_t degrid_order_temp_bytes(size_t n) {
-  size_t bytes = 0;
-  (void)hipcub::DeviceRadixSort::SortPairs(
-    nullptr, bytes, static_cast<unsigned*>(nullptr), static_cast<unsigned*>(nullptr),
-    static_cast<unsigned*>(nullptr), static_cast<unsigned*>(nullptr),
-    int(std::min<size_t>(n, 0x7fffffffull)), 0, 32);
-  return bytes;
+size_t degrid_bins_entries(size_t n) {
+  return (2 + std::min<size_t>((n + 2047) / 2048, 512)) * (patch_local_keys + 1);
 }
 
 hipError_t launch_degrid(
@@ -4014,18 +4102,43 @@ hipError_t launch_degrid(
   const unsigned long long regions = count(geo.nx) * count(geo.ny);
   const bool by_cube = slices * regions * geo.nc < key_limit;
   const unsigned long long kmax = by_cube ? slices * regions * geo.nc : slices;
-  const bool sorted = n <= 0x7fffffffull && kmax > 0 && kmax < key_limit;
+  // Bins: at most half of the records that one workgroup counts (its global
+  // atomics, one for each of its bins, at 10 G/s of the card), not fewer than
+  // 1024 for the second level's workgroups.  Keys beyond patch_local_keys bins
+  // of degrid_low_keys lose their lowest bits: 2^27 of them, more than the
+  // records of a call in practice, have next to no two records of one slice.
+  const bool sorted = kmax > 0 && kmax < key_limit;
+  const size_t batch = patch_batch(n);
+  const unsigned nb = unsigned((n + batch - 1) / batch);
+  DegridKeys dk{};
+  dk.slices = unsigned(slices);
+  dk.stride = unsigned(stride);
+  dk.region_sh = region_sh;
+  dk.regions_x = unsigned(count(geo.nx));
+  dk.regions = unsigned(by_cube ? regions : 0ull);
+  if (sorted) {
+    const unsigned long long most = std::clamp<unsigned long long>(batch / 2, 1024, patch_local_keys);
+    auto bins_at = [&](int bits) { return ((kmax - 1) >> bits) + 1; };
+    while ((1 << dk.low_bits) < degrid_low_keys && bins_at(dk.low_bits) > most) ++dk.low_bits;
+    while (bins_at(dk.low_bits + dk.drop_bits) > (unsigned long long)patch_local_keys)
+      ++dk.drop_bits;
+    dk.bins = int(bins_at(dk.low_bits + dk.drop_bits));
+  }
   DegridRec* drs = static_cast<DegridRec*>(cb.degrid_recs);
   unsigned* keys = sorted ? cb.degrid_order : nullptr;
-  unsigned* keys_sorted = cb.degrid_order + cb.order_capacity;
-  unsigned* idx = cb.degrid_order + 2 * cb.order_capacity;
-  unsigned* idx_sorted = cb.degrid_order + 3 * cb.order_capacity;
+  unsigned* sorted_idx = cb.degrid_order + cb.order_capacity;
+  uint2* pairs = reinterpret_cast<uint2*>(cb.degrid_order + 2 * cb.order_capacity);
+  unsigned* hist = cb.degrid_bins;  // counts, offsets, then the table
+  unsigned* offsets = hist + patch_local_keys + 1;
+  unsigned* table = offsets + patch_local_keys + 1;
+  if (sorted)
+    hipLaunchKernelGGL(k_zero, dim3(blocks_for(size_t(dk.bins))), dim3(block), 0, s, hist,
+                       size_t(dk.bins));
 #define HPGX_DKEYS(NP)                                                         \
   hipLaunchKernelGGL(                                                          \
-    k_degrid_keys<NP>, dim3(blocks_for(n)), dim3(block), 0, s, n, geo,         \
-    cf.groups, static_cast<const VisRec<NP>*>(records), unsigned(stride),      \
-    unsigned(slices), region_sh, unsigned(count(geo.nx)), unsigned(by_cube ? regions : 0ull), \
-    unsigned(kmax), keys, idx, drs)
+    k_degrid_keys<NP>, dim3(nb), dim3(patch_local_threads), 0, s, n, geo,      \
+    cf.groups, static_cast<const VisRec<NP>*>(records), dk, unsigned(batch),   \
+    keys, drs, hist, table)
   switch (npol) {
   case 1: HPGX_DKEYS(1); break;
   case 2: HPGX_DKEYS(2); break;
@@ -4037,12 +4150,16 @@ hipError_t launch_degrid(
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (sorted) {
-    const int bits = 32 - __builtin_clz(unsigned(kmax));
-    size_t bytes = cb.order_temp_bytes;
-    e = hipcub::DeviceRadixSort::SortPairs(cb.order_temp, bytes, keys, keys_sorted, idx,
-                                           idx_sorted, int(n), 0, bits, s);
+    hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, dk.bins, hist,
+                       offsets, static_cast<unsigned*>(nullptr));
+    hipLaunchKernelGGL(k_degrid_place, dim3(nb), dim3(patch_local_threads), 0, s, n, dk,
+                       unsigned(batch), keys, offsets, table, sorted_idx, pairs);
+    if (dk.low_bits)
+      hipLaunchKernelGGL(k_degrid_sort, dim3(unsigned(dk.bins)), dim3(degrid_sort_threads), 0, s,
+                         1 << dk.low_bits, offsets, pairs, sorted_idx);
+    e = hipGetLastError();
     if (e != hipSuccess) return e;
-    order = idx_sorted;
+    order = sorted_idx;
   }
 #define HPGX_DEGRID_P(NP, PP, KD)                                              \
   do {                                                                         \
@@ -4050,7 +4167,7 @@ hipError_t launch_degrid(
     hipLaunchKernelGGL(                                                        \
       (k_degrid<NP, PP, KD>), dim3(unsigned((n + per - 1) / per)), dim3(block), 0, s, n, geo, \
       cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,            \
-      static_cast<const VisRec<NP>*>(records), order,                          \
+      static_cast<const VisRec<NP>*>(records), order, offsets + dk.bins,       \
       reinterpret_cast<double*>(cb.degrid_acc));                               \
   } while (0)
 #define HPGX_DEGRID_K(NP, KD)                                                  \
