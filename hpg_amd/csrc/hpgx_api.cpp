@@ -463,19 +463,24 @@ int ensure_call_buffers(hpgx_state_t st) {
       dev_free(cb.tally_keys);
       cb.tally_capacity = 0;
       HPGX_HIP(st, dev_alloc(cb.tally_entries, need * hpgx::halo_entry_bytes(int(st->npol))));
-      HPGX_HIP(st, dev_alloc(cb.tally_keys, need * 2 * sizeof(unsigned)));
+      HPGX_HIP(st, dev_alloc(cb.tally_keys, need * 3 * sizeof(unsigned)));
       cb.tally_capacity = need;
+    }
+    if ((use_sub_global(st) || (st->model && !use_degrid_binned(st)))
+        && st->vis_capacity > cb.sort_capacity) {
+      dev_free(cb.sort_bins);
+      cb.sort_capacity = 0;
+      HPGX_HIP(st, dev_alloc(cb.sort_bins, hpgx::sort_bins_entries(st->vis_capacity)
+                                             * sizeof(unsigned)));
+      cb.sort_capacity = st->vis_capacity;
     }
     // the slice-ordered degridder's record order, once a model is set
     if (st->model && !use_degrid_binned(st) && st->vis_capacity > cb.order_capacity) {
       dev_free(cb.degrid_order);
       dev_free(cb.degrid_recs);
-      dev_free(cb.degrid_bins);
       cb.order_capacity = 0;
       HPGX_HIP(st, dev_alloc(cb.degrid_order, 4 * st->vis_capacity * sizeof(unsigned)));
       HPGX_HIP(st, dev_alloc(cb.degrid_recs, st->vis_capacity * hpgx::degrid_rec_bytes()));
-      HPGX_HIP(st, dev_alloc(cb.degrid_bins, hpgx::degrid_bins_entries(st->vis_capacity)
-                                               * sizeof(unsigned)));
       cb.order_capacity = st->vis_capacity;
     }
     if (need > cb.entries_capacity) {
@@ -536,7 +541,7 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.scan_temp);
   dev_free(cb.degrid_order);
   dev_free(cb.degrid_recs);
-  dev_free(cb.degrid_bins);
+  dev_free(cb.sort_bins);
   dev_free(cb.invalid_count);
   if (st->plan_z2z.valid) hipfftDestroy(st->plan_z2z.h);
   if (st->plan_c2c.valid) hipfftDestroy(st->plan_c2c.h);
@@ -907,19 +912,16 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
     c.gvis = cb.gvis + off * np;
     const double2* res = residuals ? residuals + off * np : nullptr;
     const bool sub = use_sub_global(st);
-    const size_t keys = sub ? 4 * st->nkeys : st->nkeys;
-    HPGX_HIP(st, hipMemsetAsync(c.hist, 0, (keys + 1) * sizeof(unsigned), st->stream));
     if (sub) {
       HPGX_HIP(st, hpgx::launch_tally(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, gvis_ready, src,
                      res, c, st->weights));
-      HPGX_HIP(st, hpgx::launch_scan(st->stream, keys, c));
-      HPGX_HIP(st, hpgx::launch_place(st->stream, np, m, geo, c));
     } else {
+      HPGX_HIP(st, hipMemsetAsync(c.hist, 0, (st->nkeys + 1) * sizeof(unsigned), st->stream));
       HPGX_HIP(st, hpgx::launch_count(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, true, c,
                      st->weights, true));
-      HPGX_HIP(st, hpgx::launch_scan(st->stream, keys, c));
+      HPGX_HIP(st, hpgx::launch_scan(st->stream, st->nkeys, c));
       HPGX_HIP(st, hpgx::launch_emit(
                      st->stream, np, m, geo, st->cf, st->mu, gvis_ready, src, res, c, true));
     }

@@ -84,8 +84,10 @@ struct CallBuffers {
   double2* degrid_acc;   // binned degridding: per record x polarization sums
   size_t degrid_acc_capacity;
   void* tally_entries;   // launch_tally: entries in record order (Entry4<N>)
-  void* tally_keys;      // launch_tally: (key, place within the key) per slot
+  void* tally_keys;      // and per slot its key and a (lower key bits, slot) pair
   size_t tally_capacity; // slots of both
+  unsigned* sort_bins;   // launch_tally, launch_degrid: the sort's counts, offsets
+  size_t sort_capacity;  // and places, for this many records (sort_bins_entries)
   void* patch_recs;       // launch_patch: prepared records (PatchRec<N>)
   size_t patch_capacity;
   unsigned* patch_list;   // and the tiles' lists of record indexes
@@ -93,9 +95,7 @@ struct CallBuffers {
   unsigned* patch_table;  // and the workgroups' places in them (few tiles)
   size_t patch_table_capacity;
   unsigned* degrid_order; // launch_degrid: keys, the record order, (key, record)
-                          // pairs, 4 order_capacity values,
-  unsigned* degrid_bins;  // the sort's counts, offsets and places
-                          // (degrid_bins_entries),
+                          // pairs, 4 order_capacity values
   void* degrid_recs;      // and its prepared records (DegridRec)
   size_t order_capacity;
 };
@@ -139,16 +139,13 @@ hipError_t launch_emit(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool gvis_ready, GvisSource src, const double2* residuals,
   CallBuffers& cb, bool halo_entries = false, bool quad_keys = false);
-// global quadrant bins (one polarization, haloed entries) in two passes:
-// launch_tally (counts in cb.hist, entries and their (key, place) in
-// record order), launch_scan, then launch_place (entries into their keys'
-// ranges); n x nr slots of cb.tally_entries / cb.tally_keys
+// global quadrant bins (one polarization, haloed entries): the entries in their
+// keys' order in cb.stream_entries, the keys' offsets in cb.offsets; n x nr slots
+// of cb.tally_entries / cb.tally_keys
 hipError_t launch_tally(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
   const double2* residuals, CallBuffers& cb, double* weights);
-hipError_t launch_place(hipStream_t s, int npol, size_t n, const Geometry& geo,
-                        CallBuffers& cb);
 // block-local binning (small key counts)
 int bin_blocks_for(size_t n);
 size_t bin_block_records();
@@ -219,10 +216,10 @@ hipError_t launch_degrid_finish(
 // slice-ordered degridding of the records at `records`: FP64 predictions to
 // pred64, or predicted values (residuals, and gvis in cb, when do_grid)
 // written into out_records when not null, which may be `records`.  With a
-// model, cb.degrid_order, degrid_bins, degrid_recs and degrid_acc hold at least n
+// model, cb.degrid_order, sort_bins, degrid_recs and degrid_acc hold at least n
 // records.
 size_t degrid_rec_bytes();
-size_t degrid_bins_entries(size_t n);
+size_t sort_bins_entries(size_t n);
 hipError_t launch_degrid(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, const double2* model, bool do_grid, CallBuffers& cb, double2* pred64,

@@ -12,7 +12,7 @@
 //   k_bin + k_sub / k_tile4 + k_halo   one polarization, supports narrower
 //        than a tile: records binned by the 32 x 32 tile holding their support
 //        corner (block-local bins, no global atomics; grids of more than 8192
-//        keys bin through global counters: k_tally + k_place, k_count +
+//        keys bin through global memory: k_tally + k_tally_sort, k_count +
 //        k_emit); the tile kernels accumulate the tile plus a halo of
 //        (support - 1) pixels in LDS, and k_halo folds each tile's halo into
 //        its neighbours.
@@ -567,43 +567,179 @@ __global__ __launch_bounds__(block) void k_emit(
   }
 }
 
-// Global quadrant bins in two passes over the records instead of the three
-// of k_count + k_emit: k_tally makes each record's entries (one per grid row
-// with a Mueller index, keyed by the quadrant of the support corner) once,
-// takes each entry's place within its key from the returning count, and
-// writes the entry and its (key, place) in record order (slot
-// record * nr + row); after the scan of the counts, k_place moves each
-// entry into its key's contiguous range.  Weights as k_count.
+// ---- counting sort -----------------------------------------------------------
+//
+// 32-bit keys (~0: not sorted) in two levels: the upper bits in at most
+// patch_local_keys bins, counted in LDS by the kernel that makes the keys, a
+// workgroup of patch_local_threads per batch, with one global atomic per
+// workgroup and bin (global counters of every key are bound by the 10 G/s of the
+// chip) whose result is the workgroup's place in the bin (k_sort_place); the lower low_bits within a bin in LDS (sort_bin).  As the
+// degridder's order 35 us for 1e6 records of 3e5 keys and 25 for 300,000, against
+// 130 and 104 us of hipCUB's radix sort (two-polarization residuals 752 -> 649 us).
+
+constexpr int patch_local_threads = 1024;
+constexpr int patch_local_keys = 16384;
+constexpr int sort_threads = 256;
+constexpr int sort_loads = 8;
+constexpr int sort_low_bits_max = 14;
+
+struct SortKeys {
+  int drop_bits, low_bits, bins;  // the key's bits, from the lowest
+};
+
+// block-wide exclusive scan of a[0, n) in LDS (n <= bin_quad_keys_max), returns
+// the total; `part` holds blockDim.x / wave + 1 values
+__device__ unsigned block_exclusive_scan(unsigned* a, int n, unsigned* part) {
+  const int nt = blockDim.x;
+  const int per = (n + nt - 1) / nt;
+  const int beg = min(n, int(threadIdx.x) * per);
+  const int end = min(n, beg + per);
+  unsigned sum = 0;
+  for (int k = beg; k < end; ++k) sum += a[k];
+  // inclusive wave scan of the per-thread sums
+  const int lane = threadIdx.x % wave;
+  unsigned v = sum;
+#pragma unroll
+  for (int d = 1; d < wave; d <<= 1) {
+    const unsigned t = __shfl_up(v, d, wave);
+    if (lane >= d) v += t;
+  }
+  const int w = threadIdx.x / wave;
+  if (lane == wave - 1) part[w] = v;
+  __syncthreads();
+  if (w == 0) {
+    // exclusive scan of the wave totals (at most 64 waves) by one wave
+    const int nw = nt / wave;
+    const unsigned t = lane < nw ? part[lane] : 0u;
+    unsigned incl = t;
+#pragma unroll
+    for (int d = 1; d < wave; d <<= 1) {
+      const unsigned u = __shfl_up(incl, d, wave);
+      if (lane >= d) incl += u;
+    }
+    if (lane < nw) part[lane] = incl - t;
+    if (lane == nw - 1) part[nw] = incl;
+  }
+  __syncthreads();
+  unsigned run = part[w] + v - sum;  // exclusive prefix of this thread
+  for (int k = beg; k < end; ++k) {
+    const unsigned t = a[k];
+    a[k] = run;
+    run += t;
+  }
+  const unsigned total = part[nt / wave];
+  __syncthreads();
+  return total;
+}
+
+__global__ __launch_bounds__(block) void k_zero(unsigned* __restrict__ p, size_t n) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// (lower key bits, index) pairs by bin; order given (no lower bits): the indexes
+__global__ __launch_bounds__(patch_local_threads) void k_sort_place(
+  size_t n, SortKeys sk, unsigned batch, const unsigned* __restrict__ keys,
+  const unsigned* __restrict__ offsets, const unsigned* __restrict__ table,
+  unsigned* __restrict__ order, uint2* __restrict__ pairs) {
+  __shared__ unsigned at[patch_local_keys];
+  const unsigned* row = table + size_t(blockIdx.x) * sk.bins;
+  for (int k = threadIdx.x; k < sk.bins; k += blockDim.x) at[k] = offsets[k] + row[k];
+  __syncthreads();
+  const size_t first = blockIdx.x * (size_t)batch;
+  const size_t last = min(n, first + batch);
+  for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
+    const unsigned key = keys[i];
+    if (key == ~0u) continue;
+    const unsigned pos =
+      __hip_atomic_fetch_add(at + (key >> (sk.low_bits + sk.drop_bits)), 1u, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (order)
+      order[pos] = unsigned(i);
+    else
+      pairs[pos] = make_uint2((key >> sk.drop_bits) & ((1u << sk.low_bits) - 1u), unsigned(i));
+  }
+}
+
+// a workgroup's bin, pairs [beg, end): scanned(counts) once each lower key's
+// first place is known, then put(place, index) for every pair
+template <typename S, typename F>
+__device__ __forceinline__ void sort_bin(
+  int low_bits, unsigned beg, unsigned end, const uint2* __restrict__ pairs, S scanned, F put) {
+  extern __shared__ unsigned low[];  // 2^low_bits
+  __shared__ unsigned part[sort_threads / wave + 1];
+  constexpr unsigned stride = sort_threads * sort_loads;
+  const int low_keys = 1 << low_bits;
+  for (int k = threadIdx.x; k < low_keys; k += sort_threads) low[k] = 0u;
+  __syncthreads();
+  for (int pass = 0; pass < 2; ++pass) {
+    for (size_t first = beg; first < end; first += stride) {
+      uint2 p[sort_loads];
+#pragma unroll
+      for (int j = 0; j < sort_loads; ++j) {
+        const size_t k = first + j * sort_threads + threadIdx.x;
+        p[j] = k < end ? pairs[k] : make_uint2(~0u, 0u);
+      }
+#pragma unroll
+      for (int j = 0; j < sort_loads; ++j) {
+        if (p[j].x == ~0u) continue;
+        const unsigned at = __hip_atomic_fetch_add(low + p[j].x, 1u, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (pass) put(at, p[j].y);
+      }
+    }
+    __syncthreads();
+    if (!pass) {
+      block_exclusive_scan(low, low_keys, part);
+      __syncthreads();
+      scanned(low);
+      __syncthreads();
+    }
+  }
+}
+
+// Global quadrant bins: k_tally makes each record's entries (one per grid row
+// with a Mueller index, keyed by the quadrant of the support corner) in record
+// order (slot record * nr + row) and counts the keys' bins; k_sort_place and
+// k_tally_sort then move the entries into their keys' ranges, whose offsets
+// k_tally_sort writes.  Weights as k_count.  Bound by the passes over records
+// and entries: 1e6 records on 4001 x 3750, 96 us (49, 10, 27 and two small ones),
+// against 114 with a returning global atomic per entry, a device-wide scan and
+// a memset; moving the entries already with k_sort_place costs there (24 us)
+// what it saves.
 template <int N>
-__global__ __launch_bounds__(block) void k_tally(
+__global__ __launch_bounds__(patch_local_threads) void k_tally(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int gvis_ready, int adjoint,
   const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
-  unsigned* __restrict__ hist, double* __restrict__ weights,
-  unsigned long long* __restrict__ invalid, Entry4<N>* __restrict__ tally,
-  uint2* __restrict__ tally_keys) {
+  SortKeys sk, unsigned batch, unsigned* __restrict__ hist, unsigned* __restrict__ table,
+  double* __restrict__ weights, unsigned long long* __restrict__ invalid,
+  Entry4<N>* __restrict__ tally, unsigned* __restrict__ tally_keys) {
 
   __shared__ double wblk[count_planes_lds];
+  __shared__ unsigned cnt[patch_local_keys];
+  for (int k = threadIdx.x; k < sk.bins; k += blockDim.x) cnt[k] = 0u;
   const int nplanes = geo.nr * geo.nc;
   const bool lds_w = update_weights && nplanes <= count_planes_lds;
   if (lds_w)
     for (int k = threadIdx.x; k < nplanes; k += blockDim.x) wblk[k] = 0.0;
   __syncthreads();
 
-  const size_t stride = size_t(gridDim.x) * blockDim.x;
-  const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  const size_t iters = (n + stride - 1) / stride;
+  const size_t first = blockIdx.x * (size_t)batch;
+  const size_t last = min(n, first + batch);
   const int ntiles = geo.ntx * geo.nty;
-  for (size_t it = 0; it < iters; ++it) {
-    const size_t i = i0 + it * stride;
+  // every thread runs the same number of iterations (the wave reductions
+  // below need all lanes)
+  for (size_t at = first; at < last; at += blockDim.x) {
+    const size_t i = at + threadIdx.x;
     bool counted = false;
     unsigned gcube = 0;
     double tw[4] = {0.0, 0.0, 0.0, 0.0};
-    if (i < n) {
+    if (i < last) {
       // slots of rows without an entry say so
       for (int gpol = 0; gpol < geo.nr; ++gpol)
-        tally_keys[i * geo.nr + gpol] = make_uint2(~0u, 0u);
+        tally_keys[i * geo.nr + gpol] = ~0u;
       const VisRec<N>& r = recs[i];
       const unsigned grp = r.cf_index[1];
       const unsigned cfcube = r.cf_index[0];
@@ -665,9 +801,10 @@ __global__ __launch_bounds__(block) void k_tally(
             if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
             const int key =
               bin_key((int(gcube) * geo.nr + gpol) * ntiles + ty * geo.ntx + tx, c.gx, c.gy, 1);
-            const unsigned place = atomicAdd(hist + key, 1u);
+            __hip_atomic_fetch_add(cnt + (unsigned(key) >> sk.low_bits), 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
             tally[i * geo.nr + gpol] = e;
-            tally_keys[i * geo.nr + gpol] = make_uint2(unsigned(key), place);
+            tally_keys[i * geo.nr + gpol] = unsigned(key);
           }
         }
       }
@@ -693,26 +830,41 @@ __global__ __launch_bounds__(block) void k_tally(
       }
     }
   }
-  if (lds_w) {
-    __syncthreads();
+  __syncthreads();
+  if (lds_w)
     for (int k = threadIdx.x; k < nplanes; k += blockDim.x)
       if (wblk[k] != 0.0) atomicAdd(weights + k, wblk[k]);
-  }
+  unsigned* row = table + size_t(blockIdx.x) * sk.bins;
+  for (int k = threadIdx.x; k < sk.bins; k += blockDim.x)
+    row[k] = cnt[k] ? atomicAdd(hist + k, cnt[k]) : 0u;
 }
 
+// one workgroup per bin: its entries in order of their keys, and the keys'
+// offsets
 template <int N>
-__global__ __launch_bounds__(block) void k_place(
-  size_t slots, int nr, const unsigned* __restrict__ offsets,
-  const Entry4<N>* __restrict__ tally, const uint2* __restrict__ tally_keys,
-  Entry4<N>* __restrict__ entries, unsigned* __restrict__ entry_vis) {
-  const size_t sl = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (sl >= slots) return;
-  const uint2 kp = tally_keys[sl];
-  if (kp.x == ~0u) return;
-  const unsigned pos = offsets[kp.x] + kp.y;
-  const Entry4<N> e = tally[sl];
-  entries[pos] = e;
-  if (e.h.pos & e4_gradient) entry_vis[pos] = unsigned(sl / size_t(nr));
+__global__ __launch_bounds__(sort_threads) void k_tally_sort(
+  int low_bits, size_t nkeys, int nr, const unsigned* __restrict__ bin_offsets,
+  const uint2* __restrict__ pairs, const Entry4<N>* __restrict__ tally,
+  unsigned* __restrict__ offsets, Entry4<N>* __restrict__ entries,
+  unsigned* __restrict__ entry_vis) {
+  const unsigned beg = bin_offsets[blockIdx.x], end = bin_offsets[blockIdx.x + 1];
+  const size_t key0 = size_t(blockIdx.x) << low_bits;
+  const size_t keys = min(size_t(1) << low_bits, nkeys - key0);
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) offsets[nkeys] = end;
+  if (beg == end) {
+    for (size_t k = threadIdx.x; k < keys; k += sort_threads) offsets[key0 + k] = beg;
+    return;
+  }
+  sort_bin(
+    low_bits, beg, end, pairs,
+    [&](const unsigned* first) {
+      for (size_t k = threadIdx.x; k < keys; k += sort_threads) offsets[key0 + k] = beg + first[k];
+    },
+    [&](unsigned at, unsigned slot) {
+      const Entry4<N> e = tally[slot];
+      entries[beg + at] = e;
+      if (e.h.pos & e4_gradient) entry_vis[beg + at] = slot / unsigned(nr);
+    });
 }
 
 __device__ __forceinline__ int bcast(int v, int k) {
@@ -741,52 +893,6 @@ constexpr int bin_planes_max = 1024;
 constexpr int tile_bins_max = 2048;  // bin blocks per pass (LDS of k_tile4)
 constexpr int bin_stage_bytes = 65536;  // LDS staging of k_bin's haloed entries (one
                                         // chunk for a block of one-polarization entries)
-
-// block-wide exclusive scan of a[0, n) in LDS (n <= bin_quad_keys_max), returns
-// the total; `part` holds blockDim.x / wave + 1 values
-__device__ unsigned block_exclusive_scan(unsigned* a, int n, unsigned* part) {
-  const int nt = blockDim.x;
-  const int per = (n + nt - 1) / nt;
-  const int beg = min(n, int(threadIdx.x) * per);
-  const int end = min(n, beg + per);
-  unsigned sum = 0;
-  for (int k = beg; k < end; ++k) sum += a[k];
-  // inclusive wave scan of the per-thread sums
-  const int lane = threadIdx.x % wave;
-  unsigned v = sum;
-#pragma unroll
-  for (int d = 1; d < wave; d <<= 1) {
-    const unsigned t = __shfl_up(v, d, wave);
-    if (lane >= d) v += t;
-  }
-  const int w = threadIdx.x / wave;
-  if (lane == wave - 1) part[w] = v;
-  __syncthreads();
-  if (w == 0) {
-    // exclusive scan of the wave totals (at most 64 waves) by one wave
-    const int nw = nt / wave;
-    const unsigned t = lane < nw ? part[lane] : 0u;
-    unsigned incl = t;
-#pragma unroll
-    for (int d = 1; d < wave; d <<= 1) {
-      const unsigned u = __shfl_up(incl, d, wave);
-      if (lane >= d) incl += u;
-    }
-    if (lane < nw) part[lane] = incl - t;
-    if (lane == nw - 1) part[nw] = incl;
-  }
-  __syncthreads();
-  unsigned run = part[w] + v - sum;  // exclusive prefix of this thread
-  for (int k = beg; k < end; ++k) {
-    const unsigned t = a[k];
-    a[k] = run;
-    run += t;
-  }
-  const unsigned total = part[nt / wave];
-  __syncthreads();
-  return total;
-}
-
 
 // one entry per record and plane, keyed by the tile of the support corner
 template <int N>
@@ -2207,8 +2313,6 @@ static_assert(sizeof(PatchRec<1>) == 48 && sizeof(PatchRec<4>) == 64, "PatchRec 
 // places the entries without global atomics (10 G/s over the chip: they were
 // all of the two kernels' time: 284 + 265 us for 300,000 records of supports 9-33
 // on 4096 tiles, now 48 + 19).
-constexpr int patch_local_threads = 1024;
-constexpr int patch_local_keys = 16384;
 template <int N, bool LOCAL>
 __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_prep(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
@@ -2452,11 +2556,6 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
     __syncthreads();
   }
   if (threadIdx.x == 0) offsets[keys] = total;
-}
-
-__global__ __launch_bounds__(block) void k_zero(unsigned* __restrict__ p, size_t n) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
 }
 
 // exp(i ph): ph less the nearest multiple k of pi / 2 (pi / 2 as a 53-bit
@@ -2748,14 +2847,9 @@ void k_patch(
 // ---- degridding --------------------------------------------------------
 
 // The slice-ordered degridder, for several polarizations, large supports and
-// large grids: k_degrid_keys prepares the records, k_degrid_place and
+// large grids: k_degrid_keys prepares the records, k_sort_place and
 // k_degrid_sort order them by CF slice, k_degrid sums c' x model over their
-// supports and k_degrid_finish makes predictions of the sums.  The order is a
-// counting sort in two levels, the upper bits of the keys in at most
-// patch_local_keys bins as the tile lists of k_patch (LDS counts, one global
-// atomic per workgroup and bin), the lower 2^low_bits within a bin in LDS: 4
-// short launches, 35 us for 1e6 records of 3e5 keys and 25 for 300,000, against
-// 130 and 104 us of hipCUB's radix sort (two-polarization residuals 752 -> 649 us).
+// supports and k_degrid_finish makes predictions of the sums.
 
 // a record prepared for k_degrid; sxy = 0: not degridded
 struct __align__(16) DegridRec {
@@ -2771,7 +2865,6 @@ struct DegridKeys {
   unsigned slices, stride;  // of the batch, of a group
   int region_sh;
   unsigned regions_x, regions;
-  int drop_bits, low_bits, bins;  // the key's bits, from the lowest
 };
 
 // key = the record's (grid cube, region, group, CF cube, fine offsets), ~0 for
@@ -2781,12 +2874,12 @@ struct DegridKeys {
 template <int N>
 __global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
   size_t n, Geometry geo, const GroupInfo* __restrict__ groups,
-  const VisRec<N>* __restrict__ recs, DegridKeys dk, unsigned batch, unsigned* __restrict__ keys,
+  const VisRec<N>* __restrict__ recs, DegridKeys dk, SortKeys sk, unsigned batch,
+  unsigned* __restrict__ keys,
   DegridRec* __restrict__ out, unsigned* __restrict__ hist, unsigned* __restrict__ table) {
   __shared__ unsigned cnt[patch_local_keys];
-  const int shift = dk.low_bits + dk.drop_bits;
   if (keys)
-    for (int k = threadIdx.x; k < dk.bins; k += blockDim.x) cnt[k] = 0u;
+    for (int k = threadIdx.x; k < sk.bins; k += blockDim.x) cnt[k] = 0u;
   __syncthreads();
   const size_t first = blockIdx.x * (size_t)batch;
   const size_t last = min(n, first + batch);
@@ -2815,7 +2908,7 @@ __global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
             | (fxi << 8) | (fyi << 16);
           d.nm = unsigned(g.nmueller);
           if (keys)
-            __hip_atomic_fetch_add(cnt + (key >> shift), 1u, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(cnt + (key >> (sk.low_bits + sk.drop_bits)), 1u, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
@@ -2825,74 +2918,22 @@ __global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
   }
   if (!keys) return;
   __syncthreads();
-  unsigned* row = table + size_t(blockIdx.x) * dk.bins;
-  for (int k = threadIdx.x; k < dk.bins; k += blockDim.x)
+  unsigned* row = table + size_t(blockIdx.x) * sk.bins;
+  for (int k = threadIdx.x; k < sk.bins; k += blockDim.x)
     row[k] = cnt[k] ? atomicAdd(hist + k, cnt[k]) : 0u;
 }
 
-// the records into their bins: (lower key bits, record) pairs
-__global__ __launch_bounds__(patch_local_threads) void k_degrid_place(
-  size_t n, DegridKeys dk, unsigned batch, const unsigned* __restrict__ keys,
-  const unsigned* __restrict__ offsets, const unsigned* __restrict__ table,
-  unsigned* __restrict__ order, uint2* __restrict__ pairs) {
-  __shared__ unsigned at[patch_local_keys];
-  const int shift = dk.low_bits + dk.drop_bits;
-  const unsigned* row = table + size_t(blockIdx.x) * dk.bins;
-  for (int k = threadIdx.x; k < dk.bins; k += blockDim.x) at[k] = offsets[k] + row[k];
-  __syncthreads();
-  const size_t first = blockIdx.x * (size_t)batch;
-  const size_t last = min(n, first + batch);
-  for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
-    const unsigned key = keys[i];
-    if (key == ~0u) continue;
-    const unsigned pos = __hip_atomic_fetch_add(at + (key >> shift), 1u, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (dk.low_bits)
-      pairs[pos] = make_uint2((key >> dk.drop_bits) & ((1u << dk.low_bits) - 1u), unsigned(i));
-    else
-      order[pos] = unsigned(i);  // the bins are the slices
-  }
-}
-
 // one workgroup per bin: its records in order of their lower key bits
-constexpr int degrid_sort_threads = 256;
-constexpr int degrid_sort_loads = 8;
-constexpr int degrid_low_keys = 8192;
-__global__ __launch_bounds__(degrid_sort_threads) void k_degrid_sort(
-  int low_keys, const unsigned* __restrict__ offsets, const uint2* __restrict__ pairs,
+__global__ __launch_bounds__(sort_threads) void k_degrid_sort(
+  int low_bits, const unsigned* __restrict__ offsets, const uint2* __restrict__ pairs,
   unsigned* __restrict__ order) {
-  __shared__ unsigned low[degrid_low_keys];
-  __shared__ unsigned part[degrid_sort_threads / wave + 1];
-  constexpr unsigned stride = degrid_sort_threads * degrid_sort_loads;
   const unsigned beg = offsets[blockIdx.x], end = offsets[blockIdx.x + 1];
   if (end - beg <= 1u) {
     if (threadIdx.x == 0 && end != beg) order[beg] = pairs[beg].y;
     return;
   }
-  for (int k = threadIdx.x; k < low_keys; k += degrid_sort_threads) low[k] = 0u;
-  __syncthreads();
-  for (int pass = 0; pass < 2; ++pass) {
-    for (size_t first = beg; first < end; first += stride) {
-      uint2 p[degrid_sort_loads];
-#pragma unroll
-      for (int j = 0; j < degrid_sort_loads; ++j) {
-        const size_t k = first + j * degrid_sort_threads + threadIdx.x;
-        p[j] = k < end ? pairs[k] : make_uint2(~0u, 0u);
-      }
-#pragma unroll
-      for (int j = 0; j < degrid_sort_loads; ++j) {
-        if (p[j].x == ~0u) continue;
-        const unsigned at = __hip_atomic_fetch_add(low + p[j].x, 1u, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (pass) order[beg + at] = p[j].y;
-      }
-    }
-    __syncthreads();
-    if (!pass) {
-      block_exclusive_scan(low, low_keys, part);
-      __syncthreads();
-    }
-  }
+  sort_bin(low_bits, beg, end, pairs, [](const unsigned*) {},
+           [&](unsigned at, unsigned i) { order[beg + at] = i; });
 }
 
 // sums val[0, V) of the lanes that differ in bits 1 .. MASK of their number.
@@ -3654,30 +3695,78 @@ hipError_t launch_count(
 
 size_t entry_bytes(int npol) { return sizeof(EntryHead) + sizeof(float2) * size_t(npol); }
 
+size_t patch_batch(size_t n) {
+  return std::max<size_t>(2048, ((n + 511) / 512 + 1023) / 1024 * 1024);
+}
+
+// Bins: at most half of the items that one workgroup counts (its global
+// atomics, one for each of its bins), not fewer than 1024: the second level
+// has one workgroup per bin, which of 1e6 records in 256 bins around a dense
+// uv core took 58 us and of 1024 bins 16.  Keys beyond patch_local_keys bins
+// of 2^sort_low_bits_max lose their lowest bits.
+SortKeys sort_plan(unsigned long long keys, size_t batch) {
+  const unsigned long long most =
+    std::clamp<unsigned long long>(batch / 2, 1024, patch_local_keys);
+  SortKeys sk{};
+  auto bins = [&]() { return ((keys - 1) >> (sk.low_bits + sk.drop_bits)) + 1; };
+  while (sk.low_bits < sort_low_bits_max && bins() > most) ++sk.low_bits;
+  while (bins() > (unsigned long long)patch_local_keys) ++sk.drop_bits;
+  sk.bins = int(bins());
+  return sk;
+}
+
+size_t sort_bins_entries(size_t n) {
+  return (2 + std::min<size_t>((n + 2047) / 2048, 512)) * (patch_local_keys + 1);
+}
+
+// the bins' offsets and the pairs of n keys, from the counts in cb.sort_bins
+hipError_t launch_sort_place(hipStream_t s, size_t n, size_t batch, const SortKeys& sk,
+                             const CallBuffers& cb, const unsigned* keys, unsigned* order,
+                             uint2* pairs) {
+  unsigned* hist = cb.sort_bins;
+  unsigned* offsets = hist + patch_local_keys + 1;
+  const unsigned* table = offsets + patch_local_keys + 1;
+  hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, sk.bins, hist, offsets,
+                     static_cast<unsigned*>(nullptr));
+  hipLaunchKernelGGL(k_sort_place, dim3(unsigned((n + batch - 1) / batch)),
+                     dim3(patch_local_threads), 0, s, n, sk, unsigned(batch), keys, offsets, table,
+                     order, pairs);
+  return hipGetLastError();
+}
+
 hipError_t launch_tally(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
   const double2* residuals, CallBuffers& cb, double* weights) {
   if (n == 0) return hipSuccess;
-  if (npol != 1) return hipErrorInvalidValue;
+  if (npol != 1 || n * size_t(geo.nr) > cb.tally_capacity || n > cb.sort_capacity)
+    return hipErrorInvalidValue;
+  const size_t nkeys = 4 * size_t(geo.ntx) * geo.nty * geo.nr * geo.nc;
+  const size_t batch = patch_batch(n);
+  const SortKeys sk = sort_plan(nkeys, batch);
+  if (sk.drop_bits) return hipErrorInvalidValue;
+  unsigned* hist = cb.sort_bins;
+  unsigned* offsets = hist + patch_local_keys + 1;
+  unsigned* table = offsets + patch_local_keys + 1;
+  uint2* pairs = static_cast<uint2*>(cb.tally_keys);
+  unsigned* keys = reinterpret_cast<unsigned*>(pairs + cb.tally_capacity);
+  Entry4<1>* tally = static_cast<Entry4<1>*>(cb.tally_entries);
+  hipLaunchKernelGGL(k_zero, dim3(blocks_for(size_t(sk.bins))), dim3(block), 0, s, hist,
+                     size_t(sk.bins));
   hipLaunchKernelGGL(
-    k_tally<1>, dim3(std::min(blocks_for(n), count_blocks_max)), dim3(block), 0, s,
+    k_tally<1>, dim3(unsigned((n + batch - 1) / batch)), dim3(patch_local_threads), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
     int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint), cb.gvis, residuals,
-    cb.hist, weights, cb.invalid_count, static_cast<Entry4<1>*>(cb.tally_entries),
-    static_cast<uint2*>(cb.tally_keys));
-  return hipGetLastError();
-}
-
-hipError_t launch_place(hipStream_t s, int npol, size_t n, const Geometry& geo,
-                        CallBuffers& cb) {
-  const size_t slots = n * size_t(geo.nr);
-  if (slots == 0) return hipSuccess;
-  if (npol != 1) return hipErrorInvalidValue;
+    sk, unsigned(batch), hist, table, weights, cb.invalid_count, tally, keys);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  e = launch_sort_place(s, n * size_t(geo.nr), batch * size_t(geo.nr), sk, cb, keys, nullptr,
+                        pairs);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(
-    k_place<1>, dim3(blocks_for(slots)), dim3(block), 0, s, slots, geo.nr, cb.offsets,
-    static_cast<const Entry4<1>*>(cb.tally_entries), static_cast<const uint2*>(cb.tally_keys),
-    static_cast<Entry4<1>*>(cb.stream_entries), cb.entry_vis);
+    k_tally_sort<1>, dim3(unsigned(sk.bins)), dim3(sort_threads),
+    (size_t(1) << sk.low_bits) * sizeof(unsigned), s, sk.low_bits, nkeys, geo.nr, offsets, pairs,
+    tally, cb.offsets, static_cast<Entry4<1>*>(cb.stream_entries), cb.entry_vis);
   return hipGetLastError();
 }
 
@@ -3855,9 +3944,6 @@ size_t patch_keys(const Geometry& geo) {
 }
 // records of a workgroup that counts in LDS: 2048, or more so that there are
 // at most 512 rows of places
-size_t patch_batch(size_t n) {
-  return std::max<size_t>(2048, ((n + 511) / 512 + 1023) / 1024 * 1024);
-}
 size_t patch_table_entries(const Geometry& geo, size_t n) {
   const size_t keys = patch_keys(geo);
   return keys <= size_t(patch_local_keys) ? std::min<size_t>((n + 2047) / 2048, 512) * keys : 0;
@@ -4038,9 +4124,6 @@ hipError_t launch_degrid_finish(
 }
 
 size_t degrid_rec_bytes() { return sizeof(DegridRec); }
-size_t degrid_bins_entries(size_t n) {
-  return (2 + std::min<size_t>((n + 2047) / 2048, 512)) * (patch_local_keys + 1);
-}
 
 hipError_t launch_degrid(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
@@ -4050,7 +4133,8 @@ hipError_t launch_degrid(
   if (!model)
     return launch_degrid_finish(s, npol, n, geo, cf, mu, nullptr, do_grid, records, out_records,
                                 cb, pred64);
-  if (cb.order_capacity < n || n > 0xffffffffull) return hipErrorInvalidValue;
+  if (cb.order_capacity < n || cb.sort_capacity < n || n > 0xffffffffull)
+    return hipErrorInvalidValue;
   const int P = patch_lanes(geo.nr);
   int kind = patch_kind(npol, geo, cf, mu);
   bool same_rows = true;
@@ -4102,11 +4186,8 @@ hipError_t launch_degrid(
   const unsigned long long regions = count(geo.nx) * count(geo.ny);
   const bool by_cube = slices * regions * geo.nc < key_limit;
   const unsigned long long kmax = by_cube ? slices * regions * geo.nc : slices;
-  // Bins: at most half of the records that one workgroup counts (its global
-  // atomics, one for each of its bins, at 10 G/s of the card), not fewer than
-  // 1024 for the second level's workgroups.  Keys beyond patch_local_keys bins
-  // of degrid_low_keys lose their lowest bits: 2^27 of them, more than the
-  // records of a call in practice, have next to no two records of one slice.
+  // Keys beyond the sort's 2^28 lose their lowest bits: more than the records
+  // of a call in practice, next to no two records have one slice.
   const bool sorted = kmax > 0 && kmax < key_limit;
   const size_t batch = patch_batch(n);
   const unsigned nb = unsigned((n + batch - 1) / batch);
@@ -4116,29 +4197,22 @@ hipError_t launch_degrid(
   dk.region_sh = region_sh;
   dk.regions_x = unsigned(count(geo.nx));
   dk.regions = unsigned(by_cube ? regions : 0ull);
-  if (sorted) {
-    const unsigned long long most = std::clamp<unsigned long long>(batch / 2, 1024, patch_local_keys);
-    auto bins_at = [&](int bits) { return ((kmax - 1) >> bits) + 1; };
-    while ((1 << dk.low_bits) < degrid_low_keys && bins_at(dk.low_bits) > most) ++dk.low_bits;
-    while (bins_at(dk.low_bits + dk.drop_bits) > (unsigned long long)patch_local_keys)
-      ++dk.drop_bits;
-    dk.bins = int(bins_at(dk.low_bits + dk.drop_bits));
-  }
+  const SortKeys sk = sorted ? sort_plan(kmax, batch) : SortKeys{};
   DegridRec* drs = static_cast<DegridRec*>(cb.degrid_recs);
   unsigned* keys = sorted ? cb.degrid_order : nullptr;
   unsigned* sorted_idx = cb.degrid_order + cb.order_capacity;
   uint2* pairs = reinterpret_cast<uint2*>(cb.degrid_order + 2 * cb.order_capacity);
-  unsigned* hist = cb.degrid_bins;  // counts, offsets, then the table
+  unsigned* hist = cb.sort_bins;  // counts, offsets, then the table
   unsigned* offsets = hist + patch_local_keys + 1;
   unsigned* table = offsets + patch_local_keys + 1;
   if (sorted)
-    hipLaunchKernelGGL(k_zero, dim3(blocks_for(size_t(dk.bins))), dim3(block), 0, s, hist,
-                       size_t(dk.bins));
+    hipLaunchKernelGGL(k_zero, dim3(blocks_for(size_t(sk.bins))), dim3(block), 0, s, hist,
+                       size_t(sk.bins));
 #define HPGX_DKEYS(NP)                                                         \
   hipLaunchKernelGGL(                                                          \
     k_degrid_keys<NP>, dim3(nb), dim3(patch_local_threads), 0, s, n, geo,      \
-    cf.groups, static_cast<const VisRec<NP>*>(records), dk, unsigned(batch),   \
-    keys, drs, hist, table)
+    cf.groups, static_cast<const VisRec<NP>*>(records), dk, sk,                \
+    unsigned(batch), keys, drs, hist, table)
   switch (npol) {
   case 1: HPGX_DKEYS(1); break;
   case 2: HPGX_DKEYS(2); break;
@@ -4150,13 +4224,12 @@ hipError_t launch_degrid(
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (sorted) {
-    hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, dk.bins, hist,
-                       offsets, static_cast<unsigned*>(nullptr));
-    hipLaunchKernelGGL(k_degrid_place, dim3(nb), dim3(patch_local_threads), 0, s, n, dk,
-                       unsigned(batch), keys, offsets, table, sorted_idx, pairs);
-    if (dk.low_bits)
-      hipLaunchKernelGGL(k_degrid_sort, dim3(unsigned(dk.bins)), dim3(degrid_sort_threads), 0, s,
-                         1 << dk.low_bits, offsets, pairs, sorted_idx);
+    e = launch_sort_place(s, n, batch, sk, cb, keys, sk.low_bits ? nullptr : sorted_idx, pairs);
+    if (e != hipSuccess) return e;
+    if (sk.low_bits)
+      hipLaunchKernelGGL(k_degrid_sort, dim3(unsigned(sk.bins)), dim3(sort_threads),
+                         (size_t(1) << sk.low_bits) * sizeof(unsigned), s, sk.low_bits, offsets,
+                         pairs, sorted_idx);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     order = sorted_idx;
@@ -4167,7 +4240,7 @@ hipError_t launch_degrid(
     hipLaunchKernelGGL(                                                        \
       (k_degrid<NP, PP, KD>), dim3(unsigned((n + per - 1) / per)), dim3(block), 0, s, n, geo, \
       cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,            \
-      static_cast<const VisRec<NP>*>(records), order, offsets + dk.bins,       \
+      static_cast<const VisRec<NP>*>(records), order, offsets + sk.bins,       \
       reinterpret_cast<double*>(cb.degrid_acc));                               \
   } while (0)
 #define HPGX_DEGRID_K(NP, KD)                                                  \
