@@ -305,6 +305,13 @@ bool use_patch(hpgx_state_t st) {
   return st->gridder == 5 && st->mode != HPGX_GRID_FP64 && st->fp32_tile == 2 && !sub_ok(st);
 }
 
+// a few records in one launch (k_direct), where the choice of a pipeline is
+// left to the library
+bool use_direct(hpgx_state_t st, size_t n) {
+  return st->gridder == 5 && st->sub_tiles && st->npol == 1 && halo_ok(st)
+    && (st->mode == HPGX_GRID_FP64 || st->fp32_tile == 2) && hpgx::direct_ok(n, st->geometry());
+}
+
 // k_sub on block-local haloed bins: 4 bin keys per (plane, tile) within one
 // workgroup's LDS histogram
 bool use_sub(hpgx_state_t st) {
@@ -854,6 +861,14 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
   }
   if (!do_grid) return HPGX_SUCCESS;
   const int mode = st->mode == HPGX_GRID_FP64 ? 0 : 1;
+  if (use_direct(st, n)) {
+    CallBuffers c = cb;
+    c.vis = rec_base;
+    HPGX_HIP(st, hpgx::launch_direct(
+                   st->stream, np, n, geo, st->cf, st->mu, update_weights, gvis_ready, src,
+                   residuals, c, st->weights, mode, st->grid));
+    return HPGX_SUCCESS;
+  }
   if (use_patch(st)) {
     const size_t chunk = std::min(cb.patch_capacity, cb.patch_list_capacity / patch_tiles(st));
     if (chunk == 0) return fail(st, HPGX_ERR_OTHER, "patch lists not allocated");

@@ -142,6 +142,13 @@ hipError_t launch_emit(
 // global quadrant bins (one polarization, haloed entries): the entries in their
 // keys' order in cb.stream_entries, the keys' offsets in cb.offsets; n x nr slots
 // of cb.tally_entries / cb.tally_keys
+// the whole gridding pass of a few records in one launch, on no buffers of cb
+// but vis, gvis and invalid_count
+bool direct_ok(size_t n, const Geometry& geo);
+hipError_t launch_direct(
+  hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf, const Mueller& mu,
+  bool update_weights, bool gvis_ready, GvisSource src, const double2* residuals,
+  const CallBuffers& cb, double* weights, int mode, void* grid);
 hipError_t launch_tally(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,

@@ -16,6 +16,7 @@
 //        k_emit); the tile kernels accumulate the tile plus a halo of
 //        (support - 1) pixels in LDS, and k_halo folds each tile's halo into
 //        its neighbours.
+//   k_direct   the same records where they are few, in one launch.
 //   k_patch_prep + k_patch_list + k_patch   several polarizations, larger
 //        supports: each tile's sums of all its grid rows in registers.
 // Degridding (degrid_vis, src/hpg_core.hpp:579-682): k_degrid4 reads the
@@ -2302,6 +2303,67 @@ struct __align__(16) PatchRec {
 };
 static_assert(sizeof(PatchRec<1>) == 48 && sizeof(PatchRec<4>) == 64, "PatchRec layout");
 
+// record i, whose support at c is inside the grid, prepared (sxy = 0 and
+// false: no row takes it), and its weight in each grid row
+template <int N>
+__device__ __forceinline__ bool patch_record(
+  const VisRec<N>& r, size_t i, const Coord& c, const Geometry& geo, const GroupInfo& g,
+  const double2* __restrict__ wsum, const Mueller& mu, int update_weights, int gvis_ready,
+  int adjoint, const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
+  PatchRec<N>& e, double (&tw4)[4]) {
+  const bool pos_w = r.uvw[2] > 0;
+  const unsigned cfcube = r.cf_index[0];
+  const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
+  bool any = false;
+#pragma unroll
+  for (int gp = 0; gp < 4; ++gp) {
+    tw4[gp] = 0.0;
+    if (gp >= geo.nr) continue;
+    double t = 0.0;
+#pragma unroll
+    for (int v = 0; v < N; ++v) {
+      const int m = pos_w ? mu.M[gp][v] : mu.Mc[gp][v];
+      any |= m >= 0;
+      if (update_weights && m >= 0 && m < g.nmueller) {
+        const double2 sw = wsum[g.wsum_offset
+                                + ((long long)(cfcube * g.nmueller + m) * geo.nf + fxi) * geo.nf
+                                + fyi];
+        t += hypot(sw.x, sw.y) * double(r.w[v]);
+      }
+    }
+    tw4[gp] = t;
+  }
+  e.sxy = 0u;
+  if (!any) return false;
+  const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
+  e.gx = c.gx;
+  e.gy = c.gy;
+  e.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi);
+  e.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
+  e.fl = unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0)) | (unsigned(fxi) << 8)
+    | (unsigned(fyi) << 16);
+  e.nm = unsigned(g.nmueller);
+  e.cube = r.grid_cube;
+  if (gvis_ready) {
+    for (int v = 0; v < N; ++v) e.g[v] = gvis_in[i * N + v];
+  } else {
+    const double2 phasor = cphase(r.phase);
+    if (!adjoint) {
+      for (int v = 0; v < N; ++v) e.g[v] = prephase(r.vis[v], phasor, r.w[v]);
+    } else {
+      double2 W[N];
+      degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
+      for (int v = 0; v < N; ++v) {
+        double2 d = W[v];
+        if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
+        d.y = -d.y;
+        e.g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
+      }
+    }
+  }
+  return true;
+}
+
 // Weights: each wave sums its records' weights per (grid cube, row), and
 // for grids of at most count_planes_lds planes adds the sums into the
 // workgroup's LDS, which adds into the grid weights once at its end (the
@@ -2358,55 +2420,10 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_p
       } else {
         const GroupInfo g = groups[grp];
         const Coord c = vis_coord(r, geo, g);
-        const bool pos_w = r.uvw[2] > 0;
         if (c.inside) {
-          const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
-          bool any = false;
           counted = update_weights != 0;
-#pragma unroll
-          for (int gp = 0; gp < 4; ++gp) {
-            if (gp >= geo.nr) continue;
-            double t = 0.0;
-#pragma unroll
-            for (int v = 0; v < N; ++v) {
-              const int m = pos_w ? mu.M[gp][v] : mu.Mc[gp][v];
-              any |= m >= 0;
-              if (update_weights && m >= 0 && m < g.nmueller) {
-                const double2 sw = wsum[g.wsum_offset
-                                        + ((long long)(cfcube * g.nmueller + m) * geo.nf + fxi)
-                                          * geo.nf + fyi];
-                t += hypot(sw.x, sw.y) * double(r.w[v]);
-              }
-            }
-            tw4[gp] = t;
-          }
-          if (any) {
-            const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-            e.gx = c.gx;
-            e.gy = c.gy;
-            e.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi);
-            e.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
-            e.fl = unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
-              | (unsigned(fxi) << 8) | (unsigned(fyi) << 16);
-            e.nm = unsigned(g.nmueller);
-            e.cube = gcube;
-            if (gvis_ready) {
-              for (int v = 0; v < N; ++v) e.g[v] = gvis_in[i * N + v];
-            } else {
-              const double2 phasor = cphase(r.phase);
-              if (!adjoint) {
-                for (int v = 0; v < N; ++v) e.g[v] = prephase(r.vis[v], phasor, r.w[v]);
-              } else {
-                double2 W[N];
-                degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-                for (int v = 0; v < N; ++v) {
-                  double2 d = W[v];
-                  if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
-                  d.y = -d.y;
-                  e.g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
-                }
-              }
-            }
+          if (patch_record<N>(r, i, c, geo, g, wsum, mu, update_weights, gvis_ready, adjoint,
+                              gvis_in, residuals, e, tw4)) {
             const int tx0 = c.gx / tw, tx1 = (c.gx + g.sx - 1) / tw;
             const int ty0 = c.gy / th, ty1 = (c.gy + g.sy - 1) / th;
             for (int ty = ty0; ty <= ty1; ++ty)
@@ -2843,6 +2860,216 @@ void k_patch(
   }
 }
 
+
+// ---- gridding, few records -----------------------------------------------------
+//
+// One launch in place of the three or more of the binned pipelines, for batches
+// whose time those launches are (one polarization, supports narrower than a
+// tile): one workgroup per 32 x 32 tile looks through all records for those
+// that touch it, adds the weights of those whose support corner it holds, and
+// sums them in LDS (FP64 atomics; the grid rows' planes in turn), then adds the
+// tile into the grid, of which it is the only writer.  A thread prepares a
+// record in registers, and its wave adds its threads' records one after the
+// other, a tap per lane in blocks of 8 x 8, the taps of direct_loads records
+// loaded together.  Bound by latencies: the launch, two reads of the records and
+// 0.045 us per record of the densest tile.  Supports of 7 on 512^2, uniform, back
+// to back, FP64 (FP32) grids: 200 records 25.6 (21.1) -> 9.9 us, 2000 32.3 (27.7)
+// -> 14.7; a register patch per wave in place of LDS sums took 0.33 us per record
+// of the densest tile.
+
+struct DirectArgs {
+  const GroupInfo* groups;
+  const double2* wsum;
+  const float2* gvis;
+  const double2* residuals;
+  double* weights;
+  unsigned long long* invalid;
+  int update_weights, gvis_ready, adjoint;
+};
+constexpr int direct_block = 512;
+constexpr int direct_loads = 4;
+constexpr unsigned direct_records = 2048;
+constexpr int direct_row = tile + 8;  // LDS row: four rows of a block on banks of their own
+constexpr int direct_plane = tile * direct_row;
+
+__global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(
+  Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode,
+  const VisRec<1>* __restrict__ recs, unsigned n, DirectArgs da, void* __restrict__ grid) {
+  extern __shared__ double sums[];  // per grid row: re, im
+  __shared__ unsigned short hit_i[direct_records];
+  __shared__ unsigned hits;
+  __shared__ double row_w[4];
+
+  const unsigned key = blockIdx.x;
+  const int x0 = int(key % unsigned(geo.ntx)) * tile;
+  const unsigned tq = key / unsigned(geo.ntx);
+  const int y0 = int(tq % unsigned(geo.nty)) * tile;
+  const int cube = int(tq / unsigned(geo.nty));
+  if (threadIdx.x == 0) hits = 0u;
+  if (threadIdx.x < 4) row_w[threadIdx.x] = 0.0;
+  __syncthreads();
+  for (unsigned i = threadIdx.x; i < n; i += direct_block) {
+    const VisRec<1>& r = recs[i];
+    const unsigned grp = r.cf_index[1], gcube = r.grid_cube;
+    bool valid = grp < unsigned(geo.ngroups) && gcube < unsigned(geo.nc);
+    if (valid) valid = r.cf_index[0] < unsigned(da.groups[grp].ncube);
+    if (!valid) {
+      if (key == 0) atomicAdd(da.invalid, 1ull);
+      continue;
+    }
+    if (int(gcube) != cube) continue;
+    const GroupInfo& g = da.groups[grp];
+    const Coord c = vis_coord(r, geo, g);
+    if (c.inside && c.gx < x0 + tile && c.gx + g.sx > x0 && c.gy < y0 + tile && c.gy + g.sy > y0)
+      hit_i[__hip_atomic_fetch_add(&hits, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)] =
+        (unsigned short)i;
+  }
+  __syncthreads();
+  const unsigned cnt = unsigned(uniform(int(hits)));
+  if (cnt == 0) return;
+  for (int k = threadIdx.x; k < geo.nr * 2 * direct_plane; k += direct_block) sums[k] = 0.0;
+  __syncthreads();
+
+  const unsigned w = unsigned(uniform(int(threadIdx.x) / wave));
+  const int lane = threadIdx.x % wave;
+  const int lx = lane & 7, ly = lane >> 3;
+  constexpr unsigned nw = direct_block / wave;
+  for (unsigned b0 = 0; b0 < cnt; b0 += direct_block) {
+    // lane l: record w + l * nw of the round
+    const unsigned h = b0 + w + unsigned(lane) * nw;
+    const unsigned left = cnt - b0;
+    const int mine = left > w ? int(min((left - w + nw - 1u) / nw, unsigned(wave))) : 0;
+    PatchRec<1> e{};
+    unsigned i = 0;
+    if (h < cnt) {
+      i = hit_i[h];
+      const VisRec<1>& r = recs[i];
+      const GroupInfo g = da.groups[r.cf_index[1]];
+      const Coord c = vis_coord(r, geo, g);
+      double tw4[4];
+      patch_record<1>(r, i, c, geo, g, da.wsum, mu, da.update_weights, da.gvis_ready, da.adjoint,
+                      da.gvis, da.residuals, e, tw4);
+      if (da.update_weights && c.gx >= x0 && c.gy >= y0) {
+#pragma unroll
+        for (int gp = 0; gp < 4; ++gp)
+          if (gp < geo.nr)
+            __hip_atomic_fetch_add(row_w + gp, tw4[gp], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+    const bool plain = int(e.sxy & 0xffffu) <= 8 && int(e.sxy >> 16) <= 8
+      && !(e.fl & flag_gradient);
+    const unsigned long long plain_m = __ballot(plain);
+    auto of = [&](int v, int j) { return __builtin_amdgcn_readlane(v, j); };
+    // the tap (X, Y) of record j: its value (in: there is one in the tile)
+    auto load = [&](int j, int gp, int X, int Y, bool& in, int& px) {
+      const unsigned sxy = unsigned(of(int(e.sxy), j));
+      const unsigned nm = unsigned(of(int(e.nm), j));
+      const bool pos_w = of(int(e.fl), j) & flag_pos_w;
+      const int el = pos_w ? mu.M[gp][0] : mu.Mc[gp][0];
+      const int x = of(e.gx, j) + X - x0, y = of(e.gy, j) + Y - y0;
+      in = X < int(sxy & 0xffffu) && Y < int(sxy >> 16) && unsigned(x) < unsigned(tile)
+        && unsigned(y) < unsigned(tile) && el >= 0 && unsigned(el) < nm;
+      px = y * direct_row + x;
+      const float2* cf = taps
+        + ((unsigned long long)unsigned(of(int(unsigned(e.base)), j))
+           | ((unsigned long long)unsigned(of(int(e.base >> 32), j)) << 32));
+      return in ? cf[unsigned(Y) * ((sxy & 0xffffu) * nm) + unsigned(X) * nm + unsigned(el)]
+                : make_float2(0.0f, 0.0f);
+    };
+    auto add = [&](int j, int gp, float2 cc, bool in, int px) {
+      const float2 gv = make_float2(__int_as_float(of(__float_as_int(e.g[0].x), j)),
+                                    __int_as_float(of(__float_as_int(e.g[0].y), j)));
+      if (!in) return;
+      const float2 pr = cmul(cc, gv);
+      double* dst = sums + gp * 2 * direct_plane + px;
+      __hip_atomic_fetch_add(dst, double(pr.x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(dst + direct_plane, double(pr.y), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    for (int j0 = 0; j0 < mine; j0 += direct_loads) {
+      constexpr unsigned long long all = (1ull << direct_loads) - 1ull;
+      if (((plain_m >> j0) & all) == all) {  // lanes past the last record are plain
+        for (int gp = 0; gp < geo.nr; ++gp) {
+          float2 c[direct_loads];
+          bool in[direct_loads];
+          int px[direct_loads];
+#pragma unroll
+          for (int u = 0; u < direct_loads; ++u) c[u] = load(j0 + u, gp, lx, ly, in[u], px[u]);
+#pragma unroll
+          for (int u = 0; u < direct_loads; ++u) {
+            c[u].y *= (of(int(e.fl), j0 + u) & flag_pos_w) ? -1.0f : 1.0f;
+            add(j0 + u, gp, c[u], in[u], px[u]);
+          }
+        }
+        continue;
+      }
+#pragma unroll 1
+      for (int j = j0; j < min(j0 + direct_loads, mine); ++j) {
+        const unsigned sxy = unsigned(of(int(e.sxy), j));
+        const unsigned fl = unsigned(of(int(e.fl), j));
+        const int sx = int(sxy & 0xffffu), sy = int(sxy >> 16);
+        const float imf = (fl & flag_pos_w) ? -1.0f : 1.0f;
+        double gxr = 0.0, gyr = 0.0;
+        if (fl & flag_gradient) {
+          const unsigned ri = unsigned(of(int(i), j));
+          gxr = recs[ri].grad[0];
+          gyr = recs[ri].grad[1];
+        }
+        const double phi0x = -gxr * ((sx / 2) * geo.os - (int((fl >> 8) & 255u) - geo.F));
+        const double phi0y = -gyr * ((sy / 2) * geo.os - (int((fl >> 16) & 255u) - geo.F));
+        const double dphix = gxr * geo.os, dphiy = gyr * geo.os;
+        // the support's blocks in the tile
+        const int gx = of(e.gx, j), gy = of(e.gy, j);
+        const int bx0 = max(x0 - gx, 0), bx1 = min(sx, x0 + tile - gx);
+        const int by0 = max(y0 - gy, 0), by1 = min(sy, y0 + tile - gy);
+        for (int gp = 0; gp < geo.nr; ++gp)
+          for (int Y = by0 + ly; Y - ly < by1; Y += 8) {
+            float2 c[direct_loads];
+            bool in[direct_loads];
+            int px[direct_loads];
+#pragma unroll
+            for (int u = 0; u < direct_loads; ++u)  // at most 4 blocks in a row of them
+              c[u] = load(j, gp, bx0 + lx + 8 * u, Y, in[u], px[u]);
+#pragma unroll 1
+            for (int u = 0; u < direct_loads; ++u) {
+              if (bx0 + 8 * u >= bx1) break;
+              float2 cc = u == 0 ? c[0] : u == 1 ? c[1] : u == 2 ? c[2] : c[3];
+              const bool ok = u == 0 ? in[0] : u == 1 ? in[1] : u == 2 ? in[2] : in[3];
+              const int at = u == 0 ? px[0] : u == 1 ? px[1] : u == 2 ? px[2] : px[3];
+              cc.y *= imf;
+              if (fl & flag_gradient)
+                cc = cmul(cc, narrow(cphase((phi0x + (bx0 + lx + 8 * u) * dphix)
+                                            + (phi0y + Y * dphiy))));
+              add(j, gp, cc, ok, at);
+            }
+          }
+      }
+    }
+  }
+  __syncthreads();
+  if (int(threadIdx.x) < geo.nr && row_w[threadIdx.x] != 0.0)
+    atomicAdd(da.weights + (size_t(cube) * geo.nr + threadIdx.x), row_w[threadIdx.x]);
+  for (int k = threadIdx.x; k < geo.nr * tile * tile; k += direct_block) {
+    const int gp = k / (tile * tile), px = k % (tile * tile);
+    const int x = x0 + px % tile, y = y0 + px / tile;
+    if (x >= geo.nx || y >= geo.ny) continue;
+    const double* src = sums + gp * 2 * direct_plane + (px / tile) * direct_row + px % tile;
+    const double vr = src[0], vi = src[direct_plane];
+    if (vr == 0.0 && vi == 0.0) continue;
+    const size_t gi = ((size_t(cube) * geo.nr + gp) * geo.ny + y) * geo.nx + x;
+    if (mode == 0) {
+      double2* at = static_cast<double2*>(grid) + gi;
+      const double2 g0 = *at;
+      *at = make_double2(g0.x + vr, g0.y + vi);
+    } else {
+      // one rounding of grid value + FP64 tile sum
+      float2* at = static_cast<float2*>(grid) + gi;
+      const float2 g0 = *at;
+      *at = make_float2(float(double(g0.x) + vr), float(double(g0.y) + vi));
+    }
+  }
+}
 
 // ---- degridding --------------------------------------------------------
 
@@ -4071,6 +4298,30 @@ hipError_t launch_patch(
 #undef HPGX_PATCH_P
 #undef HPGX_LIST
 #undef HPGX_PREP
+  return hipGetLastError();
+}
+
+// every tile looks through all records: their product, at 2^21 still the faster
+// (2000 records, 1024 tiles: 40.5 -> 32.5 us) and at 2^22 even (1000 records,
+// 4096 tiles: 52.3, 51.0); and not where few tiles hold them all (2000 records,
+// 4 tiles, FP32: 33.5 -> 39.6 us; 1000: 24.1 -> 21.9)
+bool direct_ok(size_t n, const Geometry& geo) {
+  const size_t tiles = size_t(geo.ntx) * geo.nty * geo.nc;
+  return n <= direct_records && n * tiles <= (size_t(1) << 21) && n <= 256 * tiles;
+}
+
+hipError_t launch_direct(
+  hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf, const Mueller& mu,
+  bool update_weights, bool gvis_ready, GvisSource src, const double2* residuals,
+  const CallBuffers& cb, double* weights, int mode, void* grid) {
+  if (n == 0) return hipSuccess;
+  if (npol != 1 || n > direct_records || geo.nr > 4) return hipErrorInvalidValue;
+  const size_t lds = size_t(geo.nr) * 2 * direct_plane * sizeof(double);
+  const DirectArgs args{cf.groups, cf.wsum, cb.gvis, residuals, weights, cb.invalid_count,
+                        int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint)};
+  hipLaunchKernelGGL(
+    k_direct, dim3(unsigned(size_t(geo.ntx) * geo.nty * geo.nc)), dim3(direct_block), lds, s, geo,
+    cf.taps, mu, mode, static_cast<const VisRec<1>*>(cb.vis), unsigned(n), args, grid);
   return hipGetLastError();
 }
 
