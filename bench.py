@@ -481,7 +481,7 @@ def pmc_summary(fetch_dir, write_dir):
         if k.startswith("k_bin"):
             per_call["fp32c"] += b
             per_call["fp64"] += b
-        elif (k.startswith("k_sub<") or k.startswith("k_quad<") or k.startswith("k_tile4<1, 1")
+        elif (k.startswith("k_sub<") or k.startswith("k_tile4<1, 1")
               or k.startswith("k_halo<HIP_vector_type<float")):
             per_call["fp32c"] += b
         elif k.startswith("k_tile4<1, 0") or k.startswith("k_halo<HIP_vector_type<double"):

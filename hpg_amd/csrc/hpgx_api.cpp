@@ -130,7 +130,7 @@ struct hpgx_state_s {
   // gridder 4), 0 = FP64 tile sums
   int fp32_tile = 2;
   // FP32-compensated grids of one polarization with supports up to 8 x 8:
-  // quadrant-keyed bins and k_sub (HPGX_SUB_TILES=0: register patches)
+  // quadrant-keyed bins and k_sub (HPGX_SUB_TILES=0: k_tile4)
   bool sub_tiles = true;
   // the finishing chain, deferred until an entry point touches the grid
   // (flush_finishing): normalize_by_weights, an in-place grid FFT and, for
@@ -301,15 +301,34 @@ bool sub_ok(hpgx_state_t st) {
 
 // register patches (k_patch)
 bool use_patch(hpgx_state_t st) {
-  if (st->gridder < 4 || st->npol > 1 || !halo_ok(st)) return true;
-  return st->gridder == 5 && st->mode != HPGX_GRID_FP64 && st->fp32_tile == 2 && !sub_ok(st);
+  return st->gridder < 4 || st->npol > 1 || !halo_ok(st);
 }
 
+// and for sparse batches of one polarization in FP32 grids that k_sub does not
+// take (supports of 9: 10,000 records on 2048^2, 2.4 a tile, 112 us by tiles and
+// halos, 69 by patches; 10,000 on 512^2, 39 a tile, 41 against 46; 1e6 on 4001^2,
+// 64 a tile, 500 against 549)
+bool sparse_patch(hpgx_state_t st) {
+  return st->gridder == 5 && st->npol == 1 && halo_ok(st) && st->mode != HPGX_GRID_FP64
+    && st->fp32_tile == 2 && !sub_ok(st);
+}
+bool use_sparse_patch(hpgx_state_t st, const CallBuffers& cb, size_t n) {
+  return sparse_patch(st) && cb.patch_capacity > 0
+    && n < 16 * st->nkeys;
+}
+
+// accumulation of k_tile4 (launch_tile_halo): FP32 grids that k_sub does not
+// take sum in FP64 (1e6 records, supports of 9, 1024^2: 161 us a call, 490 by
+// (hi, lo) pairs, 559 by register patches); the pairs under compare-and-swap on
+// request
+int tile_acc(hpgx_state_t st) { return st->gridder == 5 ? 0 : st->fp32_tile; }
+
 // a few records in one launch (k_direct), where the choice of a pipeline is
-// left to the library
+// left to the library.  FP64 grids: in an FP32 grid its one rounding per pixel
+// would show beside the tiles' and halos'
 bool use_direct(hpgx_state_t st, size_t n) {
-  return st->gridder == 5 && st->sub_tiles && st->npol == 1 && halo_ok(st)
-    && (st->mode == HPGX_GRID_FP64 || st->fp32_tile == 2) && hpgx::direct_ok(n, st->geometry());
+  return st->gridder == 5 && st->npol == 1 && halo_ok(st) && st->mode == HPGX_GRID_FP64
+    && hpgx::direct_ok(n, st->geometry());
 }
 
 // k_sub on block-local haloed bins: 4 bin keys per (plane, tile) within one
@@ -393,7 +412,7 @@ int ensure_call_buffers(hpgx_state_t st) {
     HPGX_HIP(st, dev_alloc(cb.scan_temp, cb.scan_temp_bytes));
   }
   if (st->cf.ngroups > 0) {
-    if (use_patch(st)) {
+    if (use_patch(st) || sparse_patch(st)) {
       // prepared records and tile lists for the whole batch, up to the entry
       // memory budget and 2^32 list indexes; larger batches are gridded in
       // chunks (run_grid)
@@ -869,7 +888,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
                    residuals, c, st->weights, mode, st->grid));
     return HPGX_SUCCESS;
   }
-  if (use_patch(st)) {
+  if (use_patch(st) || use_sparse_patch(st, cb, n)) {
     const size_t chunk = std::min(cb.patch_capacity, cb.patch_list_capacity / patch_tiles(st));
     if (chunk == 0) return fail(st, HPGX_ERR_OTHER, "patch lists not allocated");
     const size_t rec_bytes = visdata_size(st->npol);
@@ -880,7 +899,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
       HPGX_HIP(st, hpgx::launch_patch(
                      st->stream, np, std::min(chunk, n - off), geo, st->cf, st->mu,
                      update_weights, gvis_ready, src, residuals ? residuals + off * np : nullptr,
-                     c, st->weights, mode, st->grid));
+                     c, st->weights, mode, mode == 1 && halo_ok(st), st->grid));
     }
     return HPGX_SUCCESS;
   }
@@ -908,7 +927,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
                        block_cap, halo_x(st), halo_y(st), st->grid));
       else
         HPGX_HIP(st, hpgx::launch_tile_halo(
-                       st->stream, np, mode, st->fp32_tile, m, st->nkeys, geo, st->cf, st->mu, c,
+                       st->stream, np, mode, tile_acc(st), m, st->nkeys, geo, st->cf, st->mu, c,
                        block_cap, halo_x(st), halo_y(st), st->grid));
     }
     return HPGX_SUCCESS;
@@ -947,7 +966,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
                      halo_x(st), halo_y(st), st->grid, true));
     else
       HPGX_HIP(st, hpgx::launch_tile_halo(
-                     st->stream, np, mode, st->fp32_tile, m, st->nkeys, geo, st->cf, st->mu,
+                     st->stream, np, mode, tile_acc(st), m, st->nkeys, geo, st->cf, st->mu,
                      c, 0, halo_x(st), halo_y(st), st->grid, true));
   }
   return HPGX_SUCCESS;

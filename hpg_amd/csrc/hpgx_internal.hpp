@@ -201,7 +201,7 @@ size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy);
 hipError_t launch_patch(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
-  const double2* residuals, CallBuffers& cb, double* weights, int mode, void* grid);
+  const double2* residuals, CallBuffers& cb, double* weights, int mode, bool halo_rounds, void* grid);
 // binned degridding from the model's LDS tiles (entries of launch_bin with
 // degrid_pass).  one_plane (every record has exactly one entry): the
 // predictions are finished in the same kernel -- FP64 values to pred64, or

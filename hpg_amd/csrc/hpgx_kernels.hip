@@ -16,7 +16,7 @@
 //        k_emit); the tile kernels accumulate the tile plus a halo of
 //        (support - 1) pixels in LDS, and k_halo folds each tile's halo into
 //        its neighbours.
-//   k_direct   the same records where they are few, in one launch.
+//   k_direct   the same records, FP64 grids, where they are few: one launch.
 //   k_patch_prep + k_patch_list + k_patch   several polarizations, larger
 //        supports: each tile's sums of all its grid rows in registers.
 // Degridding (degrid_vis, src/hpg_core.hpp:579-682): k_degrid4 reads the
@@ -1311,29 +1311,34 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
 
   for (unsigned r0 = 0; r0 < total; r0 += halo_sched) {
     const unsigned rn = min(unsigned(halo_sched), total - r0);
-    // counting sort of the round's entries by bank class
-    if (threadIdx.x < halo_classes) cls[threadIdx.x] = 0u;
-    __syncthreads();
-    for (unsigned q = threadIdx.x; q < rn; q += halo_block)
-      __hip_atomic_fetch_add(cls + bank_class(entries[locate(r0 + q)].h.pos), 1u,
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned run = 0;
-      for (int c = 0; c < halo_classes; ++c) {
-        const unsigned t = cls[c];
-        cls[c] = run;
-        run += t;
+    if (rn <= wave) {  // one wave's entries: as they come
+      if (threadIdx.x < rn) sched[threadIdx.x] = locate(r0 + threadIdx.x);
+      __syncthreads();
+    } else {
+      // counting sort of the round's entries by bank class
+      if (threadIdx.x < halo_classes) cls[threadIdx.x] = 0u;
+      __syncthreads();
+      for (unsigned q = threadIdx.x; q < rn; q += halo_block)
+        __hip_atomic_fetch_add(cls + bank_class(entries[locate(r0 + q)].h.pos), 1u,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        unsigned run = 0;
+        for (int c = 0; c < halo_classes; ++c) {
+          const unsigned t = cls[c];
+          cls[c] = run;
+          run += t;
+        }
       }
+      __syncthreads();
+      for (unsigned q = threadIdx.x; q < rn; q += halo_block) {
+        const unsigned idx = locate(r0 + q);
+        const unsigned slot = __hip_atomic_fetch_add(
+          cls + bank_class(entries[idx].h.pos), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        sched[slot] = idx;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    for (unsigned q = threadIdx.x; q < rn; q += halo_block) {
-      const unsigned idx = locate(r0 + q);
-      const unsigned slot = __hip_atomic_fetch_add(
-        cls + bank_class(entries[idx].h.pos), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      sched[slot] = idx;
-    }
-    __syncthreads();
     // batch j of the round takes sorted entries rank * nbatch + j
     const unsigned nbatch = (rn + wave - 1) / wave;
     for (unsigned j = w; j < nbatch; j += nw) {
@@ -2613,11 +2618,15 @@ constexpr int patch_full = 1;  // N neighbouring elements, N even, at 16-byte
                                // alignment: two elements a load
 constexpr int patch_one = 2;   // at most one element
 
+// the records that a launch takes for a pixel: all, those whose support corner
+// lies in the pixel's 32 x 32 tile, or the others
+constexpr int patch_all = 0, patch_own = 1, patch_others = 2;
+
 template <int N, int P, int KIND>
 __global__ __launch_bounds__(patch_split(P) * patch_block)
 __attribute__((amdgpu_waves_per_eu(5)))
 void k_patch(
-  Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int ptx, int pty,
+  Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int take, int ptx, int pty,
   const unsigned* __restrict__ offsets, const unsigned* __restrict__ order,
   const unsigned* __restrict__ list, const PatchRec<N>* __restrict__ prs,
   const VisRec<N>* __restrict__ recs, void* __restrict__ grid) {
@@ -2697,7 +2706,9 @@ void k_patch(
       const unsigned long long hbase = st[je].base;
       const unsigned hsxy = st[je].sxy, hfl = st[je].fl, hnm = st[je].nm;
       const bool hit = lane % SPLIT == part && k0 + unsigned(lane) < m && hgx < bx + 2 * PW
-        && hgx + int(hsxy & 0xffffu) > bx && hgy < by + 2 * PH && hgy + int(hsxy >> 16) > by;
+        && hgx + int(hsxy & 0xffffu) > bx && hgy < by + 2 * PH && hgy + int(hsxy >> 16) > by
+        && (take == patch_all
+            || ((hgx / tile == bx / tile && hgy / tile == by / tile) == (take == patch_own)));
       unsigned long long todo = __ballot(hit);
       while (todo) {
         const int j = __builtin_ctzll(todo);
@@ -4208,7 +4219,8 @@ int patch_kind(int npol, const Geometry& geo, const DeviceCF& cf, const Mueller&
 hipError_t launch_patch(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
-  const double2* residuals, CallBuffers& cb, double* weights, int mode, void* grid) {
+  const double2* residuals, CallBuffers& cb, double* weights, int mode, bool halo_rounds,
+  void* grid) {
   if (n == 0) return hipSuccess;
   if (n > cb.patch_capacity) return hipErrorInvalidValue;
   const int P = patch_lanes(geo.nr);
@@ -4241,7 +4253,7 @@ hipError_t launch_patch(
   hipLaunchKernelGGL(                                                          \
     (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_split(PP) * patch_block), 0, s, \
     geo, cf.taps, mu,                                                          \
-    mode, ptx, pty, cb.offsets, order, cb.patch_list,                          \
+    mode, take, ptx, pty, cb.offsets, order, cb.patch_list,                          \
     static_cast<const PatchRec<NP>*>(cb.patch_recs),                           \
     static_cast<const VisRec<NP>*>(cb.vis), grid)
 #define HPGX_PATCH_K(NP, KD)                                                   \
@@ -4272,27 +4284,34 @@ hipError_t launch_patch(
   }
   if (e != hipSuccess) return e;
   switch (npol) {
-  case 1:
-    HPGX_LIST(1);
-    HPGX_PATCH_K(1, patch_one);
-    break;
-  case 2:
-    HPGX_LIST(2);
-    if (kind == patch_one) HPGX_PATCH_K(2, patch_one);
-    else if (kind == patch_full) HPGX_PATCH_K(2, patch_full);
-    else HPGX_PATCH_K(2, patch_any);
-    break;
-  case 3:
-    HPGX_LIST(3);
-    if (kind == patch_one) HPGX_PATCH_K(3, patch_one);
-    else HPGX_PATCH_K(3, patch_any);
-    break;
-  default:
-    HPGX_LIST(4);
-    if (kind == patch_one) HPGX_PATCH_K(4, patch_one);
-    else if (kind == patch_full) HPGX_PATCH_K(4, patch_full);
-    else HPGX_PATCH_K(4, patch_any);
-    break;
+  case 1: HPGX_LIST(1); break;
+  case 2: HPGX_LIST(2); break;
+  case 3: HPGX_LIST(3); break;
+  default: HPGX_LIST(4); break;
+  }
+  // FP32 grids of supports below a tile round twice a pixel, as the haloed tiles
+  // do: once with the sum of the tile's records, once with its neighbours'
+  for (int take = halo_rounds ? patch_own : patch_all; take <= (halo_rounds ? patch_others : patch_all);
+       ++take) {
+    switch (npol) {
+    case 1:
+      HPGX_PATCH_K(1, patch_one);
+      break;
+    case 2:
+      if (kind == patch_one) HPGX_PATCH_K(2, patch_one);
+      else if (kind == patch_full) HPGX_PATCH_K(2, patch_full);
+      else HPGX_PATCH_K(2, patch_any);
+      break;
+    case 3:
+      if (kind == patch_one) HPGX_PATCH_K(3, patch_one);
+      else HPGX_PATCH_K(3, patch_any);
+      break;
+    default:
+      if (kind == patch_one) HPGX_PATCH_K(4, patch_one);
+      else if (kind == patch_full) HPGX_PATCH_K(4, patch_full);
+      else HPGX_PATCH_K(4, patch_any);
+      break;
+    }
   }
 #undef HPGX_PATCH_K
 #undef HPGX_PATCH_P
