@@ -120,8 +120,8 @@ struct hpgx_state_s {
   std::vector<bool> released_set;
   // gridding pipeline: 5 = by size (use_patch): haloed tiles for one
   // polarization and small supports, register patches for all other calls
-  // (default); 4 = as 5, but FP32 grids' haloed tiles updated by LDS atomics
-  // instead of one wave per tile quadrant; 2, 3 = register patches always
+  // (default); 4 = as 5, but FP32 grids' haloed tiles updated as (hi, lo) pairs
+  // under compare-and-swap; 2, 3 = register patches always
   int gridder = 5;
   size_t nkeys = 0;
   size_t pass_blocks = 0;  // bin blocks per pass of the block-local pipelines
@@ -257,7 +257,6 @@ int ensure_cf_capacity(hpgx_state_t st, size_t taps, size_t ws) {
   return HPGX_SUCCESS;
 }
 
-// bin entries one record can produce: one per grid row per touched tile
 // block-local bins: the pipelines of choice when one workgroup's LDS holds
 // a histogram over all (plane, tile) keys
 bool use_block_local(hpgx_state_t st) {
@@ -833,7 +832,7 @@ int run_degrid_binned(hpgx_state_t st, size_t n, bool do_grid, const void* recor
     c.gvis = cb.gvis + off * np;
     HPGX_HIP(st, hpgx::launch_bin(
                    st->stream, np, m, geo, st->cf, st->mu, false, false,
-                   hpgx::GvisSource::Values, nullptr, c, block_cap, st->weights, true, true,
+                   hpgx::GvisSource::Values, nullptr, c, block_cap, st->weights, true,
                    copy_out ? static_cast<char*>(out_base) + off * rec_bytes : nullptr));
     HPGX_HIP(st, hpgx::launch_degrid_tiles(
                    st->stream, np, m, st->nkeys, geo, st->cf, st->mu, c, block_cap,
@@ -919,7 +918,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
       const bool sub = use_sub(st);
       HPGX_HIP(st, hpgx::launch_bin(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, gvis_ready, src,
-                     res, c, block_cap, st->weights, true, false, nullptr, sub));
+                     res, c, block_cap, st->weights, false, nullptr, sub));
       if (sub)
         HPGX_HIP(st, hpgx::launch_tile_sub(
                        st->stream, np, m, st->nkeys, geo, st->cf,
@@ -954,10 +953,10 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
       HPGX_HIP(st, hipMemsetAsync(c.hist, 0, (st->nkeys + 1) * sizeof(unsigned), st->stream));
       HPGX_HIP(st, hpgx::launch_count(
                      st->stream, np, m, geo, st->cf, st->mu, update_weights, true, c,
-                     st->weights, true));
+                     st->weights));
       HPGX_HIP(st, hpgx::launch_scan(st->stream, st->nkeys, c));
       HPGX_HIP(st, hpgx::launch_emit(
-                     st->stream, np, m, geo, st->cf, st->mu, gvis_ready, src, res, c, true));
+                     st->stream, np, m, geo, st->cf, st->mu, gvis_ready, src, res, c));
     }
     if (sub)
       HPGX_HIP(st, hpgx::launch_tile_sub(

@@ -17,7 +17,6 @@ constexpr int max_cf_groups = 1000;
 // grid tile edge (pixels) owned by one workgroup of the gridding kernel
 constexpr int tile = 32;
 // waves per gridding workgroup; each wave accumulates into its own tile copy
-constexpr int tile_waves = 4;
 
 // Per-group geometry of the device CF.  The device layout of group g is
 // "fine-offset sliced": for every (cube, fx, fy) -- fx, fy in [-F, F] the
@@ -125,20 +124,17 @@ size_t tiles_per_footprint(int max_sx, int max_sy);
 // exclusive scan of the global bin counts (hist -> offsets, cursor)
 hipError_t launch_scan(hipStream_t s, size_t nkeys, CallBuffers& cb);
 size_t scan_temp_bytes(size_t nkeys);
-// global bins; halo_entries: one Entry4 per record and plane in the bin of
-// the tile holding the support corner (for launch_tile_halo with
-// global_bins; with quad_keys the bin of the corner's quadrant, key 4 x tile
-// key + quadrant, for launch_tile_sub with global_bins), else one Entry per
-// touched tile
+// global bins: one Entry4 per record and plane in the bin of the tile holding the
+// support corner (for launch_tile_halo with global_bins)
 hipError_t launch_count(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool do_grid, CallBuffers& cb,
-  double* weights, bool halo_entries = false, bool quad_keys = false);
+  double* weights);
 size_t entry_bytes(int npol);
 hipError_t launch_emit(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool gvis_ready, GvisSource src, const double2* residuals,
-  CallBuffers& cb, bool halo_entries = false, bool quad_keys = false);
+  CallBuffers& cb);
 // global quadrant bins (one polarization, haloed entries): the entries in their
 // keys' order in cb.stream_entries, the keys' offsets in cb.offsets; n x nr slots
 // of cb.tally_entries / cb.tally_keys
@@ -163,7 +159,7 @@ hipError_t launch_bin(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
   const double2* residuals, CallBuffers& cb, size_t block_cap, double* weights,
-  bool halo_entries, bool degrid_pass = false, void* copy_records = nullptr,
+  bool degrid_pass = false, void* copy_records = nullptr,
   bool quad_keys = false);
 // haloed tiles (one entry per record and plane; supports below tile)
 size_t halo_entry_bytes(int npol);
@@ -184,7 +180,7 @@ size_t sub_lds_bytes(int hx, int hy);
 int sub_bins_limit();
 bool sub_supported(int hx, int hy);
 // uni: every CF group has the same support; global_bins (one polarization):
-// the entries of launch_emit with quad_keys, cb.offsets their key offsets
+// the entries of launch_tally, cb.offsets their key offsets
 hipError_t launch_tile_sub(
   hipStream_t s, int npol, size_t n, size_t ntile_keys, const Geometry& geo, const DeviceCF& cf,
   size_t taps_bytes, bool uni, const Mueller& mu, const CallBuffers& cb, size_t block_cap,

@@ -397,8 +397,7 @@ __device__ __forceinline__ int bin_key(int k, int gx, int gy, int quad_keys) {
   return 4 * k + (qx | (qy << 1));
 }
 
-// one entry per plane, in the bin of the tile holding the support corner (with
-// quad_keys of the corner's quadrant, bin_key)
+// one entry per plane, in the bin of the tile holding the support corner
 // Weights: each wave sums its records' weights per (grid cube, row), and
 // for grids of at most count_planes_lds planes adds the sums into the
 // workgroup's LDS, which adds into the grid weights once at its end (the
@@ -412,7 +411,7 @@ __global__ __launch_bounds__(block) void k_count(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int do_grid, unsigned* __restrict__ hist,
-  double* __restrict__ weights, unsigned long long* __restrict__ invalid, int quad_keys) {
+  double* __restrict__ weights, unsigned long long* __restrict__ invalid) {
 
   __shared__ double wblk[count_planes_lds];
   const int nplanes = geo.nr * geo.nc;
@@ -470,7 +469,7 @@ __global__ __launch_bounds__(block) void k_count(
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
             if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
             const int base = int(gcube * geo.nr + gpol) * ntiles;
-            atomicAdd(hist + bin_key(base + t, c.gx, c.gy, quad_keys), 1u);
+            atomicAdd(hist + bin_key(base + t, c.gx, c.gy, 0), 1u);
           }
         }
       }
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(block) void k_emit(
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int gvis_ready, int adjoint, const float2* __restrict__ gvis_in,
   const double2* __restrict__ residuals, unsigned* __restrict__ cursor,
-  void* __restrict__ entries_out, unsigned* __restrict__ entry_vis, int quad_keys) {
+  void* __restrict__ entries_out, unsigned* __restrict__ entry_vis) {
 
   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -555,7 +554,7 @@ __global__ __launch_bounds__(block) void k_emit(
     if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
     const int base = int(gcube * geo.nr + gpol) * ntiles;
     const unsigned pos =
-      atomicAdd(cursor + bin_key(base + ty * geo.ntx + tx, c.gx, c.gy, quad_keys), 1u);
+      atomicAdd(cursor + bin_key(base + ty * geo.ntx + tx, c.gx, c.gy, 0), 1u);
     // corner relative to the tile, fine offsets, flags
     const unsigned hpos = unsigned(c.gx - tx * tile) | (unsigned(c.gy - ty * tile) << 6)
       | ((e.h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u) | (grad ? e4_gradient : 0u);
@@ -3919,15 +3918,14 @@ hipError_t launch_scan(hipStream_t s, size_t nkeys, CallBuffers& cb) {
 hipError_t launch_count(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool do_grid, CallBuffers& cb,
-  double* weights, bool halo_entries, bool quad_keys) {
+  double* weights) {
   if (n == 0) return hipSuccess;
   if (npol != 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(
     k_count<1>, dim3(std::min(unsigned(blocks_for(n)), count_blocks_max)),
     dim3(block), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
-    int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count,
-    int(halo_entries && quad_keys));
+    int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count);
   return hipGetLastError();
 }
 
@@ -4011,7 +4009,7 @@ hipError_t launch_tally(
 hipError_t launch_emit(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool gvis_ready, GvisSource src, const double2* residuals,
-  CallBuffers& cb, bool halo_entries, bool quad_keys) {
+  CallBuffers& cb) {
   if (n == 0) return hipSuccess;
   const int adj = src == GvisSource::Adjoint;
   if (npol != 1) return hipErrorInvalidValue;
@@ -4019,7 +4017,7 @@ hipError_t launch_emit(
     k_emit<1>, dim3(blocks_for(n)), dim3(block), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
     int(gvis_ready), adj, cb.gvis, residuals, cb.cursor, cb.stream_entries,
-    cb.entry_vis, int(halo_entries && quad_keys));
+    cb.entry_vis);
   return hipGetLastError();
 }
 
@@ -4033,10 +4031,10 @@ hipError_t launch_bin(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
   const double2* residuals, CallBuffers& cb, size_t block_cap, double* weights,
-  bool halo_entries, bool degrid_pass, void* copy_records, bool quad_keys) {
+  bool degrid_pass, void* copy_records, bool quad_keys) {
   if (n == 0) return hipSuccess;
   if (copy_records && !degrid_pass) return hipErrorInvalidValue;
-  if (quad_keys && (!halo_entries || degrid_pass)) return hipErrorInvalidValue;
+  if (quad_keys && degrid_pass) return hipErrorInvalidValue;
   const int adj = src == GvisSource::Adjoint;
   const int dg = degrid_pass;
   const unsigned nb = unsigned(bin_blocks_for(n));
