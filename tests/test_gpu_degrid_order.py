@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
     (2, 1, 4, 2049),
     (30, 3, 8, 4097),        # 8670 slices x 3 cubes: bins of 32 keys
     (60, 70, 20, 6000),      # 100860 slices x 70 cubes: bins of 8192 keys
-    (60, 2000, 20, 3000),    # 2e8 keys: their lowest bits left out
+    (60, 3000, 20, 3000),    # 3e8 keys: their lowest bits left out
 ])
 def test_order_vs_oracle(hpg, oracle_mod, monkeypatch, ncube, nc, oversampling, n, one_slice):
     from hpg_amd import workloads
