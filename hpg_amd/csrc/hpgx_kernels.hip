@@ -2579,15 +2579,56 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
   if (threadIdx.x == 0) offsets[keys] = total;
 }
 
-// exp(i ph): ph less the nearest multiple k of pi / 2 (pi / 2 as a 53-bit
-// head, whose difference is exact, and its tail), then the Taylor series of
-// sine and cosine up to r^15 and r^16, |r| <= pi / 4 (remainders below
-// 1e-16).  As cphase, whose library call would cost the tap loops 40 registers
-// and with them a quarter of their waves.
+// 64 zeros and the 1152 bits of 2 / pi behind the point (computed from Machin's
+// formula for pi)
+__device__ const unsigned long long two_over_pi[19] = {
+  0ull,
+  0xa2f9836e4e441529ull, 0xfc2757d1f534ddc0ull, 0xdb6295993c439041ull,
+  0xfe5163abdebbc561ull, 0xb7246e3a424dd2e0ull, 0x06492eea09d1921cull,
+  0xfe1deb1cb129a73eull, 0xe88235f52ebb4484ull, 0xe99c7026b45f7e41ull,
+  0x3991d639835339f4ull, 0x9c845f8bbdf9283bull, 0x1ff897ffde05980full,
+  0xef2f118b5a0a6d1full, 0x6d367ecf27cb09b7ull, 0x4f463f669e5fea2dull,
+  0x7527bac7ebe5f17bull, 0x3d0739f78a5292eaull, 0x6bfb5fb11f8d5d08ull};
+
+// exp(i ph).  |ph| < 2^40: ph less the nearest multiple k of pi / 2 (pi / 2 as a
+// 53-bit head, whose difference is exact, and its tail).  From there on, where
+// the rounding of k itself would come to matter: Payne and Hanek's reduction
+// ("Radian reduction for trigonometric functions", 1983), ph = m 2^e times the
+// 128 bits of 2 / pi from the first that makes less than four quarter turns on,
+// to 2^-62 of one.  Then the Taylor series of sine and cosine up to r^15 and
+// r^16, |r| <= pi / 4 (remainders below 1e-16).  As cphase, whose library call
+// would cost the tap loops 40 registers and with them a quarter of their waves
+// (out of line still: its calling convention spills 20 to 100).
 __device__ __forceinline__ double2 cphase_taylor(double ph) {
-  const double k = rint(ph * 0.63661977236758134);  // 2 / pi
-  double r = __builtin_fma(-k, 1.5707963267948966, ph);
-  r = __builtin_fma(-k, 6.123233995736766e-17, r);
+  double r;
+  int q;
+  if (fabs(ph) < 1099511627776.0) {
+    const double k = rint(ph * 0.63661977236758134);  // 2 / pi
+    r = __builtin_fma(-k, 1.5707963267948966, ph);
+    r = __builtin_fma(-k, 6.123233995736766e-17, r);
+    q = int(k - 4.0 * rint(0.25 * k)) & 3;  // quadrant (0 .. 3)
+  } else {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(ph);
+    const int e = int(b >> 52) & 0x7ff;  // ph = m 2^(e - 1075)
+    const unsigned long long m = (b & 0xfffffffffffffull) | 0x10000000000000ull;
+    // the first bit that makes less than four turns: 2^-(e - 1076) in 2 / pi
+    const int at = min(e, 2046) - 1077 + 64;
+    const unsigned long long* w = two_over_pi + (at >> 6);
+    const int sh = at & 63;
+    const unsigned long long hi = sh ? (w[0] << sh) | (w[1] >> (64 - sh)) : w[0];
+    const unsigned long long lo = sh ? (w[1] << sh) | (w[2] >> (64 - sh)) : w[1];
+    const unsigned long long phi = __umul64hi(m, lo) + m * hi;
+    // phi: two bits of quarter turns, then their fraction, to the nearest
+    const long long f = (long long)(phi << 2);
+    q = int(phi >> 62) + (f < 0 ? 1 : 0);
+    r = double(f) * 8.515303950216386e-20;  // pi / 2 2^-64
+    if (b >> 63) {
+      q = -q;
+      r = -r;
+    }
+    q &= 3;
+    if (e == 0x7ff) r = ph - ph;  // not finite
+  }
   const double z = r * r;
   double s = -1.0 / 1307674368000.0;
   s = __builtin_fma(s, z, 1.0 / 6227020800.0);
@@ -2606,7 +2647,6 @@ __device__ __forceinline__ double2 cphase_taylor(double ph) {
   c = __builtin_fma(c, z, 1.0 / 24.0);
   c = __builtin_fma(c, z, -0.5);
   c = __builtin_fma(c, z, 1.0);
-  const int q = int(k - 4.0 * rint(0.25 * k)) & 3;  // quadrant (0 .. 3)
   const double re = q & 1 ? s : c, im = q & 1 ? c : s;
   return make_double2(q == 1 || q == 2 ? -re : re, q >= 2 ? -im : im);
 }
