@@ -193,8 +193,8 @@ __device__ __forceinline__ long long slice_start(
 
 __global__ void k_cf_relayout(
   const float2* __restrict__ staging, unsigned ex, unsigned ey, GroupInfo gi,
-  int os, int F, int nf, float2* __restrict__ taps, long long total) {
-  const long long o = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  int os, int F, int nf, float2* __restrict__ taps, long long total, long long block0) {
+  const long long o = (block0 + blockIdx.x) * (long long)blockDim.x + threadIdx.x;
   if (o >= total) return;
   long long q = o;
   const int m = int(q % gi.nmueller);
@@ -225,9 +225,9 @@ constexpr int relayout_block = 256;
 constexpr size_t relayout_lds = 40960;
 __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
   const float2* __restrict__ staging, unsigned ex, unsigned ey, GroupInfo gi,
-  int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc) {
+  int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc, long long block0) {
   extern __shared__ float2 win[];
-  unsigned b = blockIdx.x;
+  unsigned long long b = (unsigned long long)(block0 + blockIdx.x);
   const int X0 = int(b % unsigned(nxc)) * xc;
   b /= unsigned(nxc);
   const int Y = int(b % unsigned(gi.sy));
@@ -271,13 +271,14 @@ __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
 constexpr int wsum_block = 1024;
 __global__ __launch_bounds__(wsum_block) void k_cf_wsum(
   GroupInfo gi, int nf, const float2* __restrict__ taps,
-  double2* __restrict__ wsum, int per) {
+  double2* __restrict__ wsum, int per, long long block0) {
   __shared__ double2 part[wsum_block / wave][wave];
   const int nm = gi.nmueller;
   const long long ntap = (long long)gi.sx * gi.sy;
-  const long long slice = per ? blockIdx.x : blockIdx.x / nm;  // (cube * nf + fx) * nf + fy
+  const long long b = block0 + blockIdx.x;
+  const long long slice = per ? b : b / nm;  // (cube * nf + fx) * nf + fy
   const int step = per ? 1 : nm;
-  const float2* t = taps + gi.tap_offset + slice * ntap * nm + (per ? 0 : int(blockIdx.x % nm));
+  const float2* t = taps + gi.tap_offset + slice * ntap * nm + (per ? 0 : int(b % nm));
   const int keep = per ? per : 1;  // elements of this workgroup
   double re = 0.0, im = 0.0;
   for (long long k = threadIdx.x; k < ntap * keep; k += blockDim.x) {
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(wsum_block) void k_cf_wsum(
     re += part[w][threadIdx.x].x;
     im += part[w][threadIdx.x].y;
   }
-  const int m = per ? int(threadIdx.x) : int(blockIdx.x % nm);
+  const int m = per ? int(threadIdx.x) : int(b % nm);
   const long long nslice = (long long)nf * nf;
   const long long c = slice / nslice;
   wsum[gi.wsum_offset + (c * nm + m) * nslice + (slice - c * nslice)] = make_double2(re, im);
@@ -2668,7 +2669,7 @@ void k_patch(
   Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int take, int ptx, int pty,
   const unsigned* __restrict__ offsets, const unsigned* __restrict__ order,
   const unsigned* __restrict__ list, const PatchRec<N>* __restrict__ prs,
-  const VisRec<N>* __restrict__ recs, void* __restrict__ grid) {
+  const VisRec<N>* __restrict__ recs, void* __restrict__ grid, unsigned block0) {
 
   constexpr int PW = patch_w(P), PH = patch_h(P);
   constexpr int L = KIND == patch_one ? 1 : N;  // elements a lane loads per tap
@@ -2677,7 +2678,8 @@ void k_patch(
   __shared__ PatchRec<N> st[stage];
   __shared__ unsigned st_i[stage];
 
-  const unsigned key = order ? order[blockIdx.x] : blockIdx.x;
+  const unsigned b = block0 + blockIdx.x;
+  const unsigned key = order ? order[b] : b;
   const unsigned beg = offsets[key];
   const unsigned cnt = offsets[key + 1] - beg;
   if (cnt == 0) return;
@@ -3271,7 +3273,7 @@ void k_degrid(
   size_t n, Geometry geo, const float2* __restrict__ taps, Mueller mu, int same_rows,
   const double2* __restrict__ model, int by_xcd, const DegridRec* __restrict__ drs,
   const VisRec<N>* __restrict__ recs, const unsigned* __restrict__ order,
-  const unsigned* __restrict__ ordered, double* __restrict__ acc) {
+  const unsigned* __restrict__ ordered, double* __restrict__ acc, unsigned block0) {
 
   constexpr int R = degrid_recs;
   constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
@@ -3279,7 +3281,7 @@ void k_degrid(
 
   const int w = uniform(int(threadIdx.x) / wave);
   const int lane = threadIdx.x % wave;
-  const unsigned bi = by_xcd ? xcd_key(blockIdx.x, gridDim.x) : blockIdx.x;
+  const unsigned bi = block0 + (by_xcd ? xcd_key(blockIdx.x, gridDim.x) : blockIdx.x);
   const size_t p0 = (bi * (size_t)(block / wave) + w) * R;
   if (order) n = *ordered;  // the records that are not skipped
   if (p0 >= n) return;
@@ -3889,6 +3891,20 @@ inline unsigned blocks_for(size_t n, int b = block) {
   return unsigned((n + b - 1) / b);
 }
 
+// launch(first block, blocks) for parts of a grid of workgroups: HIP counts a
+// launch's threads in 32 bits, and a launch of more runs what is left of them
+// modulo 2^32
+template <typename F>
+hipError_t in_launches(unsigned long long blocks, int threads, F launch) {
+  const unsigned long long most = 0xffffffffull / unsigned(threads);
+  hipError_t e = hipSuccess;
+  for (unsigned long long first = 0; first < blocks && e == hipSuccess; first += most) {
+    launch(first, unsigned(std::min(most, blocks - first)));
+    e = hipGetLastError();
+  }
+  return e;
+}
+
 }  // namespace
 
 // ---- launchers -------------------------------------------------------------
@@ -3907,15 +3923,18 @@ hipError_t launch_cf_relayout(
   while (xc > 1 && lds(xc) > relayout_lds) --xc;
   const int nxc = (gi.sx + xc - 1) / xc;
   const unsigned long long blocks = (unsigned long long)nxc * gi.sy * nf * gi.ncube;
-  if (lds(xc) <= relayout_lds && blocks <= 0x7fffffffull)
+  if (lds(xc) <= relayout_lds)
+    return in_launches(blocks, relayout_block, [&](unsigned long long first, unsigned nb) {
+      hipLaunchKernelGGL(
+        k_cf_relayout_lds, dim3(nb), dim3(relayout_block), lds(xc), s, staging, ext[0], ext[1],
+        gi, os, F, nf, taps, xc, nxc, (long long)first);
+    });
+  return in_launches((total + block - 1) / block, block,
+                     [&](unsigned long long first, unsigned nb) {
     hipLaunchKernelGGL(
-      k_cf_relayout_lds, dim3(unsigned(blocks)), dim3(relayout_block), lds(xc), s, staging,
-      ext[0], ext[1], gi, os, F, nf, taps, xc, nxc);
-  else
-    hipLaunchKernelGGL(
-      k_cf_relayout, dim3(blocks_for(size_t(total))), dim3(block), 0, s, staging,
-      ext[0], ext[1], gi, os, F, nf, taps, total);
-  return hipGetLastError();
+      k_cf_relayout, dim3(nb), dim3(block), 0, s, staging, ext[0], ext[1], gi, os, F, nf, taps,
+      total, (long long)first);
+  });
 }
 
 hipError_t launch_cf_wsum(
@@ -3927,9 +3946,10 @@ hipError_t launch_cf_wsum(
   if (ns == 0) return hipSuccess;
   const long long values = (long long)gi.sx * gi.sy * (per ? per : 1);
   const int threads = values <= 1024 ? wave : values <= 8192 ? 256 : wsum_block;
-  hipLaunchKernelGGL(
-    k_cf_wsum, dim3(unsigned(ns)), dim3(threads), 0, s, gi, nf, taps, wsum, per);
-  return hipGetLastError();
+  return in_launches(ns, threads, [&](unsigned long long first, unsigned nb) {
+    hipLaunchKernelGGL(k_cf_wsum, dim3(nb), dim3(threads), 0, s, gi, nf, taps, wsum, per,
+                       (long long)first);
+  });
 }
 
 size_t tiles_per_footprint(int max_sx, int max_sy) {
@@ -4288,12 +4308,14 @@ hipError_t launch_patch(
     patch_tile_x(P), patch_tile_y(P), static_cast<const PatchRec<NP>*>(cb.patch_recs), \
     cb.hist, cb.offsets, cb.patch_list, unsigned(batch), cb.patch_table)
 #define HPGX_PATCH_P(NP, PP, KD)                                               \
-  hipLaunchKernelGGL(                                                          \
-    (k_patch<NP, PP, KD>), dim3(unsigned(keys)), dim3(patch_split(PP) * patch_block), 0, s, \
-    geo, cf.taps, mu,                                                          \
-    mode, take, ptx, pty, cb.offsets, order, cb.patch_list,                          \
-    static_cast<const PatchRec<NP>*>(cb.patch_recs),                           \
-    static_cast<const VisRec<NP>*>(cb.vis), grid)
+  e = in_launches(keys, patch_split(PP) * patch_block,                         \
+                  [&](unsigned long long first, unsigned blocks) {             \
+    hipLaunchKernelGGL(                                                        \
+      (k_patch<NP, PP, KD>), dim3(blocks), dim3(patch_split(PP) * patch_block), 0, s, \
+      geo, cf.taps, mu, mode, take, ptx, pty, cb.offsets, order, cb.patch_list, \
+      static_cast<const PatchRec<NP>*>(cb.patch_recs),                         \
+      static_cast<const VisRec<NP>*>(cb.vis), grid, unsigned(first));          \
+  })
 #define HPGX_PATCH_K(NP, KD)                                                   \
   do {                                                                         \
     if (P == 1) HPGX_PATCH_P(NP, 1, KD);                                       \
@@ -4329,6 +4351,8 @@ hipError_t launch_patch(
   }
   // FP32 grids of supports below a tile round twice a pixel, as the haloed tiles
   // do: once with the sum of the tile's records, once with its neighbours'
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
   for (int take = halo_rounds ? patch_own : patch_all; take <= (halo_rounds ? patch_others : patch_all);
        ++take) {
     switch (npol) {
@@ -4350,12 +4374,13 @@ hipError_t launch_patch(
       else HPGX_PATCH_K(4, patch_any);
       break;
     }
+    if (e != hipSuccess) return e;
   }
 #undef HPGX_PATCH_K
 #undef HPGX_PATCH_P
 #undef HPGX_LIST
 #undef HPGX_PREP
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 // every tile looks through all records: their product, at 2^21 still the faster
@@ -4544,12 +4569,14 @@ hipError_t launch_degrid(
   }
 #define HPGX_DEGRID_P(NP, PP, KD)                                              \
   do {                                                                         \
-    constexpr size_t per = size_t(block / wave) * degrid_recs;       \
-    hipLaunchKernelGGL(                                                        \
-      (k_degrid<NP, PP, KD>), dim3(unsigned((n + per - 1) / per)), dim3(block), 0, s, n, geo, \
-      cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,            \
-      static_cast<const VisRec<NP>*>(records), order, offsets + sk.bins,       \
-      reinterpret_cast<double*>(cb.degrid_acc));                               \
+    constexpr size_t per = size_t(block / wave) * degrid_recs;                 \
+    e = in_launches((n + per - 1) / per, block, [&](unsigned long long first, unsigned blocks) { \
+      hipLaunchKernelGGL(                                                      \
+        (k_degrid<NP, PP, KD>), dim3(blocks), dim3(block), 0, s, n, geo,       \
+        cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,          \
+        static_cast<const VisRec<NP>*>(records), order, offsets + sk.bins,     \
+        reinterpret_cast<double*>(cb.degrid_acc), unsigned(first));            \
+    });                                                                        \
   } while (0)
 #define HPGX_DEGRID_K(NP, KD)                                                  \
   do {                                                                         \
@@ -4580,7 +4607,6 @@ hipError_t launch_degrid(
   }
 #undef HPGX_DEGRID_K
 #undef HPGX_DEGRID_P
-  e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_degrid_finish(s, npol, n, geo, cf, mu, cb.degrid_acc, do_grid, records,
                               out_records, cb, pred64);

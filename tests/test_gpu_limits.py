@@ -69,3 +69,62 @@ def test_large_phase_gradients(hpg, oracle_mod, npol, M, nm, lo, hi):
     _set_model(hpg, gs, o, gsz)
     _check_predictions(hpg, oracle_mod, gs, o, rec)
     _check_grid(hpg, oracle_mod, gs, o, rec, 1e-6)
+
+
+def test_many_cf_cubes(hpg, oracle_mod):
+    """A CF laid out by 65536 x 87 x 3 workgroups of 256 threads: more threads
+    than 2^32."""
+    from hpg_amd import workloads
+    rng = np.random.default_rng(1)
+    plane = rng.standard_normal((91, 5)) + 1j * rng.standard_normal((91, 5))
+    values = plane.astype(np.complex64) * np.linspace(
+        1, 2, 65536, dtype=np.float32)[:, None, None, None]
+    cf = hpg.CFArray(1, [values])
+    gsz, n = (20, 130, 1, 1), 200
+    rec = workloads.random_visibilities(n, 1, gsz, (0.9, 1.1), cf, seed=2)
+    gs, o = _pair(hpg, oracle_mod, gsz, [[0]], [[0]], cf, 0, n)
+    _check_grid(hpg, oracle_mod, gs, o, rec, 1e-12)
+
+
+def test_many_patches(hpg, oracle_mod):
+    """2^31 pixels a plane: patches of 16 x 16 pixels by 512 threads each, 2^32.
+    Against the middle of the same u, v on a small grid."""
+    from hpg_amd import workloads
+    gsz, small, n = (65536, 32768, 3, 1), (64, 64, 3, 1), 200
+    M = [[0, 1], [1, -1], [-1, 0]]
+    cf = workloads.random_cf(4, [3], nmueller=2, seed=1)
+    # whole supports inside the small grid too
+    rec = workloads.random_visibilities(n, 2, small, (0.9, 1.1), cf, seed=2, margin=5)
+    gs = hpg.GridderState.create(hpg.Device.Hip, 0, n, cf, gsz, (0.9, 1.1), M, M, grid_mode=1)
+    gs.set_convolution_function(hpg.Device.Serial, cf)
+    gs.grid_visibilities(hpg.Device.Serial, rec, True)
+    o = oracle_mod.Oracle(small, (0.9, 1.1), M, M)
+    o.set_cf(cf.oversampling(), [(cf.extents(0), cf.values(0))])
+    o.grid_visibilities(_view(rec, oracle_mod), True)
+    for row, exp in enumerate(o.grid_values()[0]):
+        got = gs.grid_window(32768 - 32, 16384 - 32, 64, 64, row, 0)
+        assert np.abs(got - exp).max() <= 1e-6 * np.abs(exp).max()  # FP32 grid
+
+
+def test_many_records_degridded(hpg):
+    """2^28 + 300000 records, 16 by a workgroup of 256 threads: more threads
+    than 2^32.  The batch repeats a small one, whose predictions it repeats."""
+    import torch
+    from hpg_amd import workloads
+    gsz, part = (200, 180, 2, 1), 300_000
+    M = [[0, -1], [-1, 1]]
+    repeats = (1 << 28) // part + 2
+    n = part * repeats
+    cf = workloads.random_cf(4, [1], nmueller=2, seed=1)
+    rec = workloads.random_visibilities(part, 2, gsz, (1.0, 1.0), cf, seed=2)
+    gs = hpg.GridderState.create(hpg.Device.Hip, 0, n, cf, gsz, (1.0, 1.0), M, M)
+    gs.set_convolution_function(hpg.Device.Serial, cf)
+    model = torch.randn(gs.grid_shape, dtype=torch.complex128, device="cuda")
+    gs.set_model(hpg.Device.Serial, model)
+    one = torch.from_numpy(rec.view(np.uint8).reshape(part, -1)).cuda()
+    exp = gs.degrid_get_predicted_visibilities(hpg.Device.Serial, one)
+    got = gs.degrid_get_predicted_visibilities(hpg.Device.Serial, one.repeat(repeats, 1))
+    vis = exp[:, :16].contiguous().view(torch.float32)
+    bar = 1e-6 * vis.abs().max()
+    for k, chunk in enumerate(got.split(part)):
+        assert (chunk[:, :16].contiguous().view(torch.float32) - vis).abs().max() <= bar, k
