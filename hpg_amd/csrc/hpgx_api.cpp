@@ -1562,13 +1562,18 @@ int hpgx_grid_visibilities(
   if (int rc = ensure_call_buffers(st)) return rc;
   // Device records are read in place; degridding writes the returned records
   // straight into visibilities_out, or nowhere when they are not returned.
-  const bool dev = memory == HPGX_DEVICE;
+  // Returned records that overlap others (visibilities_out neither visibilities
+  // nor clear of them) are made from the staged copy.
+  const uintptr_t from = reinterpret_cast<uintptr_t>(vis), to = reinterpret_cast<uintptr_t>(vis_out);
+  const bool overlap = return_visibilities && vis != vis_out
+    && (from < to ? to - from : from - to) < n * visdata_size(npol);
+  const bool dev = memory == HPGX_DEVICE && !overlap;
   const void* records = nullptr;  // nullptr: the staged copy
   void* out_records = nullptr;
   if (dev) {
     records = vis;
     if (do_degrid && return_visibilities) out_records = vis_out;
-  } else if (!dev && st->tasks > 1) {
+  } else if (memory != HPGX_DEVICE && st->tasks > 1) {
     // uploaded on the next task's copy stream: overlaps the kernels of the
     // calls before
     if (int rc = upload_task_records(st, vis, n)) return rc;

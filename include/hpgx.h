@@ -185,7 +185,7 @@ HPGX_API int hpgx_has_model(hpgx_state_t state);
  * in `memory`.  With return_visibilities, the records -- with residual
  * values (do_degrid && do_grid) or predicted values (do_degrid && !do_grid)
  * for records inside the grid -- are written to visibilities_out (same
- * memory kind; may equal visibilities) once the stream reaches that point;
+ * memory kind; may equal or overlap visibilities) once the stream reaches that point;
  * they are valid after the next hpgx_fence.  HPGX_HOST records are copied
  * before the call returns.  HPGX_DEVICE records may be read in place by the
  * queued kernels, so they must be ready when the call is made and stay

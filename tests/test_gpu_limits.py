@@ -128,3 +128,38 @@ def test_many_records_degridded(hpg):
     bar = 1e-6 * vis.abs().max()
     for k, chunk in enumerate(got.split(part)):
         assert (chunk[:, :16].contiguous().view(torch.float32) - vis).abs().max() <= bar, k
+
+
+@pytest.mark.parametrize("shift", [-7, -1, 1, 7])
+@pytest.mark.parametrize("do_grid", [0, 1])
+@pytest.mark.parametrize("npol,M", [(1, [[0]]), (2, [[0, 1]])])
+def test_overlapping_device_records(hpg, npol, M, do_grid, shift):
+    """Records returned some records before or behind their own place."""
+    import ctypes
+    import torch
+    from hpg_amd import workloads
+    print(f"npol {npol} do_grid {do_grid} shift {shift}", flush=True)
+    gsz, n = (200, 180, 1, 1), 100_000
+    cf = workloads.random_cf(4, [3], nmueller=2, seed=1)
+    rec = workloads.random_visibilities(n, npol, gsz, (1.0, 1.0), cf, seed=2, margin=-3)
+    gs = hpg.GridderState.create(hpg.Device.Hip, 0, n, cf, gsz, (1.0, 1.0), M, M)
+    gs.set_convolution_function(hpg.Device.Serial, cf)
+    rng = np.random.default_rng(3)
+    gs.set_model(hpg.Device.Serial, rng.standard_normal(gsz[::-1]) + 0j)
+    exp = (gs.degrid_grid_get_residual_visibilities if do_grid
+           else gs.degrid_get_predicted_visibilities)(hpg.Device.Serial, rec)
+    size = rec.dtype.itemsize
+    src, dst = max(0, -shift) * size, max(0, shift) * size
+    buf = torch.zeros((n + abs(shift)) * size, dtype=torch.uint8, device="cuda")
+    buf[src:src + n * size] = torch.from_numpy(rec.view(np.uint8)).cuda()
+    torch.cuda.synchronize()
+    assert hpg._lib.lib().hpgx_grid_visibilities(
+        gs._h, ctypes.c_void_p(buf.data_ptr() + src), n, npol, 0, 1, 1, do_grid,
+        ctypes.c_void_p(buf.data_ptr() + dst), 1) == 0
+    gs.fence()
+    got = buf[dst:dst + n * size].cpu().numpy().view(rec.dtype)
+    for name in rec.dtype.names:
+        if name != "visibilities":
+            assert np.array_equal(got[name], exp[name]), name
+    bar = 1e-6 * np.abs(exp["visibilities"]).max()
+    assert np.abs(got["visibilities"] - exp["visibilities"]).max() <= bar
