@@ -890,6 +890,9 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
   if (use_patch(st) || use_sparse_patch(st, cb, n)) {
     const size_t chunk = std::min(cb.patch_capacity, cb.patch_list_capacity / patch_tiles(st));
     if (chunk == 0) return fail(st, HPGX_ERR_OTHER, "patch lists not allocated");
+    for (const GroupInfo& g : st->groups)
+      if (!hpgx::patch_offsets_fit(g))
+        return fail(st, HPGX_ERR_OTHER, "gridding: 16 rows of a CF slice exceed 4 GiB");
     const size_t rec_bytes = visdata_size(st->npol);
     for (size_t off = 0; off < n; off += chunk) {
       CallBuffers c = cb;

@@ -194,6 +194,9 @@ size_t patch_rec_bytes(int npol);
 // values of cb.patch_table for n records a call (0 for many tiles)
 size_t patch_table_entries(const Geometry& geo, size_t n);
 size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy);
+// the rows of a slice that one wave's pixels take have 32-bit byte offsets (not
+// so from 2^32 bytes in 16 rows on: CFs of 38 GB at the least)
+bool patch_offsets_fit(const GroupInfo& g);
 hipError_t launch_patch(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,

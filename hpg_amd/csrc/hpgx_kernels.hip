@@ -2295,18 +2295,37 @@ constexpr int patch_block = 4 * wave;
 // for the wider tiles, whose entries are cheap (two rows: 244 us against 312).
 __host__ __device__ constexpr int patch_split(int P) { return P == 4 ? 2 : 1; }
 
-// a record prepared for its tiles; sxy = 0: not gridded
+// a record prepared for its tiles; sxy = 0: not gridded.  The support's extents
+// (odd, below 2^30) are split: their lower 16 bits in sxy, and what is left of
+// them above the 36 bits of an index of 8-byte values in 512 GB, which keeps the
+// record at 64 bytes (two more words would cost a quarter of the staged records'
+// LDS, and in DegridRec a register in the loop over the taps)
 template <int N>
 struct __align__(16) PatchRec {
   int gx, gy;               // support corner
   unsigned long long base;  // first value of its CF slice (element 0, tap 0)
-  unsigned sxy;             // sx | sy << 16
+                            // | sx >> 16 << 36 | sy >> 16 << 50
+  unsigned sxy;             // low 16 bits of sx | sy << 16
   unsigned fl;              // flags | fxi << 8 | fyi << 16
   unsigned nm;              // Mueller elements of its CF group
   unsigned cube;            // grid cube
   float2 g[N];
 };
 static_assert(sizeof(PatchRec<1>) == 48 && sizeof(PatchRec<4>) == 64, "PatchRec layout");
+// the slice's index, taken apart and made (also of DegridRec)
+constexpr unsigned patch_base_hi = 0xfu;  // its bits of the upper word
+__device__ __forceinline__ void patch_pack(
+  long long slice, int sx, int sy, unsigned long long& base, unsigned& sxy) {
+  base = (unsigned long long)slice | ((unsigned long long)(unsigned(sx) >> 16) << 36)
+    | ((unsigned long long)(unsigned(sy) >> 16) << 50);
+  sxy = (unsigned(sx) & 0xffffu) | (unsigned(sy) << 16);
+}
+__device__ __forceinline__ int patch_sx(unsigned sxy, unsigned base_hi) {
+  return int((sxy & 0xffffu) | ((base_hi << 12) & 0x3fff0000u));
+}
+__device__ __forceinline__ int patch_sy(unsigned sxy, unsigned base_hi) {
+  return int((sxy >> 16) | ((base_hi >> 2) & 0x3fff0000u));
+}
 
 // record i, whose support at c is inside the grid, prepared (sxy = 0 and
 // false: no row takes it), and its weight in each grid row
@@ -2343,8 +2362,7 @@ __device__ __forceinline__ bool patch_record(
   const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
   e.gx = c.gx;
   e.gy = c.gy;
-  e.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi);
-  e.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
+  patch_pack(slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi), g.sx, g.sy, e.base, e.sxy);
   e.fl = unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0)) | (unsigned(fxi) << 8)
     | (unsigned(fyi) << 16);
   e.nm = unsigned(g.nmueller);
@@ -2498,8 +2516,9 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_l
     if (!sxy) continue;
     const int gx = prs[i].gx, gy = prs[i].gy;
     const unsigned gcube = prs[i].cube;
-    const int tx0 = gx / tw, tx1 = (gx + int(sxy & 0xffffu) - 1) / tw;
-    const int ty0 = gy / th, ty1 = (gy + int(sxy >> 16) - 1) / th;
+    const unsigned bhi = unsigned(prs[i].base >> 32);
+    const int tx0 = gx / tw, tx1 = (gx + patch_sx(sxy, bhi) - 1) / tw;
+    const int ty0 = gy / th, ty1 = (gy + patch_sy(sxy, bhi) - 1) / th;
     for (int ty = ty0; ty <= ty1; ++ty)
       for (int tx = tx0; tx <= tx1; ++tx) {
         const size_t key = (size_t(gcube) * pty + ty) * ptx + tx;
@@ -2746,8 +2765,10 @@ void k_patch(
       const int hgx = st[je].gx, hgy = st[je].gy;
       const unsigned long long hbase = st[je].base;
       const unsigned hsxy = st[je].sxy, hfl = st[je].fl, hnm = st[je].nm;
+      const unsigned hbhi = unsigned(hbase >> 32);
       const bool hit = lane % SPLIT == part && k0 + unsigned(lane) < m && hgx < bx + 2 * PW
-        && hgx + int(hsxy & 0xffffu) > bx && hgy < by + 2 * PH && hgy + int(hsxy >> 16) > by
+        && hgx + patch_sx(hsxy, hbhi) > bx && hgy < by + 2 * PH
+        && hgy + patch_sy(hsxy, hbhi) > by
         && (take == patch_all
             || ((hgx / tile == bx / tile && hgy / tile == by / tile) == (take == patch_own)));
       unsigned long long todo = __ballot(hit);
@@ -2757,21 +2778,22 @@ void k_patch(
         const int gx = __builtin_amdgcn_readlane(hgx, j);
         const int gy = __builtin_amdgcn_readlane(hgy, j);
         const unsigned blo = unsigned(__builtin_amdgcn_readlane(int(unsigned(hbase)), j));
-        const unsigned bhi = unsigned(__builtin_amdgcn_readlane(int(hbase >> 32), j));
+        const unsigned bhi = unsigned(__builtin_amdgcn_readlane(int(hbhi), j));
         const unsigned sxy = unsigned(__builtin_amdgcn_readlane(int(hsxy), j));
         const unsigned fl = unsigned(__builtin_amdgcn_readlane(int(hfl), j));
         const unsigned nm = unsigned(__builtin_amdgcn_readlane(int(hnm), j));
         const PatchRec<N>& e = st[k0 + unsigned(j)];
-        const int sx = int(sxy & 0xffffu), sy = int(sxy >> 16);
+        const int sx = patch_sx(sxy, bhi), sy = patch_sy(sxy, bhi);
         const bool pos_w = fl & flag_pos_w;
         const unsigned pm = pos_w ? ~0u : 0u;
         // the slice from the first support row within the wave's pixels on,
-        // at most 2 PH rows: offsets of 32 bits for any support
+        // at most 2 PH rows: offsets of 32 bits (patch_offsets_fit)
         const int y0 = max(by - gy, 0);
         const int rows = min(sy - y0, 2 * PH);
         const unsigned tap_bytes = nm * unsigned(sizeof(float2));
         const unsigned row_bytes = unsigned(sx) * tap_bytes;
-        const float2* first = taps + ((unsigned long long)blo | ((unsigned long long)bhi << 32))
+        const float2* first = taps
+          + ((unsigned long long)blo | ((unsigned long long)(bhi & patch_base_hi) << 32))
           + (unsigned long long)unsigned(y0) * (unsigned(sx) * nm);
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<float2*>(first), 0, int(unsigned(rows) * row_bytes), 0x00020000);
@@ -3132,9 +3154,9 @@ __global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4)
 
 // a record prepared for k_degrid; sxy = 0: not degridded
 struct __align__(16) DegridRec {
-  unsigned long long base;  // first value of its CF slice (element 0, tap 0)
+  unsigned long long base;  // as PatchRec::base
   long long corner;         // model index of its support corner, grid row 0
-  unsigned sxy;             // sx | sy << 16
+  unsigned sxy;             // as PatchRec::sxy
   unsigned fl;              // flags | fxi << 8 | fyi << 16
   unsigned nm;              // Mueller elements of its CF group
   unsigned pad;
@@ -3180,9 +3202,9 @@ __global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
             + (unsigned(c.gx) >> dk.region_sh);
           key = (gcube * dk.regions + region) * dk.slices + grp * dk.stride
             + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
-          d.base = (unsigned long long)slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi));
+          patch_pack(slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi)), g.sx, g.sy,
+                     d.base, d.sxy);
           d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
-          d.sxy = unsigned(g.sx) | (unsigned(g.sy) << 16);
           d.fl = unsigned((r.uvw[2] > 0 ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
             | (fxi << 8) | (fyi << 16);
           d.nm = unsigned(g.nmueller);
@@ -3342,11 +3364,15 @@ void k_degrid(
     constexpr int RR = decltype(rr_c)::value;
     constexpr bool GRAD = decltype(grad_c)::value;
     const unsigned sxy = lane_u32(d.sxy, r);
-    const int sx = int(sxy & 0xffffu);
-    const unsigned ntap = unsigned(sx) * (sxy >> 16);
+    const unsigned long long base = lane_u64(d.base, r);
+    const int sx = patch_sx(sxy, unsigned(base >> 32));
+    const int sy = patch_sy(sxy, unsigned(base >> 32));
+    const unsigned ntap = unsigned(sx) * unsigned(sy);  // of one slice: below 2^32 in 288 GB
     const unsigned nm = lane_u32(d.nm, r);
     const int pm = (lane_u32(d.fl, r) & flag_pos_w) ? -1 : 0;
-    const float2* cf = taps + lane_u64(d.base, r) + size_t(q) * nm;  // this lane's tap
+    const float2* cf = taps
+      + (base & (((unsigned long long)patch_base_hi << 32) | 0xffffffffull))
+      + size_t(q) * nm;  // this lane's tap
     unsigned eo[L];                                                  // its elements
     bool use[L];
 #pragma unroll
@@ -3388,7 +3414,7 @@ void k_degrid(
       const VisRec<N>& rc = recs[lane_u32(rec_i, r)];
       const double gxr = rc.grad[0], gyr = rc.grad[1];
       gp0 = -gxr * ((sx / 2) * geo.os - (int((fl >> 8) & 255u) - geo.F));
-      gp1 = -gyr * ((int(sxy >> 16) / 2) * geo.os - (int((fl >> 16) & 255u) - geo.F));
+      gp1 = -gyr * ((sy / 2) * geo.os - (int((fl >> 16) & 255u) - geo.F));
       gdx = gxr * geo.os;
       gdy = gyr * geo.os;
     }
@@ -4255,6 +4281,11 @@ size_t patch_rec_bytes(int npol) {
 size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy) {
   const int tw = patch_tile_x(patch_lanes(nr)), th = patch_tile_y(patch_lanes(nr));
   return size_t((max_sx - 1 + tw - 1) / tw + 1) * size_t((max_sy - 1 + th - 1) / th + 1);
+}
+
+bool patch_offsets_fit(const GroupInfo& g) {
+  const size_t rows = std::min(g.sy, 2 * patch_h(1));
+  return rows * size_t(g.sx) * size_t(g.nmueller) * sizeof(float2) < 0xfffffff0ull;
 }
 
 // how the rows of both signs of w take their elements of a slice

@@ -163,3 +163,23 @@ def test_overlapping_device_records(hpg, npol, M, do_grid, shift):
             assert np.array_equal(got[name], exp[name]), name
     bar = 1e-6 * np.abs(exp["visibilities"]).max()
     assert np.abs(got["visibilities"] - exp["visibilities"]).max() <= bar
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("npol,M,nm", [(1, [[0]], 1), (2, [[0, 1]], 2), (2, [[0, 1], [2, 1]], 3),
+                                       (4, DIAG, 4), (4, FULL, 16)])
+@pytest.mark.parametrize("sx,sy", [(65537, 3), (3, 65539), (65535, 1), (131075, 1)])
+def test_wide_supports(hpg, oracle_mod, sx, sy, npol, M, nm, mode):
+    """Supports of 2^16 pixels and more along one axis."""
+    from hpg_amd import workloads
+    print(f"support {sx} x {sy} npol {npol} nm {nm} mode {mode}", flush=True)
+    gsz, n = (sx + 21, sy + 21, len(M), 1), 40
+    cf = workloads.random_cf(1, [((sx - 1) // 2, (sy - 1) // 2), 1], nmueller=nm, seed=1)
+    rec = workloads.random_visibilities(n, npol, gsz, (0.9, 1.1), cf, seed=2, phase=True)
+    wide = rec["cf_index"][:, 1] == 0
+    rng = np.random.default_rng(4)
+    rec["uvw"][wide, :2] = rng.uniform(-9, 9, (wide.sum(), 2)) / np.array([0.9, 1.1])
+    gs, o = _pair(hpg, oracle_mod, gsz, M, M, cf, mode, n)
+    _set_model(hpg, gs, o, gsz)
+    _check_predictions(hpg, oracle_mod, gs, o, rec)
+    _check_grid(hpg, oracle_mod, gs, o, rec, 1e-6 if mode else 1e-12)
