@@ -2806,9 +2806,11 @@ void k_patch(
         for (int k = 0; k < 4; ++k) {
           const int dx = (k & 1) * PW, dy = (k >> 1) * PH;
           in[k] = unsigned(X + dx) < unsigned(sx) && unsigned(Y + dy) < unsigned(sy);
-          // a row without its element takes nothing
+          // a row without its element takes nothing, nor do lanes past the rows
+          // (of three rows: whole elements of none would be read at ~0u)
           if constexpr (KIND == patch_one)
             in[k] = in[k] && (eo[0] ^ (eo_x[0] & pm)) < tap_bytes;
+          if constexpr (KIND == patch_full && P == 4) in[k] = in[k] && row < geo.nr;
           const unsigned off = off0 + unsigned(dy) * row_bytes + unsigned(dx) * tap_bytes;
           if constexpr (KIND == patch_full) {
             const unsigned o = in[k] ? off + (eo[0] ^ (eo_x[0] & pm)) : ~0u;

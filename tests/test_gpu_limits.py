@@ -183,3 +183,20 @@ def test_wide_supports(hpg, oracle_mod, sx, sy, npol, M, nm, mode):
     _set_model(hpg, gs, o, gsz)
     _check_predictions(hpg, oracle_mod, gs, o, rec)
     _check_grid(hpg, oracle_mod, gs, o, rec, 1e-6 if mode else 1e-12)
+
+
+@pytest.mark.parametrize("gradient", [False, True])
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("rows,nm", [((0, 1, 2), 16), ((0, 1, 2), 12), ((3, 0, 2), 16)])
+def test_three_rows_of_neighbouring_elements(hpg, oracle_mod, rows, nm, mode, gradient):
+    """Rows of four neighbouring elements, whose patches' fourth lane has no row."""
+    from hpg_amd import workloads
+    gsz, n = (81, 64, 3, 2), 900
+    M, Mc = [FULL[r] for r in rows], [FULL[r] for r in rows[::-1]]
+    cf = workloads.random_cf(6, [(1, 3), 8], nmueller=nm, ncube=2, seed=1)
+    rec = workloads.random_visibilities(n, 4, gsz, (0.9, 1.1), cf, seed=2, phase=True, margin=-3,
+                                        gradient=gradient)
+    gs, o = _pair(hpg, oracle_mod, gsz, M, Mc, cf, mode, n)
+    _set_model(hpg, gs, o, gsz)
+    _check_predictions(hpg, oracle_mod, gs, o, rec)
+    _check_grid(hpg, oracle_mod, gs, o, rec, 1e-6 if mode or gradient else 1e-12)
