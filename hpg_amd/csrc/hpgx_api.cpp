@@ -239,6 +239,21 @@ size_t cf_taps_for(unsigned os, unsigned ngroups, const unsigned* extents,
   return taps;
 }
 
+// the Mueller elements to hold of groups of these extents
+hpgx::CfElements cf_elements(hpgx_state_t st, unsigned ngroups, const unsigned* extents) {
+  std::vector<int> used;
+  for (const std::vector<int>* rows : {&st->mueller_rows, &st->conj_mueller_rows})
+    for (int m : *rows)
+      if (m >= 0) used.push_back(m);
+  std::sort(used.begin(), used.end());
+  used.erase(std::unique(used.begin(), used.end()), used.end());
+  hpgx::CfElements ce{};
+  for (unsigned g = 0; g < ngroups && ce.n == 0; ++g)
+    if (used.empty() || unsigned(used[0]) >= extents[4 * g + 2]) ce.elem[ce.n++] = -1;
+  for (int m : used) ce.elem[ce.n++] = m;
+  return ce;
+}
+
 int ensure_cf_capacity(hpgx_state_t st, size_t taps, size_t ws) {
   if (taps > st->taps_capacity) {
     dev_free(st->cf.taps);
@@ -1329,6 +1344,7 @@ int hpgx_clone(hpgx_state_t src, hpgx_state_t* dst) {
     st->cf.taps = t;
     st->cf.wsum = w;
     st->groups = src->groups;
+    st->mu = src->mu;
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st->stream);
   if (e != hipSuccess) {
@@ -1438,6 +1454,7 @@ int hpgx_set_convolution_function(
   const int os = int(oversampling);
   const int F = (os + 1) / 2;
   const int nf = 2 * F + 1;
+  const hpgx::CfElements ce = cf_elements(st, num_groups, extents);
   std::vector<GroupInfo> groups(num_groups);
   long long toff = 0, woff = 0;
   int max_sx = 1, max_sy = 1, max_ncube = 1;
@@ -1450,7 +1467,9 @@ int hpgx_set_convolution_function(
     radii(e, oversampling, gi.rx, gi.ry);
     gi.sx = 2 * gi.rx + 1;
     gi.sy = 2 * gi.ry + 1;
-    gi.nmueller = int(e[2]);
+    while (gi.nmueller < ce.n
+           && (ce.elem[gi.nmueller] < 0 || unsigned(ce.elem[gi.nmueller]) < e[2]))
+      ++gi.nmueller;
     gi.ncube = int(e[3]);
     gi.tap_offset = toff;
     gi.wsum_offset = woff;
@@ -1465,7 +1484,12 @@ int hpgx_set_convolution_function(
     even_nm = even_nm && gi.nmueller % 2 == 0;
     max_stage = std::max(max_stage, size_t(e[0]) * e[1] * e[2] * e[3]);
   }
-  if (int rc = ensure_cf_capacity(st, size_t(toff), size_t(woff))) return rc;
+  // the region that the shape asks for (hpgx_convolution_function_region_size),
+  // of which the held elements take a part
+  size_t ws = 0;
+  const size_t taps = cf_taps_for(oversampling, num_groups, extents, &ws);
+  if (int rc = ensure_cf_capacity(st, std::max(taps, size_t(toff)), std::max(ws, size_t(woff))))
+    return rc;
   if (memory != HPGX_DEVICE && max_stage > st->staging_capacity) {
     dev_free(st->staging);
     st->staging_capacity = 0;
@@ -1481,7 +1505,8 @@ int hpgx_set_convolution_function(
                                   hipMemcpyHostToDevice, st->stream));
       src = st->staging;
     }
-    HPGX_HIP(st, hpgx::launch_cf_relayout(st->stream, src, e, groups[g], os, F, nf, st->cf.taps));
+    HPGX_HIP(st, hpgx::launch_cf_relayout(st->stream, src, e, groups[g], ce, os, F, nf,
+                                          st->cf.taps));
     HPGX_HIP(st, hpgx::launch_cf_wsum(st->stream, groups[g], nf, st->cf.taps, st->cf.wsum));
     if (memory != HPGX_DEVICE) HPGX_HIP(st, hipStreamSynchronize(st->stream));
   }
@@ -1490,6 +1515,17 @@ int hpgx_set_convolution_function(
                                 hipMemcpyHostToDevice, st->stream));
   HPGX_HIP(st, hipStreamSynchronize(st->stream));
   st->groups = groups;
+  // the Mueller rows in terms of the held elements
+  for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < 4; ++c) {
+      const size_t k = size_t(r) * st->npol + size_t(c);
+      const bool in = unsigned(r) < st->gsize[2] && unsigned(c) < st->npol;
+      auto held = [&](int m) {
+        return m < 0 ? -1 : int(std::find(ce.elem, ce.elem + ce.n, m) - ce.elem);
+      };
+      st->mu.M[r][c] = in ? held(st->mueller_rows[k]) : -1;
+      st->mu.Mc[r][c] = in ? held(st->conj_mueller_rows[k]) : -1;
+    }
   st->cf.os = os;
   st->cf.F = F;
   st->cf.nf = nf;

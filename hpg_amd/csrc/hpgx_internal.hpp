@@ -16,7 +16,6 @@ constexpr int cf_padding = 2;
 constexpr int max_cf_groups = 1000;
 // grid tile edge (pixels) owned by one workgroup of the gridding kernel
 constexpr int tile = 32;
-// waves per gridding workgroup; each wave accumulates into its own tile copy
 
 // Per-group geometry of the device CF.  The device layout of group g is
 // "fine-offset sliced": for every (cube, fx, fy) -- fx, fy in [-F, F] the
@@ -25,18 +24,30 @@ constexpr int tile = 32;
 // elements side by side (a record reads all of them, so whole lines of its
 // slice, wherever a tile border cuts the support):
 //   taps[tap_offset + ((((cube * nf + fx + F) * nf + fy + F) * sx * sy
-//        + Y * sx + X) * nmueller + m]
-//   = CFArray(ix, iy, m, cube, g), ix = (X + padding) * os + fx, iy likewise,
-// which is the element the reference reaches through its 6-D layout
+//        + Y * sx + X) * nmueller + k]
+//   = CFArray(ix, iy, elem[k], cube, g), ix = (X + padding) * os + fx, iy
+// likewise, which is the element the reference reaches through its 6-D layout
 // (src/hpg_impl.hpp:221-281, src/hpg_core.hpp:422-446: major * os + minor).
-// wsum[wsum_offset + ((cube * nmueller + m) * nf + fx + F) * nf + fy + F]
+// wsum[wsum_offset + ((cube * nmueller + k) * nf + fx + F) * nf + fy + F]
 // is the FP64 sum of that element's taps of the slice.
+// Only elements that some Mueller row names are held (CfElements, ascending;
+// the rows that the kernels see count in them): a tap's neighbours in memory
+// are then values that the calls read.  One polarization on a CF of 16 elements,
+// 1e6 records, supports of 7: 320 us with all 16 side by side, 134 with the one.
 struct GroupInfo {
   long long tap_offset;
   long long wsum_offset;
   int sx, sy;          // support 2r + 1 per axis
   int rx, ry;          // radii (src/hpg.hpp:687-694)
-  int nmueller, ncube;
+  int nmueller, ncube;  // held elements (the first so many of CfElements)
+};
+
+// the Mueller elements held, ascending; -1: none of the CFArray's, all zero,
+// first and named by no row, where a group has none of those that rows name (so
+// that every group has one: lanes without an element read it)
+struct CfElements {
+  int n;
+  int elem[33];  // two matrices of 4 x 4, and the -1
 };
 
 struct Mueller {
@@ -114,7 +125,7 @@ struct DeviceCF {
 
 hipError_t launch_cf_relayout(
   hipStream_t s, const float2* staging, const unsigned ext[4],
-  const GroupInfo& gi, int os, int F, int nf, float2* taps);
+  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, float2* taps);
 hipError_t launch_cf_wsum(
   hipStream_t s, const GroupInfo& gi, int nf, const float2* taps,
   double2* wsum);

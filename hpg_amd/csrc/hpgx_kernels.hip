@@ -192,12 +192,13 @@ __device__ __forceinline__ long long slice_start(
 // ---- CF ingestion ----------------------------------------------------
 
 __global__ void k_cf_relayout(
-  const float2* __restrict__ staging, unsigned ex, unsigned ey, GroupInfo gi,
-  int os, int F, int nf, float2* __restrict__ taps, long long total, long long block0) {
+  const float2* __restrict__ staging, unsigned ex, unsigned ey, unsigned em, GroupInfo gi,
+  CfElements ce, int os, int F, int nf, float2* __restrict__ taps, long long total,
+  long long block0) {
   const long long o = (block0 + blockIdx.x) * (long long)blockDim.x + threadIdx.x;
   if (o >= total) return;
   long long q = o;
-  const int m = int(q % gi.nmueller);
+  const int m = ce.elem[q % gi.nmueller];
   q /= gi.nmueller;
   const int X = int(q % gi.sx);
   q /= gi.sx;
@@ -210,8 +211,8 @@ __global__ void k_cf_relayout(
   const long long ix = (long long)(X + cf_padding) * os + (fxi - F);
   const long long iy = (long long)(Y + cf_padding) * os + (fyi - F);
   float2 v = make_float2(0.0f, 0.0f);
-  if (ix >= 0 && iy >= 0 && ix < ex && iy < ey)
-    v = staging[((long long)(c * gi.nmueller + m) * ey + iy) * ex + ix];
+  if (m >= 0 && ix >= 0 && iy >= 0 && ix < ex && iy < ey)
+    v = staging[(((long long)c * em + m) * ey + iy) * ex + ix];
   taps[gi.tap_offset + o] = v;
 }
 
@@ -224,8 +225,9 @@ __global__ void k_cf_relayout(
 constexpr int relayout_block = 256;
 constexpr size_t relayout_lds = 40960;
 __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
-  const float2* __restrict__ staging, unsigned ex, unsigned ey, GroupInfo gi,
-  int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc, long long block0) {
+  const float2* __restrict__ staging, unsigned ex, unsigned ey, unsigned em, GroupInfo gi,
+  CfElements ce, int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc,
+  long long block0) {
   extern __shared__ float2 win[];
   unsigned long long b = (unsigned long long)(block0 + blockIdx.x);
   const int X0 = int(b % unsigned(nxc)) * xc;
@@ -239,14 +241,16 @@ __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
   const int width = (xc - 1) * os + nf;
   const long long ix0 = (long long)(X0 + cf_padding) * os - F;
   const long long iy = (long long)(Y + cf_padding) * os + (fyi - F);
-  for (int m = 0; m < nm; ++m)
+  for (int m = 0; m < nm; ++m) {
+    const int em_m = ce.elem[m];
     for (int k = threadIdx.x; k < width; k += relayout_block) {
       const long long ix = ix0 + k;
       float2 v = make_float2(0.0f, 0.0f);
-      if (ix >= 0 && iy >= 0 && ix < ex && iy < ey)
-        v = staging[((long long)(c * nm + m) * ey + iy) * ex + ix];
+      if (em_m >= 0 && ix >= 0 && iy >= 0 && ix < ex && iy < ey)
+        v = staging[(((long long)c * em + em_m) * ey + iy) * ex + ix];
       win[m * width + k] = v;
     }
+  }
   __syncthreads();
   const unsigned run = unsigned(cols) * unsigned(nm);
   for (unsigned k = threadIdx.x; k < run * unsigned(nf); k += relayout_block) {
@@ -3939,7 +3943,7 @@ hipError_t in_launches(unsigned long long blocks, int threads, F launch) {
 
 hipError_t launch_cf_relayout(
   hipStream_t s, const float2* staging, const unsigned ext[4],
-  const GroupInfo& gi, int os, int F, int nf, float2* taps) {
+  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, float2* taps) {
   const long long total =
     (long long)gi.ncube * gi.nmueller * nf * nf * gi.sx * gi.sy;
   if (total == 0) return hipSuccess;
@@ -3955,13 +3959,13 @@ hipError_t launch_cf_relayout(
     return in_launches(blocks, relayout_block, [&](unsigned long long first, unsigned nb) {
       hipLaunchKernelGGL(
         k_cf_relayout_lds, dim3(nb), dim3(relayout_block), lds(xc), s, staging, ext[0], ext[1],
-        gi, os, F, nf, taps, xc, nxc, (long long)first);
+        ext[2], gi, ce, os, F, nf, taps, xc, nxc, (long long)first);
     });
   return in_launches((total + block - 1) / block, block,
                      [&](unsigned long long first, unsigned nb) {
     hipLaunchKernelGGL(
-      k_cf_relayout, dim3(nb), dim3(block), 0, s, staging, ext[0], ext[1], gi, os, F, nf, taps,
-      total, (long long)first);
+      k_cf_relayout, dim3(nb), dim3(block), 0, s, staging, ext[0], ext[1], ext[2], gi, ce, os, F,
+      nf, taps, total, (long long)first);
   });
 }
 
