@@ -164,6 +164,7 @@ struct hpgx_state_s {
     g.F = cf.F;
     g.nf = cf.nf;
     g.ngroups = cf.ngroups;
+    g.planar = cf.planar;
     g.ntx = (g.nx + hpgx::tile - 1) / hpgx::tile;
     g.nty = (g.ny + hpgx::tile - 1) / hpgx::tile;
     return g;
@@ -284,12 +285,12 @@ int halo_x(hpgx_state_t st) { return std::max(1, st->cf.max_sx) - 1; }
 int halo_y(hpgx_state_t st) { return std::max(1, st->cf.max_sy) - 1; }
 
 // haloed tiles: supports narrower than a tile, tile + halo within LDS
-bool halo_ok(hpgx_state_t st) {
+bool halo_fits(hpgx_state_t st, int hx, int hy) {
   if (st->gridder != 4 && st->gridder != 5) return false;
-  const int hx = halo_x(st), hy = halo_y(st);
   return hx < hpgx::halo_tile_limit() && hy < hpgx::halo_tile_limit()
     && hpgx::halo_lds_bytes(hx, hy, 1) <= 65536;
 }
+bool halo_ok(hpgx_state_t st) { return halo_fits(st, halo_x(st), halo_y(st)); }
 
 // haloed tiles fed by block-local bins (grids of up to bin_keys_limit keys)
 bool use_halo(hpgx_state_t st) { return halo_ok(st) && use_block_local(st); }
@@ -356,12 +357,10 @@ bool use_sub(hpgx_state_t st) {
 // counters): grids of more keys than the block-local histogram holds
 bool use_sub_global(hpgx_state_t st) { return sub_ok(st) && use_halo_global(st); }
 
-// every CF group has the same support and number of Mueller elements
+// every CF group has the same support
 bool uniform_support(hpgx_state_t st) {
   for (const GroupInfo& g : st->groups)
-    if (g.sx != st->groups[0].sx || g.sy != st->groups[0].sy
-        || g.nmueller != st->groups[0].nmueller)
-      return false;
+    if (g.sx != st->groups[0].sx || g.sy != st->groups[0].sy) return false;
   return !st->groups.empty();
 }
 
@@ -1458,7 +1457,7 @@ int hpgx_set_convolution_function(
   std::vector<GroupInfo> groups(num_groups);
   long long toff = 0, woff = 0;
   int max_sx = 1, max_sy = 1, max_ncube = 1;
-  int min_nm = num_groups ? INT_MAX : 0, max_nm = 0;
+  int min_nm = num_groups ? INT_MAX : 0;
   bool even_nm = true;
   size_t max_stage = 0;
   for (unsigned g = 0; g < num_groups; ++g) {
@@ -1480,10 +1479,11 @@ int hpgx_set_convolution_function(
     max_sy = std::max(max_sy, gi.sy);
     max_ncube = std::max(max_ncube, gi.ncube);
     min_nm = std::min(min_nm, gi.nmueller);
-    max_nm = std::max(max_nm, gi.nmueller);
     even_nm = even_nm && gi.nmueller % 2 == 0;
     max_stage = std::max(max_stage, size_t(e[0]) * e[1] * e[2] * e[3]);
   }
+  // the layout of the kernels that the state's calls take (halo_ok)
+  const bool planar = st->npol == 1 && halo_fits(st, max_sx - 1, max_sy - 1);
   // the region that the shape asks for (hpgx_convolution_function_region_size),
   // of which the held elements take a part
   size_t ws = 0;
@@ -1506,8 +1506,9 @@ int hpgx_set_convolution_function(
       src = st->staging;
     }
     HPGX_HIP(st, hpgx::launch_cf_relayout(st->stream, src, e, groups[g], ce, os, F, nf,
-                                          st->cf.taps));
-    HPGX_HIP(st, hpgx::launch_cf_wsum(st->stream, groups[g], nf, st->cf.taps, st->cf.wsum));
+                                          planar, st->cf.taps));
+    HPGX_HIP(st, hpgx::launch_cf_wsum(st->stream, groups[g], nf, planar, st->cf.taps,
+                                      st->cf.wsum));
     if (memory != HPGX_DEVICE) HPGX_HIP(st, hipStreamSynchronize(st->stream));
   }
   if (num_groups > 0)
@@ -1534,8 +1535,8 @@ int hpgx_set_convolution_function(
   st->cf.max_sy = max_sy;
   st->cf.max_ncube = max_ncube;
   st->cf.min_nm = min_nm;
-  st->cf.max_nm = max_nm;
   st->cf.even_nm = even_nm;
+  st->cf.planar = planar;
   return ensure_call_buffers(st);
 }
 

@@ -30,6 +30,11 @@ constexpr int tile = 32;
 // (src/hpg_impl.hpp:221-281, src/hpg_core.hpp:422-446: major * os + minor).
 // wsum[wsum_offset + ((cube * nmueller + k) * nf + fx + F) * nf + fy + F]
 // is the FP64 sum of that element's taps of the slice.
+// Planar (one polarization, supports that the tile kernels take: a record reads
+// one element for a grid row): the slice's elements one after the other instead,
+//   ... * nf + fy + F) * nmueller + k) * sx * sy + Y * sx + X]
+// (one polarization in four grid rows of an element each, 500,000 records,
+// supports of 15, FP64: 896 us side by side, 678 so; predicted 1034, 606).
 // Only elements that some Mueller row names are held (CfElements, ascending;
 // the rows that the kernels see count in them): a tap's neighbours in memory
 // are then values that the calls read.  One polarization on a CF of 16 elements,
@@ -63,6 +68,7 @@ struct Geometry {
   int F;               // max |fine offset| = (os + 1) / 2
   int nf;              // 2F + 1
   int ngroups;
+  int planar;          // the CF layout (GroupInfo)
   int ntx, nty;        // tiles per plane along x and y
 };
 
@@ -117,17 +123,19 @@ struct DeviceCF {
   int os, F, nf, ngroups;
   int max_sx, max_sy;
   int max_ncube;  // CF cubes of the group with the most
-  int min_nm, max_nm;  // Mueller elements of the groups with the fewest and the most
+  int min_nm;     // Mueller elements of the group with the fewest
   bool even_nm;   // every group has an even number of them
+  bool planar;    // the layout (GroupInfo)
 };
 
 // ---- launchers (hpgx_kernels.hip) -------------------------------------
 
 hipError_t launch_cf_relayout(
   hipStream_t s, const float2* staging, const unsigned ext[4],
-  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, float2* taps);
+  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, bool planar,
+  float2* taps);
 hipError_t launch_cf_wsum(
-  hipStream_t s, const GroupInfo& gi, int nf, const float2* taps,
+  hipStream_t s, const GroupInfo& gi, int nf, bool planar, const float2* taps,
   double2* wsum);
 
 size_t tiles_per_footprint(int max_sx, int max_sy);

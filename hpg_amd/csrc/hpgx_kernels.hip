@@ -178,32 +178,43 @@ __device__ __forceinline__ void degrid_norms(
   }
 }
 
-// index of the first tap of Mueller element m in the CF slice (cube, fx,
-// fy); the element's tap t follows at t * g.nmueller
-// (UNIT: its CF group has one element)
-template <bool UNIT = false>
+// index of the first value of the CF slice (cube, fx, fy); its Mueller
+// element m follows at m, tap t at t * g.nmueller, or (planar) at m * ntap, t
 __device__ __forceinline__ long long slice_start(
+  const GroupInfo& g, int nf, int cube, int fxi, int fyi) {
+  const long long slice = ((long long)cube * nf + fxi) * nf + fyi;
+  return g.tap_offset + slice * ((long long)g.sx * g.sy * g.nmueller);
+}
+// of its element m in the planar form
+__device__ __forceinline__ long long plane_start(
   const GroupInfo& g, int nf, int cube, int m, int fxi, int fyi) {
   const long long slice = ((long long)cube * nf + fxi) * nf + fyi;
-  const long long ntap = (long long)g.sx * g.sy;
-  return UNIT ? g.tap_offset + slice * ntap : g.tap_offset + slice * (ntap * g.nmueller) + m;
+  return g.tap_offset + (slice * g.nmueller + m) * ((long long)g.sx * g.sy);
 }
 
 // ---- CF ingestion ----------------------------------------------------
 
 __global__ void k_cf_relayout(
   const float2* __restrict__ staging, unsigned ex, unsigned ey, unsigned em, GroupInfo gi,
-  CfElements ce, int os, int F, int nf, float2* __restrict__ taps, long long total,
+  CfElements ce, int os, int F, int nf, int planar, float2* __restrict__ taps, long long total,
   long long block0) {
   const long long o = (block0 + blockIdx.x) * (long long)blockDim.x + threadIdx.x;
   if (o >= total) return;
   long long q = o;
-  const int m = ce.elem[q % gi.nmueller];
-  q /= gi.nmueller;
+  int k = 0;
+  if (!planar) {
+    k = int(q % gi.nmueller);
+    q /= gi.nmueller;
+  }
   const int X = int(q % gi.sx);
   q /= gi.sx;
   const int Y = int(q % gi.sy);
   q /= gi.sy;
+  if (planar) {
+    k = int(q % gi.nmueller);
+    q /= gi.nmueller;
+  }
+  const int m = ce.elem[k];
   const int fyi = int(q % nf);
   q /= nf;
   const int fxi = int(q % nf);
@@ -226,7 +237,7 @@ constexpr int relayout_block = 256;
 constexpr size_t relayout_lds = 40960;
 __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
   const float2* __restrict__ staging, unsigned ex, unsigned ey, unsigned em, GroupInfo gi,
-  CfElements ce, int os, int F, int nf, float2* __restrict__ taps, int xc, int nxc,
+  CfElements ce, int os, int F, int nf, int planar, float2* __restrict__ taps, int xc, int nxc,
   long long block0) {
   extern __shared__ float2 win[];
   unsigned long long b = (unsigned long long)(block0 + blockIdx.x);
@@ -256,11 +267,19 @@ __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
   for (unsigned k = threadIdx.x; k < run * unsigned(nf); k += relayout_block) {
     const int fxi = int(k / run);
     const unsigned t = k - unsigned(fxi) * run;
-    const int X = int(t / unsigned(nm));
-    const int m = int(t - unsigned(X) * unsigned(nm));
-    taps[gi.tap_offset
-         + ((((long long)c * nf + fxi) * nf + fyi) * gi.sy + Y) * gi.sx * nm
-         + (long long)X0 * nm + t] = win[m * width + X * os + fxi];
+    const long long slice = ((long long)c * nf + fxi) * nf + fyi;
+    int X, m;
+    long long at;
+    if (planar) {
+      m = int(t / unsigned(cols));
+      X = int(t) - m * cols;
+      at = ((slice * nm + m) * gi.sy + Y) * gi.sx + X0 + X;
+    } else {
+      X = int(t / unsigned(nm));
+      m = int(t - unsigned(X) * unsigned(nm));
+      at = (slice * gi.sy + Y) * gi.sx * nm + (long long)X0 * nm + t;
+    }
+    taps[gi.tap_offset + at] = win[m * width + X * os + fxi];
   }
 }
 
@@ -269,20 +288,21 @@ __global__ __launch_bounds__(relayout_block) void k_cf_relayout_lds(
 // slice's size: large supports have few slices): thread t sums the values t,
 // t + threads, ... (coalesced reads), which with per = 2^k <= 64 elements all
 // belong to element t mod per, then a fixed-order reduction.  Other numbers of
-// elements (per = 0): one workgroup per slice and element.  FP64 sums of FP32
+// elements, and planar slices (per = 0): one workgroup per slice and element.  FP64 sums of FP32
 // taps: exact while the taps' exponents span fewer than about 29 bits, else
 // within a few FP64 ulps of any other order
 constexpr int wsum_block = 1024;
 __global__ __launch_bounds__(wsum_block) void k_cf_wsum(
   GroupInfo gi, int nf, const float2* __restrict__ taps,
-  double2* __restrict__ wsum, int per, long long block0) {
+  double2* __restrict__ wsum, int per, int planar, long long block0) {
   __shared__ double2 part[wsum_block / wave][wave];
   const int nm = gi.nmueller;
   const long long ntap = (long long)gi.sx * gi.sy;
   const long long b = block0 + blockIdx.x;
   const long long slice = per ? b : b / nm;  // (cube * nf + fx) * nf + fy
-  const int step = per ? 1 : nm;
-  const float2* t = taps + gi.tap_offset + slice * ntap * nm + (per ? 0 : int(b % nm));
+  const int step = per || planar ? 1 : nm;
+  const float2* t = taps + gi.tap_offset + slice * ntap * nm
+    + (per ? 0 : (b % nm) * (planar ? ntap : 1));
   const int keep = per ? per : 1;  // elements of this workgroup
   double re = 0.0, im = 0.0;
   for (long long k = threadIdx.x; k < ntap * keep; k += blockDim.x) {
@@ -1239,8 +1259,7 @@ __host__ __device__ inline int halo_pixels(int hx, int hy) {
 constexpr int acc_f64 = 0;
 constexpr int acc_f32_cas = 2;
 
-// UNIT: every CF group has one Mueller element
-template <int N, int MODE, int ACC, bool UNIT>
+template <int N, int MODE, int ACC>
 __global__ __launch_bounds__(halo_block) void k_tile4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
@@ -1360,7 +1379,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
       const int grp = int(e.h.gpk & 0xffffu);
       const int cfcube = int(e.h.gpk >> 16);
       const GroupInfo g = groups[grp];
-      const int sx = g.sx, sy = g.sy, nm = UNIT ? 1 : g.nmueller;
+      const int sx = g.sx, sy = g.sy;
       const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
       const float imf = pos_w ? -1.0f : 1.0f;
       const float2* slice[N];
@@ -1368,7 +1387,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
       for (int v = 0; v < N; ++v) {
         const int m = row[v];
         use[v] = m >= 0 && m < g.nmueller;
-        slice[v] = taps + slice_start<UNIT>(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
+        slice[v] = taps + plane_start(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
       }
       double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
       if (grad) {
@@ -1485,7 +1504,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
 #pragma unroll
             for (int v = 0; v < N; ++v) {
               float2 tv = make_float2(0.0f, 0.0f);
-              if (ok[k]) tv = slice[v][(t0 + k) * nm];
+              if (ok[k]) tv = slice[v][t0 + k];
               c[k][v] = use[v] ? tv : make_float2(0.0f, 0.0f);
             }
           }
@@ -1767,7 +1786,7 @@ __device__ __forceinline__ float2 screen_f32(double phi) {
 // one wave, one lane per tap, to the wave's FP32 region
 template <int N>
 __device__ __forceinline__ void sub_gradient_entry(
-  unsigned w0, int nm, const unsigned* slice, const float2* g, unsigned ri, unsigned pos,
+  unsigned w0, const unsigned* slice, const float2* g, unsigned ri, unsigned pos,
   const Geometry& geo, const float2* __restrict__ taps, const VisRec<N>* __restrict__ recs,
   int QX, float2* region) {
   const int lane = int(threadIdx.x % wave);
@@ -1792,7 +1811,7 @@ __device__ __forceinline__ void sub_gradient_entry(
   float h_r = 0.0f, h_i = 0.0f;
   for (int v = 0; v < N; ++v) {
     if (!((use >> v) & 1u)) continue;
-    float2 cc = taps[size_t(slice[v]) + size_t(tp) * nm];
+    float2 cc = taps[size_t(slice[v]) + size_t(tp)];
     cc.y *= imf;
     const float2 pr = cmul(cmul(cc, scr), g[v]);
     if constexpr (N == 1) {
@@ -2006,15 +2025,14 @@ void k_sub(
   // reads past taps_bytes return 0
   const __amdgpu_buffer_rsrc_t tap_rsrc = __builtin_amdgcn_make_buffer_rsrc(
     const_cast<float2*>(taps), 0, int(taps_bytes), 0x00020000);
-  // lanes holding a tap of a support (sx, sy) of a CF group with nm Mueller
-  // elements, and their tap byte offset
-  auto support_lanes = [&](int sx, int sy, int nm, unsigned& off) {
+  // lanes holding a tap of a support (sx, sy), and their tap byte offset
+  auto support_lanes = [&](int sx, int sy, unsigned& off) {
     const bool ok = lane_x < sx && lane_y < sy;
-    off = unsigned(ok ? (lane_y * sx + lane_x) * nm : 0) * unsigned(sizeof(float2));
+    off = unsigned(ok ? lane_y * sx + lane_x : 0) * unsigned(sizeof(float2));
     return ok;
   };
   unsigned tap_off = 0;
-  const bool uni_ok = UNI ? support_lanes(group0.sx, group0.sy, group0.nmueller, tap_off) : true;
+  const bool uni_ok = UNI ? support_lanes(group0.sx, group0.sy, tap_off) : true;
   int tap_key = -1;
   unsigned long long tap_lanes = 0ull;
 
@@ -2075,14 +2093,14 @@ void k_sub(
         const int m = pos_w ? row_m[v] : row_mc[v];
         const bool u = m >= 0 && m < g.nmueller;
         use |= u ? 1u << v : 0u;
-        p_sl[v] = unsigned(slice_start(g, geo.nf, cfcube, u ? m : 0, fxi, fyi));
+        p_sl[v] = unsigned(plane_start(g, geo.nf, cfcube, u ? m : 0, fxi, fyi));
         if (u && !grad) {
           p_gx[v] = e.g[v].x;
           p_gy[v] = e.g[v].y;
         }
       }
       const unsigned base = unsigned((ly - qy * quad_edge) * QX + (lx - qx * quad_edge));
-      p_key = unsigned(g.sx) | (unsigned(g.sy) << 6) | (unsigned(g.nmueller) << 12);
+      p_key = unsigned(g.sx) | (unsigned(g.sy) << 6);
       normal = !grad && use != 0u;
       if constexpr (PK) {
         p_addr = (p_sl[0] << sub_pk_shift) | (normal ? base | (pos_w ? sub_pk_flip : 0u) : 0u);
@@ -2109,7 +2127,7 @@ void k_sub(
         const int key_s = __builtin_amdgcn_readlane(int(p_key), j);
         if (key_s != tap_key) {
           tap_key = key_s;
-          tap_lanes = __ballot(support_lanes(key_s & 63, (key_s >> 6) & 63, key_s >> 12, tap_off));
+          tap_lanes = __ballot(support_lanes(key_s & 63, key_s >> 6, tap_off));
         }
         ring_lanes[r] = tap_lanes;
       }
@@ -2223,7 +2241,7 @@ void k_sub(
         const unsigned w0 = (gbase * unsigned(QX) + ((gpos & 63u) - unsigned(qx * quad_edge)))
           | (unsigned(gg.sx) << 12) | (unsigned(gg.sy) << 18) | (guse << 24)
           | (gpos_w ? quad_pos_w : 0u);
-        sub_gradient_entry<N>(w0, gg.nmueller, sl, gv, entry_vis[ej], ge.h.pos, geo, taps, recs,
+        sub_gradient_entry<N>(w0, sl, gv, entry_vis[ej], ge.h.pos, geo, taps, recs,
                               QX, region);
       }
       if (last_half && ((rd + 1u) % unsigned(sub_fold_rounds) == 0u || rd + 1u == nrounds)) {
@@ -2366,7 +2384,7 @@ __device__ __forceinline__ bool patch_record(
   const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
   e.gx = c.gx;
   e.gy = c.gy;
-  patch_pack(slice_start(g, geo.nf, int(cfcube), 0, fxi, fyi), g.sx, g.sy, e.base, e.sxy);
+  patch_pack(slice_start(g, geo.nf, int(cfcube), fxi, fyi), g.sx, g.sy, e.base, e.sxy);
   e.fl = unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0)) | (unsigned(fxi) << 8)
     | (unsigned(fyi) << 16);
   e.nm = unsigned(g.nmueller);
@@ -2680,6 +2698,7 @@ constexpr int patch_any = 0;   // any of the N elements, one load each
 constexpr int patch_full = 1;  // N neighbouring elements, N even, at 16-byte
                                // alignment: two elements a load
 constexpr int patch_one = 2;   // at most one element
+constexpr int patch_plane = 3;  // k_patch: that, of planar slices (one polarization)
 
 // the records that a launch takes for a pixel: all, those whose support corner
 // lies in the pixel's 32 x 32 tile, or the others
@@ -2695,7 +2714,9 @@ void k_patch(
   const VisRec<N>* __restrict__ recs, void* __restrict__ grid, unsigned block0) {
 
   constexpr int PW = patch_w(P), PH = patch_h(P);
-  constexpr int L = KIND == patch_one ? 1 : N;  // elements a lane loads per tap
+  constexpr bool PLANAR = KIND == patch_plane;
+  constexpr bool ONE = KIND == patch_one || PLANAR;
+  constexpr int L = ONE ? 1 : N;  // elements a lane loads per tap
   constexpr int SPLIT = patch_split(P);
   constexpr unsigned stage = SPLIT * patch_block;
   __shared__ PatchRec<N> st[stage];
@@ -2737,14 +2758,14 @@ void k_patch(
     for (int v = 0; v < N; ++v) {
       const int m0 = mu.Mc[r][v], m1 = mu.M[r][v];
       constexpr unsigned es = unsigned(sizeof(float2));
-      const int k = KIND == patch_one ? 0 : v;
+      const int k = ONE ? 0 : v;
       if (m0 >= 0) {
         eo[k] = unsigned(m0) * es;
-        if (KIND == patch_one) vs = unsigned(v);
+        if (ONE) vs = unsigned(v);
       }
       if (m1 >= 0) {
         eo_x[k] = unsigned(m1) * es;
-        if (KIND == patch_one) vs_x = unsigned(v);
+        if (ONE) vs_x = unsigned(v);
       }
     }
   }
@@ -2794,13 +2815,19 @@ void k_patch(
         // at most 2 PH rows: offsets of 32 bits (patch_offsets_fit)
         const int y0 = max(by - gy, 0);
         const int rows = min(sy - y0, 2 * PH);
-        const unsigned tap_bytes = nm * unsigned(sizeof(float2));
+        const unsigned elem_bytes = nm * unsigned(sizeof(float2));
+        // planar (one polarization): an element's taps lie side by side, the next
+        // element `plane` taps on
+        const unsigned plane = PLANAR ? unsigned(sx) * unsigned(sy) : 1u;
+        const unsigned tap_bytes = PLANAR ? unsigned(sizeof(float2)) : elem_bytes;
         const unsigned row_bytes = unsigned(sx) * tap_bytes;
         const float2* first = taps
           + ((unsigned long long)blo | ((unsigned long long)(bhi & patch_base_hi) << 32))
-          + (unsigned long long)unsigned(y0) * (unsigned(sx) * nm);
+          + (unsigned long long)unsigned(y0) * (unsigned(sx) * (PLANAR ? 1u : nm));
+        const unsigned bytes = unsigned(rows) * row_bytes
+          + (PLANAR ? (elem_bytes - unsigned(sizeof(float2))) * plane : 0u);
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<float2*>(first), 0, int(unsigned(rows) * row_bytes), 0x00020000);
+          const_cast<float2*>(first), 0, int(bytes), 0x00020000);
         const int X = bx + px - gx;
         const int Y = by + py - gy;
         const unsigned off0 = unsigned(Y - y0) * row_bytes + unsigned(X) * tap_bytes;
@@ -2812,8 +2839,8 @@ void k_patch(
           in[k] = unsigned(X + dx) < unsigned(sx) && unsigned(Y + dy) < unsigned(sy);
           // a row without its element takes nothing, nor do lanes past the rows
           // (of three rows: whole elements of none would be read at ~0u)
-          if constexpr (KIND == patch_one)
-            in[k] = in[k] && (eo[0] ^ (eo_x[0] & pm)) < tap_bytes;
+          if constexpr (ONE)
+            in[k] = in[k] && (eo[0] ^ (eo_x[0] & pm)) < elem_bytes;
           if constexpr (KIND == patch_full && P == 4) in[k] = in[k] && row < geo.nr;
           const unsigned off = off0 + unsigned(dy) * row_bytes + unsigned(dx) * tap_bytes;
           if constexpr (KIND == patch_full) {
@@ -2830,7 +2857,10 @@ void k_patch(
             for (int v = 0; v < L; ++v) {
               const unsigned ev = eo[v] ^ (eo_x[v] & pm);
               const v2i_t q = __builtin_amdgcn_raw_buffer_load_b64(
-                rsrc, int(in[k] && (KIND == patch_one || ev < tap_bytes) ? off + ev : ~0u), 0, 0);
+                rsrc,
+                int(in[k] && (ONE || ev < elem_bytes)
+                      ? off + (PLANAR ? ev * plane : ev) : ~0u),
+                0, 0);
               c[k][v] = make_float2(__int_as_float(q.x), __int_as_float(q.y));
             }
           }
@@ -2864,7 +2894,7 @@ void k_patch(
         float2 g[L], gs[L];
 #pragma unroll
         for (int v = 0; v < L; ++v) {
-          g[v] = KIND == patch_one ? e.g[vs ^ (vs_x & pm)] : e.g[v];
+          g[v] = ONE ? e.g[vs ^ (vs_x & pm)] : e.g[v];
           gs[v] = make_float2(imf * g[v].x, imf * g[v].y);
         }
 #pragma unroll
@@ -2880,7 +2910,7 @@ void k_patch(
               sr += double(pr);
               si += double(pi);
             } else {
-              const bool use = (eo[v] ^ (eo_x[v] & pm)) < tap_bytes;
+              const bool use = (eo[v] ^ (eo_x[v] & pm)) < elem_bytes;
               sr += use ? double(pr) : 0.0;
               si += use ? double(pi) : 0.0;
             }
@@ -3054,7 +3084,7 @@ __global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4)
       const float2* cf = taps
         + ((unsigned long long)unsigned(of(int(unsigned(e.base)), j))
            | ((unsigned long long)unsigned(of(int(e.base >> 32), j)) << 32));
-      return in ? cf[unsigned(Y) * ((sxy & 0xffffu) * nm) + unsigned(X) * nm + unsigned(el)]
+      return in ? cf[(unsigned(el) * (sxy >> 16) + unsigned(Y)) * (sxy & 0xffffu) + unsigned(X)]
                 : make_float2(0.0f, 0.0f);
     };
     auto add = [&](int j, int gp, float2 cc, bool in, int px) {
@@ -3208,7 +3238,7 @@ __global__ __launch_bounds__(patch_local_threads) void k_degrid_keys(
             + (unsigned(c.gx) >> dk.region_sh);
           key = (gcube * dk.regions + region) * dk.slices + grp * dk.stride
             + (cfcube * unsigned(geo.nf) + fxi) * unsigned(geo.nf) + fyi;
-          patch_pack(slice_start(g, geo.nf, int(cfcube), 0, int(fxi), int(fyi)), g.sx, g.sy,
+          patch_pack(slice_start(g, geo.nf, int(cfcube), int(fxi), int(fyi)), g.sx, g.sy,
                      d.base, d.sxy);
           d.corner = ((long long)gcube * geo.nr * geo.ny + c.gy) * geo.nx + c.gx;
           d.fl = unsigned((r.uvw[2] > 0 ? flag_pos_w : 0) | (grad ? flag_gradient : 0))
@@ -3376,16 +3406,18 @@ void k_degrid(
     const unsigned ntap = unsigned(sx) * unsigned(sy);  // of one slice: below 2^32 in 288 GB
     const unsigned nm = lane_u32(d.nm, r);
     const int pm = (lane_u32(d.fl, r) & flag_pos_w) ? -1 : 0;
+    const bool planar = N == 1 && geo.planar;
+    const unsigned step = planar ? 1u : nm;  // from tap to tap
     const float2* cf = taps
       + (base & (((unsigned long long)patch_base_hi << 32) | 0xffffffffull))
-      + size_t(q) * nm;  // this lane's tap
+      + size_t(q) * step;  // this lane's tap
     unsigned eo[L];                                                  // its elements
     bool use[L];
 #pragma unroll
     for (int v = 0; v < L; ++v) {
       const int m = el[v] ^ (el_x[v] & pm);
       use[v] = m >= 0 && m < int(nm);
-      eo[v] = unsigned(use[v] ? m : 0);
+      eo[v] = unsigned(use[v] ? m : 0) * (planar ? ntap : 1u);
     }
     const double2* mp[RR];
     unsigned flip[RR];  // w <= 0: the imaginary parts' sign
@@ -3442,7 +3474,7 @@ void k_degrid(
 #pragma unroll
           for (int v = 0; v < L; ++v) c[u][v] = cf[eo[v]];
         }
-        cf += size_t(TPS) * nm;
+        cf += size_t(TPS) * step;
 #pragma unroll
         for (int k = 0; k < RR; ++k) m[u][k] = mp[k][off];
         if constexpr (GRAD)
@@ -3556,8 +3588,7 @@ __device__ __noinline__ double2 degrid_screen(double2 m, double ph) {
 // cphase out of line, for the same reason
 __device__ __noinline__ double2 cphase_call(double ph) { return cphase(ph); }
 
-// UNIT: every CF group has one Mueller element
-template <int N, bool UNIT>
+template <int N>
 __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 1))) void k_degrid4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
@@ -3648,7 +3679,7 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
     const int grp = int(eh.gpk & 0xffffu);
     const int cfcube = int(eh.gpk >> 16);
     const GroupInfo g = groups[grp];
-    const int sx = g.sx, sy = g.sy, nm = UNIT ? 1 : g.nmueller;
+    const int sx = g.sx, sy = g.sy;
     // degridding uses the other Mueller matrix and the opposite conjugation
     // of gridding (src/hpg_core.hpp:598-600)
     const int* row = pos_w ? mu.Mc[gpol] : mu.M[gpol];
@@ -3658,7 +3689,7 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
     for (int v = 0; v < N; ++v) {
       const int m = row[v];
       use[v] = m >= 0 && m < g.nmueller;
-      slice[v] = taps + slice_start<UNIT>(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
+      slice[v] = taps + plane_start(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
     }
     double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
     if (grad) {
@@ -3714,7 +3745,7 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
 #pragma unroll
           for (int v = 0; v < N; ++v) {
             float2 tv = make_float2(0.0f, 0.0f);
-            if (ok[k]) tv = slice[v][(t0 + k) * nm];
+            if (ok[k]) tv = slice[v][t0 + k];
             c[k][v] = tv;
           }
         }
@@ -3943,7 +3974,8 @@ hipError_t in_launches(unsigned long long blocks, int threads, F launch) {
 
 hipError_t launch_cf_relayout(
   hipStream_t s, const float2* staging, const unsigned ext[4],
-  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, float2* taps) {
+  const GroupInfo& gi, const CfElements& ce, int os, int F, int nf, bool planar,
+  float2* taps) {
   const long long total =
     (long long)gi.ncube * gi.nmueller * nf * nf * gi.sx * gi.sy;
   if (total == 0) return hipSuccess;
@@ -3959,28 +3991,28 @@ hipError_t launch_cf_relayout(
     return in_launches(blocks, relayout_block, [&](unsigned long long first, unsigned nb) {
       hipLaunchKernelGGL(
         k_cf_relayout_lds, dim3(nb), dim3(relayout_block), lds(xc), s, staging, ext[0], ext[1],
-        ext[2], gi, ce, os, F, nf, taps, xc, nxc, (long long)first);
+        ext[2], gi, ce, os, F, nf, int(planar), taps, xc, nxc, (long long)first);
     });
   return in_launches((total + block - 1) / block, block,
                      [&](unsigned long long first, unsigned nb) {
     hipLaunchKernelGGL(
       k_cf_relayout, dim3(nb), dim3(block), 0, s, staging, ext[0], ext[1], ext[2], gi, ce, os, F,
-      nf, taps, total, (long long)first);
+      nf, int(planar), taps, total, (long long)first);
   });
 }
 
 hipError_t launch_cf_wsum(
-  hipStream_t s, const GroupInfo& gi, int nf, const float2* taps,
+  hipStream_t s, const GroupInfo& gi, int nf, bool planar, const float2* taps,
   double2* wsum) {
   const int nm = gi.nmueller;
-  const int per = nm > 0 && nm <= wave && (nm & (nm - 1)) == 0 ? nm : 0;
+  const int per = !planar && nm > 0 && nm <= wave && (nm & (nm - 1)) == 0 ? nm : 0;
   const long long ns = (long long)gi.ncube * (per ? 1 : nm) * nf * nf;
   if (ns == 0) return hipSuccess;
   const long long values = (long long)gi.sx * gi.sy * (per ? per : 1);
   const int threads = values <= 1024 ? wave : values <= 8192 ? 256 : wsum_block;
   return in_launches(ns, threads, [&](unsigned long long first, unsigned nb) {
     hipLaunchKernelGGL(k_cf_wsum, dim3(nb), dim3(threads), 0, s, gi, nf, taps, wsum, per,
-                       (long long)first);
+                       int(planar), (long long)first);
   });
 }
 
@@ -4219,7 +4251,7 @@ hipError_t launch_tile_sub(
   // by tap index below sub_pk_taps
   static_assert(9 * wave < int(sub_pk_flip), "region pixel in the packed word");
   const bool pk = npol == 1 && taps_bytes / sizeof(float2) < sub_pk_taps;
-  if (npol != 1) return hipErrorInvalidValue;
+  if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
   if (pk) HPGX_SUB_PX(HPGX_SUB_1, 1, true) else HPGX_SUB_PX(HPGX_SUB_1, 1, false)
 #undef HPGX_SUB_PX
 #undef HPGX_SUB_1
@@ -4243,12 +4275,11 @@ hipError_t launch_tile_halo(
   if (lds > 65536) return hipErrorInvalidValue;
 #define HPGX_TILE4(MD, AC)                                                     \
   hipLaunchKernelGGL(                                                          \
-    cf.max_nm == 1 ? (k_tile4<1, MD, AC, true>) : (k_tile4<1, MD, AC, false>), \
-    dim3(unsigned(nkeys)), dim3(halo_block), lds, s,                           \
+    (k_tile4<1, MD, AC>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s,                           \
     geo, cf.groups, cf.taps, mu, table, nb, block_cap,                         \
     static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,            \
     static_cast<const VisRec<1>*>(cb.vis), hx, hy, grid, cb.halo, cb.halo_set)
-  if (npol != 1) return hipErrorInvalidValue;
+  if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
   if (mode == 0)
     HPGX_TILE4(0, acc_f64);
   else if (acc == 0)
@@ -4394,7 +4425,8 @@ hipError_t launch_patch(
        ++take) {
     switch (npol) {
     case 1:
-      HPGX_PATCH_K(1, patch_one);
+      if (cf.planar) HPGX_PATCH_K(1, patch_plane);
+      else HPGX_PATCH_K(1, patch_one);
       break;
     case 2:
       if (kind == patch_one) HPGX_PATCH_K(2, patch_one);
@@ -4434,7 +4466,7 @@ hipError_t launch_direct(
   bool update_weights, bool gvis_ready, GvisSource src, const double2* residuals,
   const CallBuffers& cb, double* weights, int mode, void* grid) {
   if (n == 0) return hipSuccess;
-  if (npol != 1 || n > direct_records || geo.nr > 4) return hipErrorInvalidValue;
+  if (npol != 1 || !cf.planar || n > direct_records || geo.nr > 4) return hipErrorInvalidValue;
   const size_t lds = size_t(geo.nr) * 2 * direct_plane * sizeof(double);
   const DirectArgs args{cf.groups, cf.wsum, cb.gvis, residuals, weights, cb.invalid_count,
                         int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint)};
@@ -4454,19 +4486,12 @@ hipError_t launch_degrid_tiles(
   const int nb = bin_blocks_for(n);
   const size_t lds = halo_lds_bytes(hx, hy, nb);
   if (lds > 65536) return hipErrorInvalidValue;
-#define HPGX_DEGRID4(UNIT)                                                     \
-  hipLaunchKernelGGL(                                                          \
-    (k_degrid4<1, UNIT>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo, \
-    cf.groups, cf.taps, mu, cb.off_table, nb, block_cap,                       \
-    static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,            \
-    static_cast<const VisRec<1>*>(cb.vis), hx, hy, model, acc, int(one_plane), \
-    cf.wsum, int(do_grid), static_cast<VisRec<1>*>(out_recs), cb.gvis, pred64)
-  if (npol != 1) return hipErrorInvalidValue;
-  if (cf.max_nm == 1)
-    HPGX_DEGRID4(true);
-  else
-    HPGX_DEGRID4(false);
-#undef HPGX_DEGRID4
+  if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(
+    k_degrid4<1>, dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo, cf.groups, cf.taps, mu,
+    cb.off_table, nb, block_cap, static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,
+    static_cast<const VisRec<1>*>(cb.vis), hx, hy, model, acc, int(one_plane), cf.wsum,
+    int(do_grid), static_cast<VisRec<1>*>(out_recs), cb.gvis, pred64);
   return hipGetLastError();
 }
 
