@@ -453,6 +453,13 @@ int ensure_call_buffers(hpgx_state_t st) {
         HPGX_HIP(st, dev_alloc(cb.patch_table, table * sizeof(unsigned)));
         cb.patch_table_capacity = table;
       }
+      const size_t slots = hpgx::patch_split_slots(recs * tiles);
+      if (slots > cb.patch_split_slots) {
+        dev_free(cb.patch_split);
+        cb.patch_split_slots = 0;
+        HPGX_HIP(st, dev_alloc(cb.patch_split, hpgx::patch_split_bytes(slots)));
+        cb.patch_split_slots = slots;
+      }
     }
     // bin entries for the whole batch, up to the entry memory budget; larger
     // batches are gridded in chunks (run_grid)
@@ -568,6 +575,7 @@ void free_state(hpgx_state_t st) {
   dev_free(cb.patch_recs);
   dev_free(cb.patch_list);
   dev_free(cb.patch_table);
+  dev_free(cb.patch_split);
   dev_free(cb.hist);
   dev_free(cb.offsets);
   dev_free(cb.cursor);
@@ -1048,6 +1056,10 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
     c.scan_temp = p;
     c.scan_temp_bytes = st->cb.scan_temp_bytes;
     p += up(c.scan_temp_bytes);
+    // (a few slots for split lists: 4 MB of the 64)
+    c.patch_split_slots = std::min<size_t>(256, hpgx::patch_split_slots(n * tiles));
+    c.patch_split = p;
+    p += up(hpgx::patch_split_bytes(c.patch_split_slots));
     const size_t used = size_t(p - static_cast<char*>(base)) + 2 * 256;
     auto fits = [&](size_t r) {
       return used + r * (rec + tiles * sizeof(unsigned))

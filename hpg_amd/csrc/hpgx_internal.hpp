@@ -110,6 +110,8 @@ struct CallBuffers {
   size_t patch_list_capacity;
   unsigned* patch_table;  // and the workgroups' places in them (few tiles)
   size_t patch_table_capacity;
+  void* patch_split;      // and the chunks of split lists: their sums and slots
+  size_t patch_split_slots;
   unsigned* degrid_order; // launch_degrid: keys, the record order, (key, record)
                           // pairs, 4 order_capacity values
   void* degrid_recs;      // and its prepared records (DegridRec)
@@ -212,6 +214,11 @@ size_t patch_keys(const Geometry& geo);
 size_t patch_rec_bytes(int npol);
 // values of cb.patch_table for n records a call (0 for many tiles)
 size_t patch_table_entries(const Geometry& geo, size_t n);
+// slots of cb.patch_split for lists of so many entries in all, at most
+// patch_slots_max, and the bytes they take
+constexpr size_t patch_slots_max = 2048;
+size_t patch_split_slots(size_t entries);
+size_t patch_split_bytes(size_t slots);
 size_t patch_tiles_per_footprint(int nr, int max_sx, int max_sy);
 // the rows of a slice that one wave's pixels take have 32-bit byte offsets (not
 // so from 2^32 bytes in 16 rows on: CFs of 38 GB at the least)

@@ -2348,6 +2348,20 @@ __device__ __forceinline__ int patch_sx(unsigned sxy, unsigned base_hi) {
 __device__ __forceinline__ int patch_sy(unsigned sxy, unsigned base_hi) {
   return int((sxy >> 16) | ((base_hi >> 2) & 0x3fff0000u));
 }
+// of a uniform record: supports of 65536 pixels and more by a branch, whose
+// instructions would lengthen the loops' scalar chains (228 -> 231 us, two
+// polarizations, 300,000 records)
+__device__ __forceinline__ void patch_unpack(
+  unsigned sxy, unsigned& base_hi, int& sx, int& sy) {
+  sx = int(sxy & 0xffffu);
+  sy = int(sxy >> 16);
+  if (__builtin_expect(base_hi > patch_base_hi, 0)) {
+    asm volatile("");  // kept a branch
+    sx = patch_sx(sxy, base_hi);
+    sy = patch_sy(sxy, base_hi);
+    base_hi &= patch_base_hi;
+  }
+}
 
 // record i, whose support at c is inside the grid, prepared (sxy = 0 and
 // false: no row takes it), and its weight in each grid row
@@ -2561,15 +2575,80 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_l
 // them (200,000 records, supports 9-25: 1172 -> 1071 us, two polarizations,
 // 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
 // in place of hipCUB's scan (10 us).  order null: the scan alone.
+//
+// A list of two chunks or more is split: one workgroup for each chunk of it, in
+// slots next to each other (the last of a tile's to end adds up their sums in the
+// slots' order), or a dense uv core would be one workgroup's serial chain.  The
+// chunk is the least, from patch_chunk_min on, that leaves the launch enough slots:
+// a list of two chunks or more has 1.5 slots a chunk of its entries at most.
+// Two polarizations, FP64: 100,000 records of supports 5 within a few pixels 28.5 ->
+// 0.41 ms (1.8 by haloed LDS tiles), 200,000 on 128^2, supports 3, 2.38 -> 0.21
+// (0.37), 10,000 on 256^2 104 -> 91 us (75); least chunks of 16 and 64 are 5 and 4%
+// slower there.  With a fence of the device's scope instead of stores past the L2s
+// 116 us: it writes a whole L2 back for every chunk.
+constexpr unsigned patch_chunk_min = 32;
+constexpr unsigned patch_none = ~0u;  // in the tiles' order: a split one
+constexpr int patch_values = 8 * patch_block;
+// device scope: past the XCDs' own L2s
+__device__ __forceinline__ void patch_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double patch_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+struct PatchSplit {
+  unsigned slots;  // of the launch; 0: no list is split
+  char* base;
+  // slots taken, chunk
+  __host__ __device__ unsigned* ctl() const { return reinterpret_cast<unsigned*>(base); }
+  // a slot's patch_values sums
+  __device__ double* sums(unsigned slot) const {
+    return reinterpret_cast<double*>(base + 256) + size_t(slot) * patch_values;
+  }
+  // (tile, chunk's number) of every slot
+  __device__ uint2* items() const { return reinterpret_cast<uint2*>(sums(slots)); }
+  // of a tile's first slot, for each of two k_patch launches
+  __device__ unsigned* tickets() const { return reinterpret_cast<unsigned*>(items() + slots); }
+};
+__device__ __forceinline__ unsigned patch_chunk(unsigned total, unsigned slots) {
+  return max(patch_chunk_min, unsigned(1.5 * double(total) / double(slots)) + 1u);
+}
+// the slots of a tile whose list has cnt entries, taken from *taken
+__device__ __forceinline__ void patch_take(
+  const PatchSplit& ps, unsigned chunk, unsigned key, unsigned cnt, unsigned* taken, int scope) {
+  const unsigned m = (cnt + chunk - 1u) / chunk;
+  const unsigned at = scope == __HIP_MEMORY_SCOPE_WORKGROUP
+    ? __hip_atomic_fetch_add(taken, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+    : atomicAdd(taken, m);
+  ps.tickets()[at] = ps.tickets()[ps.slots + at] = 0u;
+  for (unsigned i = 0; i < m; ++i) ps.items()[at + i] = make_uint2(key, i);
+}
+// the same for more tiles than k_patch_scan takes, and their order, as they come
+__global__ __launch_bounds__(block) void k_patch_split(
+  size_t keys, const unsigned* __restrict__ offsets, unsigned* __restrict__ order,
+  PatchSplit ps) {
+  const size_t k = blockIdx.x * (size_t)block + threadIdx.x;
+  if (k >= keys) return;
+  const unsigned chunk = patch_chunk(offsets[keys], ps.slots);
+  if (k == 0) ps.ctl()[1] = chunk;
+  const unsigned cnt = offsets[k + 1] - offsets[k];
+  const bool split = cnt >= 2u * chunk;
+  order[k] = split ? patch_none : unsigned(k);
+  if (split)
+    patch_take(ps, chunk, unsigned(k), cnt, ps.ctl(), __HIP_MEMORY_SCOPE_AGENT);
+}
+
 constexpr int patch_scan_threads = 1024;
 constexpr int patch_scan_keys = patch_local_keys;
 constexpr int patch_classes = 6;
 __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
   int keys, const unsigned* __restrict__ hist, unsigned* __restrict__ offsets,
-  unsigned* __restrict__ order) {
+  unsigned* __restrict__ order, PatchSplit ps) {
   __shared__ unsigned a[patch_scan_keys + 1];
   __shared__ unsigned part[patch_scan_threads / wave + 1];
   __shared__ unsigned cls[patch_classes];
+  __shared__ unsigned taken;
+  if (threadIdx.x == 0) taken = 0u;
   for (int k = threadIdx.x; k < keys; k += patch_scan_threads) a[k] = hist[k];
   if (threadIdx.x < patch_classes) cls[threadIdx.x] = 0u;
   __syncthreads();
@@ -2582,6 +2661,7 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
   }
   const int lane = threadIdx.x % wave;
   const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
+  const unsigned chunk = ps.slots ? patch_chunk(total, ps.slots) : 0x7fffffffu;
   // class 0: over four times the mean, ..., the last: empty
   auto class_of = [&](int k) {
     const unsigned long long c = (unsigned long long)(a[k + 1] - a[k]) * unsigned(keys);
@@ -2603,8 +2683,14 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
           at = __hip_atomic_fetch_add(cls + c, unsigned(__builtin_popcountll(m)),
                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         at = unsigned(__builtin_amdgcn_readlane(int(at), lead));
-        if (pass == 1 && q == c)
-          order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] = unsigned(k);
+        if (pass == 1 && q == c) {
+          const unsigned cnt = a[k + 1] - a[k];
+          const bool split = cnt >= 2u * chunk;
+          order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] =
+            split ? patch_none : unsigned(k);
+          if (split)
+            patch_take(ps, chunk, unsigned(k), cnt, &taken, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
       }
     }
     __syncthreads();
@@ -2618,7 +2704,13 @@ __global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) offsets[keys] = total;
+  if (threadIdx.x == 0) {
+    offsets[keys] = total;
+    if (ps.slots) {
+      ps.ctl()[0] = taken;
+      ps.ctl()[1] = chunk;
+    }
+  }
 }
 
 // 64 zeros and the 1152 bits of 2 / pi behind the point (computed from Machin's
@@ -2711,7 +2803,7 @@ void k_patch(
   Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode, int take, int ptx, int pty,
   const unsigned* __restrict__ offsets, const unsigned* __restrict__ order,
   const unsigned* __restrict__ list, const PatchRec<N>* __restrict__ prs,
-  const VisRec<N>* __restrict__ recs, void* __restrict__ grid, unsigned block0) {
+  const VisRec<N>* __restrict__ recs, void* __restrict__ grid, unsigned block0, PatchSplit ps) {
 
   constexpr int PW = patch_w(P), PH = patch_h(P);
   constexpr bool PLANAR = KIND == patch_plane;
@@ -2722,10 +2814,36 @@ void k_patch(
   __shared__ PatchRec<N> st[stage];
   __shared__ unsigned st_i[stage];
 
+  // the slots of split lists first, then every tile
   const unsigned b = block0 + blockIdx.x;
-  const unsigned key = order ? order[b] : b;
-  const unsigned beg = offsets[key];
-  const unsigned cnt = offsets[key + 1] - beg;
+  const bool split = b < ps.slots;
+  unsigned key;
+  uint2 ctl = make_uint2(0u, 0u), it = make_uint2(0u, 0u);
+  if (split) {
+    ctl = *reinterpret_cast<const uint2*>(ps.ctl());
+    it = ps.items()[b];
+    if (b >= ctl.x) return;
+    key = it.x;
+  } else {
+    key = order ? order[b - ps.slots] : b - ps.slots;
+    if (key == patch_none) return;
+  }
+  unsigned beg = offsets[key];
+  unsigned cnt = offsets[key + 1] - beg;
+  // what the end of a chunk needs, in LDS: scalar registers held through the loop
+  // would spill others
+  __shared__ unsigned chunk_slot, chunk_slot0, chunk_count;
+  __shared__ PatchSplit chunk_ps;
+  if (split) {
+    if (threadIdx.x == 0) {
+      chunk_slot = b;
+      chunk_slot0 = b - it.y;
+      chunk_count = (cnt + ctl.y - 1u) / ctl.y;
+      chunk_ps = ps;
+    }
+    beg += it.y * ctl.y;
+    cnt = min(ctl.y, cnt - it.y * ctl.y);
+  }
   if (cnt == 0) return;
   const int tx = int(key % unsigned(ptx));
   const int tq = int(key / unsigned(ptx));
@@ -2803,12 +2921,13 @@ void k_patch(
         const int gx = __builtin_amdgcn_readlane(hgx, j);
         const int gy = __builtin_amdgcn_readlane(hgy, j);
         const unsigned blo = unsigned(__builtin_amdgcn_readlane(int(unsigned(hbase)), j));
-        const unsigned bhi = unsigned(__builtin_amdgcn_readlane(int(hbhi), j));
+        unsigned bhi = unsigned(__builtin_amdgcn_readlane(int(hbhi), j));
         const unsigned sxy = unsigned(__builtin_amdgcn_readlane(int(hsxy), j));
         const unsigned fl = unsigned(__builtin_amdgcn_readlane(int(hfl), j));
         const unsigned nm = unsigned(__builtin_amdgcn_readlane(int(hnm), j));
         const PatchRec<N>& e = st[k0 + unsigned(j)];
-        const int sx = patch_sx(sxy, bhi), sy = patch_sy(sxy, bhi);
+        int sx, sy;
+        patch_unpack(sxy, bhi, sx, sy);
         const bool pos_w = fl & flag_pos_w;
         const unsigned pm = pos_w ? ~0u : 0u;
         // the slice from the first support row within the wave's pixels on,
@@ -2822,7 +2941,7 @@ void k_patch(
         const unsigned tap_bytes = PLANAR ? unsigned(sizeof(float2)) : elem_bytes;
         const unsigned row_bytes = unsigned(sx) * tap_bytes;
         const float2* first = taps
-          + ((unsigned long long)blo | ((unsigned long long)(bhi & patch_base_hi) << 32))
+          + ((unsigned long long)blo | ((unsigned long long)bhi << 32))
           + (unsigned long long)unsigned(y0) * (unsigned(sx) * (PLANAR ? 1u : nm));
         const unsigned bytes = unsigned(rows) * row_bytes
           + (PLANAR ? (elem_bytes - unsigned(sizeof(float2))) * plane : 0u);
@@ -2936,8 +3055,8 @@ void k_patch(
       }
     }
     __syncthreads();
-    if (part > 0) return;
     for (int o = 1; o < SPLIT; ++o) {
+      if (part > 0) break;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const double* q = sums + ((size_t(w + 4 * (o - 1)) * 8 + 2 * k) * wave + lane);
@@ -2946,14 +3065,54 @@ void k_patch(
       }
     }
   }
+  if (split) {
+    const unsigned chunks = unsigned(uniform(int(chunk_count)));
+    // this chunk's sums into its slot; the tile's last chunk to get here goes on
+    // with those of all of them
+    __shared__ unsigned ticket;
+    const PatchSplit cs = chunk_ps;
+    if (part == 0) {
+      double* q = cs.sums(chunk_slot) + threadIdx.x;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        patch_store(q + 2 * k * patch_block, ar[k]);
+        patch_store(q + (2 * k + 1) * patch_block, ai[k]);
+      }
+    }
+    // written through to where every XCD reads them, before the ticket
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      ticket = atomicAdd(cs.tickets() + (take == patch_others ? cs.slots : 0u) + chunk_slot0, 1u);
+    __syncthreads();
+    if (ticket + 1u != chunks) return;
+    if (part == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ar[k] = ai[k] = 0.0;
+      const double* q = cs.sums(chunk_slot0) + threadIdx.x;
+#pragma unroll 1
+      for (unsigned c = 0; c < chunks; ++c, q += patch_values) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = patch_load(q + k * patch_block);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          ar[k] += v[2 * k];
+          ai[k] += v[2 * k + 1];
+        }
+      }
+    }
+  }
 
   // the tile's only writer: a plain read-modify-write of each pixel
-  if (row >= geo.nr) return;
+  if (part > 0 || row >= geo.nr) return;
   const size_t plane = (size_t(cube) * geo.nr + row) * size_t(geo.ny) * geo.nx;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int x = bx + px + (k & 1) * PW, y = by + py + (k >> 1) * PH;
     if (x >= geo.nx || y >= geo.ny) continue;
+    // a patch that nothing was added to stays as it is
+    if (!__any(ar[k] != 0.0 || ai[k] != 0.0)) continue;
     const size_t gi = plane + size_t(y) * geo.nx + x;
     if (mode == 0) {
       double2* gp = static_cast<double2*>(grid) + gi;
@@ -3400,16 +3559,17 @@ void k_degrid(
     constexpr int RR = decltype(rr_c)::value;
     constexpr bool GRAD = decltype(grad_c)::value;
     const unsigned sxy = lane_u32(d.sxy, r);
-    const unsigned long long base = lane_u64(d.base, r);
-    const int sx = patch_sx(sxy, unsigned(base >> 32));
-    const int sy = patch_sy(sxy, unsigned(base >> 32));
+    const unsigned base_lo = lane_u32(unsigned(d.base), r);
+    unsigned base_hi = lane_u32(unsigned(d.base >> 32), r);
+    int sx, sy;
+    patch_unpack(sxy, base_hi, sx, sy);
     const unsigned ntap = unsigned(sx) * unsigned(sy);  // of one slice: below 2^32 in 288 GB
     const unsigned nm = lane_u32(d.nm, r);
     const int pm = (lane_u32(d.fl, r) & flag_pos_w) ? -1 : 0;
     const bool planar = N == 1 && geo.planar;
     const unsigned step = planar ? 1u : nm;  // from tap to tap
     const float2* cf = taps
-      + (base & (((unsigned long long)patch_base_hi << 32) | 0xffffffffull))
+      + ((unsigned long long)base_lo | ((unsigned long long)base_hi << 32))
       + size_t(q) * step;  // this lane's tap
     unsigned eo[L];                                                  // its elements
     bool use[L];
@@ -4087,7 +4247,7 @@ hipError_t launch_sort_place(hipStream_t s, size_t n, size_t batch, const SortKe
   unsigned* offsets = hist + patch_local_keys + 1;
   const unsigned* table = offsets + patch_local_keys + 1;
   hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, sk.bins, hist, offsets,
-                     static_cast<unsigned*>(nullptr));
+                     static_cast<unsigned*>(nullptr), PatchSplit{});
   hipLaunchKernelGGL(k_sort_place, dim3(unsigned((n + batch - 1) / batch)),
                      dim3(patch_local_threads), 0, s, n, sk, unsigned(batch), keys, offsets, table,
                      order, pairs);
@@ -4307,6 +4467,13 @@ size_t patch_table_entries(const Geometry& geo, size_t n) {
   const size_t keys = patch_keys(geo);
   return keys <= size_t(patch_local_keys) ? std::min<size_t>((n + 2047) / 2048, 512) * keys : 0;
 }
+// slots for the split lists of so many entries in all, and their memory
+size_t patch_split_slots(size_t entries) {
+  return std::min<size_t>(patch_slots_max, entries * 3 / (2 * patch_chunk_min));
+}
+size_t patch_split_bytes(size_t slots) {
+  return slots * (patch_values * sizeof(double) + sizeof(uint2) + 2 * sizeof(unsigned)) + 256;
+}
 size_t patch_rec_bytes(int npol) {
   switch (npol) {
   case 1: return sizeof(PatchRec<1>);
@@ -4356,6 +4523,11 @@ hipError_t launch_patch(
   // a kernel, not a memset: a captured graph may replay it
   hipLaunchKernelGGL(k_zero, dim3(blocks_for(keys + 1)), dim3(block), 0, s, cb.hist, keys + 1);
   const bool local = keys <= size_t(patch_local_keys);
+  PatchSplit ps{};
+  ps.slots = unsigned(std::min(
+    cb.patch_split_slots,
+    patch_split_slots(n * patch_tiles_per_footprint(geo.nr, cf.max_sx, cf.max_sy))));
+  ps.base = static_cast<char*>(cb.patch_split);
   const size_t batch = patch_batch(n);
   const unsigned nb = local ? unsigned((n + batch - 1) / batch) : 0u;
   if (local && nb * keys > cb.patch_table_capacity) return hipErrorInvalidValue;
@@ -4376,13 +4548,13 @@ hipError_t launch_patch(
     patch_tile_x(P), patch_tile_y(P), static_cast<const PatchRec<NP>*>(cb.patch_recs), \
     cb.hist, cb.offsets, cb.patch_list, unsigned(batch), cb.patch_table)
 #define HPGX_PATCH_P(NP, PP, KD)                                               \
-  e = in_launches(keys, patch_split(PP) * patch_block,                         \
+  e = in_launches(ps.slots + keys, patch_split(PP) * patch_block,              \
                   [&](unsigned long long first, unsigned blocks) {             \
     hipLaunchKernelGGL(                                                        \
       (k_patch<NP, PP, KD>), dim3(blocks), dim3(patch_split(PP) * patch_block), 0, s, \
       geo, cf.taps, mu, mode, take, ptx, pty, cb.offsets, order, cb.patch_list, \
       static_cast<const PatchRec<NP>*>(cb.patch_recs),                         \
-      static_cast<const VisRec<NP>*>(cb.vis), grid, unsigned(first));          \
+      static_cast<const VisRec<NP>*>(cb.vis), grid, unsigned(first), ps);      \
   })
 #define HPGX_PATCH_K(NP, KD)                                                   \
   do {                                                                         \
@@ -4403,12 +4575,19 @@ hipError_t launch_patch(
   if (local) {
     order = cb.cursor;
     hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, int(keys), cb.hist,
-                       cb.offsets, cb.cursor);
+                       cb.offsets, cb.cursor, ps);
     e = hipGetLastError();
   } else {
     size_t bytes = cb.scan_temp_bytes;
     e = hipcub::DeviceScan::ExclusiveSum(cb.scan_temp, bytes, cb.hist, cb.offsets, int(keys + 1),
                                          s);
+    if (ps.slots && e == hipSuccess) {
+      hipLaunchKernelGGL(k_zero, dim3(1), dim3(block), 0, s, ps.ctl(), size_t(2));
+      order = cb.cursor;
+      hipLaunchKernelGGL(k_patch_split, dim3(blocks_for(keys)), dim3(block), 0, s, keys,
+                         cb.offsets, cb.cursor, ps);
+      e = hipGetLastError();
+    }
   }
   if (e != hipSuccess) return e;
   switch (npol) {
