@@ -3140,11 +3140,11 @@ void k_patch(
 // tile into the grid, of which it is the only writer.  A thread prepares a
 // record in registers, and its wave adds its threads' records one after the
 // other, a tap per lane in blocks of 8 x 8, the taps of direct_loads records
-// loaded together.  Bound by latencies: the launch, two reads of the records and
-// 0.045 us per record of the densest tile.  Supports of 7 on 512^2, uniform, back
-// to back, FP64 (FP32) grids: 200 records 25.6 (21.1) -> 9.9 us, 2000 32.3 (27.7)
-// -> 14.7; a register patch per wave in place of LDS sums took 0.33 us per record
-// of the densest tile.
+// loaded together; where it has many, a record per lane.  Bound by latencies: the
+// launch, two reads of the records and what the densest tile takes.  Supports of 7
+// on 512^2, uniform, back to back: 200 records 25.6 -> 9.9 us, 2000 32.3 -> 14.7; a
+// register patch per wave in place of LDS sums took 0.33 us per record of the densest
+// tile.
 
 struct DirectArgs {
   const GroupInfo* groups;
@@ -3157,6 +3157,14 @@ struct DirectArgs {
 };
 constexpr int direct_block = 512;
 constexpr int direct_loads = 4;
+// A wave's lanes take a record each, tap by tap, where the supports have at most so
+// many taps for each of its records (the time goes with the taps then, not with
+// the records).  2000 records, sigma 2 pixels: supports 3 76 -> 37 us, 7 107 -> 80, 9
+// 375 -> 103, 25 880 -> 450; 1500 on 128^2, supports 25 242 -> 107.  Limits of 1.5 and
+// 20: 500 records of supports 25 there 122 us, 117 so.
+constexpr float direct_lane_plain = 2.0f, direct_lane = 40.0f;
+constexpr int direct_lane_min = 5;
+constexpr int direct_lane_loads = 8;  // 4: 118 us for the 1500
 constexpr unsigned direct_records = 2048;
 constexpr int direct_row = tile + 8;  // LDS row: four rows of a block on banks of their own
 constexpr int direct_plane = tile * direct_row;
@@ -3229,6 +3237,75 @@ __global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4)
     const bool plain = int(e.sxy & 0xffffu) <= 8 && int(e.sxy >> 16) <= 8
       && !(e.fl & flag_gradient);
     const unsigned long long plain_m = __ballot(plain);
+    // many records in the wave: each lane its own, tap by tap
+    const float most = float(mine) * (plain_m == ~0ull ? direct_lane_plain : direct_lane);
+    if (__builtin_expect(mine >= direct_lane_min, 0)
+        && !__any(float(int(e.sxy & 0xffffu) * int(e.sxy >> 16)) > most)) {
+      if (!e.sxy) continue;
+      const int sx = int(e.sxy & 0xffffu), sy = int(e.sxy >> 16);
+      const bool pos_w = e.fl & flag_pos_w, grad = e.fl & flag_gradient;
+      const float imf = pos_w ? -1.0f : 1.0f;
+      double gxr = 0.0, gyr = 0.0;
+      if (grad) {
+        gxr = recs[i].grad[0];
+        gyr = recs[i].grad[1];
+      }
+      const double phi0x = -gxr * ((sx / 2) * geo.os - (int((e.fl >> 8) & 255u) - geo.F));
+      const double phi0y = -gyr * ((sy / 2) * geo.os - (int((e.fl >> 16) & 255u) - geo.F));
+      const double dphix = gxr * geo.os, dphiy = gyr * geo.os;
+      // the support's part in the tile
+      const int bx0 = max(x0 - e.gx, 0), bx1 = min(sx, x0 + tile - e.gx);
+      const int by0 = max(y0 - e.gy, 0), by1 = min(sy, y0 + tile - e.gy);
+      const int nt = (bx1 - bx0) * (by1 - by0);
+      for (int gp = 0; gp < geo.nr; ++gp) {
+        const int el = pos_w ? mu.M[gp][0] : mu.Mc[gp][0];
+        if (el < 0 || unsigned(el) >= e.nm) continue;
+        const float2* cf = taps + e.base + unsigned(el) * unsigned(sx * sy);
+        double* dst = sums + gp * 2 * direct_plane;
+        auto add_at = [&](int X, int Y, float2 cc) {
+          const float2 pr = cmul(cc, e.g[0]);
+          double* at = dst + (e.gy + Y - y0) * direct_row + e.gx + X - x0;
+          __hip_atomic_fetch_add(at, double(pr.x), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add(at + direct_plane, double(pr.y), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        if (grad) {  // apart: its registers would be the whole kernel's
+#pragma unroll 1
+          for (int Y = by0; Y < by1; ++Y)
+#pragma unroll 1
+            for (int X = bx0; X < bx1; ++X) {
+              float2 cc = cf[Y * sx + X];
+              cc.y *= imf;
+              add_at(X, Y, cmul(cc, narrow(cphase_taylor((phi0x + X * dphix)
+                                                         + (phi0y + Y * dphiy)))));
+            }
+          continue;
+        }
+        int X = bx0, Y = by0;
+        for (int t0 = 0; t0 < nt; t0 += direct_lane_loads) {
+          float2 c[direct_lane_loads];
+          int Xk[direct_lane_loads], Yk[direct_lane_loads];
+#pragma unroll
+          for (int k = 0; k < direct_lane_loads; ++k) {
+            Xk[k] = X;
+            Yk[k] = Y;
+            c[k] = t0 + k < nt ? cf[Y * sx + X] : make_float2(0.0f, 0.0f);
+            if (++X == bx1) {
+              X = bx0;
+              ++Y;
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < direct_lane_loads; ++k) {
+            if (t0 + k >= nt) continue;
+            c[k].y *= imf;
+            add_at(Xk[k], Yk[k], c[k]);
+          }
+        }
+      }
+      continue;
+    }
     auto of = [&](int v, int j) { return __builtin_amdgcn_readlane(v, j); };
     // the tap (X, Y) of record j: its value (in: there is one in the tile)
     auto load = [&](int j, int gp, int X, int Y, bool& in, int& px) {
