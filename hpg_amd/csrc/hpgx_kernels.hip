@@ -2423,6 +2423,186 @@ __device__ __forceinline__ bool patch_record(
   return true;
 }
 
+// For tiles of at most patch_scan_keys: the exclusive scan of their counts, and
+// their order by falling count class, so that the tiles of a dense uv core
+// start first: in grid order they came in the middle, and the chip waited for
+// them (200,000 records, supports 9-25: 1172 -> 1071 us, two polarizations,
+// 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
+// in place of hipCUB's scan (10 us).  order null: the scan alone.
+//
+// A list of two chunks or more is split: one workgroup for each chunk of it, in
+// slots next to each other (the last of a tile's to end adds up their sums in the
+// slots' order), or a dense uv core would be one workgroup's serial chain.  The
+// chunk is the least, from patch_chunk_min on, that leaves the launch enough slots:
+// a list of two chunks or more has 1.5 slots a chunk of its entries at most.
+// Two polarizations, FP64: 100,000 records of supports 5 within a few pixels 28.5 ->
+// 0.41 ms (1.8 by haloed LDS tiles), 200,000 on 128^2, supports 3, 2.38 -> 0.21
+// (0.37), 10,000 on 256^2 104 -> 91 us (75); least chunks of 16 and 64 are 5 and 4%
+// slower there.  With a fence of the device's scope instead of stores past the L2s
+// 116 us: it writes a whole L2 back for every chunk.
+constexpr unsigned patch_chunk_min = 32;
+constexpr unsigned patch_none = ~0u;  // in the tiles' order: a split one
+constexpr int patch_values = 8 * patch_block;
+// device scope: past the XCDs' own L2s
+__device__ __forceinline__ void patch_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double patch_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+struct PatchSplit {
+  unsigned slots;  // of the launch; 0: no list is split
+  char* base;
+  // slots taken, chunk
+  __host__ __device__ unsigned* ctl() const { return reinterpret_cast<unsigned*>(base); }
+  // a slot's patch_values sums
+  __device__ double* sums(unsigned slot) const {
+    return reinterpret_cast<double*>(base + 256) + size_t(slot) * patch_values;
+  }
+  // (tile, chunk's number) of every slot
+  __device__ uint2* items() const { return reinterpret_cast<uint2*>(sums(slots)); }
+  // of a tile's first slot, for each of two k_patch launches
+  __device__ unsigned* tickets() const { return reinterpret_cast<unsigned*>(items() + slots); }
+};
+__device__ __forceinline__ unsigned patch_chunk(unsigned total, unsigned slots) {
+  return max(patch_chunk_min, unsigned(1.5 * double(total) / double(slots)) + 1u);
+}
+// the slots of a tile whose list has cnt entries, taken from *taken
+__device__ __forceinline__ void patch_take(
+  const PatchSplit& ps, unsigned chunk, unsigned key, unsigned cnt, unsigned* taken, int scope) {
+  const unsigned m = (cnt + chunk - 1u) / chunk;
+  const unsigned at = scope == __HIP_MEMORY_SCOPE_WORKGROUP
+    ? __hip_atomic_fetch_add(taken, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+    : atomicAdd(taken, m);
+  ps.tickets()[at] = ps.tickets()[ps.slots + at] = 0u;
+  for (unsigned i = 0; i < m; ++i) ps.items()[at + i] = make_uint2(key, i);
+}
+// the same for more tiles than k_patch_scan takes, and their order, as they come
+__global__ __launch_bounds__(block) void k_patch_split(
+  size_t keys, const unsigned* __restrict__ offsets, unsigned* __restrict__ order,
+  PatchSplit ps) {
+  const size_t k = blockIdx.x * (size_t)block + threadIdx.x;
+  if (k >= keys) return;
+  const unsigned chunk = patch_chunk(offsets[keys], ps.slots);
+  if (k == 0) ps.ctl()[1] = chunk;
+  const unsigned cnt = offsets[k + 1] - offsets[k];
+  const bool split = cnt >= 2u * chunk;
+  order[k] = split ? patch_none : unsigned(k);
+  if (split)
+    patch_take(ps, chunk, unsigned(k), cnt, ps.ctl(), __HIP_MEMORY_SCOPE_AGENT);
+}
+
+constexpr int patch_scan_threads = 1024;
+constexpr int patch_scan_keys = patch_local_keys;
+constexpr int patch_classes = 6;
+constexpr unsigned patch_split_bit = 8u;
+// a: the counts in LDS, keys + 1 values, afterwards the offsets
+__device__ __forceinline__ void patch_scan(
+  int keys, unsigned* a, unsigned* __restrict__ offsets, unsigned* __restrict__ order,
+  const PatchSplit& ps) {
+  __shared__ unsigned part[patch_scan_threads / wave + 1];
+  __shared__ unsigned cls[patch_classes];
+  __shared__ unsigned taken;
+  if (threadIdx.x == 0) taken = 0u;
+  if (threadIdx.x < patch_classes) cls[threadIdx.x] = 0u;
+  __syncthreads();
+  const unsigned total = block_exclusive_scan(a, keys, part);
+  if (threadIdx.x == 0) a[keys] = total;
+  __syncthreads();
+  if (!order) {
+    for (int k = threadIdx.x; k <= keys; k += patch_scan_threads) offsets[k] = a[k];
+    return;
+  }
+  const int lane = threadIdx.x % wave;
+  const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
+  const unsigned chunk = ps.slots ? patch_chunk(total, ps.slots) : 0x7fffffffu;
+  // class 0: over four times the mean, ..., the last: empty; with patch_split_bit
+  // that of a split list
+  auto class_of = [&](int k) {
+    const unsigned cnt = a[k + 1] - a[k];
+    const unsigned long long c = (unsigned long long)cnt * unsigned(keys);
+    const unsigned q = c > 4ull * total ? 0 : c > 2ull * total ? 1 : c > total ? 2
+      : 4ull * c > total ? 3 : c ? 4 : 5;
+    return q | (cnt >= 2u * chunk ? patch_split_bit : 0u);
+  };
+  static_assert(patch_scan_keys <= 16 * patch_scan_threads, "four bits a round in classes");
+  unsigned long long classes = 0;  // of this thread's tiles, from the first pass
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int r = 0; r < rounds; ++r) {
+      const int k = r * patch_scan_threads + int(threadIdx.x);
+      unsigned q = ~0u;
+      if (k < keys) {
+        if (pass == 0) {
+          q = class_of(k);
+          classes |= (unsigned long long)q << (4 * r);
+          offsets[k] = a[k];
+        } else {
+          q = unsigned(classes >> (4 * r)) & 15u;
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < patch_classes; ++c) {
+        const bool mine = (q & ~patch_split_bit) == unsigned(c);
+        const unsigned long long m = __ballot(mine);
+        if (!m) continue;
+        const int lead = __builtin_ctzll(m);
+        unsigned at = 0;
+        if (lane == lead)
+          at = __hip_atomic_fetch_add(cls + c, unsigned(__builtin_popcountll(m)),
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        at = unsigned(__builtin_amdgcn_readlane(int(at), lead));
+        if (pass == 1 && mine) {
+          const bool split = q & patch_split_bit;
+          order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] =
+            split ? patch_none : unsigned(k);
+          if (split)
+            patch_take(ps, chunk, unsigned(k), a[k + 1] - a[k], &taken,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      }
+    }
+    __syncthreads();
+    if (pass == 0 && threadIdx.x == 0) {
+      unsigned run = 0;
+      for (int c = 0; c < patch_classes; ++c) {
+        const unsigned t = cls[c];
+        cls[c] = run;
+        run += t;
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    offsets[keys] = total;
+    if (ps.slots) {
+      ps.ctl()[0] = taken;
+      ps.ctl()[1] = chunk;
+    }
+  }
+}
+__global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
+  int keys, const unsigned* __restrict__ hist, unsigned* __restrict__ offsets,
+  unsigned* __restrict__ order, PatchSplit ps) {
+  __shared__ unsigned a[patch_scan_keys + 1];
+  for (int k = threadIdx.x; k < keys; k += patch_scan_threads) a[k] = hist[k];
+  patch_scan(keys, a, offsets, order, ps);
+}
+
+// f(tile) for the tiles that a prepared record touches
+template <int N, typename F>
+__device__ __forceinline__ void patch_tiles(
+  const PatchRec<N>& e, int pty, int ptx, int tw, int th, F f) {
+  const unsigned sxy = e.sxy;
+  if (!sxy) return;
+  const int gx = e.gx, gy = e.gy;
+  const unsigned bhi = unsigned(e.base >> 32);
+  const int tx0 = gx / tw, tx1 = (gx + patch_sx(sxy, bhi) - 1) / tw;
+  const int ty0 = gy / th, ty1 = (gy + patch_sy(sxy, bhi) - 1) / th;
+  const int cube = int(e.cube) * pty;
+  for (int ty = ty0; ty <= ty1; ++ty)
+    for (int tx = tx0; tx <= tx1; ++tx) f((cube + ty) * ptx + tx);
+}
+
 // Weights: each wave sums its records' weights per (grid cube, row), and
 // for grids of at most count_planes_lds planes adds the sums into the
 // workgroup's LDS, which adds into the grid weights once at its end (the
@@ -2433,19 +2613,24 @@ __device__ __forceinline__ bool patch_record(
 // keeps each tile's place for it in its row of `table`, so that k_patch_list
 // places the entries without global atomics (10 G/s over the chip: they were
 // all of the two kernels' time: 284 + 265 us for 300,000 records of supports 9-33
-// on 4096 tiles, now 48 + 19).
+// on 4096 tiles, now 48 + 19).  A single workgroup (patch_batch) does the scan and
+// the lists too (offsets not null), three launches fewer: 300 records of two
+// polarizations 70 -> 64 us with the call's end waited for.
 template <int N, bool LOCAL>
-__global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_prep(
+__global__ __launch_bounds__(LOCAL ? patch_local_threads : block)
+__attribute__((amdgpu_waves_per_eu(4))) void k_patch_prep(
   const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int gvis_ready, int adjoint,
   const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
   int ptx, int pty, int tw, int th, PatchRec<N>* __restrict__ out,
   unsigned* __restrict__ hist, double* __restrict__ weights,
-  unsigned long long* __restrict__ invalid, unsigned batch, unsigned* __restrict__ table) {
+  unsigned long long* __restrict__ invalid, unsigned batch, unsigned* __restrict__ table,
+  unsigned* __restrict__ offsets, unsigned* __restrict__ order, unsigned* __restrict__ list,
+  PatchSplit ps) {
 
   __shared__ double wblk[count_planes_lds];
-  __shared__ unsigned cnt[LOCAL ? patch_local_keys : 1];
+  __shared__ unsigned cnt[LOCAL ? patch_local_keys + 1 : 1];
   const int keys = ptx * pty * geo.nc;
   if constexpr (LOCAL)
     for (int k = threadIdx.x; k < keys; k += blockDim.x) cnt[k] = 0u;
@@ -2525,6 +2710,16 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_p
     for (int k = threadIdx.x; k < nplanes; k += blockDim.x)
       if (wblk[k] != 0.0) atomicAdd(weights + k, wblk[k]);
   if constexpr (LOCAL) {
+    if (offsets) {
+      patch_scan(keys, cnt, offsets, order, ps);
+      for (size_t i = threadIdx.x; i < n; i += blockDim.x)  // its own records
+        patch_tiles(out[i], pty, ptx, tw, th, [&](int key) {
+          const unsigned at = __hip_atomic_fetch_add(cnt + key, 1u, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+          list[at] = unsigned(i);
+        });
+      return;
+    }
     unsigned* row = table + size_t(blockIdx.x) * keys;
     for (int k = threadIdx.x; k < keys; k += blockDim.x)
       row[k] = cnt[k] ? atomicAdd(hist + k, cnt[k]) : 0u;
@@ -2548,168 +2743,15 @@ __global__ __launch_bounds__(LOCAL ? patch_local_threads : block) void k_patch_l
   }
   const size_t last = min(n, first + (LOCAL ? size_t(batch) : size_t(blockDim.x)));
   for (size_t i = first + threadIdx.x; i < last; i += blockDim.x) {
-    const unsigned sxy = prs[i].sxy;
-    if (!sxy) continue;
-    const int gx = prs[i].gx, gy = prs[i].gy;
-    const unsigned gcube = prs[i].cube;
-    const unsigned bhi = unsigned(prs[i].base >> 32);
-    const int tx0 = gx / tw, tx1 = (gx + patch_sx(sxy, bhi) - 1) / tw;
-    const int ty0 = gy / th, ty1 = (gy + patch_sy(sxy, bhi) - 1) / th;
-    for (int ty = ty0; ty <= ty1; ++ty)
-      for (int tx = tx0; tx <= tx1; ++tx) {
-        const size_t key = (size_t(gcube) * pty + ty) * ptx + tx;
-        unsigned pos;
-        if constexpr (LOCAL)
-          pos = __hip_atomic_fetch_add(at + key, 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-        else
-          pos = offsets[key] + atomicSub(hist + key, 1u) - 1u;
-        list[pos] = unsigned(i);
-      }
-  }
-}
-
-// For tiles of at most patch_scan_keys: the exclusive scan of their counts, and
-// their order by falling count class, so that the tiles of a dense uv core
-// start first: in grid order they came in the middle, and the chip waited for
-// them (200,000 records, supports 9-25: 1172 -> 1071 us, two polarizations,
-// 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
-// in place of hipCUB's scan (10 us).  order null: the scan alone.
-//
-// A list of two chunks or more is split: one workgroup for each chunk of it, in
-// slots next to each other (the last of a tile's to end adds up their sums in the
-// slots' order), or a dense uv core would be one workgroup's serial chain.  The
-// chunk is the least, from patch_chunk_min on, that leaves the launch enough slots:
-// a list of two chunks or more has 1.5 slots a chunk of its entries at most.
-// Two polarizations, FP64: 100,000 records of supports 5 within a few pixels 28.5 ->
-// 0.41 ms (1.8 by haloed LDS tiles), 200,000 on 128^2, supports 3, 2.38 -> 0.21
-// (0.37), 10,000 on 256^2 104 -> 91 us (75); least chunks of 16 and 64 are 5 and 4%
-// slower there.  With a fence of the device's scope instead of stores past the L2s
-// 116 us: it writes a whole L2 back for every chunk.
-constexpr unsigned patch_chunk_min = 32;
-constexpr unsigned patch_none = ~0u;  // in the tiles' order: a split one
-constexpr int patch_values = 8 * patch_block;
-// device scope: past the XCDs' own L2s
-__device__ __forceinline__ void patch_store(double* p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double patch_load(const double* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-struct PatchSplit {
-  unsigned slots;  // of the launch; 0: no list is split
-  char* base;
-  // slots taken, chunk
-  __host__ __device__ unsigned* ctl() const { return reinterpret_cast<unsigned*>(base); }
-  // a slot's patch_values sums
-  __device__ double* sums(unsigned slot) const {
-    return reinterpret_cast<double*>(base + 256) + size_t(slot) * patch_values;
-  }
-  // (tile, chunk's number) of every slot
-  __device__ uint2* items() const { return reinterpret_cast<uint2*>(sums(slots)); }
-  // of a tile's first slot, for each of two k_patch launches
-  __device__ unsigned* tickets() const { return reinterpret_cast<unsigned*>(items() + slots); }
-};
-__device__ __forceinline__ unsigned patch_chunk(unsigned total, unsigned slots) {
-  return max(patch_chunk_min, unsigned(1.5 * double(total) / double(slots)) + 1u);
-}
-// the slots of a tile whose list has cnt entries, taken from *taken
-__device__ __forceinline__ void patch_take(
-  const PatchSplit& ps, unsigned chunk, unsigned key, unsigned cnt, unsigned* taken, int scope) {
-  const unsigned m = (cnt + chunk - 1u) / chunk;
-  const unsigned at = scope == __HIP_MEMORY_SCOPE_WORKGROUP
-    ? __hip_atomic_fetch_add(taken, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-    : atomicAdd(taken, m);
-  ps.tickets()[at] = ps.tickets()[ps.slots + at] = 0u;
-  for (unsigned i = 0; i < m; ++i) ps.items()[at + i] = make_uint2(key, i);
-}
-// the same for more tiles than k_patch_scan takes, and their order, as they come
-__global__ __launch_bounds__(block) void k_patch_split(
-  size_t keys, const unsigned* __restrict__ offsets, unsigned* __restrict__ order,
-  PatchSplit ps) {
-  const size_t k = blockIdx.x * (size_t)block + threadIdx.x;
-  if (k >= keys) return;
-  const unsigned chunk = patch_chunk(offsets[keys], ps.slots);
-  if (k == 0) ps.ctl()[1] = chunk;
-  const unsigned cnt = offsets[k + 1] - offsets[k];
-  const bool split = cnt >= 2u * chunk;
-  order[k] = split ? patch_none : unsigned(k);
-  if (split)
-    patch_take(ps, chunk, unsigned(k), cnt, ps.ctl(), __HIP_MEMORY_SCOPE_AGENT);
-}
-
-constexpr int patch_scan_threads = 1024;
-constexpr int patch_scan_keys = patch_local_keys;
-constexpr int patch_classes = 6;
-__global__ __launch_bounds__(patch_scan_threads) void k_patch_scan(
-  int keys, const unsigned* __restrict__ hist, unsigned* __restrict__ offsets,
-  unsigned* __restrict__ order, PatchSplit ps) {
-  __shared__ unsigned a[patch_scan_keys + 1];
-  __shared__ unsigned part[patch_scan_threads / wave + 1];
-  __shared__ unsigned cls[patch_classes];
-  __shared__ unsigned taken;
-  if (threadIdx.x == 0) taken = 0u;
-  for (int k = threadIdx.x; k < keys; k += patch_scan_threads) a[k] = hist[k];
-  if (threadIdx.x < patch_classes) cls[threadIdx.x] = 0u;
-  __syncthreads();
-  const unsigned total = block_exclusive_scan(a, keys, part);
-  if (threadIdx.x == 0) a[keys] = total;
-  __syncthreads();
-  if (!order) {
-    for (int k = threadIdx.x; k <= keys; k += patch_scan_threads) offsets[k] = a[k];
-    return;
-  }
-  const int lane = threadIdx.x % wave;
-  const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
-  const unsigned chunk = ps.slots ? patch_chunk(total, ps.slots) : 0x7fffffffu;
-  // class 0: over four times the mean, ..., the last: empty
-  auto class_of = [&](int k) {
-    const unsigned long long c = (unsigned long long)(a[k + 1] - a[k]) * unsigned(keys);
-    return c > 4ull * total ? 0 : c > 2ull * total ? 1 : c > total ? 2 : 4ull * c > total ? 3
-      : c ? 4 : 5;
-  };
-  for (int pass = 0; pass < 2; ++pass) {
-    for (int r = 0; r < rounds; ++r) {
-      const int k = r * patch_scan_threads + int(threadIdx.x);
-      const int q = k < keys ? class_of(k) : -1;
-      if (pass == 0 && k < keys) offsets[k] = a[k];
-#pragma unroll
-      for (int c = 0; c < patch_classes; ++c) {
-        const unsigned long long m = __ballot(q == c);
-        if (!m) continue;
-        const int lead = __builtin_ctzll(m);
-        unsigned at = 0;
-        if (lane == lead)
-          at = __hip_atomic_fetch_add(cls + c, unsigned(__builtin_popcountll(m)),
-                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        at = unsigned(__builtin_amdgcn_readlane(int(at), lead));
-        if (pass == 1 && q == c) {
-          const unsigned cnt = a[k + 1] - a[k];
-          const bool split = cnt >= 2u * chunk;
-          order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] =
-            split ? patch_none : unsigned(k);
-          if (split)
-            patch_take(ps, chunk, unsigned(k), cnt, &taken, __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-      }
-    }
-    __syncthreads();
-    if (pass == 0 && threadIdx.x == 0) {
-      unsigned run = 0;
-      for (int c = 0; c < patch_classes; ++c) {
-        const unsigned t = cls[c];
-        cls[c] = run;
-        run += t;
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    offsets[keys] = total;
-    if (ps.slots) {
-      ps.ctl()[0] = taken;
-      ps.ctl()[1] = chunk;
-    }
+    patch_tiles(prs[i], pty, ptx, tw, th, [&](int key) {
+      unsigned pos;
+      if constexpr (LOCAL)
+        pos = __hip_atomic_fetch_add(at + key, 1u, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+      else
+        pos = offsets[key] + atomicSub(hist + key, 1u) - 1u;
+      list[pos] = unsigned(i);
+    });
   }
 }
 
@@ -4292,8 +4334,17 @@ hipError_t launch_count(
 
 size_t entry_bytes(int npol) { return sizeof(EntryHead) + sizeof(float2) * size_t(npol); }
 
+// records of a workgroup that counts in LDS: all of a small batch (which one
+// workgroup then prepares whole), 1024 (a record a thread) where 2048 would leave
+// most of the chip idle (10,000 records, two polarizations, 256^2: 90 -> 84 us), then
+// 2048, or more so that there are at most 512 workgroups
 size_t patch_batch(size_t n) {
+  if (n > 2048 && n <= 16384) return 1024;
   return std::max<size_t>(2048, ((n + 511) / 512 + 1023) / 1024 * 1024);
+}
+// workgroups of up to n records a call at most
+size_t patch_batches(size_t n) {
+  return std::min<size_t>(std::max<size_t>((n + 2047) / 2048, 16), 512);
 }
 
 // Bins: at most half of the items that one workgroup counts (its global
@@ -4313,7 +4364,7 @@ SortKeys sort_plan(unsigned long long keys, size_t batch) {
 }
 
 size_t sort_bins_entries(size_t n) {
-  return (2 + std::min<size_t>((n + 2047) / 2048, 512)) * (patch_local_keys + 1);
+  return (2 + patch_batches(n)) * (patch_local_keys + 1);
 }
 
 // the bins' offsets and the pairs of n keys, from the counts in cb.sort_bins
@@ -4538,11 +4589,9 @@ int patch_tiles_y(const Geometry& geo) {
 size_t patch_keys(const Geometry& geo) {
   return size_t(patch_tiles_x(geo)) * patch_tiles_y(geo) * geo.nc;
 }
-// records of a workgroup that counts in LDS: 2048, or more so that there are
-// at most 512 rows of places
 size_t patch_table_entries(const Geometry& geo, size_t n) {
   const size_t keys = patch_keys(geo);
-  return keys <= size_t(patch_local_keys) ? std::min<size_t>((n + 2047) / 2048, 512) * keys : 0;
+  return keys <= size_t(patch_local_keys) ? patch_batches(n) * keys : 0;
 }
 // slots for the split lists of so many entries in all, and their memory
 size_t patch_split_slots(size_t entries) {
@@ -4597,8 +4646,6 @@ hipError_t launch_patch(
   const int ptx = patch_tiles_x(geo), pty = patch_tiles_y(geo);
   const size_t keys = patch_keys(geo);
   const int kind = patch_kind(npol, geo, cf, mu);
-  // a kernel, not a memset: a captured graph may replay it
-  hipLaunchKernelGGL(k_zero, dim3(blocks_for(keys + 1)), dim3(block), 0, s, cb.hist, keys + 1);
   const bool local = keys <= size_t(patch_local_keys);
   PatchSplit ps{};
   ps.slots = unsigned(std::min(
@@ -4608,6 +4655,10 @@ hipError_t launch_patch(
   const size_t batch = patch_batch(n);
   const unsigned nb = local ? unsigned((n + batch - 1) / batch) : 0u;
   if (local && nb * keys > cb.patch_table_capacity) return hipErrorInvalidValue;
+  const bool one = local && nb == 1;  // one workgroup prepares, scans and lists
+  // a kernel, not a memset: a captured graph may replay it
+  if (!one)
+    hipLaunchKernelGGL(k_zero, dim3(blocks_for(keys + 1)), dim3(block), 0, s, cb.hist, keys + 1);
 #define HPGX_PREP(NP)                                                          \
   hipLaunchKernelGGL(                                                          \
     local ? (k_patch_prep<NP, true>) : (k_patch_prep<NP, false>),              \
@@ -4616,7 +4667,8 @@ hipError_t launch_patch(
     static_cast<const VisRec<NP>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,    \
     int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint), cb.gvis, residuals, \
     ptx, pty, patch_tile_x(P), patch_tile_y(P), static_cast<PatchRec<NP>*>(cb.patch_recs), \
-    cb.hist, weights, cb.invalid_count, unsigned(batch), cb.patch_table)
+    cb.hist, weights, cb.invalid_count, unsigned(batch), cb.patch_table,       \
+    one ? cb.offsets : nullptr, cb.cursor, cb.patch_list, ps)
 #define HPGX_LIST(NP)                                                          \
   hipLaunchKernelGGL(                                                          \
     local ? (k_patch_list<NP, true>) : (k_patch_list<NP, false>),              \
@@ -4649,7 +4701,9 @@ hipError_t launch_patch(
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const unsigned* order = nullptr;
-  if (local) {
+  if (one) {
+    order = cb.cursor;
+  } else if (local) {
     order = cb.cursor;
     hipLaunchKernelGGL(k_patch_scan, dim3(1), dim3(patch_scan_threads), 0, s, int(keys), cb.hist,
                        cb.offsets, cb.cursor, ps);
@@ -4667,11 +4721,13 @@ hipError_t launch_patch(
     }
   }
   if (e != hipSuccess) return e;
-  switch (npol) {
-  case 1: HPGX_LIST(1); break;
-  case 2: HPGX_LIST(2); break;
-  case 3: HPGX_LIST(3); break;
-  default: HPGX_LIST(4); break;
+  if (!one) {
+    switch (npol) {
+    case 1: HPGX_LIST(1); break;
+    case 2: HPGX_LIST(2); break;
+    case 3: HPGX_LIST(3); break;
+    default: HPGX_LIST(4); break;
+    }
   }
   // FP32 grids of supports below a tile round twice a pixel, as the haloed tiles
   // do: once with the sum of the tile's records, once with its neighbours'
