@@ -383,12 +383,8 @@ size_t patch_tiles(hpgx_state_t st) {
     int(st->gsize[2]), std::max(1, st->cf.max_sx), std::max(1, st->cf.max_sy));
 }
 
-size_t entries_per_record(hpgx_state_t st) {
-  const size_t planes = size_t(std::max(1u, st->gsize[2]));
-  if (use_halo(st) || use_halo_global(st)) return planes;
-  return planes
-    * hpgx::tiles_per_footprint(std::max(1, st->cf.max_sx), std::max(1, st->cf.max_sy));
-}
+// bin entries of a record: one in each plane of its grid cube
+size_t entries_per_record(hpgx_state_t st) { return std::max(1u, st->gsize[2]); }
 
 // device memory for bin entries (HPGX_ENTRY_BUDGET_MB; default 16 GiB,
 // under 6% of an MI355X's 288 GB: batches whose entries exceed it are
@@ -1016,28 +1012,7 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
                   + std::to_string(hpgx::bin_keys_limit())
                   + " (plane, 32x32 tile) keys are not supported (this grid has "
                   + std::to_string(st->nkeys) + ")");
-  const bool halo = use_halo(st);
-  const size_t epr = entries_per_record(st);
-  const size_t block_cap = hpgx::bin_block_records() * epr;
-  const size_t esize =
-    halo ? hpgx::halo_entry_bytes(int(st->npol)) : hpgx::entry_bytes(int(st->npol));
   auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t halo_bytes =
-    halo ? up(st->nkeys * hpgx::halo_pixels_per_key(halo_x(st), halo_y(st)) * sizeof(double2))
-    : 0;
-  const size_t set_bytes = halo ? up(st->nkeys * sizeof(unsigned)) : 0;
-  const size_t per_block =
-    (bin_keys(st) + 1) * sizeof(unsigned) + block_cap * esize + block_cap * sizeof(unsigned);
-  const size_t fixed = halo_bytes + set_bytes + 3 * 256;
-  const size_t fit = noalloc_scratch_bytes > fixed ? (noalloc_scratch_bytes - fixed) / per_block : 0;
-  const size_t bins_max = halo ? halo_bins_limit(st) : size_t(hpgx::tile_bins_limit());
-  const size_t needed = (n + hpgx::bin_block_records() - 1) / hpgx::bin_block_records();
-  const size_t blocks = std::min({needed, bins_max, fit});
-  if (blocks == 0)
-    return fail(st, HPGX_ERR_OTHER,
-                "hpgx_grid_visibilities_noalloc: one bin block of this grid and CF needs "
-                  + std::to_string(fixed + per_block) + " bytes of scratch; the fixed scratch holds "
-                  + std::to_string(noalloc_scratch_bytes));
   char* p = static_cast<char*>(base);
   c = CallBuffers{};
   // skipped records are counted in the state's own counter (read by
@@ -1081,6 +1056,23 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
     pass_blocks = 0;
     return HPGX_SUCCESS;
   }
+  // (!use_patch: haloed entries)
+  const size_t block_cap = hpgx::bin_block_records() * entries_per_record(st);
+  const size_t esize = hpgx::halo_entry_bytes(int(st->npol));
+  const size_t halo_values = st->nkeys * hpgx::halo_pixels_per_key(halo_x(st), halo_y(st));
+  const size_t halo_bytes = up(halo_values * sizeof(double2));
+  const size_t set_bytes = up(st->nkeys * sizeof(unsigned));
+  const size_t per_block =
+    (bin_keys(st) + 1) * sizeof(unsigned) + block_cap * esize + block_cap * sizeof(unsigned);
+  const size_t fixed = halo_bytes + set_bytes + 3 * 256;
+  const size_t fit = noalloc_scratch_bytes > fixed ? (noalloc_scratch_bytes - fixed) / per_block : 0;
+  const size_t needed = (n + hpgx::bin_block_records() - 1) / hpgx::bin_block_records();
+  const size_t blocks = std::min({needed, halo_bins_limit(st), fit});
+  if (blocks == 0)
+    return fail(st, HPGX_ERR_OTHER,
+                "hpgx_grid_visibilities_noalloc: one bin block of this grid and CF needs "
+                  + std::to_string(fixed + per_block) + " bytes of scratch; the fixed scratch holds "
+                  + std::to_string(noalloc_scratch_bytes));
   c.off_table = reinterpret_cast<unsigned*>(p);
   c.off_table_capacity = blocks * (bin_keys(st) + 1);
   p += up(c.off_table_capacity * sizeof(unsigned));
@@ -1089,14 +1081,12 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
   p += up(c.entries_capacity * esize);
   c.entry_vis = reinterpret_cast<unsigned*>(p);
   p += up(c.entries_capacity * sizeof(unsigned));
-  if (halo) {
-    c.halo = reinterpret_cast<double2*>(p);
-    c.halo_capacity = st->nkeys * hpgx::halo_pixels_per_key(halo_x(st), halo_y(st));
-    p += halo_bytes;
-    c.halo_set = reinterpret_cast<unsigned*>(p);
-    c.halo_set_capacity = st->nkeys;
-    p += set_bytes;
-  }
+  c.halo = reinterpret_cast<double2*>(p);
+  c.halo_capacity = halo_values;
+  p += halo_bytes;
+  c.halo_set = reinterpret_cast<unsigned*>(p);
+  c.halo_set_capacity = st->nkeys;
+  p += set_bytes;
   if (size_t(p - static_cast<char*>(base)) > noalloc_scratch_bytes)
     return fail(st, HPGX_ERR_OTHER, "hpgx_grid_visibilities_noalloc: scratch layout overflow");
   pass_blocks = blocks;

@@ -140,8 +140,6 @@ hipError_t launch_cf_wsum(
   hipStream_t s, const GroupInfo& gi, int nf, bool planar, const float2* taps,
   double2* wsum);
 
-size_t tiles_per_footprint(int max_sx, int max_sy);
-
 // exclusive scan of the global bin counts (hist -> offsets, cursor)
 hipError_t launch_scan(hipStream_t s, size_t nkeys, CallBuffers& cb);
 size_t scan_temp_bytes(size_t nkeys);
@@ -151,7 +149,6 @@ hipError_t launch_count(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool do_grid, CallBuffers& cb,
   double* weights);
-size_t entry_bytes(int npol);
 hipError_t launch_emit(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool gvis_ready, GvisSource src, const double2* residuals,

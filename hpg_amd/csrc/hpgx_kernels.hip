@@ -4295,12 +4295,6 @@ hipError_t launch_cf_wsum(
   });
 }
 
-size_t tiles_per_footprint(int max_sx, int max_sy) {
-  const size_t tx = size_t((max_sx - 1 + tile - 1) / tile + 1);
-  const size_t ty = size_t((max_sy - 1 + tile - 1) / tile + 1);
-  return tx * ty;
-}
-
 size_t scan_temp_bytes(size_t nkeys) {
   size_t bytes = 0;
   (void)hipcub::DeviceScan::ExclusiveSum(
@@ -4331,8 +4325,6 @@ hipError_t launch_count(
     int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count);
   return hipGetLastError();
 }
-
-size_t entry_bytes(int npol) { return sizeof(EntryHead) + sizeof(float2) * size_t(npol); }
 
 // records of a workgroup that counts in LDS: all of a small batch (which one
 // workgroup then prepares whole), 1024 (a record a thread) where 2048 would leave

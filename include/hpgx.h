@@ -211,9 +211,9 @@ HPGX_API int hpgx_grid_visibilities(
  * entries, offset table and halo values live in a fixed
  * HPGX_NOALLOC_SCRATCH_BYTES device array of the library, and a batch whose
  * bins exceed it is gridded in several passes.  Grids of more than 8192
- * (plane, 32x32 tile) keys, or a grid and CF for which one bin block of 4096
- * records does not fit the scratch, are rejected with HPGX_ERR_OTHER and a
- * message.  The records must be ready when the call is made and stay
+ * (plane, 32x32 tile) keys, or (one polarization, supports below a tile) a grid
+ * and CF whose halo values and one bin block of 4096 records do not fit the
+ * scratch, are rejected with HPGX_ERR_OTHER and a message.  The records must be ready when the call is made and stay
  * unchanged until the next hpgx_fence.  Every call on one GPU uses that GPU's
  * one scratch array: calls that may overlap in time on the same GPU (states
  * on different streams, or several host threads) race and must be ordered by

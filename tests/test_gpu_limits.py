@@ -259,3 +259,33 @@ def test_few_of_a_cf_s_elements(hpg, oracle_mod, case, radii, mode, gradient):
     gs.grid_visibilities(hpg.Device.Serial, rec2, True)
     o.grid_visibilities(_view(rec2, oracle_mod), True)
     assert np.abs(gs.grid_values() - o.grid_values()).max() <= bar * np.abs(o.grid_values()).max()
+
+
+def test_noalloc_register_patches(hpg):
+    """Without allocations, calls by register patches need neither halos nor
+    bins: they fit where the halo values alone (4096 keys of 1280 pixels, 84 MB)
+    would not.  1e-12: the same products in another order of FP64 sums."""
+    import ctypes
+    import torch
+    from hpg_amd import _lib, workloads
+    gsz, n = (1024, 1024, 4, 1), 700
+    cf = workloads.random_cf(4, [8], nmueller=4, seed=91)
+    rec = workloads.random_visibilities(n, 4, gsz, (1.0, 1.0), cf, seed=92, phase=True)
+    dev = torch.from_numpy(rec.view(np.uint8).copy()).cuda()
+    torch.cuda.synchronize()
+    states = []
+    for noalloc in (False, True):
+        gs = hpg.GridderState.create(hpg.Device.Hip, 0, n, cf, gsz, (1.0, 1.0), DIAG)
+        gs.set_convolution_function(hpg.Device.Serial, cf)
+        if noalloc:
+            rc = _lib.lib().hpgx_grid_visibilities_noalloc(
+                gs._h, ctypes.c_void_p(dev.data_ptr()), n, 4, 1)
+            assert rc == 0, _lib.error_message(gs._h)
+        else:
+            gs.grid_visibilities(hpg.Device.Serial, dev)
+        gs.fence()
+        states.append(gs)
+    exp = states[0].grid_values()
+    assert np.abs(exp).max() > 0
+    assert np.abs(states[1].grid_values() - exp).max() <= 1e-12 * np.abs(exp).max()
+    np.testing.assert_allclose(states[1].grid_weights(), states[0].grid_weights(), rtol=1e-12)
