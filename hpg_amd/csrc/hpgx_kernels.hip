@@ -3581,6 +3581,14 @@ __device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
 // records a wave takes (eight of one element a row, or of two polarizations,
 // measured slower: their registers cost a wave per SIMD)
 constexpr int degrid_recs = 4;
+// rounds of loads between sums put aside, where a row uses one element: its taps
+// then fill 16 to 64 lanes, whose sums of up to thousands of taps round more than
+// 64 lanes' with shorter ones.  Predictions of four rows' error against 64 bits and
+// the call: supports of 33 to 65, 50,000 records, 7.3e-16 in one chain of two
+// roundings a tap (1170 us), 4.5e-16 with one rounding for two taps, 3.4e-16 with
+// parts too (1190 us; 3.8e-16 by 64 lanes a row); 9 to 33, 1e6, 3.7e-16 (3070 us) and
+// 2.9e-16 (3062)
+constexpr unsigned degrid_part = 8;
 
 // One wave takes R records in a row of the order; those of one slice share
 // every CF value it loads (per tap of 4 x 4 elements a record reads 64 bytes
@@ -3614,6 +3622,7 @@ void k_degrid(
   constexpr int R = degrid_recs;
   constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
   constexpr int TPS = wave / P;                 // taps a step
+  __shared__ double part[KIND == patch_one ? R * L * 2 * block : 1];
 
   const int w = uniform(int(threadIdx.x) / wave);
   const int lane = threadIdx.x % wave;
@@ -3767,37 +3776,55 @@ void k_degrid(
           off += wrap;
         }
       }
+      // the steps' products added up, then to the sums: one rounding of a sum for
+      // U taps in place of two for each
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int k = 0; k < RR; ++k) {
 #pragma unroll
-        for (int k = 0; k < RR; ++k) {
-          const double mx = m[u][k].x;
-          const double my = __hiloint2double(
-            int(unsigned(__double2hiint(m[u][k].y)) ^ flip[k]), __double2loint(m[u][k].y));
+        for (int v = 0; v < L; ++v) {
+          if (KIND == patch_any && !use[v]) continue;
+          double tr = 0.0, ti = 0.0;
 #pragma unroll
-          for (int v = 0; v < L; ++v) {
-            if (KIND == patch_any && !use[v]) continue;
+          for (int u = 0; u < U; ++u) {
+            const double mx = m[u][k].x;
+            const double my = __hiloint2double(
+              int(unsigned(__double2hiint(m[u][k].y)) ^ flip[k]), __double2loint(m[u][k].y));
             const double cx = double(c[u][v].x), cy = double(c[u][v].y);
-            double& a = val[(k * L + v) * 2];
-            double& b = val[(k * L + v) * 2 + 1];
-            a = __builtin_fma(cx, mx, a);
-            a = __builtin_fma(-cy, my, a);
-            b = __builtin_fma(cx, my, b);
-            b = __builtin_fma(cy, mx, b);
+            tr = u ? __builtin_fma(cx, mx, tr) : cx * mx;
+            tr = __builtin_fma(-cy, my, tr);
+            ti = u ? __builtin_fma(cx, my, ti) : cx * my;
+            ti = __builtin_fma(cy, mx, ti);
           }
+          val[(k * L + v) * 2] += tr;
+          val[(k * L + v) * 2 + 1] += ti;
         }
       }
     };
     constexpr int U = GRAD || RR * (L + 1) > 12 ? 1 : 2;
     const unsigned full = ntap / TPS;
     unsigned s = 0;
+    bool kept = false;
 #pragma unroll 1
-    for (; s + U <= full; s += U) steps(std::integral_constant<int, U>{});
+    for (; s + U <= full; s += U) {
+      steps(std::integral_constant<int, U>{});
+      if (KIND == patch_one && (s / U) % degrid_part == degrid_part - 1) {
+#pragma unroll
+        for (int k = 0; k < RR * L * 2; ++k) {
+          double* p = part + k * block + threadIdx.x;
+          *p = kept ? *p + val[k] : val[k];
+          val[k] = 0.0;
+        }
+        kept = true;
+      }
+    }
     if constexpr (U > 1) {
 #pragma unroll 1
       for (; s < full; ++s) steps(std::integral_constant<int, 1>{});
     }
     if (full * TPS + unsigned(q) < ntap) steps(std::integral_constant<int, 1>{});
+    if (kept)
+#pragma unroll
+      for (int k = 0; k < RR * L * 2; ++k) val[k] += part[k * block + threadIdx.x];
     // the other sign's imaginary parts, then the sums over the taps (and,
     // but for patch_one, the rows)
 #pragma unroll
