@@ -462,7 +462,7 @@ int ensure_call_buffers(hpgx_state_t st) {
     const size_t epr = entries_per_record(st);
     // (register patches: the bins of the binned degridder only)
     const bool halo = use_patch(st) ? use_degrid_binned(st) : use_halo(st) || use_halo_global(st);
-    const size_t per_entry = hpgx::halo_entry_bytes(int(st->npol)) + sizeof(unsigned);
+    const size_t per_entry = hpgx::halo_entry_bytes() + sizeof(unsigned);
     // entries per pass: at least one record's, and below 2^32 (bin counts,
     // offsets and entry indexes are 32-bit)
     const size_t budget = std::min<size_t>(std::max(entry_budget_bytes() / per_entry, epr),
@@ -504,7 +504,7 @@ int ensure_call_buffers(hpgx_state_t st) {
       dev_free(cb.tally_entries);
       dev_free(cb.tally_keys);
       cb.tally_capacity = 0;
-      HPGX_HIP(st, dev_alloc(cb.tally_entries, need * hpgx::halo_entry_bytes(int(st->npol))));
+      HPGX_HIP(st, dev_alloc(cb.tally_entries, need * hpgx::halo_entry_bytes()));
       HPGX_HIP(st, dev_alloc(cb.tally_keys, need * 3 * sizeof(unsigned)));
       cb.tally_capacity = need;
     }
@@ -529,7 +529,7 @@ int ensure_call_buffers(hpgx_state_t st) {
       dev_free(cb.stream_entries);
       dev_free(cb.entry_vis);
       cb.entries_capacity = 0;
-      HPGX_HIP(st, dev_alloc(cb.stream_entries, need * hpgx::halo_entry_bytes(int(st->npol))));
+      HPGX_HIP(st, dev_alloc(cb.stream_entries, need * hpgx::halo_entry_bytes()));
       HPGX_HIP(st, dev_alloc(cb.entry_vis, need * sizeof(unsigned)));
       cb.entries_capacity = need;
     }
@@ -902,7 +902,7 @@ int run_grid_with(hpgx_state_t st, CallBuffers& cb, size_t pass_blocks, size_t n
     c.vis = rec_base;
     HPGX_HIP(st, hpgx::launch_direct(
                    st->stream, np, n, geo, st->cf, st->mu, update_weights, gvis_ready, src,
-                   residuals, c, st->weights, mode, st->grid));
+                   residuals, c, st->weights, static_cast<double2*>(st->grid)));
     return HPGX_SUCCESS;
   }
   if (use_patch(st) || use_sparse_patch(st, cb, n)) {
@@ -1058,7 +1058,7 @@ int noalloc_plan(hpgx_state_t st, void* base, size_t n, CallBuffers& c, size_t& 
   }
   // (!use_patch: haloed entries)
   const size_t block_cap = hpgx::bin_block_records() * entries_per_record(st);
-  const size_t esize = hpgx::halo_entry_bytes(int(st->npol));
+  const size_t esize = hpgx::halo_entry_bytes();
   const size_t halo_values = st->nkeys * hpgx::halo_pixels_per_key(halo_x(st), halo_y(st));
   const size_t halo_bytes = up(halo_values * sizeof(double2));
   const size_t set_bytes = up(st->nkeys * sizeof(unsigned));

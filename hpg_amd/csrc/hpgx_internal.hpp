@@ -88,7 +88,7 @@ struct CallBuffers {
   size_t entries_capacity;  // entries of stream_entries
   void* scan_temp;
   size_t scan_temp_bytes;
-  void* stream_entries;  // compact binned entries (Entry<N>), sorted by key
+  void* stream_entries;  // compact binned entries (Entry4), sorted by key
   unsigned* entry_vis;   // record index of entries with a phase gradient
   unsigned* off_table;   // block-local bins: per bin block, nkeys + 1 offsets
   size_t off_table_capacity;
@@ -99,7 +99,7 @@ struct CallBuffers {
   unsigned long long* invalid_count;
   double2* degrid_acc;   // binned degridding: per record x polarization sums
   size_t degrid_acc_capacity;
-  void* tally_entries;   // launch_tally: entries in record order (Entry4<N>)
+  void* tally_entries;   // launch_tally: entries in record order (Entry4)
   void* tally_keys;      // and per slot its key and a (lower key bits, slot) pair
   size_t tally_capacity; // slots of both
   unsigned* sort_bins;   // launch_tally, launch_degrid: the sort's counts, offsets
@@ -153,16 +153,16 @@ hipError_t launch_emit(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool gvis_ready, GvisSource src, const double2* residuals,
   CallBuffers& cb);
-// global quadrant bins (one polarization, haloed entries): the entries in their
-// keys' order in cb.stream_entries, the keys' offsets in cb.offsets; n x nr slots
-// of cb.tally_entries / cb.tally_keys
 // the whole gridding pass of a few records in one launch, on no buffers of cb
 // but vis, gvis and invalid_count
 bool direct_ok(size_t n, const Geometry& geo);
 hipError_t launch_direct(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf, const Mueller& mu,
   bool update_weights, bool gvis_ready, GvisSource src, const double2* residuals,
-  const CallBuffers& cb, double* weights, int mode, void* grid);
+  const CallBuffers& cb, double* weights, double2* grid);
+// global quadrant bins (one polarization, haloed entries): the entries in their
+// keys' order in cb.stream_entries, the keys' offsets in cb.offsets; n x nr slots
+// of cb.tally_entries / cb.tally_keys
 hipError_t launch_tally(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf,
   const Mueller& mu, bool update_weights, bool gvis_ready, GvisSource src,
@@ -180,12 +180,12 @@ hipError_t launch_bin(
   bool degrid_pass = false, void* copy_records = nullptr,
   bool quad_keys = false);
 // haloed tiles (one entry per record and plane; supports below tile)
-size_t halo_entry_bytes(int npol);
+size_t halo_entry_bytes();
 size_t halo_pixels_per_key(int hx, int hy);
 int halo_tile_limit();
 size_t halo_lds_bytes(int hx, int hy, int nbins);
-// acc (FP32 grids): 0 FP64 tile sums, 1 FP32 two-sum via returning atomics,
-// 2 FP32 two-sum of (hi, lo) pairs under compare-and-swap
+// acc (FP32 grids): 0 FP64 tile sums, else FP32 two-sum of (hi, lo) pairs under
+// compare-and-swap
 hipError_t launch_tile_halo(
   hipStream_t s, int npol, int mode, int acc, size_t n, size_t nkeys, const Geometry& geo,
   const DeviceCF& cf, const Mueller& mu, const CallBuffers& cb, size_t block_cap,
@@ -194,7 +194,6 @@ hipError_t launch_tile_halo(
 // most 8 x 8 (hx, hy <= 7), bins of launch_bin with quad_keys; ntile_keys
 // (plane, tile) keys, whose offset-table rows hold 4 ntile_keys + 1 values;
 // CF taps of at most 2^32 - 1 bytes
-size_t sub_lds_bytes(int hx, int hy);
 int sub_bins_limit();
 bool sub_supported(int hx, int hy);
 // uni: every CF group has the same support; global_bins (one polarization):

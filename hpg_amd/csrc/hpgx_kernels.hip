@@ -1,9 +1,10 @@
 // HIP kernels of the MI355X gridding device (gfx950, wave64).
 //
-// Build with -ffp-contract=off: every FP32 product and FP64 sum below is
-// rounded where the reference's source rounds it (no fused multiply-add), so
-// that the FP64-grid mode reproduces the reference's per-tap values bit for
-// bit and differs from it only by the order of FP64 accumulation.
+// Build with -ffp-contract=off: a product or sum is fused only where the code
+// says so.  FP64 grids without phase gradients hold the reference's per-tap FP32
+// values bit for bit, and differ from it only by the order of FP64 accumulation.
+// Fused by intent: the FP32 products of k_sub (FP32 grids), the FP64 products of
+// k_degrid, and cphase_taylor's reduction and series.
 //
 // Gridding (VisibilityGridder::kernel, src/hpg_core.hpp:1082-1253) is
 // re-organized for the device in two stages: binning, then one workgroup per
@@ -346,17 +347,14 @@ __device__ __forceinline__ unsigned long long pack_pair(float hi, float lo) {
     | ((unsigned long long)__float_as_uint(lo) << 32);
 }
 
-// the pair (hi, lo) after adding h (+ the low-order part l, when HAS_L)
-// to it: hi' = fl(hi + h), lo' = fl(lo + (err + l)) with err the exact
-// rounding error of the first sum (two-sum)
-template <bool HAS_L>
-__device__ __forceinline__ unsigned long long pair_plus(
-  unsigned long long pair, float h, float l) {
+// the pair (hi, lo) after adding h to it: hi' = fl(hi + h), lo' = fl(lo + err)
+// with err the exact rounding error of the first sum (two-sum)
+__device__ __forceinline__ unsigned long long pair_plus(unsigned long long pair, float h) {
   const float hi = __uint_as_float(unsigned(pair));
   const float lo = __uint_as_float(unsigned(pair >> 32));
   float sum, err;
   two_sum(hi, h, sum, err);
-  return pack_pair(sum, HAS_L ? lo + (err + l) : lo + err);
+  return pack_pair(sum, lo + err);
 }
 
 // compare-and-swap of the pair at a from `expect` to `desired`; on failure
@@ -369,15 +367,15 @@ __device__ __forceinline__ bool pair_swap(
 
 // retries until the update of the pair at a lands; every retry follows a
 // successful update of the same pair by another lane or wave
-template <bool HAS_L>
 __device__ __forceinline__ void pair_add(
-  unsigned long long* a, unsigned long long expect, float h, float l) {
-  while (!pair_swap(a, expect, pair_plus<HAS_L>(expect, h, l))) {
+  unsigned long long* a, unsigned long long expect, float h) {
+  while (!pair_swap(a, expect, pair_plus(expect, h))) {
   }
 }
 
 // ---- gridding, global bins ---------------------------------------------------
 //
+// (and the kernels of the next two sections: one polarization)
 // k_count   one thread per visibility: skip rule, weights, bin counts
 // k_emit    one thread per visibility: writes one compact Entry4 per grid plane
 //           -- support corner, fine offsets, CF group and cube, pre-phased
@@ -386,15 +384,11 @@ __device__ __forceinline__ void pair_add(
 //           gathering per-visibility records
 
 // an entry under construction in k_bin
-struct EntryHead {
+struct Entry {
   int gx, gy;
   unsigned fpk;  // fxi | fyi << 8 | flags << 16
   unsigned gpk;  // grp | cfcube << 16
-};
-template <int N>
-struct Entry {
-  EntryHead h;
-  float2 g[N];
+  float2 g;
 };
 
 // entries of the haloed-tile pipeline (k_tile4): one per (record, plane),
@@ -403,20 +397,17 @@ struct Entry4Head {
   unsigned pos;  // lx | ly << 6 | fxi << 12 | fyi << 20 | flags << 28
   unsigned gpk;  // grp | cfcube << 16
 };
-template <int N>
 struct Entry4 {
   Entry4Head h;
-  float2 g[N];
+  float2 g;
 };
 constexpr unsigned e4_pos_w = 1u << 28;
 constexpr unsigned e4_gradient = 1u << 29;
-// k_emit writes this layout as 2 + 2N 32-bit words
-static_assert(sizeof(Entry4<1>) == 16 && sizeof(Entry4<4>) == 40, "Entry4 layout");
+static_assert(sizeof(Entry4) == 16, "Entry4 layout");
 
-// bin key of tile key k for a support corner (gx, gy): k itself, or with
-// quad_keys 4 k + the quadrant of the corner within its tile
-__device__ __forceinline__ int bin_key(int k, int gx, int gy, int quad_keys) {
-  if (!quad_keys) return k;
+// quadrant key of tile key k for a support corner (gx, gy): 4 k + the quadrant
+// of the corner within its tile
+__device__ __forceinline__ int quad_key(int k, int gx, int gy) {
   const int qx = (gx % tile) >= tile / 2 ? 1 : 0;
   const int qy = (gy % tile) >= tile / 2 ? 1 : 0;
   return 4 * k + (qx | (qy << 1));
@@ -431,9 +422,8 @@ __device__ __forceinline__ int bin_key(int k, int gx, int gy, int quad_keys) {
 constexpr int count_planes_lds = 64;
 constexpr unsigned count_blocks_max = 2048;
 
-template <int N>
 __global__ __launch_bounds__(block) void k_count(
-  const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
+  const VisRec<1>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int do_grid, unsigned* __restrict__ hist,
   double* __restrict__ weights, unsigned long long* __restrict__ invalid) {
@@ -456,7 +446,7 @@ __global__ __launch_bounds__(block) void k_count(
     unsigned gcube = 0;
     double tw[4] = {0.0, 0.0, 0.0, 0.0};
     if (i < n) {
-      const VisRec<N>& r = recs[i];
+      const VisRec<1>& r = recs[i];
       const unsigned grp = r.cf_index[1];
       const unsigned cfcube = r.cf_index[0];
       gcube = r.grid_cube;
@@ -473,28 +463,24 @@ __global__ __launch_bounds__(block) void k_count(
           const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
             const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
-            double t = 0.0;
-            for (int v = 0; v < N; ++v) {
-              const int m = row[v];
-              double mag = 0.0;
-              if (m >= 0 && m < g.nmueller) {
-                const double2 sw = wsum[g.wsum_offset
-                                        + ((long long)(cfcube * g.nmueller + m) * geo.nf
-                                           + fxi) * geo.nf + fyi];
-                mag = hypot(sw.x, sw.y);
-              }
-              t += mag * double(r.w[v]);
+            const int m = row[0];
+            double mag = 0.0;
+            if (m >= 0 && m < g.nmueller) {
+              const double2 sw = wsum[g.wsum_offset
+                                      + ((long long)(cfcube * g.nmueller + m) * geo.nf
+                                         + fxi) * geo.nf + fyi];
+              mag = hypot(sw.x, sw.y);
             }
-            tw[gpol] = t;
+            tw[gpol] = mag * double(r.w[0]);
           }
         }
         if (c.inside && do_grid) {
           const int ntiles = geo.ntx * geo.nty;
           const int t = tiles_begin(c.gy) * geo.ntx + tiles_begin(c.gx);
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
-            if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
+            if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], 1)) continue;
             const int base = int(gcube * geo.nr + gpol) * ntiles;
-            atomicAdd(hist + bin_key(base + t, c.gx, c.gy, 0), 1u);
+            atomicAdd(hist + base + t, 1u);
           }
         }
       }
@@ -527,17 +513,16 @@ __global__ __launch_bounds__(block) void k_count(
   }
 }
 
-template <int N>
 __global__ __launch_bounds__(block) void k_emit(
-  const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
+  const VisRec<1>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int gvis_ready, int adjoint, const float2* __restrict__ gvis_in,
   const double2* __restrict__ residuals, unsigned* __restrict__ cursor,
-  void* __restrict__ entries_out, unsigned* __restrict__ entry_vis) {
+  Entry4* __restrict__ entries, unsigned* __restrict__ entry_vis) {
 
   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const VisRec<N>& r = recs[i];
+  const VisRec<1>& r = recs[i];
   const unsigned grp = r.cf_index[1];
   const unsigned cfcube = r.cf_index[0];
   const unsigned gcube = r.grid_cube;
@@ -550,44 +535,33 @@ __global__ __launch_bounds__(block) void k_emit(
   const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
   const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
 
-  Entry<N> e;
-  e.h.gx = c.gx;
-  e.h.gy = c.gy;
-  e.h.fpk = unsigned(fxi) | (unsigned(fyi) << 8)
-    | (unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0)) << 16);
+  const int tx = tiles_begin(c.gx), ty = tiles_begin(c.gy);
+  // corner relative to the tile, fine offsets, flags
+  Entry4 e;
+  e.h.pos = unsigned(c.gx - tx * tile) | (unsigned(c.gy - ty * tile) << 6)
+    | (unsigned(fxi) << 12) | (unsigned(fyi) << 20) | (pos_w ? e4_pos_w : 0u)
+    | (grad ? e4_gradient : 0u);
   e.h.gpk = grp | (cfcube << 16);
   if (gvis_ready) {
-    for (int v = 0; v < N; ++v) e.g[v] = gvis_in[i * N + v];
+    e.g = gvis_in[i];
   } else {
     const double2 phasor = cphase(r.phase);
     if (!adjoint) {
-      for (int v = 0; v < N; ++v) e.g[v] = prephase(r.vis[v], phasor, r.w[v]);
+      e.g = prephase(r.vis[0], phasor, r.w[0]);
     } else {
-      double2 W[N];
-      degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-      for (int v = 0; v < N; ++v) {
-        double2 d = W[v];
-        if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
-        d.y = -d.y;
-        e.g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
-      }
+      double2 d;
+      degrid_norms<1>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, &d);
+      if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
+      d.y = -d.y;
+      e.g = narrow(kdiv(cmul(residuals[i], phasor), d));
     }
   }
   const int ntiles = geo.ntx * geo.nty;
-  const int tx = tiles_begin(c.gx), ty = tiles_begin(c.gy);
   for (int gpol = 0; gpol < geo.nr; ++gpol) {
-    if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
+    if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], 1)) continue;
     const int base = int(gcube * geo.nr + gpol) * ntiles;
-    const unsigned pos =
-      atomicAdd(cursor + bin_key(base + ty * geo.ntx + tx, c.gx, c.gy, 0), 1u);
-    // corner relative to the tile, fine offsets, flags
-    const unsigned hpos = unsigned(c.gx - tx * tile) | (unsigned(c.gy - ty * tile) << 6)
-      | ((e.h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u) | (grad ? e4_gradient : 0u);
-    unsigned* q = static_cast<unsigned*>(entries_out) + size_t(pos) * (2 + 2 * N);
-    q[0] = hpos;
-    q[1] = e.h.gpk;
-    float2* qg = reinterpret_cast<float2*>(q + 2);
-    for (int v = 0; v < N; ++v) qg[v] = e.g[v];
+    const unsigned pos = atomicAdd(cursor + base + ty * geo.ntx + tx, 1u);
+    entries[pos] = e;
     if (grad) entry_vis[pos] = unsigned(i);
   }
 }
@@ -732,15 +706,14 @@ __device__ __forceinline__ void sort_bin(
 // against 114 with a returning global atomic per entry, a device-wide scan and
 // a memset; moving the entries already with k_sort_place costs there (24 us)
 // what it saves.
-template <int N>
 __global__ __launch_bounds__(patch_local_threads) void k_tally(
-  const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
+  const VisRec<1>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int gvis_ready, int adjoint,
   const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
   SortKeys sk, unsigned batch, unsigned* __restrict__ hist, unsigned* __restrict__ table,
   double* __restrict__ weights, unsigned long long* __restrict__ invalid,
-  Entry4<N>* __restrict__ tally, unsigned* __restrict__ tally_keys) {
+  Entry4* __restrict__ tally, unsigned* __restrict__ tally_keys) {
 
   __shared__ double wblk[count_planes_lds];
   __shared__ unsigned cnt[patch_local_keys];
@@ -765,7 +738,7 @@ __global__ __launch_bounds__(patch_local_threads) void k_tally(
       // slots of rows without an entry say so
       for (int gpol = 0; gpol < geo.nr; ++gpol)
         tally_keys[i * geo.nr + gpol] = ~0u;
-      const VisRec<N>& r = recs[i];
+      const VisRec<1>& r = recs[i];
       const unsigned grp = r.cf_index[1];
       const unsigned cfcube = r.cf_index[0];
       gcube = r.grid_cube;
@@ -782,50 +755,43 @@ __global__ __launch_bounds__(patch_local_threads) void k_tally(
           counted = true;
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
             const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
-            double t = 0.0;
-            for (int v = 0; v < N; ++v) {
-              const int m = row[v];
-              double mag = 0.0;
-              if (m >= 0 && m < g.nmueller) {
-                const double2 sw = wsum[g.wsum_offset
-                                        + ((long long)(cfcube * g.nmueller + m) * geo.nf
-                                           + fxi) * geo.nf + fyi];
-                mag = hypot(sw.x, sw.y);
-              }
-              t += mag * double(r.w[v]);
+            const int m = row[0];
+            double mag = 0.0;
+            if (m >= 0 && m < g.nmueller) {
+              const double2 sw = wsum[g.wsum_offset
+                                      + ((long long)(cfcube * g.nmueller + m) * geo.nf
+                                         + fxi) * geo.nf + fyi];
+              mag = hypot(sw.x, sw.y);
             }
-            tw[gpol] = t;
+            tw[gpol] = mag * double(r.w[0]);
           }
         }
         if (c.inside) {
           const bool grad = r.grad[0] != 0.0 || r.grad[1] != 0.0;
-          Entry4<N> e;
+          Entry4 e;
           const int tx = tiles_begin(c.gx), ty = tiles_begin(c.gy);
           e.h.pos = unsigned(c.gx - tx * tile) | (unsigned(c.gy - ty * tile) << 6)
             | (unsigned(fxi) << 12) | (unsigned(fyi) << 20) | (pos_w ? e4_pos_w : 0u)
             | (grad ? e4_gradient : 0u);
           e.h.gpk = grp | (cfcube << 16);
           if (gvis_ready) {
-            for (int v = 0; v < N; ++v) e.g[v] = gvis_in[i * N + v];
+            e.g = gvis_in[i];
           } else {
             const double2 phasor = cphase(r.phase);
             if (!adjoint) {
-              for (int v = 0; v < N; ++v) e.g[v] = prephase(r.vis[v], phasor, r.w[v]);
+              e.g = prephase(r.vis[0], phasor, r.w[0]);
             } else {
-              double2 W[N];
-              degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-              for (int v = 0; v < N; ++v) {
-                double2 d = W[v];
-                if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
-                d.y = -d.y;
-                e.g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
-              }
+              double2 d;
+              degrid_norms<1>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, &d);
+              if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
+              d.y = -d.y;
+              e.g = narrow(kdiv(cmul(residuals[i], phasor), d));
             }
           }
           for (int gpol = 0; gpol < geo.nr; ++gpol) {
-            if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], N)) continue;
+            if (!row_has_index(pos_w ? mu.M[gpol] : mu.Mc[gpol], 1)) continue;
             const int key =
-              bin_key((int(gcube) * geo.nr + gpol) * ntiles + ty * geo.ntx + tx, c.gx, c.gy, 1);
+              quad_key((int(gcube) * geo.nr + gpol) * ntiles + ty * geo.ntx + tx, c.gx, c.gy);
             __hip_atomic_fetch_add(cnt + (unsigned(key) >> sk.low_bits), 1u, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
             tally[i * geo.nr + gpol] = e;
@@ -866,11 +832,10 @@ __global__ __launch_bounds__(patch_local_threads) void k_tally(
 
 // one workgroup per bin: its entries in order of their keys, and the keys'
 // offsets
-template <int N>
 __global__ __launch_bounds__(sort_threads) void k_tally_sort(
   int low_bits, size_t nkeys, int nr, const unsigned* __restrict__ bin_offsets,
-  const uint2* __restrict__ pairs, const Entry4<N>* __restrict__ tally,
-  unsigned* __restrict__ offsets, Entry4<N>* __restrict__ entries,
+  const uint2* __restrict__ pairs, const Entry4* __restrict__ tally,
+  unsigned* __restrict__ offsets, Entry4* __restrict__ entries,
   unsigned* __restrict__ entry_vis) {
   const unsigned beg = bin_offsets[blockIdx.x], end = bin_offsets[blockIdx.x + 1];
   const size_t key0 = size_t(blockIdx.x) << low_bits;
@@ -886,7 +851,7 @@ __global__ __launch_bounds__(sort_threads) void k_tally_sort(
       for (size_t k = threadIdx.x; k < keys; k += sort_threads) offsets[key0 + k] = beg + first[k];
     },
     [&](unsigned at, unsigned slot) {
-      const Entry4<N> e = tally[slot];
+      const Entry4 e = tally[slot];
       entries[beg + at] = e;
       if (e.h.pos & e4_gradient) entry_vis[beg + at] = slot / unsigned(nr);
     });
@@ -920,15 +885,14 @@ constexpr int bin_stage_bytes = 65536;  // LDS staging of k_bin's haloed entries
                                         // chunk for a block of one-polarization entries)
 
 // one entry per record and plane, keyed by the tile of the support corner
-template <int N>
 __global__ __launch_bounds__(bin_threads) void k_bin(
-  const VisRec<N>* __restrict__ recs, size_t n, Geometry geo,
+  const VisRec<1>* __restrict__ recs, size_t n, Geometry geo,
   const GroupInfo* __restrict__ groups, const double2* __restrict__ wsum,
   Mueller mu, int update_weights, int gvis_ready, int adjoint, int degrid_pass,
   const float2* __restrict__ gvis_in, const double2* __restrict__ residuals,
   unsigned* __restrict__ off_table, void* __restrict__ entries_out,
   unsigned* __restrict__ entry_vis, size_t block_cap, double* __restrict__ weights,
-  unsigned long long* __restrict__ invalid, VisRec<N>* __restrict__ copy_recs, int quad_keys) {
+  unsigned long long* __restrict__ invalid, VisRec<1>* __restrict__ copy_recs, int quad_keys) {
 
   __shared__ unsigned cnt[bin_quad_keys_max];
   __shared__ double wl[bin_planes_max];
@@ -960,7 +924,7 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
         atomicAdd(weights + k, acc[gpol]);
     }
   };
-  Entry<N> e[bin_recs_per_thread];
+  Entry e[bin_recs_per_thread];
   bool keep[bin_recs_per_thread];
   unsigned gc[bin_recs_per_thread];
   unsigned ninvalid = 0;
@@ -971,21 +935,20 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
 #pragma unroll
   for (int gp = 0; gp < 4; ++gp) {
     if (gp >= geo.nr) continue;
-    rows_m |= row_has_index(mu.M[gp], N) ? 1u << gp : 0u;
-    rows_mc |= row_has_index(mu.Mc[gp], N) ? 1u << gp : 0u;
+    rows_m |= row_has_index(mu.M[gp], 1) ? 1u << gp : 0u;
+    rows_mc |= row_has_index(mu.Mc[gp], 1) ? 1u << gp : 0u;
   }
   const bool one_group = geo.ngroups == 1;
   const GroupInfo group0 = groups[0];
 
-  // N == 1: the thread's records are loaded whole, two at a time, so that
-  // two records' loads are in flight at once rather than one record (and its
-  // chain of dependent loads) at a time; four would spill the 128 registers
-  // a 1024-thread block allows, larger records load per record
-  constexpr bool hoist = N == 1;
-  constexpr int words = int(sizeof(VisRec<N>) / sizeof(unsigned long long));
-  static_assert(sizeof(VisRec<N>) % sizeof(unsigned long long) == 0, "8-byte record words");
+  // the thread's records are loaded whole, two at a time, so that two records'
+  // loads are in flight at once rather than one record (and its chain of
+  // dependent loads) at a time; four would spill the 128 registers a
+  // 1024-thread block allows
+  constexpr int words = int(sizeof(VisRec<1>) / sizeof(unsigned long long));
+  static_assert(sizeof(VisRec<1>) % sizeof(unsigned long long) == 0, "8-byte record words");
   static_assert(bin_recs_per_thread % 2 == 0, "records loaded in pairs");
-  VisRec<N> rc[hoist ? 2 : 1];
+  VisRec<1> rc[2];
   // the place of each of this thread's entries (one per record and
   // grid row with an index; ~0u for none) within its key, from the count's
   // returned value, then (after the scan) its block-local position; the
@@ -998,38 +961,25 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
 
 #pragma unroll
   for (int j = 0; j < bin_recs_per_thread; ++j) {
-    if constexpr (hoist) {
-      if (j % 2 == 0) {
+    if (j % 2 == 0) {
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const size_t i = b * bin_records + size_t(j + jj) * bin_threads + threadIdx.x;
-          if (i >= n) continue;
-          const unsigned long long* src = reinterpret_cast<const unsigned long long*>(recs + i);
-          unsigned long long wds[words];
+      for (int jj = 0; jj < 2; ++jj) {
+        const size_t i = b * bin_records + size_t(j + jj) * bin_threads + threadIdx.x;
+        if (i >= n) continue;
+        const unsigned long long* src = reinterpret_cast<const unsigned long long*>(recs + i);
+        unsigned long long wds[words];
 #pragma unroll
-          for (int k = 0; k < words; ++k) wds[k] = src[k];
-          __builtin_memcpy(&rc[jj], wds, sizeof(VisRec<N>));
-        }
+        for (int k = 0; k < words; ++k) wds[k] = src[k];
+        __builtin_memcpy(&rc[jj], wds, sizeof(VisRec<1>));
       }
     }
     keep[j] = false;
     const size_t i = b * bin_records + size_t(j) * bin_threads + threadIdx.x;
     if (i >= n) continue;
-    // N == 2: the whole record in registers first, so its fields load in one
-    // round instead of one round per dependent use
-    VisRec<N> r_copy;
-    if constexpr (N == 2) {
-      const unsigned long long* src = reinterpret_cast<const unsigned long long*>(recs + i);
-      unsigned long long wds[words];
-#pragma unroll
-      for (int k = 0; k < words; ++k) wds[k] = src[k];
-      __builtin_memcpy(&r_copy, wds, sizeof(r_copy));
-    }
-    const VisRec<N>& r = hoist ? rc[j % 2] : N == 2 ? r_copy : recs[i];
+    const VisRec<1>& r = rc[j % 2];
     // degridding that returns the batch: every record is written to the
     // returned batch here, whose values the degridding kernels then replace
     if (copy_recs) {
-      constexpr int words = int(sizeof(VisRec<N>) / sizeof(unsigned long long));
       const unsigned long long* src = reinterpret_cast<const unsigned long long*>(&r);
       unsigned long long* dst = reinterpret_cast<unsigned long long*>(copy_recs + i);
 #pragma unroll
@@ -1053,34 +1003,31 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
     const int fxi = c.fx + geo.F, fyi = c.fy + geo.F;
     keep[j] = true;
     gc[j] = gcube;
-    e[j].h.gx = c.gx;
-    e[j].h.gy = c.gy;
-    e[j].h.fpk = unsigned(fxi) | (unsigned(fyi) << 8)
+    e[j].gx = c.gx;
+    e[j].gy = c.gy;
+    e[j].fpk = unsigned(fxi) | (unsigned(fyi) << 8)
       | (unsigned((pos_w ? flag_pos_w : 0) | (grad ? flag_gradient : 0)) << 16);
-    e[j].h.gpk = grp | (cfcube << 16);
+    e[j].gpk = grp | (cfcube << 16);
     if (degrid_pass) {
       // degridding reads the model: entries carry no values
-      for (int v = 0; v < N; ++v) e[j].g[v] = make_float2(0.0f, 0.0f);
+      e[j].g = make_float2(0.0f, 0.0f);
     } else if (gvis_ready) {
-      for (int v = 0; v < N; ++v) e[j].g[v] = gvis_in[i * N + v];
+      e[j].g = gvis_in[i];
     } else {
       const double2 phasor = cphase(r.phase);
       if (!adjoint) {
-        for (int v = 0; v < N; ++v) e[j].g[v] = prephase(r.vis[v], phasor, r.w[v]);
+        e[j].g = prephase(r.vis[0], phasor, r.w[0]);
       } else {
-        double2 W[N];
-        degrid_norms<N>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, W);
-        for (int v = 0; v < N; ++v) {
-          double2 d = W[v];
-          if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
-          d.y = -d.y;
-          e[j].g[v] = narrow(kdiv(cmul(residuals[i * N + v], phasor), d));
-        }
+        double2 d;
+        degrid_norms<1>(geo, g, wsum, mu, pos_w, cfcube, fxi, fyi, &d);
+        if (d.x == 0.0 && d.y == 0.0) d = make_double2(1.0, 0.0);
+        d.y = -d.y;
+        e[j].g = narrow(kdiv(cmul(residuals[i], phasor), d));
       }
     }
     if (update_weights) {
-      // twgt = sum_v |sum_XY cf'| * w_v (src/hpg_core.hpp:877-885); grid
-      // rows and polarizations unrolled, so the Mueller indices are scalars
+      // twgt = |sum_XY cf'| * w (src/hpg_core.hpp:877-885); grid rows
+      // unrolled, so the Mueller indices are scalars
       // and the slice-sum loads of all rows issue together
       if (int(gcube) != wcube) {
         if (wcube >= 0) flush_weights(wcube, wacc);
@@ -1091,20 +1038,15 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
 #pragma unroll
       for (int gp = 0; gp < 4; ++gp) {
         if (gp >= geo.nr) continue;
-        double t = 0.0;
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          const int m = pos_w ? mu.M[gp][v] : mu.Mc[gp][v];
-          double mag = 0.0;
-          if (m >= 0 && m < g.nmueller) {
-            const double2 sw = wsum[g.wsum_offset
-                                    + ((long long)(cfcube * g.nmueller + m) * geo.nf + fxi)
-                                      * geo.nf + fyi];
-            mag = hypot(sw.x, sw.y);
-          }
-          t += mag * double(r.w[v]);
+        const int m = pos_w ? mu.M[gp][0] : mu.Mc[gp][0];
+        double mag = 0.0;
+        if (m >= 0 && m < g.nmueller) {
+          const double2 sw = wsum[g.wsum_offset
+                                  + ((long long)(cfcube * g.nmueller + m) * geo.nf + fxi)
+                                    * geo.nf + fyi];
+          mag = hypot(sw.x, sw.y);
         }
-        wacc[gp] += t;
+        wacc[gp] += mag * double(r.w[0]);
       }
     }
     const int t = tiles_begin(c.gy) * geo.ntx + tiles_begin(c.gx);
@@ -1113,7 +1055,7 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
       if (!((rows >> gpol) & 1u)) continue;
       const int base = (int(gcube) * geo.nr + gpol) * ntiles;
       const unsigned place = __hip_atomic_fetch_add(
-        cnt + bin_key(base + t, c.gx, c.gy, quad_keys), 1u,
+        cnt + (quad_keys ? quad_key(base + t, c.gx, c.gy) : base + t), 1u,
         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -1160,9 +1102,9 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
   for (int j = 0; j < bin_recs_per_thread; ++j) {
     if (!keep[j]) continue;
     const size_t i = size_t(j) * bin_threads + threadIdx.x;
-    const bool pos_w = (e[j].h.fpk >> 16) & flag_pos_w;
-    const bool grad = (e[j].h.fpk >> 16) & flag_gradient;
-    const int t = tiles_begin(e[j].h.gy) * geo.ntx + tiles_begin(e[j].h.gx);
+    const bool pos_w = (e[j].fpk >> 16) & flag_pos_w;
+    const bool grad = (e[j].fpk >> 16) & flag_gradient;
+    const int t = tiles_begin(e[j].gy) * geo.ntx + tiles_begin(e[j].gx);
     const unsigned rows = (pos_w != bool(degrid_pass)) ? rows_m : rows_mc;
     for (int gpol = 0; gpol < geo.nr; ++gpol) {
       if (!((rows >> gpol) & 1u)) continue;
@@ -1172,7 +1114,8 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (r == gpol) place = hpos[j][r];
-      const unsigned pos = cnt[bin_key(base + t, e[j].h.gx, e[j].h.gy, quad_keys)] + place;
+      const unsigned pos =
+        cnt[quad_keys ? quad_key(base + t, e[j].gx, e[j].gy) : base + t] + place;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (r == gpol) hpos[j][r] = pos;
@@ -1181,26 +1124,26 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
   }
   // chunks of the block's entry range: each thread puts its entries of
   // the chunk into LDS, then the block copies the chunk out contiguously
-  // (scattered 16 to 40-byte stores would each write a partial line)
-  constexpr unsigned ewords = unsigned(sizeof(Entry4<N>) / sizeof(unsigned long long));
-  constexpr unsigned chunk = unsigned(bin_stage_bytes / sizeof(Entry4<N>));
+  // (scattered 16-byte stores would each write a partial line)
+  constexpr unsigned ewords = unsigned(sizeof(Entry4) / sizeof(unsigned long long));
+  constexpr unsigned chunk = unsigned(bin_stage_bytes / sizeof(Entry4));
   __shared__ unsigned long long stage[chunk * ewords];
-  Entry4<N>* staged = reinterpret_cast<Entry4<N>*>(stage);
+  Entry4* staged = reinterpret_cast<Entry4*>(stage);
   unsigned long long* dst =
-    reinterpret_cast<unsigned long long*>(static_cast<Entry4<N>*>(entries_out) + b * block_cap);
+    reinterpret_cast<unsigned long long*>(static_cast<Entry4*>(entries_out) + b * block_cap);
   for (unsigned c0 = 0; c0 < btotal; c0 += chunk) {
 #pragma unroll
     for (int j = 0; j < bin_recs_per_thread; ++j) {
       if (!keep[j]) continue;
-      const bool pos_w = (e[j].h.fpk >> 16) & flag_pos_w;
-      const bool grad = (e[j].h.fpk >> 16) & flag_gradient;
-      Entry4<N> q;
-      q.h.pos = unsigned(e[j].h.gx - tiles_begin(e[j].h.gx) * tile)
-        | (unsigned(e[j].h.gy - tiles_begin(e[j].h.gy) * tile) << 6)
-        | ((e[j].h.fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u)
+      const bool pos_w = (e[j].fpk >> 16) & flag_pos_w;
+      const bool grad = (e[j].fpk >> 16) & flag_gradient;
+      Entry4 q;
+      q.h.pos = unsigned(e[j].gx - tiles_begin(e[j].gx) * tile)
+        | (unsigned(e[j].gy - tiles_begin(e[j].gy) * tile) << 6)
+        | ((e[j].fpk & 0xffffu) << 12) | (pos_w ? e4_pos_w : 0u)
         | (grad ? e4_gradient : 0u);
-      q.h.gpk = e[j].h.gpk;
-      for (int v = 0; v < N; ++v) q.g[v] = e[j].g[v];
+      q.h.gpk = e[j].gpk;
+      q.g = e[j].g;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (hpos[j][r] - c0 < chunk) staged[hpos[j][r] - c0] = q;
@@ -1214,7 +1157,7 @@ __global__ __launch_bounds__(bin_threads) void k_bin(
 
 // ---- gridding, haloed tiles ---------------------------------------------
 //
-// k_bin<N, true> writes one Entry4 per (record, plane) into the bin of the
+// k_bin writes one Entry4 per (record, plane) into the bin of the
 // tile that holds the support corner.  The workgroup of a key accumulates
 // the tile plus a halo of hx = max_sx - 1 columns and hy = max_sy - 1 rows on
 // its high sides (R = (tile + hx) x (tile + hy) pixels in LDS), so every tap
@@ -1259,12 +1202,12 @@ __host__ __device__ inline int halo_pixels(int hx, int hy) {
 constexpr int acc_f64 = 0;
 constexpr int acc_f32_cas = 2;
 
-template <int N, int MODE, int ACC>
+template <int MODE, int ACC>
 __global__ __launch_bounds__(halo_block) void k_tile4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
-  int nbins, size_t block_cap, const Entry4<N>* __restrict__ entries,
-  const unsigned* __restrict__ entry_vis, const VisRec<N>* __restrict__ recs,
+  int nbins, size_t block_cap, const Entry4* __restrict__ entries,
+  const unsigned* __restrict__ entry_vis, const VisRec<1>* __restrict__ recs,
   int hx, int hy, void* __restrict__ grid, double2* __restrict__ halo,
   unsigned* __restrict__ halo_set) {
   static_assert(MODE == 1 || ACC == acc_f64, "FP64 grids accumulate in FP64");
@@ -1368,7 +1311,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
       const unsigned sp = rank * nbatch + j;
       if (sp >= rn) continue;
       const unsigned idx = sched[sp];
-      const Entry4<N> e = entries[idx];
+      const Entry4 e = entries[idx];
       const unsigned pos = e.h.pos;
       const int lx = int(pos & 63u);
       const int ly = int((pos >> 6) & 63u);
@@ -1382,13 +1325,9 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
       const int sx = g.sx, sy = g.sy;
       const int* row = pos_w ? mu.M[gpol] : mu.Mc[gpol];
       const float imf = pos_w ? -1.0f : 1.0f;
-      const float2* slice[N];
-      bool use[N];
-      for (int v = 0; v < N; ++v) {
-        const int m = row[v];
-        use[v] = m >= 0 && m < g.nmueller;
-        slice[v] = taps + plane_start(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
-      }
+      const int m = row[0];
+      const bool use = m >= 0 && m < g.nmueller;
+      const float2* slice = taps + plane_start(g, geo.nf, int(cfcube), use ? m : 0, fxi, fyi);
       double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
       if (grad) {
         const unsigned i = entry_vis[idx];
@@ -1399,64 +1338,30 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
         dphix = gxr * geo.os;
         dphiy = gyr * geo.os;
       }
-      // the value of one tap: hi (FP32) and, for N > 1, the low-order part
-      // of the FP64 sum over the polarizations; d = the FP64 value
-      auto tap_value = [&](const float2* cv, int X, int Y, float& h_r, float& h_i,
-                           float& l_r, float& l_i, double& d_r, double& d_i) {
-        float2 scr = make_float2(1.0f, 0.0f);
-        if (grad) scr = narrow(cphase((phi0x + X * dphix) + (phi0y + Y * dphiy)));
-        if constexpr (N == 1) {
-          float2 cc = cv[0];
-          cc.y *= imf;
-          if (grad) cc = cmul(cc, scr);
-          const float2 pr = cmul(cc, e.g[0]);
-          h_r = pr.x;
-          h_i = pr.y;
-          l_r = 0.0f;
-          l_i = 0.0f;
-          d_r = double(pr.x);
-          d_i = double(pr.y);
-        } else {
-          double sr = 0.0, si = 0.0;
-#pragma unroll
-          for (int v = 0; v < N; ++v) {
-            if (!use[v]) continue;
-            float2 cc = cv[v];
-            cc.y *= imf;
-            if (grad) cc = cmul(cc, scr);
-            const float2 pr = cmul(cc, e.g[v]);
-            sr += double(pr.x);
-            si += double(pr.y);
-          }
-          d_r = sr;
-          d_i = si;
-          h_r = float(sr);
-          h_i = float(si);
-          l_r = float(sr - double(h_r));
-          l_i = float(si - double(h_i));
-        }
+      // the value of one tap
+      auto tap_value = [&](float2 cc, int X, int Y) {
+        cc.y *= imf;
+        if (grad) cc = cmul(cc, narrow(cphase((phi0x + X * dphix) + (phi0y + Y * dphiy))));
+        return cmul(cc, e.g);
       };
       // adds the M taps held in the arrays to LDS pixels li[0..M) (ok[m]:
       // tap present).  The compare-and-swap form reads each pixel just
       // before its swap: the wave's LDS operations execute in order, so two
       // lanes of one wave only race on a pixel when their corners coincide;
       // failed swaps are retried after the last tap.
-      auto accumulate = [&](auto m_c, const int* li, const bool* ok, const float* h_r,
-                            const float* h_i, const float* l_r, const float* l_i,
-                            const double* d_r, const double* d_i) {
+      auto accumulate = [&](auto m_c, const int* li, const bool* ok, const float2* p) {
         constexpr int M = decltype(m_c)::value;
         if constexpr (ACC == acc_f64) {
 #pragma unroll
           for (int m = 0; m < M; ++m) {
             if (!ok[m]) continue;
-            __hip_atomic_fetch_add(acc64 + li[m], d_r[m], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(acc64 + li[m], double(p[m].x), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(acc64 + R + li[m], d_i[m], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(acc64 + R + li[m], double(p[m].y), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
           }
         } else {
           // pixel li holds (H_re, L_re) at pairs[li], (H_im, L_im) at pairs[R + li]
-          constexpr bool has_l = N > 1;
           unsigned long long er[M], ei[M];
           bool okr[M], oki[M];
 #pragma unroll
@@ -1464,15 +1369,14 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
             if (!ok[m]) continue;
             er[m] = pairs[li[m]];
             ei[m] = pairs[R + li[m]];
-            okr[m] = pair_swap(pairs + li[m], er[m], pair_plus<has_l>(er[m], h_r[m], l_r[m]));
-            oki[m] = pair_swap(pairs + R + li[m], ei[m],
-                               pair_plus<has_l>(ei[m], h_i[m], l_i[m]));
+            okr[m] = pair_swap(pairs + li[m], er[m], pair_plus(er[m], p[m].x));
+            oki[m] = pair_swap(pairs + R + li[m], ei[m], pair_plus(ei[m], p[m].y));
           }
 #pragma unroll
           for (int m = 0; m < M; ++m) {
             if (!ok[m]) continue;
-            if (!okr[m]) pair_add<has_l>(pairs + li[m], er[m], h_r[m], l_r[m]);
-            if (!oki[m]) pair_add<has_l>(pairs + R + li[m], ei[m], h_i[m], l_i[m]);
+            if (!okr[m]) pair_add(pairs + li[m], er[m], p[m].x);
+            if (!oki[m]) pair_add(pairs + R + li[m], ei[m], p[m].y);
           }
         }
       };
@@ -1487,9 +1391,7 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
           constexpr bool FULL = decltype(full)::value;
           bool ok[halo_chunk];
           int li[halo_chunk];
-          float h_r[halo_chunk], h_i[halo_chunk], l_r[halo_chunk], l_i[halo_chunk];
-          double d_r[halo_chunk], d_i[halo_chunk];
-          float2 c[halo_chunk][N];
+          float2 c[halo_chunk], p[halo_chunk];
           int Xk[halo_chunk], Yk[halo_chunk];
 #pragma unroll
           for (int k = 0; k < halo_chunk; ++k) {
@@ -1501,18 +1403,14 @@ __global__ __launch_bounds__(halo_block) void k_tile4(
             cx = eol ? 0 : cx;
             cy += eol ? 1 : 0;
             lc += eol ? 1 + wrap : 1;
-#pragma unroll
-            for (int v = 0; v < N; ++v) {
-              float2 tv = make_float2(0.0f, 0.0f);
-              if (ok[k]) tv = slice[v][t0 + k];
-              c[k][v] = use[v] ? tv : make_float2(0.0f, 0.0f);
-            }
+            float2 tv = make_float2(0.0f, 0.0f);
+            if (ok[k]) tv = slice[t0 + k];
+            c[k] = use ? tv : make_float2(0.0f, 0.0f);
           }
 #pragma unroll
           for (int k = 0; k < halo_chunk; ++k)
-            tap_value(c[k], Xk[k], Yk[k], h_r[k], h_i[k], l_r[k], l_i[k], d_r[k], d_i[k]);
-          accumulate(std::integral_constant<int, halo_chunk>{}, li, ok, h_r, h_i, l_r, l_i,
-                     d_r, d_i);
+            p[k] = tap_value(c[k], Xk[k], Yk[k]);
+          accumulate(std::integral_constant<int, halo_chunk>{}, li, ok, p);
         };
         int t0 = 0;
         for (; t0 + halo_chunk <= ntap; t0 += halo_chunk) do_chunk(std::true_type{}, t0);
@@ -1784,16 +1682,14 @@ __device__ __forceinline__ float2 screen_f32(double phi) {
 // an entry with a phase gradient: its CF taps times the phase screen
 // exp(i phi(X, Y)) (FP64 phase as the reference's, screen_f32), added by
 // one wave, one lane per tap, to the wave's FP32 region
-template <int N>
 __device__ __forceinline__ void sub_gradient_entry(
-  unsigned w0, const unsigned* slice, const float2* g, unsigned ri, unsigned pos,
-  const Geometry& geo, const float2* __restrict__ taps, const VisRec<N>* __restrict__ recs,
+  unsigned w0, unsigned slice, float2 g, unsigned ri, unsigned pos,
+  const Geometry& geo, const float2* __restrict__ taps, const VisRec<1>* __restrict__ recs,
   int QX, float2* region) {
   const int lane = int(threadIdx.x % wave);
   const int base = int(w0 & 4095u);
   const int sx = int((w0 >> 12) & 63u);
   const int sy = int((w0 >> 18) & 63u);
-  const unsigned use = (w0 >> 24) & 15u;
   const float imf = (w0 & quad_pos_w) ? -1.0f : 1.0f;
   const int fxi = int((pos >> 12) & 255u);
   const int fyi = int((pos >> 20) & 255u);
@@ -1807,28 +1703,13 @@ __device__ __forceinline__ void sub_gradient_entry(
   if (X >= sx || Y >= sy) return;
   const int tp = Y * sx + X;
   const float2 scr = screen_f32((phi0x + X * dphix) + (phi0y + Y * dphiy));
-  double sr = 0.0, si = 0.0;
-  float h_r = 0.0f, h_i = 0.0f;
-  for (int v = 0; v < N; ++v) {
-    if (!((use >> v) & 1u)) continue;
-    float2 cc = taps[size_t(slice[v]) + size_t(tp)];
-    cc.y *= imf;
-    const float2 pr = cmul(cmul(cc, scr), g[v]);
-    if constexpr (N == 1) {
-      h_r = pr.x;
-      h_i = pr.y;
-    }
-    sr += double(pr.x);
-    si += double(pr.y);
-  }
-  if constexpr (N > 1) {
-    h_r = float(sr);
-    h_i = float(si);
-  }
+  float2 cc = taps[size_t(slice) + size_t(tp)];
+  cc.y *= imf;
+  const float2 pr = cmul(cmul(cc, scr), g);
   float2* a = region + base + Y * QX + X;
   float2 t = *a;
-  t.x += h_r;
-  t.y += h_i;
+  t.x += pr.x;
+  t.y += pr.y;
   *a = t;
 }
 
@@ -1915,14 +1796,14 @@ __device__ __forceinline__ unsigned sub_locate(
 // no bounds test.  UNI: every CF group has the same support, whose lane mask
 // then holds for the whole call.  PK: see sub_pk_flip.  GB: global bins
 // (sub_tables).
-template <int N, int PX, bool UNI, bool PK, bool GB>
-__global__ __launch_bounds__(sub_block) __attribute__((amdgpu_waves_per_eu(N == 1 ? 8 : 4)))
+template <int PX, bool UNI, bool PK, bool GB>
+__global__ __launch_bounds__(sub_block) __attribute__((amdgpu_waves_per_eu(8)))
 void k_sub(
   Geometry geo, const GroupInfo* __restrict__ groups, const float2* __restrict__ taps,
   unsigned taps_bytes, Mueller mu, const unsigned* __restrict__ off_table, int nbins,
   size_t block_cap,
-  const Entry4<N>* __restrict__ entries, const unsigned* __restrict__ entry_vis,
-  const VisRec<N>* __restrict__ recs, int hx, int hy, float2* __restrict__ grid,
+  const Entry4* __restrict__ entries, const unsigned* __restrict__ entry_vis,
+  const VisRec<1>* __restrict__ recs, int hx, int hy, float2* __restrict__ grid,
   double2* __restrict__ halo, unsigned* __restrict__ halo_set) {
   // eight FP32 regions of QP = PX * 64 pixels (float2); in the flush the
   // same bytes hold the four quadrants' (hi, lo) pairs (float4, Q each)
@@ -2000,13 +1881,8 @@ void k_sub(
 
   const bool one_group = geo.ngroups == 1;
   const GroupInfo group0 = groups[0];
-  // this plane's Mueller rows for both signs of w
-  int row_m[N], row_mc[N];
-#pragma unroll
-  for (int v = 0; v < N; ++v) {
-    row_m[v] = mu.M[gpol][v];
-    row_mc[v] = mu.Mc[gpol][v];
-  }
+  // this plane's Mueller elements for both signs of w
+  const int row_m = mu.M[gpol][0], row_mc = mu.Mc[gpol][0];
   // the quadrant's list, taken by its two waves alternately 64 entries at
   // a time (fewer partly filled batches than an even split, whose per-batch
   // costs outweigh its balance)
@@ -2059,7 +1935,7 @@ void k_sub(
     const unsigned i = b0 + unsigned(lane);
     const bool valid = i < total;
     unsigned ei = 0;
-    Entry4<N> e{};
+    Entry4 e{};
     if (valid) {
       ei = locate(i);
       e = entries[ei];
@@ -2068,13 +1944,8 @@ void k_sub(
     // w-sign flip (bit 31: conj(c) for w > 0) -- 0 for slots that add
     // nothing.  PK: the region pixel | sub_pk_flip | slice << sub_pk_shift
     unsigned p_addr = 0, p_key = 0;
-    unsigned p_sl[N];
-    float p_gx[N], p_gy[N];
-#pragma unroll
-    for (int v = 0; v < N; ++v) {
-      p_sl[v] = 0u;
-      p_gx[v] = p_gy[v] = 0.0f;
-    }
+    unsigned p_sl = 0u;
+    float p_gx = 0.0f, p_gy = 0.0f;
     bool grad = false, normal = false;
     if (valid) {
       const unsigned pos = e.h.pos;
@@ -2087,27 +1958,22 @@ void k_sub(
       const int grp = int(e.h.gpk & 0xffffu);
       const int cfcube = int(e.h.gpk >> 16);
       const GroupInfo g = one_group ? group0 : groups[grp];
-      unsigned use = 0;
-#pragma unroll
-      for (int v = 0; v < N; ++v) {
-        const int m = pos_w ? row_m[v] : row_mc[v];
-        const bool u = m >= 0 && m < g.nmueller;
-        use |= u ? 1u << v : 0u;
-        p_sl[v] = unsigned(plane_start(g, geo.nf, cfcube, u ? m : 0, fxi, fyi));
-        if (u && !grad) {
-          p_gx[v] = e.g[v].x;
-          p_gy[v] = e.g[v].y;
-        }
+      const int m = pos_w ? row_m : row_mc;
+      const bool use = m >= 0 && m < g.nmueller;
+      p_sl = unsigned(plane_start(g, geo.nf, cfcube, use ? m : 0, fxi, fyi));
+      if (use && !grad) {
+        p_gx = e.g.x;
+        p_gy = e.g.y;
       }
       const unsigned base = unsigned((ly - qy * quad_edge) * QX + (lx - qx * quad_edge));
       p_key = unsigned(g.sx) | (unsigned(g.sy) << 6);
-      normal = !grad && use != 0u;
+      normal = !grad && use;
       if constexpr (PK) {
-        p_addr = (p_sl[0] << sub_pk_shift) | (normal ? base | (pos_w ? sub_pk_flip : 0u) : 0u);
+        p_addr = (p_sl << sub_pk_shift) | (normal ? base | (pos_w ? sub_pk_flip : 0u) : 0u);
       } else {
         if (normal) p_addr = base * unsigned(sizeof(float2)) | (pos_w ? 0x80000000u : 0u);
       }
-      grad = grad && use != 0u;
+      grad = grad && use;
     }
     const unsigned long long nmask = __ballot(normal);
     const unsigned long long gtodo = __ballot(valid && grad);
@@ -2118,7 +1984,7 @@ void k_sub(
     // (the fetches run on the whole wave: a lane's prepared values are read
     // from it while it is active); the slot's other values are read from
     // its lane when it is added
-    float2 ring[sub_ring][N];
+    float2 ring[sub_ring];
     unsigned ring_pk[sub_ring];               // PK: the slot's word
     unsigned long long ring_lanes[sub_ring];  // !UNI: lanes of the slot's support
     auto fetch = [&](int j) {
@@ -2136,15 +2002,12 @@ void k_sub(
         ring_pk[r] = pk;
         const v2i_t raw = __builtin_amdgcn_raw_buffer_load_b64(
           tap_rsrc, int(tap_off), int((pk >> sub_pk_shift) * unsigned(sizeof(float2))), 0);
-        ring[r][0] = make_float2(__int_as_float(raw.x), __int_as_float(raw.y));
+        ring[r] = make_float2(__int_as_float(raw.x), __int_as_float(raw.y));
       } else {
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          const int slv = __builtin_amdgcn_readlane(int(p_sl[v]), j);
-          const v2i_t raw = __builtin_amdgcn_raw_buffer_load_b64(
-            tap_rsrc, int(tap_off), slv * int(sizeof(float2)), 0);
-          ring[r][v] = make_float2(__int_as_float(raw.x), __int_as_float(raw.y));
-        }
+        const int slv = __builtin_amdgcn_readlane(int(p_sl), j);
+        const v2i_t raw = __builtin_amdgcn_raw_buffer_load_b64(
+          tap_rsrc, int(tap_off), slv * int(sizeof(float2)), 0);
+        ring[r] = make_float2(__int_as_float(raw.x), __int_as_float(raw.y));
       }
     };
     auto add = [&](int j) {
@@ -2162,38 +2025,22 @@ void k_sub(
       // UNI: the slot loops run on the support's lanes only
       bool on;
       if constexpr (UNI) on = true; else on = __builtin_amdgcn_inverse_ballot_w64(ring_lanes[r]);
-      float h_r = 0.0f, h_i = 0.0f;
-      double sr = 0.0, si = 0.0;
-#pragma unroll
-      for (int v = 0; v < N; ++v) {
-        const unsigned ux = unsigned(__builtin_amdgcn_readlane(__float_as_int(p_gx[v]), j));
-        const unsigned uy = unsigned(__builtin_amdgcn_readlane(__float_as_int(p_gy[v]), j));
-        const float gx = __uint_as_float(ux), gy = __uint_as_float(uy);
-        // conj(c) g for w > 0: c.y g.y and c.y g.x enter with the sign flipped
-        const float gcx = __uint_as_float(uy ^ flip), gcy = __uint_as_float(ux ^ flip);
-        // the FP32 complex product, each part as one product and one fused
-        // multiply-add
-        const float2 c = ring[r][v];
-        const float pr = __builtin_fmaf(c.x, gx, -(c.y * gcx));
-        const float pi = __builtin_fmaf(c.x, gy, c.y * gcy);
-        if constexpr (N == 1) {
-          h_r = pr;
-          h_i = pi;
-        } else {
-          sr += double(pr);
-          si += double(pi);
-        }
-      }
-      if constexpr (N > 1) {
-        h_r = float(sr);
-        h_i = float(si);
-      }
+      const unsigned ux = unsigned(__builtin_amdgcn_readlane(__float_as_int(p_gx), j));
+      const unsigned uy = unsigned(__builtin_amdgcn_readlane(__float_as_int(p_gy), j));
+      const float gx = __uint_as_float(ux), gy = __uint_as_float(uy);
+      // conj(c) g for w > 0: c.y g.y and c.y g.x enter with the sign flipped
+      const float gcx = __uint_as_float(uy ^ flip), gcy = __uint_as_float(ux ^ flip);
+      // the FP32 complex product, each part as one product and one fused
+      // multiply-add
+      const float2 c = ring[r];
+      const float pr = __builtin_fmaf(c.x, gx, -(c.y * gcx));
+      const float pi = __builtin_fmaf(c.x, gy, c.y * gcy);
       if (on) {
         float2* a =
           reinterpret_cast<float2*>(reinterpret_cast<char*>(sregions) + addr + lane_addr);
         float2 tv = *a;
-        tv.x += h_r;
-        tv.y += h_i;
+        tv.x += pr;
+        tv.y += pi;
         *a = tv;
       }
     };
@@ -2222,27 +2069,18 @@ void k_sub(
         // the entry again (a scalar load), so that the batch's raw entries
         // need not stay in registers through the loop above
         const unsigned ej = unsigned(__builtin_amdgcn_readlane(int(ei), j));
-        const Entry4<N> ge = entries[ej];
+        const Entry4 ge = entries[ej];
         const unsigned gpos = ge.h.pos;
         const bool gpos_w = gpos & e4_pos_w;
         const GroupInfo gg = one_group ? group0 : groups[ge.h.gpk & 0xffffu];
-        unsigned guse = 0;
-        unsigned sl[N];
-        float2 gv[N];
-#pragma unroll
-        for (int v = 0; v < N; ++v) {
-          const int m = gpos_w ? row_m[v] : row_mc[v];
-          guse |= (m >= 0 && m < gg.nmueller) ? 1u << v : 0u;
-          sl[v] = PK ? unsigned(__builtin_amdgcn_readlane(int(p_addr), j)) >> sub_pk_shift
-                     : unsigned(__builtin_amdgcn_readlane(int(p_sl[v]), j));
-          gv[v] = ge.g[v];
-        }
+        const unsigned sl =
+          PK ? unsigned(__builtin_amdgcn_readlane(int(p_addr), j)) >> sub_pk_shift
+             : unsigned(__builtin_amdgcn_readlane(int(p_sl), j));
         const unsigned gbase = ((gpos >> 6) & 63u) - unsigned(qy * quad_edge);
         const unsigned w0 = (gbase * unsigned(QX) + ((gpos & 63u) - unsigned(qx * quad_edge)))
-          | (unsigned(gg.sx) << 12) | (unsigned(gg.sy) << 18) | (guse << 24)
+          | (unsigned(gg.sx) << 12) | (unsigned(gg.sy) << 18)
           | (gpos_w ? quad_pos_w : 0u);
-        sub_gradient_entry<N>(w0, sl, gv, entry_vis[ej], ge.h.pos, geo, taps, recs,
-                              QX, region);
+        sub_gradient_entry(w0, sl, ge.g, entry_vis[ej], ge.h.pos, geo, taps, recs, QX, region);
       }
       if (last_half && ((rd + 1u) % unsigned(sub_fold_rounds) == 0u || rd + 1u == nrounds)) {
         __syncthreads();
@@ -3207,13 +3045,16 @@ constexpr int direct_loads = 4;
 constexpr float direct_lane_plain = 2.0f, direct_lane = 40.0f;
 constexpr int direct_lane_min = 5;
 constexpr int direct_lane_loads = 8;  // 4: 118 us for the 1500
+// of a call (hit_i, 16 bits each); below what launches cost up to 8000: 240 tiles,
+// supports of 7, binned and in one launch 2000 30.9, 15.6 us, 4000 37.0, 20.6, 8000
+// 36.4, 30.9
 constexpr unsigned direct_records = 2048;
 constexpr int direct_row = tile + 8;  // LDS row: four rows of a block on banks of their own
 constexpr int direct_plane = tile * direct_row;
 
 __global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4))) void k_direct(
-  Geometry geo, const float2* __restrict__ taps, Mueller mu, int mode,
-  const VisRec<1>* __restrict__ recs, unsigned n, DirectArgs da, void* __restrict__ grid) {
+  Geometry geo, const float2* __restrict__ taps, Mueller mu,
+  const VisRec<1>* __restrict__ recs, unsigned n, DirectArgs da, double2* __restrict__ grid) {
   extern __shared__ double sums[];  // per grid row: re, im
   __shared__ unsigned short hit_i[direct_records];
   __shared__ unsigned hits;
@@ -3446,16 +3287,8 @@ __global__ __launch_bounds__(direct_block) __attribute__((amdgpu_waves_per_eu(4)
     const double vr = src[0], vi = src[direct_plane];
     if (vr == 0.0 && vi == 0.0) continue;
     const size_t gi = ((size_t(cube) * geo.nr + gp) * geo.ny + y) * geo.nx + x;
-    if (mode == 0) {
-      double2* at = static_cast<double2*>(grid) + gi;
-      const double2 g0 = *at;
-      *at = make_double2(g0.x + vr, g0.y + vi);
-    } else {
-      // one rounding of grid value + FP64 tile sum
-      float2* at = static_cast<float2*>(grid) + gi;
-      const float2 g0 = *at;
-      *at = make_float2(float(double(g0.x) + vr), float(double(g0.y) + vi));
-    }
+    const double2 g0 = grid[gi];
+    grid[gi] = make_double2(g0.x + vr, g0.y + vi);
   }
 }
 
@@ -3581,13 +3414,14 @@ __device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
 // records a wave takes (eight of one element a row, or of two polarizations,
 // measured slower: their registers cost a wave per SIMD)
 constexpr int degrid_recs = 4;
-// rounds of loads between sums put aside, where a row uses one element: its taps
-// then fill 16 to 64 lanes, whose sums of up to thousands of taps round more than
-// 64 lanes' with shorter ones.  Predictions of four rows' error against 64 bits and
-// the call: supports of 33 to 65, 50,000 records, 7.3e-16 in one chain of two
-// roundings a tap (1170 us), 4.5e-16 with one rounding for two taps, 3.4e-16 with
-// parts too (1190 us; 3.8e-16 by 64 lanes a row); 9 to 33, 1e6, 3.7e-16 (3070 us) and
-// 2.9e-16 (3062)
+// Rounds of loads between sums put aside, where a row uses one element: its taps
+// then fill 16 to 64 lanes, and a sum of n taps rounds like sqrt(n / 2) of its last
+// steps.  Error against 64 bits and the call: four rows, supports of 33 to 65, 50,000
+// records, 7.3e-16 in one chain of two roundings a tap (1170 us), 4.5e-16 by pairs of
+// steps (k_degrid), 3.4e-16 with parts too (1190; 3.8e-16 by 64 lanes a row); 9 to 33,
+// 1e6 records, 3.7e-16 (3070 us) and 2.9e-16 (3062); two rows, 9 to 33, 100,000 records,
+// 3.3e-16 (237) and 2.9e-16 (243).  Parts of two rounds in place of the pairs for two
+// rows: 3.0e-16, and 666 us for 670 of a two-polarization residual call.
 constexpr unsigned degrid_part = 8;
 
 // One wave takes R records in a row of the order; those of one slice share
@@ -3876,7 +3710,7 @@ void k_degrid(
   }
 }
 
-// Binned degridding (supports below a tile): the entries of k_bin<N, true>
+// Binned degridding (supports below a tile): the entries of k_bin
 // in degrid mode (record index beside every entry) are processed one
 // workgroup per (plane, tile) key.  The workgroup loads the model's tile +
 // halo region of its plane into LDS with coalesced reads, then one lane per
@@ -3894,14 +3728,13 @@ __device__ __noinline__ double2 degrid_screen(double2 m, double ph) {
 // cphase out of line, for the same reason
 __device__ __noinline__ double2 cphase_call(double ph) { return cphase(ph); }
 
-template <int N>
-__global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N == 1 ? 4 : 1))) void k_degrid4(
+__global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(4))) void k_degrid4(
   Geometry geo, const GroupInfo* __restrict__ groups,
   const float2* __restrict__ taps, Mueller mu, const unsigned* __restrict__ off_table,
-  int nbins, size_t block_cap, const Entry4<N>* __restrict__ entries,
-  const unsigned* __restrict__ entry_vis, const VisRec<N>* recs,
+  int nbins, size_t block_cap, const Entry4* __restrict__ entries,
+  const unsigned* __restrict__ entry_vis, const VisRec<1>* recs,
   int hx, int hy, const double2* __restrict__ model, double2* __restrict__ acc,
-  int one_plane, const double2* __restrict__ wsum, int do_grid, VisRec<N>* out_recs,
+  int one_plane, const double2* __restrict__ wsum, int do_grid, VisRec<1>* out_recs,
   float2* __restrict__ gvis, double2* __restrict__ pred64) {
   // one_plane: each record has exactly one entry, so the lane finishes the
   // prediction itself (the end of degrid_vis and the degridding branch of
@@ -3990,13 +3823,9 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
     // of gridding (src/hpg_core.hpp:598-600)
     const int* row = pos_w ? mu.Mc[gpol] : mu.M[gpol];
     const float imf = pos_w ? 1.0f : -1.0f;
-    const float2* slice[N];
-    bool use[N];
-    for (int v = 0; v < N; ++v) {
-      const int m = row[v];
-      use[v] = m >= 0 && m < g.nmueller;
-      slice[v] = taps + plane_start(g, geo.nf, int(cfcube), use[v] ? m : 0, fxi, fyi);
-    }
+    const int m = row[0];
+    const bool use = m >= 0 && m < g.nmueller;
+    const float2* slice = taps + plane_start(g, geo.nf, int(cfcube), use ? m : 0, fxi, fyi);
     double phi0x = 0.0, phi0y = 0.0, dphix = 0.0, dphiy = 0.0;
     if (grad) {
       const double gxr = recs[i].grad[0];
@@ -4006,23 +3835,19 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
       dphix = gxr * geo.os;
       dphiy = gyr * geo.os;
     }
-    double2 a[N];
-    for (int v = 0; v < N; ++v) a[v] = make_double2(0.0, 0.0);
-    // c' x model for one tap, added to a[]
-    auto add_tap = [&](const float2* cv, double2 m, int X, int Y) {
+    double2 a = make_double2(0.0, 0.0);
+    // c' x model for one tap, added to a
+    auto add_tap = [&](float2 cc, double2 m, int X, int Y) {
       if (grad) {
         const double phX = phi0x + X * dphix;
         const double phY = phi0y + Y * dphiy;
         m = degrid_screen(m, -phX - phY);
       }
-#pragma unroll
-      for (int v = 0; v < N; ++v) {
-        if (!use[v]) continue;
-        float2 cc = cv[v];
+      if (use) {
         cc.y *= imf;
         const double2 p = cmul(cc, m);
-        a[v].x += p.x;
-        a[v].y += p.y;
+        a.x += p.x;
+        a.y += p.y;
       }
     };
     // any support: taps in slice order (t = Y * sx + X), halo_chunk at a
@@ -4037,7 +3862,7 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
         bool ok[halo_chunk];
         int Xk[halo_chunk], Yk[halo_chunk];
         double2 mv[halo_chunk];
-        float2 c[halo_chunk][N];
+        float2 c[halo_chunk];
 #pragma unroll
         for (int k = 0; k < halo_chunk; ++k) {
           ok[k] = FULL || t0 + k < ntap;
@@ -4048,12 +3873,9 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
           cx = eol ? 0 : cx;
           cy += eol ? 1 : 0;
           lc += eol ? 1 + wrap : 1;
-#pragma unroll
-          for (int v = 0; v < N; ++v) {
-            float2 tv = make_float2(0.0f, 0.0f);
-            if (ok[k]) tv = slice[v][t0 + k];
-            c[k][v] = tv;
-          }
+          float2 tv = make_float2(0.0f, 0.0f);
+          if (ok[k]) tv = slice[t0 + k];
+          c[k] = tv;
         }
 #pragma unroll
         for (int k = 0; k < halo_chunk; ++k)
@@ -4065,38 +3887,30 @@ __global__ __launch_bounds__(halo_block) __attribute__((amdgpu_waves_per_eu(N ==
     };
     run_chunks();
     if (!one_plane) {
-      for (int v = 0; v < N; ++v) {
-        double2* dst = acc + size_t(i) * N + v;
-        atomicAdd(&dst->x, a[v].x);
-        atomicAdd(&dst->y, a[v].y);
-      }
+      atomicAdd(&acc[i].x, a.x);
+      atomicAdd(&acc[i].y, a.y);
       continue;
     }
-    double2 W[N];
-    degrid_norms<N>(geo, g, wsum, mu, pos_w, unsigned(cfcube), fxi, fyi, W);
+    double2 W;
+    degrid_norms<1>(geo, g, wsum, mu, pos_w, unsigned(cfcube), fxi, fyi, &W);
     const double2 phasor = cphase_call(recs[i].phase);
     const double2 conj_phasor = make_double2(phasor.x, -phasor.y);
-    double2 pred_d[N];
-    for (int v = 0; v < N; ++v) {
-      const double2 d = (W[v].x != 0.0 || W[v].y != 0.0) ? W[v] : make_double2(1.0, 0.0);
-      pred_d[v] = cmul(kdiv(a[v], d), conj_phasor);
-    }
+    const double2 d = (W.x != 0.0 || W.y != 0.0) ? W : make_double2(1.0, 0.0);
+    const double2 pred_d = cmul(kdiv(a, d), conj_phasor);
     if (pred64) {
-      for (int v = 0; v < N; ++v) pred64[size_t(i) * N + v] = pred_d[v];
+      pred64[i] = pred_d;
       continue;
     }
-    for (int v = 0; v < N; ++v) {
-      const float2 pred = narrow(pred_d[v]);
-      if (do_grid) {
-        float2 val = recs[i].vis[v];
-        val.x -= pred.x;
-        val.y -= pred.y;
-        const float wv = recs[i].w[v];
-        if (out_recs) out_recs[i].vis[v] = val;
-        gvis[size_t(i) * N + v] = prephase(val, phasor, wv);
-      } else if (out_recs) {
-        out_recs[i].vis[v] = pred;
-      }
+    const float2 pred = narrow(pred_d);
+    if (do_grid) {
+      float2 val = recs[i].vis[0];
+      val.x -= pred.x;
+      val.y -= pred.y;
+      const float wv = recs[i].w[0];
+      if (out_recs) out_recs[i].vis[0] = val;
+      gvis[i] = prephase(val, phasor, wv);
+    } else if (out_recs) {
+      out_recs[i].vis[0] = pred;
     }
   }
 }
@@ -4346,7 +4160,7 @@ hipError_t launch_count(
   if (n == 0) return hipSuccess;
   if (npol != 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(
-    k_count<1>, dim3(std::min(unsigned(blocks_for(n)), count_blocks_max)),
+    k_count, dim3(std::min(unsigned(blocks_for(n)), count_blocks_max)),
     dim3(block), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
     int(update_weights), int(do_grid), cb.hist, weights, cb.invalid_count);
@@ -4417,11 +4231,11 @@ hipError_t launch_tally(
   unsigned* table = offsets + patch_local_keys + 1;
   uint2* pairs = static_cast<uint2*>(cb.tally_keys);
   unsigned* keys = reinterpret_cast<unsigned*>(pairs + cb.tally_capacity);
-  Entry4<1>* tally = static_cast<Entry4<1>*>(cb.tally_entries);
+  Entry4* tally = static_cast<Entry4*>(cb.tally_entries);
   hipLaunchKernelGGL(k_zero, dim3(blocks_for(size_t(sk.bins))), dim3(block), 0, s, hist,
                      size_t(sk.bins));
   hipLaunchKernelGGL(
-    k_tally<1>, dim3(unsigned((n + batch - 1) / batch)), dim3(patch_local_threads), 0, s,
+    k_tally, dim3(unsigned((n + batch - 1) / batch)), dim3(patch_local_threads), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
     int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint), cb.gvis, residuals,
     sk, unsigned(batch), hist, table, weights, cb.invalid_count, tally, keys);
@@ -4431,9 +4245,9 @@ hipError_t launch_tally(
                         pairs);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(
-    k_tally_sort<1>, dim3(unsigned(sk.bins)), dim3(sort_threads),
+    k_tally_sort, dim3(unsigned(sk.bins)), dim3(sort_threads),
     (size_t(1) << sk.low_bits) * sizeof(unsigned), s, sk.low_bits, nkeys, geo.nr, offsets, pairs,
-    tally, cb.offsets, static_cast<Entry4<1>*>(cb.stream_entries), cb.entry_vis);
+    tally, cb.offsets, static_cast<Entry4*>(cb.stream_entries), cb.entry_vis);
   return hipGetLastError();
 }
 
@@ -4445,10 +4259,10 @@ hipError_t launch_emit(
   const int adj = src == GvisSource::Adjoint;
   if (npol != 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(
-    k_emit<1>, dim3(blocks_for(n)), dim3(block), 0, s,
+    k_emit, dim3(blocks_for(n)), dim3(block), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
-    int(gvis_ready), adj, cb.gvis, residuals, cb.cursor, cb.stream_entries,
-    cb.entry_vis);
+    int(gvis_ready), adj, cb.gvis, residuals, cb.cursor,
+    static_cast<Entry4*>(cb.stream_entries), cb.entry_vis);
   return hipGetLastError();
 }
 
@@ -4471,7 +4285,7 @@ hipError_t launch_bin(
   const unsigned nb = unsigned(bin_blocks_for(n));
   if (npol != 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(
-    k_bin<1>, dim3(nb), dim3(bin_threads), 0, s,
+    k_bin, dim3(nb), dim3(bin_threads), 0, s,
     static_cast<const VisRec<1>*>(cb.vis), n, geo, cf.groups, cf.wsum, mu,
     int(update_weights), int(gvis_ready), adj, dg, cb.gvis, residuals,
     cb.off_table, cb.stream_entries, cb.entry_vis, block_cap, weights,
@@ -4479,9 +4293,7 @@ hipError_t launch_bin(
   return hipGetLastError();
 }
 
-size_t halo_entry_bytes(int npol) {
-  return sizeof(Entry4Head) + sizeof(float2) * size_t(npol);
-}
+size_t halo_entry_bytes() { return sizeof(Entry4); }
 size_t halo_pixels_per_key(int hx, int hy) { return size_t(halo_pixels(hx, hy)); }
 int halo_tile_limit() { return tile; }
 size_t halo_lds_bytes(int hx, int hy, int nbins) {
@@ -4509,11 +4321,6 @@ hipError_t launch_halo(
   return hipGetLastError();
 }
 
-size_t sub_lds_bytes(int hx, int hy) {
-  const int px = ((quad_edge + hx) * (quad_edge + hy) + wave - 1) / wave;
-  const int pxc = px <= 4 ? 4 : px <= 6 ? 6 : px <= 8 ? 8 : 9;
-  return size_t(sub_waves) * pxc * wave * sizeof(float2);
-}
 int sub_bins_limit() { return sub_bins_max; }
 bool sub_supported(int hx, int hy) { return hx >= 0 && hy >= 0 && hx < 8 && hy < 8; }
 
@@ -4524,44 +4331,42 @@ hipError_t launch_tile_sub(
   if (ntile_keys == 0 || n == 0) return hipSuccess;
   const int nb = global_bins ? 1 : bin_blocks_for(n);
   // segment starts are 16-bit offsets within a bin block; CF taps are
-  // addressed by 32-bit byte offsets; global bins for one polarization
-  if (!sub_supported(hx, hy) || taps_bytes > 0xffffffffull) return hipErrorInvalidValue;
-  if (global_bins ? npol != 1 : (nb > sub_bins_max || block_cap > 65536))
+  // addressed by 32-bit byte offsets
+  if (npol != 1 || !cf.planar || !sub_supported(hx, hy) || taps_bytes > 0xffffffffull)
     return hipErrorInvalidValue;
+  if (!global_bins && (nb > sub_bins_max || block_cap > 65536)) return hipErrorInvalidValue;
   const unsigned* offs = global_bins ? cb.offsets : cb.off_table;
   const int Q = (quad_edge + hx) * (quad_edge + hy);
   const int px = (Q + wave - 1) / wave;  // 4 .. 9
   const int pxc = px <= 4 ? 4 : px <= 6 ? 6 : px <= 8 ? 8 : 9;
   const size_t dyn = size_t(sub_waves) * pxc * wave * sizeof(float2);
-#define HPGX_SUB_G(NP, PX, PK, GB)                                             \
+#define HPGX_SUB_G(PX, PK, GB)                                                 \
   hipLaunchKernelGGL(                                                          \
-    uni ? (k_sub<NP, PX, true, PK, GB>) : (k_sub<NP, PX, false, PK, GB>),      \
+    uni ? (k_sub<PX, true, PK, GB>) : (k_sub<PX, false, PK, GB>),              \
     dim3(unsigned(ntile_keys)), dim3(sub_block), dyn, s,                       \
     geo, cf.groups, cf.taps, unsigned(taps_bytes), mu, offs, nb,               \
     block_cap,                                                                 \
-    static_cast<const Entry4<NP>*>(cb.stream_entries), cb.entry_vis,           \
-    static_cast<const VisRec<NP>*>(cb.vis), hx, hy, static_cast<float2*>(grid),\
+    static_cast<const Entry4*>(cb.stream_entries), cb.entry_vis,               \
+    static_cast<const VisRec<1>*>(cb.vis), hx, hy, static_cast<float2*>(grid), \
     cb.halo, cb.halo_set)
-#define HPGX_SUB_1(NP, PX, PK)                                                 \
+#define HPGX_SUB(PX, PK)                                                       \
   do {                                                                         \
-    if (global_bins) HPGX_SUB_G(1, PX, PK, true);                              \
-    else HPGX_SUB_G(1, PX, PK, false);                                         \
+    if (global_bins) HPGX_SUB_G(PX, PK, true);                                 \
+    else HPGX_SUB_G(PX, PK, false);                                            \
   } while (0)
-#define HPGX_SUB_PX(HPGX_SUB, NP, PK)                                          \
+#define HPGX_SUB_PX(PK)                                                        \
   switch (pxc) {                                                               \
-  case 4: HPGX_SUB(NP, 4, PK); break;                                          \
-  case 6: HPGX_SUB(NP, 6, PK); break;                                          \
-  case 8: HPGX_SUB(NP, 8, PK); break;                                          \
-  default: HPGX_SUB(NP, 9, PK); break;                                         \
+  case 4: HPGX_SUB(4, PK); break;                                              \
+  case 6: HPGX_SUB(6, PK); break;                                              \
+  case 8: HPGX_SUB(8, PK); break;                                              \
+  default: HPGX_SUB(9, PK); break;                                             \
   }
   // one word per slot: region pixels below sub_pk_flip, slices addressed
   // by tap index below sub_pk_taps
   static_assert(9 * wave < int(sub_pk_flip), "region pixel in the packed word");
-  const bool pk = npol == 1 && taps_bytes / sizeof(float2) < sub_pk_taps;
-  if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
-  if (pk) HPGX_SUB_PX(HPGX_SUB_1, 1, true) else HPGX_SUB_PX(HPGX_SUB_1, 1, false)
+  if (taps_bytes / sizeof(float2) < sub_pk_taps) HPGX_SUB_PX(true) else HPGX_SUB_PX(false)
 #undef HPGX_SUB_PX
-#undef HPGX_SUB_1
+#undef HPGX_SUB
 #undef HPGX_SUB_G
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -4582,9 +4387,9 @@ hipError_t launch_tile_halo(
   if (lds > 65536) return hipErrorInvalidValue;
 #define HPGX_TILE4(MD, AC)                                                     \
   hipLaunchKernelGGL(                                                          \
-    (k_tile4<1, MD, AC>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s,                           \
+    (k_tile4<MD, AC>), dim3(unsigned(nkeys)), dim3(halo_block), lds, s,                           \
     geo, cf.groups, cf.taps, mu, table, nb, block_cap,                         \
-    static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,            \
+    static_cast<const Entry4*>(cb.stream_entries), cb.entry_vis,            \
     static_cast<const VisRec<1>*>(cb.vis), hx, hy, grid, cb.halo, cb.halo_set)
   if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
   if (mode == 0)
@@ -4783,10 +4588,11 @@ hipError_t launch_patch(
   return hipSuccess;
 }
 
-// every tile looks through all records: their product, at 2^21 still the faster
-// (2000 records, 1024 tiles: 40.5 -> 32.5 us) and at 2^22 even (1000 records,
-// 4096 tiles: 52.3, 51.0); and not where few tiles hold them all (2000 records,
-// 4 tiles, FP32: 33.5 -> 39.6 us; 1000: 24.1 -> 21.9)
+// Every tile looks through all records: their product, at 2^21 still the faster
+// (supports of 7, binned and in one launch: 2000 records on 1024 tiles 38.8, 35.1 us;
+// 3000 42.9, 44.7).  And not where few tiles hold them all, which is even for wide
+// supports (1500 of 25 on 16 tiles 106, 107 us; narrow ones would still gain: 2000 of 7
+// on 4 tiles 39.7, 25.5).
 bool direct_ok(size_t n, const Geometry& geo) {
   const size_t tiles = size_t(geo.ntx) * geo.nty * geo.nc;
   return n <= direct_records && n * tiles <= (size_t(1) << 21) && n <= 256 * tiles;
@@ -4795,7 +4601,7 @@ bool direct_ok(size_t n, const Geometry& geo) {
 hipError_t launch_direct(
   hipStream_t s, int npol, size_t n, const Geometry& geo, const DeviceCF& cf, const Mueller& mu,
   bool update_weights, bool gvis_ready, GvisSource src, const double2* residuals,
-  const CallBuffers& cb, double* weights, int mode, void* grid) {
+  const CallBuffers& cb, double* weights, double2* grid) {
   if (n == 0) return hipSuccess;
   if (npol != 1 || !cf.planar || n > direct_records || geo.nr > 4) return hipErrorInvalidValue;
   const size_t lds = size_t(geo.nr) * 2 * direct_plane * sizeof(double);
@@ -4803,7 +4609,7 @@ hipError_t launch_direct(
                         int(update_weights), int(gvis_ready), int(src == GvisSource::Adjoint)};
   hipLaunchKernelGGL(
     k_direct, dim3(unsigned(size_t(geo.ntx) * geo.nty * geo.nc)), dim3(direct_block), lds, s, geo,
-    cf.taps, mu, mode, static_cast<const VisRec<1>*>(cb.vis), unsigned(n), args, grid);
+    cf.taps, mu, static_cast<const VisRec<1>*>(cb.vis), unsigned(n), args, grid);
   return hipGetLastError();
 }
 
@@ -4819,8 +4625,8 @@ hipError_t launch_degrid_tiles(
   if (lds > 65536) return hipErrorInvalidValue;
   if (npol != 1 || !cf.planar) return hipErrorInvalidValue;
   hipLaunchKernelGGL(
-    k_degrid4<1>, dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo, cf.groups, cf.taps, mu,
-    cb.off_table, nb, block_cap, static_cast<const Entry4<1>*>(cb.stream_entries), cb.entry_vis,
+    k_degrid4, dim3(unsigned(nkeys)), dim3(halo_block), lds, s, geo, cf.groups, cf.taps, mu,
+    cb.off_table, nb, block_cap, static_cast<const Entry4*>(cb.stream_entries), cb.entry_vis,
     static_cast<const VisRec<1>*>(cb.vis), hx, hy, model, acc, int(one_plane), cf.wsum,
     int(do_grid), static_cast<VisRec<1>*>(out_recs), cb.gvis, pred64);
   return hipGetLastError();
