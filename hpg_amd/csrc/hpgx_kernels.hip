@@ -3414,15 +3414,17 @@ __device__ __forceinline__ int reduce_lanes(double* val, int lane, int& at) {
 // records a wave takes (eight of one element a row, or of two polarizations,
 // measured slower: their registers cost a wave per SIMD)
 constexpr int degrid_recs = 4;
-// Rounds of loads between sums put aside, where a row uses one element: its taps
-// then fill 16 to 64 lanes, and a sum of n taps rounds like sqrt(n / 2) of its last
-// steps.  Error against 64 bits and the call: four rows, supports of 33 to 65, 50,000
-// records, 7.3e-16 in one chain of two roundings a tap (1170 us), 4.5e-16 by pairs of
-// steps (k_degrid), 3.4e-16 with parts too (1190; 3.8e-16 by 64 lanes a row); 9 to 33,
-// 1e6 records, 3.7e-16 (3070 us) and 2.9e-16 (3062); two rows, 9 to 33, 100,000 records,
-// 3.3e-16 (237) and 2.9e-16 (243).  Parts of two rounds in place of the pairs for two
-// rows: 3.0e-16, and 666 us for 670 of a two-polarization residual call.
+// Rounds of loads between sums put aside, where a row uses one element and the
+// supports are long: its taps then fill 16 to 64 lanes, and a sum of n taps rounds
+// like sqrt(n / 2) of its last steps.  Error against 64 bits and the call: four rows,
+// supports of 33 to 65, 50,000 records, 7.3e-16 in one chain of two roundings a tap
+// (1170 us), 4.5e-16 by pairs of steps (k_degrid), 3.4e-16 with parts too (1190; 3.8e-16
+// by 64 lanes a row); 9 to 33, 1e6 records, 3.7e-16 (3070 us) and 2.9e-16 (3062); two
+// rows, 9 to 33, 100,000 records, 3.3e-16 (237) and 2.9e-16 (243).
 constexpr unsigned degrid_part = 8;
+// and the steps of a chain that stays whole: two rows, supports of 7 to 17 (9 steps),
+// 2.7e-16 either way, the kernel 222 us whole and 233 in pairs
+constexpr int degrid_whole = 16;
 
 // One wave takes R records in a row of the order; those of one slice share
 // every CF value it loads (per tap of 4 x 4 elements a record reads 64 bytes
@@ -3445,7 +3447,7 @@ constexpr unsigned degrid_part = 8;
 // record a lane.  Two steps' loads at once where a row uses one element (3.3 ms
 // one by one).  Three waves per SIMD for several: at four the sums spill
 // (15.9 ms the first).
-template <int N, int P, int KIND>
+template <int N, int P, int KIND, bool LONG>
 __global__ __launch_bounds__(block) __attribute__((amdgpu_waves_per_eu(KIND == patch_one ? 4 : 3)))
 void k_degrid(
   size_t n, Geometry geo, const float2* __restrict__ taps, Mueller mu, int same_rows,
@@ -3456,7 +3458,8 @@ void k_degrid(
   constexpr int R = degrid_recs;
   constexpr int L = KIND == patch_one ? 1 : N;  // elements of a row
   constexpr int TPS = wave / P;                 // taps a step
-  __shared__ double part[KIND == patch_one ? R * L * 2 * block : 1];
+  constexpr bool parts = KIND == patch_one && LONG;
+  __shared__ double part[parts ? R * L * 2 * block : 1];
 
   const int w = uniform(int(threadIdx.x) / wave);
   const int lane = threadIdx.x % wave;
@@ -3610,27 +3613,29 @@ void k_degrid(
           off += wrap;
         }
       }
-      // the steps' products added up, then to the sums: one rounding of a sum for
-      // U taps in place of two for each
+      // LONG: the steps' products added up, then to the sums: one rounding of a sum
+      // for U taps in place of two for each
 #pragma unroll
       for (int k = 0; k < RR; ++k) {
 #pragma unroll
         for (int v = 0; v < L; ++v) {
           if (KIND == patch_any && !use[v]) continue;
-          double tr = 0.0, ti = 0.0;
+          double& a = val[(k * L + v) * 2];
+          double& b = val[(k * L + v) * 2 + 1];
+          double tr = LONG ? 0.0 : a, ti = LONG ? 0.0 : b;
 #pragma unroll
           for (int u = 0; u < U; ++u) {
             const double mx = m[u][k].x;
             const double my = __hiloint2double(
               int(unsigned(__double2hiint(m[u][k].y)) ^ flip[k]), __double2loint(m[u][k].y));
             const double cx = double(c[u][v].x), cy = double(c[u][v].y);
-            tr = u ? __builtin_fma(cx, mx, tr) : cx * mx;
+            tr = u || !LONG ? __builtin_fma(cx, mx, tr) : cx * mx;
             tr = __builtin_fma(-cy, my, tr);
-            ti = u ? __builtin_fma(cx, my, ti) : cx * my;
+            ti = u || !LONG ? __builtin_fma(cx, my, ti) : cx * my;
             ti = __builtin_fma(cy, mx, ti);
           }
-          val[(k * L + v) * 2] += tr;
-          val[(k * L + v) * 2 + 1] += ti;
+          a = LONG ? a + tr : tr;
+          b = LONG ? b + ti : ti;
         }
       }
     };
@@ -3641,7 +3646,7 @@ void k_degrid(
 #pragma unroll 1
     for (; s + U <= full; s += U) {
       steps(std::integral_constant<int, U>{});
-      if (KIND == patch_one && (s / U) % degrid_part == degrid_part - 1) {
+      if (parts && (s / U) % degrid_part == degrid_part - 1) {
 #pragma unroll
         for (int k = 0; k < RR * L * 2; ++k) {
           double* p = part + k * block + threadIdx.x;
@@ -4766,12 +4771,15 @@ hipError_t launch_degrid(
     if (e != hipSuccess) return e;
     order = sorted_idx;
   }
+  const bool longer = (long long)cf.max_sx * cf.max_sy > (long long)degrid_whole * (wave / P);
 #define HPGX_DEGRID_P(NP, PP, KD)                                              \
   do {                                                                         \
     constexpr size_t per = size_t(block / wave) * degrid_recs;                 \
     e = in_launches((n + per - 1) / per, block, [&](unsigned long long first, unsigned blocks) { \
       hipLaunchKernelGGL(                                                      \
-        (k_degrid<NP, PP, KD>), dim3(blocks), dim3(block), 0, s, n, geo,       \
+        longer || KD != patch_one ? (k_degrid<NP, PP, KD, true>)               \
+                                  : (k_degrid<NP, PP, KD, KD != patch_one>),   \
+        dim3(blocks), dim3(block), 0, s, n, geo,                               \
         cf.taps, mu, int(same_rows), model, int(region_sh < 31), drs,          \
         static_cast<const VisRec<NP>*>(records), order, offsets + sk.bins,     \
         reinterpret_cast<double*>(cb.degrid_acc), unsigned(first));            \
