@@ -2268,9 +2268,9 @@ __device__ __forceinline__ bool patch_record(
 // 7-17: 280 -> 244 us).  One workgroup, 11 us for 4096 tiles and 19 us for 8836,
 // in place of hipCUB's scan (10 us).  order null: the scan alone.
 //
-// A list of two chunks or more is split: one workgroup for each chunk of it, in
-// slots next to each other (the last of a tile's to end adds up their sums in the
-// slots' order), or a dense uv core would be one workgroup's serial chain.  The
+// A list of two chunks or more (patch_full_chip) is split: one workgroup for each
+// chunk of it, in slots next to each other (the last of a tile's to end adds up their
+// sums in the slots' order), or a dense uv core would be one workgroup's serial chain.  The
 // chunk is the least, from patch_chunk_min on, that leaves the launch enough slots:
 // a list of two chunks or more has 1.5 slots a chunk of its entries at most.
 // Two polarizations, FP64: 100,000 records of supports 5 within a few pixels 28.5 ->
@@ -2279,6 +2279,12 @@ __device__ __forceinline__ bool patch_record(
 // slower there.  With a fence of the device's scope instead of stores past the L2s
 // 116 us: it writes a whole L2 back for every chunk.
 constexpr unsigned patch_chunk_min = 32;
+// Even lists of tiles that fill the chip by themselves, two workgroups a CU and more,
+// would only pay for the chunks' sums: where a quarter of the tiles are over the mean,
+// lists of 1.5 times the mean and more are split (30,000 records: 384^2, four
+// polarizations, FP32, 576 tiles 173 us split, 149 not; 512^2, two, 512 tiles 99, 88;
+// 100,000 of a Gaussian core there stay split, 135 us for 197).
+constexpr unsigned patch_full_chip = 512;
 constexpr unsigned patch_none = ~0u;  // in the tiles' order: a split one
 constexpr int patch_values = 8 * patch_block;
 // device scope: past the XCDs' own L2s
@@ -2333,7 +2339,6 @@ __global__ __launch_bounds__(block) void k_patch_split(
 constexpr int patch_scan_threads = 1024;
 constexpr int patch_scan_keys = patch_local_keys;
 constexpr int patch_classes = 6;
-constexpr unsigned patch_split_bit = 8u;
 // a: the counts in LDS, keys + 1 values, afterwards the offsets
 __device__ __forceinline__ void patch_scan(
   int keys, unsigned* a, unsigned* __restrict__ offsets, unsigned* __restrict__ order,
@@ -2353,15 +2358,14 @@ __device__ __forceinline__ void patch_scan(
   }
   const int lane = threadIdx.x % wave;
   const int rounds = (keys + patch_scan_threads - 1) / patch_scan_threads;
-  const unsigned chunk = ps.slots ? patch_chunk(total, ps.slots) : 0x7fffffffu;
-  // class 0: over four times the mean, ..., the last: empty; with patch_split_bit
-  // that of a split list
+  const unsigned chunk = ps.slots ? patch_chunk(total, ps.slots) : 0u;
+  __shared__ unsigned least;  // the shortest list that is split
+  // class 0: over four times the mean, 2: over the mean, ..., the last: empty
   auto class_of = [&](int k) {
     const unsigned cnt = a[k + 1] - a[k];
     const unsigned long long c = (unsigned long long)cnt * unsigned(keys);
-    const unsigned q = c > 4ull * total ? 0 : c > 2ull * total ? 1 : c > total ? 2
-      : 4ull * c > total ? 3 : c ? 4 : 5;
-    return q | (cnt >= 2u * chunk ? patch_split_bit : 0u);
+    return c > 4ull * total ? 0u : c > 2ull * total ? 1u : c > total ? 2u
+      : 4ull * c > total ? 3u : c ? 4u : 5u;
   };
   static_assert(patch_scan_keys <= 16 * patch_scan_threads, "four bits a round in classes");
   unsigned long long classes = 0;  // of this thread's tiles, from the first pass
@@ -2380,7 +2384,7 @@ __device__ __forceinline__ void patch_scan(
       }
 #pragma unroll
       for (int c = 0; c < patch_classes; ++c) {
-        const bool mine = (q & ~patch_split_bit) == unsigned(c);
+        const bool mine = q == unsigned(c);
         const unsigned long long m = __ballot(mine);
         if (!m) continue;
         const int lead = __builtin_ctzll(m);
@@ -2390,11 +2394,12 @@ __device__ __forceinline__ void patch_scan(
                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         at = unsigned(__builtin_amdgcn_readlane(int(at), lead));
         if (pass == 1 && mine) {
-          const bool split = q & patch_split_bit;
+          const unsigned cnt = a[k + 1] - a[k];
+          const bool split = cnt >= least;
           order[at + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)))] =
             split ? patch_none : unsigned(k);
           if (split)
-            patch_take(ps, chunk, unsigned(k), a[k + 1] - a[k], &taken,
+            patch_take(ps, chunk, unsigned(k), cnt, &taken,
                        __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
@@ -2407,6 +2412,9 @@ __device__ __forceinline__ void patch_scan(
         cls[c] = run;
         run += t;
       }
+      const bool even = unsigned(keys) >= patch_full_chip && 4u * cls[3] >= unsigned(keys);
+      least = !ps.slots ? ~0u
+        : max(2u * chunk, even ? unsigned(3ull * total / (2ull * unsigned(keys))) + 1u : 0u);
     }
     __syncthreads();
   }

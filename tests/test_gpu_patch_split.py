@@ -44,3 +44,14 @@ def test_split_lists_vs_oracle(hpg, oracle_mod, gsz, radius, n, sigma, npol, M, 
     bar = 1e-6 if mode else 1e-12
     assert np.abs(gs.grid_values() - exp).max() <= bar * np.abs(exp).max()
     np.testing.assert_allclose(gs.grid_weights(), o.grid_weights(), rtol=1e-12)
+
+
+@pytest.mark.parametrize("npol,M,nm,gsz", [
+    (2, [[0, -1], [-1, 1]], 2, (512, 512)),  # 512 tiles of 32 x 16
+    (2, [[0, -1], [-1, 1]], 2, (512, 496)),  # one row of tiles fewer
+    (4, FULL, 16, (384, 370)),               # 576 of 16 x 16
+])
+@pytest.mark.parametrize("sigma", [None, 30.0])
+def test_many_tiles_vs_oracle(hpg, oracle_mod, npol, M, nm, gsz, sigma):
+    """Even lists, which stay whole where the tiles fill the chip, and a core's."""
+    test_split_lists_vs_oracle(hpg, oracle_mod, gsz, 3, 50_000, sigma, npol, M, nm, 0)
